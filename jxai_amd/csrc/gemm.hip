@@ -73,15 +73,16 @@ struct Stage {
 // Block-unit form: the unit ratios of each stage's blocks, [stage][block][row]
 // (an empty base otherwise: every byte of LDS counts where two workgroups
 // share a CU).
-template <int BN, bool RX>
+template <int GW, int BN, bool RX>
 struct RxStage {
     float rx[2][HB * BN];
+    float rd[GW * 64];  // [wave][gate, up][32 rows] the super-block's weight-unit ratios
 };
-template <int BN>
-struct RxStage<BN, false> {};
+template <int GW, int BN>
+struct RxStage<GW, BN, false> {};
 
-template <int HL, int BN, bool RX>
-struct GemmSmem : RxStage<BN, RX> {
+template <int GW, int HL, int BN, bool RX>
+struct GemmSmem : RxStage<GW, BN, RX> {
     Stage<HL, BN> st[2];
     int src[BN];  // activation row (token or pair) of each staged pair
 };
@@ -203,9 +204,7 @@ struct WRaw<T_Q4_K> {
     __device__ static uint32_t soff(const QMat& W, int rt, int n) {
         return (uint32_t)(((size_t)rt * W.nkb * 32 + n) * 16);
     }
-    __device__ static uint32_t moff(const QMat& W, int rt, int n) {
-        return (uint32_t)(((size_t)rt * W.nkb * (MN_SB / 16) + n) * 16);
-    }
+    __device__ static uint32_t moff(const QMat&, int, int n) { return (uint32_t)(n * 16); }
     // PAR: the parity of h (even half-units carry the header, odd ones the min pieces), so each of the
     // two alternating register sets holds only the fields its parity uses
     __device__ static uint32_t xoff(const QMat&, int, int, int) { return 0; }
@@ -332,6 +331,16 @@ struct Arr {
 // The MFMAs take the activations as operand A and the weights as operand B,
 // so in each 32x32 result lane (n, g) holds weight row n (its scales are the
 // lane's own) and registers r span pairs 8*(r/4) + 4g + r%4.
+// Block-unit gate/up (Q4_K / Q5_K) has them the other way round: lane (n, g)
+// holds pair n and registers r span weight rows.  The factor that changes
+// every 32 of K there is the pair's (its block unit), the row's changes every
+// 256, so each accumulator element's per-block factor is one value of the
+// lane, a 4-byte LDS read per pair tile and block, instead of 16 values in 16
+// registers from four 16-byte reads: LDS reads per 32-block 12 -> 6 (2 of
+// them 4 bytes), 256 VGPRs with spills -> 219 without.  h's 32-row Q8_0 blocks
+// then end in the registers of lanes n and n + 32 and need no LDS transpose.
+// Mixtral-shaped 2048 tokens gate/up 1737 -> 1638 us, 512 tokens 583 -> 545 us,
+// DeepSeek-V2-Lite-shaped 1555 tokens 398 -> 372 us (HIP events, one box).
 template <int TYPE, bool GATEUP, int GW, int TM, int TN, int WPE, int BN>
 __global__ void __launch_bounds__(GW * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8 hq, float* hf, int hf_ld,
@@ -358,7 +367,7 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
     constexpr int PB = St::PB, CPP = St::CPP, PPI = 64 / CPP;  // row bytes, chunks, rows per DMA
     constexpr int PER = BN / PPI / GW;  // 1 KB staging loads per wave and half-unit
     static_assert(PER * PPI * GW == BN, "staging split");
-    __shared__ GemmSmem<HL, BN, UNIT> sm;
+    __shared__ GemmSmem<GW, HL, BN, UNIT> sm;
     int ti, sub, rg;
     // the grid covers the tile upper bound; the items of the tiles that exist are spread over the XCDs
     // as if the grid were exact, and the rest exit (otherwise the XCDs whose ranges hold the missing
@@ -419,6 +428,12 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
     const uint8_t* pesrc = reinterpret_cast<const uint8_t*>(UNIT ? in.pu : in.pe) + src0 * (size_t)(H * 4);
     const uint8_t* xmsrc = reinterpret_cast<const uint8_t*>(UNIT ? in.xu : in.xm) + src0 * (size_t)(in.KU * 48);
     const uint8_t* rxsrc = UNIT ? reinterpret_cast<const uint8_t*>(in.rx) + src0 * (size_t)(H * HB * 4) : nullptr;
+    const uint8_t* rdsrc = nullptr;
+    if constexpr (UNIT)
+        if (active) {
+            const QMat& W = g ? W1 : W0;
+            rdsrc = W.mn + (size_t)e * W.mn_es + (size_t)rt0 * W.nkb * MN_SB + MN_RD + n * 4;
+        }
     auto stage = [&](int h) {
         St& S = sm.st[h & 1];
         const uint8_t* base = qsrc + (size_t)h * GB;
@@ -431,7 +446,10 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                     for (int pc = 0; pc < 3; ++pc) dma16(xb + xoff + pc * 16, S.xm + pc * (BN * 8) + 64 * sj * 8);
             }
         }
-        if constexpr (UNIT) {  // unit ratios of the half-unit's blocks, [block][pair]
+        if constexpr (UNIT) {
+            // the super-block's weight-unit ratios of the wave's own rows (lanes 0-31 gate, 32-63 up)
+            if (!(h & 1) && active) dma4(rdsrc + (size_t)(h >> 1) * MN_SB, sm.rd + wave * 64);
+            // unit ratios of the half-unit's blocks, [block][pair]
             if (wave < BN / 64) {
                 const uint8_t* rb = rxsrc + (size_t)h * (HB * 4) + rxoff;
 #pragma unroll
@@ -453,9 +471,9 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
         const QMat& W = (GATEUP && i == 1) ? W1 : W0;
         qbase[i] = W.qs + (size_t)e * W.qs_es;
         sbase[i] = W.sc + (size_t)e * W.sc_es;
-        mbase[i] = Q4K ? W.mn + (size_t)e * W.mn_es : nullptr;
         xbase[i] = W.ex ? W.ex + (size_t)e * W.ex_es : nullptr;
         const int rt = min(GATEUP ? rt0 : rt0 + i, W.nrt - 1);
+        mbase[i] = Q4K ? W.mn + (size_t)e * W.mn_es + (size_t)rt * W.nkb * MN_SB : nullptr;
         qo[i] = WRaw<TYPE>::qoff(W, rt, n, g);
         so[i] = WRaw<TYPE>::soff(W, rt, n);
         mo[i] = WRaw<TYPE>::moff(W, rt, n);
@@ -515,7 +533,26 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
         if (!active) return;
         const uint8_t* sa = sm.st[ODD].q + pg * TN * 32 * PB;
         if constexpr (SUPER) {
-            if (!ODD) {
+            if constexpr (UNIT) {
+                if (!ODD) {  // into the super-block's weight units (rows 8 ii + 4 g .. of the wave's tiles)
+                    const float* rd = sm.rd + wave * 64 + 4 * g;
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) {
+                        hdr[i] = cur[i].cs;
+#pragma unroll
+                        for (int ii = 0; ii < 4; ++ii) {
+                            const float4 v = *reinterpret_cast<const float4*>(rd + 32 * i + 8 * ii);
+#pragma unroll
+                            for (int t = 0; t < TN; ++t) {
+                                acc[i][t][4 * ii] *= v.x;
+                                acc[i][t][4 * ii + 1] *= v.y;
+                                acc[i][t][4 * ii + 2] *= v.z;
+                                acc[i][t][4 * ii + 3] *= v.w;
+                            }
+                        }
+                    }
+                }
+            } else if (!ODD) {
 #pragma unroll
                 for (int i = 0; i < TM; ++i) {
                     float d;
@@ -539,7 +576,8 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                         (void)d;
                     }
                 }
-            } else if constexpr (Q4K) {
+            }
+            if constexpr (Q4K) if (ODD) {
                 // min term, once per super-block: acc += sum_j (dx_j sum q_j) (-dmin m_j / unit) on bf16
                 // 3-piece splits (the activation side in xm, the weight side from the min table); six of
                 // the nine piece products (all above 2^-24 relative) in three MFMAs, (MFMA, lane half) ->
@@ -557,9 +595,14 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                         const int pr = 32 * t + n;
                         const b8 x0 = *reinterpret_cast<const b8*>(xm + (g ? 1 : 0) * BN * 8 + pr * 8);
                         const b8 x1 = *reinterpret_cast<const b8*>(xm + (g ? 2 : 0) * BN * 8 + pr * 8);
-                        acc[i][t] = mfma16b(x0, wm[0], acc[i][t]);
-                        acc[i][t] = mfma16b(x1, wm[1], acc[i][t]);
-                        if constexpr (GATEUP) acc[i][t] = mfma16b(x0, wm[2], acc[i][t]);
+                        if constexpr (UNIT) {
+                            acc[i][t] = mfma16b(wm[0], x0, acc[i][t]);
+                            acc[i][t] = mfma16b(wm[1], x1, acc[i][t]);
+                            acc[i][t] = mfma16b(wm[2], x0, acc[i][t]);
+                        } else {
+                            acc[i][t] = mfma16b(x0, wm[0], acc[i][t]);
+                            acc[i][t] = mfma16b(x1, wm[1], acc[i][t]);
+                        }
                     }
                 }
             }
@@ -622,32 +665,18 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                     }
                 }
             };
-            // block-unit form: each pair tile's 16 unit ratios of a block (register r <-> pair
-            // 8 (r / 4) + 4 g + r % 4), read from LDS one step ahead (measured faster than reading
-            // the second pair tile's at the block's first step, which saves registers)
-            float4 rxv[UNIT ? TN : 1][4];
+            // block-unit form: the lane's pair's unit ratio of a block, read from LDS one step ahead
+            float rxv[UNIT ? TN : 1];
             const float* rxs = nullptr;
-            if constexpr (UNIT) rxs = sm.rx[ODD] + pbase + 4 * g;
+            if constexpr (UNIT) rxs = sm.rx[ODD] + pbase + n;
+            auto read_rx1 = [&](int jj, int t) { rxv[t] = rxs[jj * BN + 32 * t]; };
             auto read_rx = [&](int jj) {
 #pragma unroll
-                for (int t = 0; t < TN; ++t)
-#pragma unroll
-                    for (int ii = 0; ii < 4; ++ii)
-                        rxv[t][ii] = *reinterpret_cast<const float4*>(rxs + jj * BN + 32 * t + 8 * ii);
-            };
-            auto read_rx1 = [&](int jj, int t) {
-#pragma unroll
-                for (int ii = 0; ii < 4; ++ii)
-                    rxv[t][ii] = *reinterpret_cast<const float4*>(rxs + jj * BN + 32 * t + 8 * ii);
+                for (int t = 0; t < TN; ++t) read_rx1(jj, t);
             };
             auto rescale = [&](int i, int t) {
 #pragma unroll
-                for (int ii = 0; ii < 4; ++ii) {
-                    acc[i][t][4 * ii] *= rxv[t][ii].x;
-                    acc[i][t][4 * ii + 1] *= rxv[t][ii].y;
-                    acc[i][t][4 * ii + 2] *= rxv[t][ii].z;
-                    acc[i][t][4 * ii + 3] *= rxv[t][ii].w;
-                }
+                for (int r = 0; r < 16; ++r) acc[i][t][r] *= rxv[t];
             };
             read_av(0, av[0]);
             convert(0, wv[0]);
@@ -671,17 +700,17 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                     if (b == 0) {
                         if (jj == 0) {
                             rescale(0, 0);
-                            acc[0][0] = mfma16(av[b][0][0], wv[b][0], acc[0][0]);
+                            acc[0][0] = mfma16(wv[b][0], av[b][0][0], acc[0][0]);
                             rescale(1, 0);
-                            acc[1][0] = mfma16(av[b][0][0], wv[b][1], acc[1][0]);
+                            acc[1][0] = mfma16(wv[b][1], av[b][0][0], acc[1][0]);
                         } else {
-                            acc[0][0] = mfma16(av[b][0][0], wv[b][0], acc[0][0]);
-                            acc[1][0] = mfma16(av[b][0][0], wv[b][1], acc[1][0]);
+                            acc[0][0] = mfma16(wv[b][0], av[b][0][0], acc[0][0]);
+                            acc[1][0] = mfma16(wv[b][1], av[b][0][0], acc[1][0]);
                         }
                         rescale(0, 1);
-                        acc[0][1] = mfma16(av[b][1][0], wv[b][0], acc[0][1]);
+                        acc[0][1] = mfma16(wv[b][0], av[b][1][0], acc[0][1]);
                         rescale(1, 1);
-                        acc[1][1] = mfma16(av[b][1][0], wv[b][1], acc[1][1]);
+                        acc[1][1] = mfma16(wv[b][1], av[b][1][0], acc[1][1]);
                         if (jj + 1 < HB) read_rx1(jj + 1, 0);
                         if (jj == 0) {
 #pragma unroll
@@ -698,10 +727,10 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                         }
                         __builtin_amdgcn_sched_barrier(0);
                     } else {
-                        acc[0][0] = mfma16(av[b][0][0], wv[b][0], acc[0][0]);
-                        acc[1][0] = mfma16(av[b][0][0], wv[b][1], acc[1][0]);
-                        acc[0][1] = mfma16(av[b][1][0], wv[b][0], acc[0][1]);
-                        acc[1][1] = mfma16(av[b][1][0], wv[b][1], acc[1][1]);
+                        acc[0][0] = mfma16(wv[b][0], av[b][0][0], acc[0][0]);
+                        acc[1][0] = mfma16(wv[b][1], av[b][0][0], acc[1][0]);
+                        acc[0][1] = mfma16(wv[b][0], av[b][1][0], acc[0][1]);
+                        acc[1][1] = mfma16(wv[b][1], av[b][1][0], acc[1][1]);
                         if (jj + 1 < HB) {
                             rescale(0, 0);
                             rescale(1, 0);
@@ -721,14 +750,8 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                     for (int t = 0; t < TN; ++t)
 #pragma unroll
                         for (int i = 0; i < TM; ++i) {
-#pragma unroll
-                            for (int ii = 0; ii < 4; ++ii) {
-                                acc[i][t][4 * ii] *= rxv[t][ii].x;
-                                acc[i][t][4 * ii + 1] *= rxv[t][ii].y;
-                                acc[i][t][4 * ii + 2] *= rxv[t][ii].z;
-                                acc[i][t][4 * ii + 3] *= rxv[t][ii].w;
-                            }
-                            acc[i][t] = mfma16(av[b][t][0], wv[b][i], acc[i][t]);
+                            rescale(i, t);
+                            acc[i][t] = mfma16(wv[b][i], av[b][t][0], acc[i][t]);
                         }
 #pragma unroll
                     for (int k = 0; k < TN * TM; ++k) {
@@ -742,7 +765,9 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
 #pragma unroll
                         for (int t = 0; t < TN; ++t)
 #pragma unroll
-                            for (int i = 0; i < TM; ++i) acc[i][t] = mfma16(av[b][t][hl], wv[b][i], acc[i][t]);
+                            for (int i = 0; i < TM; ++i)
+                                acc[i][t] = UNIT ? mfma16(wv[b][i], av[b][t][hl], acc[i][t])
+                                                 : mfma16(av[b][t][hl], wv[b][i], acc[i][t]);
                 }
                 if (UNIT && !(TN == 2 && TM == 2) && b == 1 && st + 1 < 2 * HB) read_rx((st + 1) >> 1);
                 if (st + 1 < 2 * HB) {
@@ -915,6 +940,66 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
     }
 
     // ------------------------------------------------------------ epilogue
+    if constexpr (UNIT) {
+        if (!active) return;
+        // Lane (n, g) holds pair 32 t + n and rows 8 (r / 4) + 4 g + r % 4 of the wave's gate and up tiles: back
+        // to natural units, h = act(gate) * up, and h's block of 32 rows (row tile rt0) split over the lanes of
+        // both halves.
+        const float* pe = sm.st[(h1 - 1) & 1].pe + pbase + n;
+        const float* ug = reinterpret_cast<const float*>(W0.mn + (size_t)e * W0.mn_es + ((size_t)rt0 * W0.nkb + W0.nkb - 1) * MN_SB + MN_U) + 4 * g;
+        const float* uu = reinterpret_cast<const float*>(W1.mn + (size_t)e * W1.mn_es + ((size_t)rt0 * W1.nkb + W1.nkb - 1) * MN_SB + MN_U) + 4 * g;
+#pragma unroll
+        for (int t = 0; t < TN; ++t) {
+            const float pv = pe[32 * t];
+            float v[16];
+#pragma unroll
+            for (int ii = 0; ii < 4; ++ii) {
+                const float4 a = *reinterpret_cast<const float4*>(ug + 8 * ii), b = *reinterpret_cast<const float4*>(uu + 8 * ii);
+                const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    v[4 * ii + c] = gated(acc[0][t][4 * ii + c] * (pv * av[c]), acc[1][t][4 * ii + c] * (pv * bv[c]), W0.act);
+            }
+            const int pr = pbase + 32 * t + n;
+            const size_t p = (size_t)(p0 + pr);
+            const bool valid = pr < cnt;
+            if (hf && valid) {
+                float* fd = hf + p * (size_t)hf_ld + rt0 * 32 + 4 * g;
+#pragma unroll
+                for (int ii = 0; ii < 4; ++ii)
+                    *reinterpret_cast<float4*>(fd + 8 * ii) = make_float4(v[4 * ii], v[4 * ii + 1], v[4 * ii + 2], v[4 * ii + 3]);
+            }
+            if (!hq.q) continue;
+            // Q8_0 of the block (quantize_row_q8_0): both halves' lanes hold the same scale and sum
+            float amax = 0.0f;
+#pragma unroll
+            for (int c = 0; c < 16; ++c) amax = fmaxf(amax, __builtin_fabsf(v[c]));
+            amax = fmaxf(amax, __shfl_xor(amax, 32));
+            const float d = amax / 127.0f;
+            const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
+            int s = 0;
+            uint32_t w[4];
+#pragma unroll
+            for (int c = 0; c < 16; ++c) {
+                float r = round_away(v[c] * id);
+                r = fminf(fmaxf(r, -127.0f), 127.0f);
+                const int q = (int)r;
+                s += q;
+                if ((c & 3) == 0) w[c >> 2] = 0;
+                w[c >> 2] |= ((uint32_t)q & 0xFFu) << (8 * (c & 3));
+            }
+            s += __shfl_xor(s, 32);
+            // word ii of half g is rows 8 ii + 4 g ..: exchange so half g stores rows 16 g .. 16 g + 15
+            const auto x0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+            const auto x1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+            if (valid) {
+                *reinterpret_cast<uint4*>(hq.q + p * (size_t)hq.K + rt0 * 32 + 16 * g) = make_uint4(x0[0], x0[1], x1[0], x1[1]);
+                if (g == 0)
+                    hq.s[p * (size_t)(hq.K / 32) + rt0] = make_float2(f16_to_f32(f32_to_f16_trunc(d)), (float)s);
+            }
+        }
+        return;
+    }
     if (active) {  // back to natural units: the row's unit (RESCALE) and the token's exponent
         const float* pe = sm.st[(h1 - 1) & 1].pe + pbase;
 #pragma unroll
@@ -934,7 +1019,7 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                     }
             }
     }
-    if constexpr (GATEUP) {
+    if constexpr (GATEUP && !UNIT) {
         // h = SiLU(g) * u in registers, written transposed to LDS: [pair][row of the workgroup]
         constexpr int HLD = A_::RW * 32 + 4;              // h row stride (floats)
         float* hs = reinterpret_cast<float*>(&sm.st[0]);  // [128 pairs][HLD], over both stage buffers
@@ -996,7 +1081,7 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
             qd[1] = make_uint4(w[4], w[5], w[6], w[7]);
             hq.s[p * (size_t)(hq.K / 32) + blk] = make_float2(f16_to_f32(f32_to_f16_trunc(d)), (float)s);
         }
-    } else {
+    } else if constexpr (!GATEUP) {
         if (!active) return;
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
@@ -1054,6 +1139,14 @@ __global__ void __launch_bounds__(256) k_min_table(QMat m, uint8_t* mn) {
     for (int c = 0; c < 3; ++c)
         *reinterpret_cast<uint4*>(base + c * 512) = make_uint4(pw[c][0], pw[c][1], pw[c][2], pw[c][3]);
     *reinterpret_cast<uint4*>(base + MN_CS) = make_uint4(cw[0], cw[1], cw[2], cw[3]);
+    float up = 1.0f;  // the previous super-block's unit (1 before the first)
+    if (t % m.nkb) {
+        const float dp = f16_to_f32(*reinterpret_cast<const uint32_t*>(m.sc + ((t - 1) * 32 + row) * 16) & 0xFFFFu);
+        up = dp == 0.0f ? 1.0f : dp;
+    }
+    float* ru = reinterpret_cast<float*>(mn + t * MN_SB + MN_RD) + row;
+    ru[0] = up / u;
+    ru[(MN_U - MN_RD) / 4] = u;
 }
 
 void launch_min_table(const QMat& m, uint8_t* mn, hipStream_t st) {

@@ -22,7 +22,8 @@ namespace jx {
 //         sc  [e][rt][sb][32 rows][16 B] = the 16 int8 sub-block scales
 //         ex  [e][rt][sb][32] fp16 d
 // Byte totals of qs+sc(+ex) equal the GGUF tensor (18/34/144/22/176/210 B per block).
-constexpr int MN_SB = 2048, MN_CS = 1536;  // QMat::mn bytes per (row tile, super-block); scales offset
+// QMat::mn bytes per (row tile, super-block); offsets of the scales, the unit ratios and the units
+constexpr int MN_SB = 2304, MN_CS = 1536, MN_RD = 2048, MN_U = 2176;
 
 struct QMat {
     int type = 0;
@@ -47,7 +48,8 @@ struct QMat {
     // and for matrices only the GEMVs read): per (expert, row tile, super-block) MN_SB
     // bytes, 3 x [32 rows][16 B] = the bf16 pieces (hi, mid, lo) of -dmin * m_j / u for
     // the 8 sub-blocks j, u = d (1 where d is zero), then at MN_CS [32 rows][16 B] = the
-    // fp16 A-operand scales s1 of the 8 sub-blocks.
+    // fp16 A-operand scales s1 of the 8 sub-blocks, at MN_RD [32 rows] fp32 u(s-1) / u(s) of super-block s
+    // (u(-1) = 1) and at MN_U [32 rows] fp32 u(s).
     const uint8_t* mn = nullptr;
     size_t mn_es = 0;  // per-expert stride (bytes)
     // Gated activation applied to this matrix's outputs when it is the gate of
