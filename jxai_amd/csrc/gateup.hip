@@ -1,0 +1,538 @@
+// Prefill gate/up: grouped GEMM on the matrix cores, one exact product per 32-block.
+//
+// The reference's dots (vec_dot_{q4_0,q8_0,q4_K,q5_K}_q8_0, src/quant.cpp:3307-3730)
+// sum each 32-element block exactly in integers and scale it by (weight scale x
+// activation scale).  Here, per 32-block and 32 x 32 result tile:
+//   S  = the block's integer sums, one MFMA with a zero accumulator
+//   P  = (weight scale of the row) x (activation scale of the pair), one MFMA of
+//        inner length 2 (the outer product)
+//   acc = fma(S, P, acc), 16 per lane
+// so the VALU does nothing but the accumulation: no operand is converted and no
+// accumulator rescaled.  Forms of S:
+//   Q4_0, Q4_K, Q5_K  v_mfma_scale_f32_32x32x64_f8f6f4 on FP6 (e2m3) operands.  FP6 holds
+//        0..15 with a sign exactly in units of 1/8 (the code's low bits are the value),
+//        and -16.  The weight q (Q4_0: q - 8, Q5_K: q - 16) is one digit; the Q8_0 quant
+//        is sign * (16 a + b), two digits, its lanes' block scales 2^4 and 1.  K = 64 of the
+//        instruction is the block's 32 weights twice, against the a's and the b's.
+//        |S| < 2^17: exact in fp32.
+//   Q8_0  v_mfma_i32_32x32x32_i8 on the quants as they are, converted to fp32 for the fma
+//        (|S| < 2^19).  (FP6 would need two weight digits and a second MFMA.)
+// P is exact up to one rounding: bf16 pieces of the scales (FP6 form: d or d * sc_j, 3
+// pieces; dx, 2 pieces) or the fp16 scales themselves (Q8_0).  The Q4_K / Q5_K min term
+// -dmin * sum_j m_j * (dx_j * sum q_j) (Q5_K: plus 16 d sc_j for the offset) is three bf16
+// MFMAs on 3-piece splits once per super-block, straight into acc.  Only the fp32 rounding of
+// the accumulation differs from the reference; it matters, because h = SiLU(g) * u is
+// re-quantized to Q8_0 (a relative error of 2^-11 in g and u moves ~1.4% of h's quants by
+// one step, ~2.6e-3 relative in the layer output).
+//
+// Work split: the dispatch tables cut each expert's pairs into tiles of MFMA_BN; a workgroup
+// owns 64 of a tile's pairs and 128 gate rows with the same 128 up rows, so SwiGLU and h's
+// Q8_0 blocks are settled in registers.  4 waves, each a gate and an up row tile x two
+// pair tiles (32 x 32 each).  Weights are MFMA operand A: lane (n, g) = (lane % 32, lane / 32) of
+// a result holds pair n and, in register r, row 8 (r / 4) + 4 g + r % 4.
+//
+// Data movement: activations go global -> LDS by DMA per half-unit (128 of K, double-buffered,
+// 16-byte chunks XOR-swizzled by row so operand reads are conflict-free).  Each wave's
+// weights stream into a register ring one half-unit ahead: a block's registers are
+// reloaded for the next half-unit as soon as its products are issued, so loads are spread
+// over the half-unit and the barrier waits only for the DMA (vmcnt counts in order, and the
+// ring's loads are younger).
+#include <stddef.h>
+
+#include <algorithm>
+
+#include "jxmoe_gemm.h"
+
+namespace jx {
+
+namespace {
+
+typedef int v6i __attribute__((ext_vector_type(6)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+
+enum : int { GU_F6 = 0, GU_F6_MIN = 1, GU_I8 = 2 };
+
+constexpr int GU_BN = 64;     // pairs per workgroup
+constexpr int GU_WAVES = 4;   // row-tile slots
+constexpr int GU_RC = 8;      // row groups per band (work_item)
+
+// One staged half-unit of GU_BN activation rows.
+template <int KIND>
+struct GuStage {
+    static constexpr int PB = KIND == GU_I8 ? 128 : 256;  // bytes per row
+    uint8_t q[GU_BN * PB];                                // row r, chunk c at chunk c ^ (r % (PB / 16))
+    float sx[KIND == GU_I8 ? GU_BN * 8 : 4];              // [block pair][row][2 blocks](scale, sum)
+    uint16_t xm[KIND == GU_F6_MIN ? 3 * GU_BN * 8 : 8];   // [piece][row][8 sub-blocks] bf16 of dx * sum(q)
+    // the waves' min-term weight pieces: gate hi, gate mid, up hi, up mid, gate lo, up lo, each [32 rows][16 B]
+    uint8_t wm[KIND == GU_F6_MIN ? GU_WAVES * 3072 : 16];
+};
+
+template <int KIND>
+struct alignas(16) GuSmem {
+    GuStage<KIND> st[2];
+    int src[GU_BN];  // token of each staged pair
+};
+
+// What a workgroup reads of x.
+struct GuIn {
+    const uint8_t* q;    // rows of operand bytes (ActH::q6, or the Q8_0 quants)
+    const uint8_t* s;    // Q8_0 form: rows of (scale, sum)
+    const uint8_t* xm;   // min-term pieces (ActH::x6)
+    int K, KU;
+};
+
+__device__ __forceinline__ v6i join6(v4i a, v2i b) {
+    return __builtin_shufflevector(a, __builtin_shufflevector(b, b, 0, 1, -1, -1), 0, 1, 2, 3, 4, 5);
+}
+
+// 32 x 32 sums of 32 FP6 products of each lane half (element blocks scaled by 2^(sa - 127), 2^(sb - 127)).
+__device__ __forceinline__ v16f mfma_fp6(v6i a, v6i b, int sa, int sb) {
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(__builtin_shufflevector(a, a, 0, 1, 2, 3, 4, 5, -1, -1),
+                                                           __builtin_shufflevector(b, b, 0, 1, 2, 3, 4, 5, -1, -1), v16f{},
+                                                           2, 2, 0, sa, 0, sb);
+}
+
+// Keeps a uniform address in scalar registers, so loads take it with a 32-bit lane offset (the compiler
+// would otherwise add the lane offsets first and hold 64-bit vector addresses).
+typedef const __attribute__((address_space(1))) uint8_t gbyte;
+__device__ __forceinline__ gbyte* scalar(const uint8_t* p) {
+    gbyte* g = (gbyte*)p;
+    asm("" : "+s"(g));
+    return g;
+}
+// The lane offset beside it: redefined where it is used, so its widening stays in the load's own block.
+__device__ __forceinline__ uint32_t here(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+template <typename T>
+__device__ __forceinline__ T gload(gbyte* p) {
+    return *reinterpret_cast<const __attribute__((address_space(1))) T*>(p);
+}
+// 64 lanes x 16 bytes from src + off (per lane) into LDS at byte `lds` (wave-uniform), lane i at lds + 16 i.  In
+// asm because the compiler, which counts the builtin as a flat access, then waits for every load in flight
+// before it uses any.  It has no result registers; the waits are the kernel's own (vmcnt counts in order, so the
+// compiler's counted waits for the weights only get stricter).  Nothing else in the kernel uses m0.
+__device__ __forceinline__ void dma16g(gbyte* src, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(src) : "memory");
+}
+// The same from per-lane addresses.
+__device__ __forceinline__ void dma16v(const uint8_t* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+
+// The weight ring: one 32-block of a row tile.
+template <int KIND>
+struct Wt {
+    v6i w;  // row n's FP6 codes
+    v2i p;  // its scale's bf16 pieces
+    __device__ __forceinline__ void load(gbyte* q, gbyte*, uint32_t o0, uint32_t o1) {
+        w = join6(gload<v4i>(q + o0), gload<v2i>(q + 512 + o1));
+        p = gload<v2i>(q + 768 + o1);
+    }
+};
+template <>
+struct Wt<GU_I8> {
+    v4i w;       // elements 16g .. 16g+15 of row n's block
+    uint16_t d;  // its fp16 scale
+    __device__ __forceinline__ void load(gbyte* q, gbyte* s, uint32_t o0, uint32_t o1) {
+        w = gload<v4i>(q + o0);
+        d = gload<uint16_t>(s + o1);
+    }
+};
+
+// VGPRs 256 of 256 at two waves per SIMD: acc 64, two (S, P) sets 64, the weight ring 64 (FP6), operands 16.
+template <int KIND>
+__global__ void __launch_bounds__(GU_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ8 hq, float* hf, int hf_ld) {
+    constexpr bool I8 = KIND == GU_I8, MIN = KIND == GU_F6_MIN;
+    using St = GuStage<KIND>;
+    constexpr int PB = St::PB, CPP = PB / 16, PPI = 64 / CPP;  // row bytes, chunks, rows per DMA
+    constexpr int PER = GU_BN / PPI / GU_WAVES;                // 1 KB DMAs per wave and half-unit
+    __shared__ GuSmem<KIND> sm;
+    int ti, sub, rg;
+    // the grid covers the tile upper bound; the items of the tiles that exist are spread over the XCDs as if
+    // the grid were exact, and the rest exit
+    int n_eff = n_items;
+    if (!grp.identity) n_eff = min(n_items, R * *grp.n_tiles * (MFMA_BN / GU_BN));
+    const int LB = (int)blockIdx.x;
+    if ((LB >> 3) >= (n_eff >> 3) + ((LB & 7) < (n_eff & 7) ? 1 : 0)) return;
+    work_item(LB, n_eff, R, MFMA_BN / GU_BN, RC, ti, sub, rg);
+    int e, p0, cnt;
+    if (!pair_tile(grp, ti, e, p0, cnt)) return;  // whole workgroup
+    e = __builtin_amdgcn_readfirstlane(e);  // uniform: the weight addresses stay scalar
+    p0 = __builtin_amdgcn_readfirstlane(p0) + sub * GU_BN;  // this workgroup's part of the tile
+    cnt = __builtin_amdgcn_readfirstlane(cnt) - sub * GU_BN;
+    if (cnt <= 0) return;
+    cnt = min(cnt, GU_BN);
+
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // a wave past the matrix repeats the last row tile and drops its results
+    const bool active = rg * GU_WAVES + wave < W0.nrt;
+    const int rt0 = min(rg * GU_WAVES + wave, W0.nrt - 1);
+
+    if (tid < GU_BN) {
+        const int p = p0 + min(tid, cnt - 1);
+        sm.src[tid] = grp.identity ? p : grp.pair_tok[p];
+    }
+    __syncthreads();
+
+    const int KB = in.K / 32, H = in.K / 128;
+    // an expert's pairs are in token order, so the buffers are based at the first source row in 64 bits and
+    // per-lane offsets stay below 2^32 (jx_moe_forward refuses larger batches)
+    const size_t src0 = (size_t)(uint32_t)__builtin_amdgcn_readfirstlane(sm.src[0]);
+    const int rowb = H * PB;  // global bytes per row: q6 64 B per block, quants 32 B
+    uint32_t soff[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int r = PPI * (wave * PER + k) + lane / CPP;
+        soff[k] = (uint32_t)(sm.src[r] - (int)src0) * (uint32_t)rowb + (uint32_t)(((lane % CPP) ^ (r % CPP)) << 4);
+    }
+    const uint32_t srow = (uint32_t)(sm.src[lane] - (int)src0);  // wave 0: the row of its side loads
+    const uint8_t* qsrc = in.q + src0 * (size_t)rowb;
+    const uint32_t xoff = srow * (uint32_t)(I8 ? KB * 8 : in.KU * 48);
+    const uint8_t* xsrc = (I8 ? in.s : in.xm) + src0 * (size_t)(I8 ? KB * 8 : in.KU * 48);
+
+    const uint8_t* wb[2];   // the wave's gate and up row tiles
+    const uint8_t* wsb[2];  // Q8_0: their scales
+    const uint8_t* wmb[2];  // their min-term pieces
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const QMat& W = i ? W1 : W0;
+        wb[i] = (I8 ? W.qs + (size_t)e * W.qs_es : W.g6 + (size_t)e * W.g6_es) + (size_t)rt0 * KB * 1024;
+        wsb[i] = W.sc + (size_t)e * W.sc_es + (size_t)rt0 * KB * 64;
+        wmb[i] = MIN ? W.g6m + (size_t)e * W.g6m_es + (size_t)rt0 * in.KU * G6M_SB : nullptr;
+    }
+    const uint8_t* wlo = MIN ? (g ? wmb[1] : wmb[0]) + 1024 + n * 16 : nullptr;
+
+    // LDS address of a stage's parts
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)&sm;
+    auto stage = [&](int h, int buf) {
+        const uint32_t S = lds0 + buf * (uint32_t)sizeof(St);
+        gbyte* base = scalar(qsrc + (size_t)h * PB);
+#pragma unroll
+        for (int k = 0; k < PER; ++k) dma16g(base, soff[k], S + (wave * PER + k) * 1024);
+        if constexpr (I8) {
+            if (wave == 0) {
+                gbyte* b = scalar(xsrc + (size_t)h * (HB * 8));
+                dma16g(b, xoff, S + offsetof(St, sx));
+                dma16g(b + 16, xoff, S + offsetof(St, sx) + GU_BN * 16);
+            }
+        }
+        if constexpr (MIN) {
+            if (h & 1) {  // the super-block's min-term pieces, used at the end of its second half
+                const uint32_t sb = (uint32_t)(h >> 1) * G6M_SB;
+                const uint32_t d = S + offsetof(St, wm) + wave * 3072;
+                gbyte *m0 = scalar(wmb[0] + sb), *m1 = scalar(wmb[1] + sb);
+                dma16g(m0, (uint32_t)lane * 16, d);
+                dma16g(m1, (uint32_t)lane * 16, d + 1024);
+                dma16v(wlo + sb, d + 2048);
+                if (wave == 0) {
+                    gbyte* b = scalar(xsrc + (size_t)(h >> 1) * 48);
+#pragma unroll
+                    for (int pc = 0; pc < 3; ++pc) dma16g(b + pc * 16, xoff, S + offsetof(St, xm) + pc * (GU_BN * 16));
+                }
+            }
+        }
+    };
+
+    v16f acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[i][t] = v16f{};
+    v16f S[2], P[2];  // the block sums and scale products of the last two tiles
+    v16i Si[2];
+    Wt<KIND> ring[HB][2];
+
+    // operand B: byte offsets of this lane's chunks of block 0 in pair tile 0 (codes or quants; code tail and
+    // pieces, or the scale)
+    const uint32_t lb0 = (uint32_t)(n * PB + ((g ^ (n % CPP)) << 4));
+    const uint32_t lb1 = I8 ? (uint32_t)n * 16 : (uint32_t)(n * PB + ((8 ^ (n % CPP)) << 4) + 8 * g);
+    const uint32_t lo0 = (uint32_t)(I8 ? lane : n) * 16, lo1 = (uint32_t)n * (I8 ? 2 : 8);
+    auto load = [&](int h, int j, uint32_t o0, uint32_t o1) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            ring[j][i].load(scalar(wb[i] + (size_t)(uint32_t)h * (HB * 1024) + j * 1024),
+                            I8 ? scalar(wsb[i] + (size_t)(uint32_t)h * (HB * 64) + j * 64) : nullptr, o0, o1);
+    };
+    // acc of tile (i, t) takes the sums of set c
+    auto fold = [&](int i, int t, int c) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            acc[i][t][r] = __builtin_fmaf(I8 ? (float)Si[c][r] : S[c][r], P[c][r], acc[i][t][r]);
+        asm volatile("" : "+v"(acc[i][t]));  // here, not where acc is next read: (S, P) stay two sets
+    };
+    const int sa = 130, sbx = g ? 130 : 134;  // 2^3 takes the codes' 1/8 away; the a digits count 16
+    const uint32_t gmask = g ? 0u : 0xFFFFu;
+
+    stage(0, 0);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int j = 0; j < HB; ++j) {
+        load(0, j, lo0, lo1);
+        __builtin_amdgcn_sched_barrier(0);  // in the ring's order: the loop waits by count
+    }
+
+    auto half = [&](int h, bool odd) {
+        // this half-unit's DMAs are older than the ring loads (Q8_0 16, FP6 24); the other waves' reads of the other stage are done
+        if constexpr (I8) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(24) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (h + 1 < H) stage(h + 1, odd ? 0 : 1);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        const St& cur = sm.st[odd ? 1 : 0];
+        const int hn = min(h + 1, H - 1);
+        const uint32_t o0 = here(lo0), o1 = here(lo1);
+        // operand B of pair tile t, block j
+        v6i bf[2];
+        v2i bp[2];
+        v4i bi[2];
+        int bd[2];
+        // chunk c of row r sits at chunk c ^ (r % CPP): the lane's offset for block j is an XOR away from block 0's
+        const uint32_t b0 = here(lb0), b1 = here(lb1);
+        auto read_b = [&](int t, int j) {
+            const uint8_t* q = cur.q + t * 32 * PB;
+            if constexpr (I8) {
+                bi[t] = *reinterpret_cast<const v4i*>(q + (b0 ^ (j << 5)));
+                bd[t] = *reinterpret_cast<const int*>(reinterpret_cast<const uint8_t*>(cur.sx) + (j >> 1) * (GU_BN * 16) +
+                                                      t * 512 + (j & 1) * 8 + b1);
+            } else {
+                const v4i a = *reinterpret_cast<const v4i*>(q + (b0 ^ (j << 5)));
+                const v2i b = *reinterpret_cast<const v2i*>(q + (b1 ^ (j << 4)));
+                bf[t] = join6(a, b);
+                bp[t] = *reinterpret_cast<const v2i*>(q + (b1 ^ ((4 + j) << 4)));
+            }
+        };
+        read_b(0, 0);
+        read_b(1, 0);
+#pragma unroll
+        for (int j = 0; j < HB; ++j) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int i = k & 1, t = k >> 1, c = k & 1;
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (I8) {
+                    Si[c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[j][i].w, bi[t], v16i{}, 0, 0, 0);
+                    const uint32_t dx = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)__int_as_float(bd[t])) & gmask;
+                    P[c] = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(h4, v2i{(int)(uint32_t)ring[j][i].d, 0}),
+                                                               __builtin_bit_cast(h4, v2i{(int)dx, 0}), v16f{}, 0, 0, 0);
+                } else {
+                    S[c] = mfma_fp6(ring[j][i].w, bf[t], sa, sbx);
+                    P[c] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(s4, ring[j][i].p),
+                                                                   __builtin_bit_cast(s4, bp[t]), v16f{}, 0, 0, 0);
+                }
+                if (j > 0 || k > 0) fold((k + 3) & 1, ((k + 3) & 3) >> 1, c ^ 1);  // the tile before
+                if (i == 1 && j + 1 < HB) read_b(t, j + 1);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);  // VALU
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            load(hn, j, o0, o1);
+        }
+        fold(1, 1, 1);
+        if constexpr (MIN) {
+            if (odd) {
+                // acc += sum_j (dx_j sum q_j)(-dmin m_j): six of the nine piece products (all above 2^-24
+                // relative) in three MFMAs, (MFMA, lane half) -> (weight piece, activation piece):
+                // (0,0) h.h (0,1) h.m (1,0) m.h (1,1) h.l (2,0) l.h (2,1) m.m
+                const uint8_t* wm = cur.wm + wave * 3072 + n * 16;
+                b8 x0[2], x1[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const uint16_t* xp = cur.xm + (32 * t + n) * 8;
+                    x0[t] = *reinterpret_cast<const b8*>(xp + (g ? 1 : 0) * GU_BN * 8);
+                    x1[t] = *reinterpret_cast<const b8*>(xp + (g ? 2 : 0) * GU_BN * 8);
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const b8 w0 = *reinterpret_cast<const b8*>(wm + i * 1024);
+                    const b8 w1 = *reinterpret_cast<const b8*>(wm + i * 1024 + (g ? 0 : 512));
+                    const b8 w2 = *reinterpret_cast<const b8*>(wm + (g ? i * 1024 + 512 : 2048 + i * 512));
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        acc[i][t] = mfma16b(w0, x0[t], acc[i][t]);
+                        acc[i][t] = mfma16b(w1, x1[t], acc[i][t]);
+                        acc[i][t] = mfma16b(w2, x0[t], acc[i][t]);
+                    }
+                }
+            }
+        }
+    };
+    for (int h = 0; h < H; h += 2) {
+        half(h, false);
+        if (h + 1 < H) half(h + 1, true);
+    }
+
+    // h = act(gate) * up, and h's block of 32 rows (row tile rt0) split over lanes n and n + 32
+    if (!active) return;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        float v[16];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) v[c] = gated(acc[0][t][c], acc[1][t][c], W0.act);
+        const int pr = 32 * t + n;
+        const size_t p = (size_t)(p0 + pr);
+        const bool valid = pr < cnt;
+        if (hf && valid) {
+            float* fd = hf + p * (size_t)hf_ld + rt0 * 32 + 4 * g;
+#pragma unroll
+            for (int ii = 0; ii < 4; ++ii)
+                *reinterpret_cast<float4*>(fd + 8 * ii) = make_float4(v[4 * ii], v[4 * ii + 1], v[4 * ii + 2], v[4 * ii + 3]);
+        }
+        if (!hq.q) continue;
+        // Q8_0 of the block (quantize_row_q8_0): both halves' lanes hold the same scale and sum
+        float amax = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) amax = fmaxf(amax, __builtin_fabsf(v[c]));
+        amax = fmaxf(amax, __shfl_xor(amax, 32));
+        const float d = amax / 127.0f;
+        const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
+        int s = 0;
+        uint32_t w[4];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            float r = round_away(v[c] * id);
+            r = fminf(fmaxf(r, -127.0f), 127.0f);
+            const int q = (int)r;
+            s += q;
+            if ((c & 3) == 0) w[c >> 2] = 0;
+            w[c >> 2] |= ((uint32_t)q & 0xFFu) << (8 * (c & 3));
+        }
+        s += __shfl_xor(s, 32);
+        // word ii of half g is rows 8 ii + 4 g ..: exchange so half g stores rows 16 g .. 16 g + 15
+        const auto x0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
+        const auto x1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
+        if (valid) {
+            *reinterpret_cast<uint4*>(hq.q + p * (size_t)hq.K + rt0 * 32 + 16 * g) = make_uint4(x0[0], x0[1], x1[0], x1[1]);
+            if (g == 0) hq.s[p * (size_t)(hq.K / 32) + rt0] = make_float2(f16_to_f32(f32_to_f16_trunc(d)), (float)s);
+        }
+    }
+}
+
+// The FP6 weight form of a repacked Q4_0 / Q4_K / Q5_K matrix (QMat::g6), one thread per (expert, row tile,
+// 32-block, row): the block's 32 codes, element i at bit 6 i, then the scale's bf16 pieces.
+__global__ void __launch_bounds__(256) k_g6_table(QMat m, int KB, uint8_t* out) {
+    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= (size_t)m.n_mats * m.nrt * KB * 32) return;
+    const size_t t = idx / 32;  // (e * nrt + rt) * KB + b
+    const int row = (int)(idx % 32), b = (int)(t % KB);
+    const size_t er = t / KB;   // e * nrt + rt
+    uint32_t lo[8];             // the 32 quants, a byte each
+    float scale;
+    if (m.type == T_Q4_0) {
+        const uint4 q = ld16(m.qs + (t * 32 + row) * 16);
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lo[i] = w[i] & 0x0F0F0F0Fu, lo[4 + i] = (w[i] >> 4) & 0x0F0F0F0Fu;
+        scale = f16_to_f32(*reinterpret_cast<const uint16_t*>(m.sc + (t * 32 + row) * 2));
+    } else {
+        const int j = b & 7;
+        const size_t u = er * m.nkb + (b >> 3);  // super-block
+        const uint8_t* qs = m.qs + (u * 8 + (j >> 1) * 2) * 512 + row * 16;
+        const uint4 q0 = ld16(qs), q1 = ld16(qs + 512);
+        const uint32_t w[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) lo[i] = (w[i] >> (j & 1 ? 4 : 0)) & 0x0F0F0F0Fu;
+        if (m.type == T_Q5_K) {
+            const uint8_t* ex = m.ex + u * 1024 + row * 16;
+            const uint4 h0 = ld16(ex), h1 = ld16(ex + 512);
+            const uint32_t hb[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) lo[i] |= ((hb[i] >> j) & 0x01010101u) << 4;
+        }
+        const uint4 hd = ld16(m.sc + (u * 32 + row) * 16);
+        int sc, mn;
+        hdr_scale_min(hd, j, sc, mn);
+        scale = f16_to_f32(hd.x & 0xFFFFu) * (float)sc;  // exact: 11 x 6 bits
+    }
+    const int off = m.type == T_Q4_0 ? 8 : m.type == T_Q5_K ? 16 : 0;
+    uint32_t c[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        const int v = (int)((lo[i >> 2] >> (8 * (i & 3))) & 0xFFu) - off;
+        const uint32_t code = v < 0 ? 32u | (uint32_t)-v : (uint32_t)v;
+        c[(6 * i) / 32] |= code << ((6 * i) % 32);
+        if ((6 * i) % 32 > 26) c[(6 * i) / 32 + 1] |= code >> (32 - (6 * i) % 32);
+    }
+    uint16_t p0, p1, p2;
+    split3(scale, p0, p1, p2);
+    uint8_t* o = out + t * 1024 + row * 16;
+    *reinterpret_cast<uint4*>(o) = make_uint4(c[0], c[1], c[2], c[3]);
+    *reinterpret_cast<uint2*>(o + 512 - row * 8) = make_uint2(c[4], c[5]);
+    *reinterpret_cast<uint2*>(o + 768 - row * 8) = make_uint2((uint32_t)p0 | (uint32_t)p1 << 16, p2);
+}
+
+// The min-term pieces of a repacked Q4_K / Q5_K matrix (QMat::g6m), one thread per (expert, row tile,
+// super-block, row): -dmin * m_j (exact in fp32), for Q5_K plus 16 d sc_j (its codes are q - 16).
+__global__ void __launch_bounds__(256) k_g6_min_table(QMat m, uint8_t* out) {
+    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= (size_t)m.n_mats * m.nrt * m.nkb * 32) return;
+    const size_t t = idx / 32;
+    const int row = (int)(idx % 32);
+    const uint4 hd = ld16(m.sc + (t * 32 + row) * 16);
+    const float d = f16_to_f32(hd.x & 0xFFFFu), dmin = f16_to_f32(hd.x >> 16);
+    uint32_t pw[3][4] = {};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        int sc, mv;
+        hdr_scale_min(hd, j, sc, mv);
+        float v = -dmin * (float)mv;
+        if (m.type == T_Q5_K) v = __builtin_fmaf(16.0f * d, (float)sc, v);
+        uint16_t p[3];
+        split3(v, p[0], p[1], p[2]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) pw[c][j / 2] |= (uint32_t)p[c] << (16 * (j & 1));
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+        *reinterpret_cast<uint4*>(out + t * G6M_SB + c * 512 + row * 16) = make_uint4(pw[c][0], pw[c][1], pw[c][2], pw[c][3]);
+}
+
+template <int KIND>
+void launch_kind(const QMat& g, const QMat& u, const GuIn& in, const Groups& grp, int tiles_ub, const ActQ8& hq,
+                 float* hf, hipStream_t st) {
+    const int R = (g.nrt + GU_WAVES - 1) / GU_WAVES;
+    const int n_items = R * tiles_ub * (MFMA_BN / GU_BN);
+    if (n_items <= 0) return;
+    hipLaunchKernelGGL(k_gateup<KIND>, dim3(n_items), dim3(GU_WAVES * 64), 0, st, g, u, in, grp, R, n_items,
+                       std::min(GU_RC, R), hq, hf, ((g.rows + 255) / 256) * 256);
+}
+
+}  // namespace
+
+bool gemm_gateup_ok(int type) { return type == T_Q8_0 || g6_type(type); }
+
+void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, hipStream_t st) {
+    const int KB = m.cols / 32;
+    const size_t n = (size_t)m.n_mats * m.nrt * KB * 32;
+    hipLaunchKernelGGL(k_g6_table, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m, KB, g6);
+    if (!g6m) return;
+    const size_t ns = (size_t)m.n_mats * m.nrt * m.nkb * 32;
+    hipLaunchKernelGGL(k_g6_min_table, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, st, m, g6m);
+}
+
+void launch_mfma_gateup(const QMat& g, const QMat& u, const ActH& xin, const ActQ8& xq, const Groups& grp, int tiles_ub,
+                        const ActQ8& hq, float* hf, hipStream_t st) {
+    GuIn in{xin.q6, nullptr, reinterpret_cast<const uint8_t*>(xin.x6), g.cols, (g.cols + 255) / 256};
+    if (g.type == T_Q8_0) {
+        in.q = reinterpret_cast<const uint8_t*>(xq.q);
+        in.s = reinterpret_cast<const uint8_t*>(xq.s);
+        launch_kind<GU_I8>(g, u, in, grp, tiles_ub, hq, hf, st);
+        return;
+    }
+    // the caller allocates the forms its matrices need; a missing one is a caller bug, and nothing is launched
+    // on null pointers
+    if (!g.g6 || !u.g6 || !in.q) return;
+    if (g.type == T_Q4_0) launch_kind<GU_F6>(g, u, in, grp, tiles_ub, hq, hf, st);
+    else if (g.g6m && u.g6m && in.xm) launch_kind<GU_F6_MIN>(g, u, in, grp, tiles_ub, hq, hf, st);
+}
+
+}  // namespace jx

@@ -1,45 +1,29 @@
-// Prefill regime (many tokens per expert): grouped GEMM on the matrix cores.
+// Prefill regime (many tokens per expert), down projection: grouped GEMM on the
+// matrix cores (gate/up: gateup.hip).
 //
-// The reference's dots (vec_dot_{q4_0,q8_0,q4_K}_q8_0, src/quant.cpp:3307-3573)
-// sum each 32-element block exactly and scale it by (weight scale x
-// activation scale).  Scaling every 32-K block on the VALU would cost more
-// than the matrix core's own work, so the scales ride in fp16 MFMA operands
-// that fp16 holds exactly:
-//   A (weights)      Q4_K: sc_j * q  (0..945)   Q4_0: q - 8   Q8_0: q
-//   B (activations)  Q4_K gate/up: the Q8_0 quants q (block-unit form); acc is
-//                    kept in units of the current block's dx per pair and
-//                    multiplied by u(b-1) / u(b) once per 32-block, so a block's
-//                    exact integer MFMA sum lands in the block's own units.
-//                    Otherwise: dx * q * 2^-E as an exact fp16 hi/lo pair (an
-//                    11-bit scale times |q| <= 127 has <= 18 significant bits;
-//                    hi + lo carry 22), two MFMAs per product (down: hi only)
-// Every product is exact in fp32, so each block's sum equals the reference's
-// integer block sum times (sc_j and) dx up to fp32 rounding of the
-// accumulation (and of the block-unit ratios).  (The exactness matters: h = SiLU(g) * u is re-quantized to
-// Q8_0 before the down projection, and a relative error of 2^-11 in g and u
-// moves ~1.4% of h's quants by one step, ~2.6e-3 relative in the layer output.)
+// The scales ride in fp16 MFMA operands:
+//   A (weights)      Q4_K: sc_j * q  (0..945)   Q4_0: q - 8   Q8_0: q   (exact;
+//                    Q6_K: sc_j * (q - 32), rounded once)
+//   B (activations)  dx * q * 2^-E (or h * 2^-E) in fp16: relative error <= 2^-12, nothing
+//                    downstream re-quantizes
 // What is left on the VALU: the accumulator is kept in units of the current
-// weight scale d of its row (Q4_K: per 256-K super-block; Q4_0 / Q8_0: per
+// weight scale d of its row (K-quants: per 256-K super-block; Q4_0 / Q5_0 / Q8_0: per
 // 32-block; 1 where d is zero, the weight operand then zeroed) and rescaled
 // by d_prev / d_cur when the period changes; the token's exponent 2^E (one
 // per row) and the last unit are applied once at the end.  The Q4_K min term
-// -dmin * sum_j m_j * (dx_j * sum q_j) is three bf16 MFMAs on exact 3-piece
-// splits once per super-block, straight into acc.  Only the fp32 rounding of
-// the accumulation differs from the reference.
+// -dmin * sum_j m_j * (dx_j * sum q_j) is two bf16 MFMAs on 3-piece
+// splits once per super-block, straight into acc.
 //
 // Work split: the dispatch tables cut each expert's pairs into tiles of
-// MFMA_BN = 128 (token, expert) pairs; a workgroup owns a tile (down) or half
-// of one (gate/up: 64 pairs) and a group of weight rows -- gate/up: 128 gate
-// rows and the same 128 up rows (one half-unit of the down projection's K, so
-// h's Q8_0 blocks are settled inside the workgroup); down: 128 rows.  A wave
-// owns TM row tiles x TN pair tiles of 32 (MFMA 32x32 edges): every B operand
-// read from LDS feeds TM MFMAs and every A operand converted in registers
+// MFMA_BN = 128 (token, expert) pairs; a workgroup owns a tile (or half of one) and
+// 128 weight rows.  A wave
+// owns TM row tiles x TN pair tiles of 32 (MFMA 32x32 edges): every activation operand
+// read from LDS feeds TM MFMAs and every weight operand converted in registers
 // feeds TN.  Activations are staged per 128-K half-unit into LDS with direct
 // global->LDS loads (double-buffered; 16-byte chunks XOR-swizzled by pair so
-// the B reads are bank-conflict free).  Each wave streams its own weight rows
+// the operand reads are bank-conflict free).  Each wave streams its own weight rows
 // from HBM into registers one half-unit ahead and converts them there.
-// Workgroups are numbered XCD-major so the ~32 resident on one XCD share a
-// pair tile, whose activations then stay in that XCD's L2.
+// Workgroups are numbered XCD-major (work_item).
 //
 // MFMA operand layout (v_mfma_f32_32x32x16_f16): lane (n, g) = (lane % 32,
 // lane / 32) holds A[row n][k = 8g + i] and B[k = 8g + i][col n], i < 8; the
@@ -49,138 +33,29 @@
 // order-free).
 #include <algorithm>
 
-#include "jxmoe_device.h"
-#include "jxmoe_kernels.h"
+#include "jxmoe_gemm.h"
 
 namespace jx {
 
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-
-constexpr int HB = 4;  // 32-blocks per staged half-unit
-
-// One staged half-unit of BN activation rows: HL = 2 stages fp16 hi and lo
-// (256 bytes each per row), HL = 1 hi only (or the block-unit form's fp16
-// quants).
-template <int HL, int BN>
+// One staged half-unit of BN activation rows: fp16 hi, 256 bytes per row.
+template <int BN>
 struct Stage {
-    static constexpr int PB = 256 * HL;   // bytes per row
+    static constexpr int PB = 256;        // bytes per row
     static constexpr int CPP = PB / 16;   // 16-byte chunks per row
     uint8_t q[BN * PB];                   // row r, chunk c at chunk (c ^ (r % CPP))
-    float pe[BN];                         // 2^E (block-unit form: the unit) of each row
+    float pe[BN];                         // 2^E of each row
     uint16_t xm[3 * BN * 8];              // Q4_K: [piece][row][8 sub-blocks] bf16 of dx * sum(q)
 };
 
-// Block-unit form: the unit ratios of each stage's blocks, [stage][block][row]
-// (an empty base otherwise: every byte of LDS counts where two workgroups
-// share a CU).
-template <int GW, int BN, bool RX>
-struct RxStage {
-    float rx[2][HB * BN];
-    float rd[GW * 64];  // [wave][gate, up][32 rows] the super-block's weight-unit ratios
+template <int BN>
+struct GemmSmem {
+    Stage<BN> st[2];
+    int src[BN];  // activation row of each staged pair
 };
-template <int GW, int BN>
-struct RxStage<GW, BN, false> {};
-
-template <int GW, int HL, int BN, bool RX>
-struct GemmSmem : RxStage<GW, BN, RX> {
-    Stage<HL, BN> st[2];
-    int src[BN];  // activation row (token or pair) of each staged pair
-};
-
-typedef __attribute__((address_space(3))) void* lds_ptr;
-
-// 64 lanes x 16 (4) bytes from per-lane global addresses into LDS at `base`
-// (wave-uniform), lane i at base + 16 i (4 i).
-__device__ __forceinline__ void dma16(const void* src, void* base) {
-    __builtin_amdgcn_global_load_lds(src, (lds_ptr)base, 16, 0, 0);
-}
-__device__ __forceinline__ void dma4(const void* src, void* base) {
-    __builtin_amdgcn_global_load_lds(src, (lds_ptr)base, 4, 0, 0);
-}
 
 __device__ __forceinline__ h2v splat(float v) {
     const _Float16 h = (_Float16)v;
     return h2v{h, h};
-}
-
-__device__ __forceinline__ v16f mfma16(h8 a, h8 b, v16f c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-__device__ __forceinline__ v16f mfma16b(b8 a, b8 b, v16f c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-
-// Exact 3-piece bf16 split of an fp32 value with at most 24 significant bits
-// (truncation keeps each remainder exact).
-__device__ __forceinline__ void split3(float v, uint16_t& h, uint16_t& m, uint16_t& l) {
-    const uint32_t bh = __float_as_uint(v) & 0xFFFF0000u;
-    const float r1 = v - __uint_as_float(bh);
-    const uint32_t bm = __float_as_uint(r1) & 0xFFFF0000u;
-    const float r2 = r1 - __uint_as_float(bm);
-    h = (uint16_t)(bh >> 16);
-    m = (uint16_t)(bm >> 16);
-    l = (uint16_t)(__float_as_uint(r2) >> 16);
-}
-
-// Exact fp16 hi/lo pair of dx * q (see the header comment).
-__device__ __forceinline__ void split2h(float v, uint16_t& h, uint16_t& l) {
-    const _Float16 a = (_Float16)v;
-    const _Float16 b = (_Float16)(v - (float)a);
-    h = __builtin_bit_cast(uint16_t, a);
-    l = __builtin_bit_cast(uint16_t, b);
-}
-
-// (scale, min) j of a Q4_K header in registers (get_scale_min_k4,
-// src/quant.cpp:1107-1115).
-__device__ __forceinline__ void hdr_scale_min(const uint4& hd, int j, int& sc, int& mn) {
-    const uint32_t s0 = hd.y, s1 = hd.z, s2 = hd.w;  // scales[0..3], [4..7], [8..11]
-    const int sh = 8 * (j & 3);
-    if (j < 4) {
-        sc = (s0 >> sh) & 63;
-        mn = (s1 >> sh) & 63;
-    } else {
-        const uint32_t b = (s2 >> sh) & 0xFF;
-        sc = (b & 0x0F) | ((((s0 >> sh) >> 6) & 3) << 4);
-        mn = (b >> 4) | ((((s1 >> sh) >> 6) & 3) << 4);
-    }
-}
-
-// ---------------------------------------------------------------- tiles
-__device__ __forceinline__ bool pair_tile(const Groups& grp, int ti, int& e, int& p0, int& cnt) {
-    if (grp.identity) {
-        e = 0;
-        p0 = ti * MFMA_BN;
-        cnt = min(MFMA_BN, grp.n_tok - p0);
-        return cnt > 0;
-    }
-    if (ti >= *grp.n_tiles) return false;
-    const int4 t = grp.tiles[ti];
-    e = t.x;
-    p0 = t.y;
-    cnt = t.z;
-    return true;
-}
-
-// Workgroup -> (pair tile, part of the tile, row group).  Numbering is
-// XCD-major (hardware deals workgroups round-robin over the 8 XCDs, so XCD x
-// runs a contiguous range of items), and within it bands of RC row groups
-// sweep every pair tile: the ~64 workgroups resident on one XCD then cover
-// about RC row groups x 64 / RC tile parts, and each weight row group and each
-// staged activation tile is fetched into that XCD's L2 once for several
-// workgroups.  RC = R: all row groups of a tile part before the next part.
-__device__ __forceinline__ void work_item(int L, int n_items, int R, int S, int RC, int& ti, int& sub, int& rg) {
-    const int x = L & 7, s = L >> 3;
-    const int q = n_items >> 3, rem = n_items & 7;
-    const int i = x * q + min(x, rem) + s;
-    const int TS = n_items / R;             // tile parts
-    const int band = i / (RC * TS);         // full bands hold RC * TS items; the last one fewer rows
-    const int rows = min(RC, R - band * RC);
-    const int j = i - band * RC * TS;
-    const int ts = j / rows;
-    rg = band * RC + (j - ts * rows);
-    ti = ts / S;
-    sub = ts - ti * S;
 }
 
 // ---------------------------------------------------------------- weights
@@ -316,58 +191,33 @@ struct Parity {
 
 // Wave arrangement of a workgroup owning BN pairs (a dispatch tile of
 // MFMA_BN, or a part of one): NPG pair groups of TN pair tiles (32 pairs each)
-// side by side, RW row slots.  Gate/up: row slot s takes row tile s of the
-// gate matrix and the same tile of the up matrix (TM = 2: tile 0 gate, tile 1
-// up), so SwiGLU needs no exchange.  Down: row slot s takes TM row tiles.
-template <bool GATEUP, int GW, int TM, int TN, int BN>
+// side by side, RW row slots of TM row tiles.
+template <int GW, int TM, int TN, int BN>
 struct Arr {
     static constexpr int NPG = BN / (32 * TN);
     static constexpr int RW = GW / NPG;
-    static constexpr int WROWS = GATEUP ? RW : RW * TM;  // row tiles of each matrix per workgroup
+    static constexpr int WROWS = RW * TM;  // row tiles per workgroup
     static_assert(NPG * TN * 32 == BN && NPG * RW == GW && MFMA_BN % BN == 0, "wave arrangement");
-    static_assert(!GATEUP || TM == 2, "gate/up: a gate and an up tile per wave");
 };
 
 // The MFMAs take the activations as operand A and the weights as operand B,
 // so in each 32x32 result lane (n, g) holds weight row n (its scales are the
 // lane's own) and registers r span pairs 8*(r/4) + 4g + r%4.
-// Block-unit gate/up (Q4_K / Q5_K) has them the other way round: lane (n, g)
-// holds pair n and registers r span weight rows.  The factor that changes
-// every 32 of K there is the pair's (its block unit), the row's changes every
-// 256, so each accumulator element's per-block factor is one value of the
-// lane, a 4-byte LDS read per pair tile and block, instead of 16 values in 16
-// registers from four 16-byte reads: LDS reads per 32-block 12 -> 6 (2 of
-// them 4 bytes), 256 VGPRs with spills -> 219 without.  h's 32-row Q8_0 blocks
-// then end in the registers of lanes n and n + 32 and need no LDS transpose.
-// Mixtral-shaped 2048 tokens gate/up 1737 -> 1638 us, 512 tokens 583 -> 545 us,
-// DeepSeek-V2-Lite-shaped 1555 tokens 398 -> 372 us (HIP events, one box).
-template <int TYPE, bool GATEUP, int GW, int TM, int TN, int WPE, int BN>
+template <int TYPE, int GW, int TM, int TN, int WPE, int BN>
 __global__ void __launch_bounds__(GW * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8 hq, float* hf, int hf_ld,
-        float* y, int KS, size_t ystride) {
-    constexpr int NTH = GW * 64;
+k_wgemm(QMat W0, ActH in, Groups grp, int R, int n_items, int RC, float* y, int KS, size_t ystride) {
     // K-quants (Q4_K / Q5_K / Q6_K): acc is kept in units of the current super-block's d (per weight
     // row) and rescaled by d_prev / d_cur at each super-block (fp32 rounding ~2^-24 per step); Q4_K and
     // Q5_K carry the min term (Q4K below), Q6_K has none and signed sub-block scales per 16 of K
     constexpr bool Q4K = TYPE == T_Q4_K || TYPE == T_Q5_K;
     constexpr bool K6 = TYPE == T_Q6_K;
     constexpr bool SUPER = Q4K || K6;
-    static_assert(!(K6 && GATEUP), "Q6_K gate/up runs on the GEMVs (its sc * q operand is not exact in fp16)");
-    constexpr bool RESCALE = true;
-    // Q4_K gate/up: block-unit activations -- the exact quants q as the operand and acc kept in units of
-    // the current block's dx per pair, rescaled by u(b-1) / u(b) (one multiply per accumulator element
-    // and 32-block) before the block's MFMAs; the weight scale d stays per super-block.  Q4_0 / Q8_0
-    // gate/up (d per block as well): exact hi + lo activation operands.  (h is re-quantized after
-    // SwiGLU, so gate/up products stay exact.)  Down: the hi half only (relative error <= 2^-12 per
-    // activation, no re-quantization downstream).
-    constexpr bool UNIT = Q4K && GATEUP;
-    constexpr int HL = GATEUP && !UNIT ? 2 : 1;
-    constexpr int GB = UNIT ? 256 : 512;  // global bytes per row and half-unit
-    using St = Stage<HL, BN>;
+    constexpr int GB = 512;  // global bytes per row and half-unit (hi, lo)
+    using St = Stage<BN>;
     constexpr int PB = St::PB, CPP = St::CPP, PPI = 64 / CPP;  // row bytes, chunks, rows per DMA
     constexpr int PER = BN / PPI / GW;  // 1 KB staging loads per wave and half-unit
     static_assert(PER * PPI * GW == BN, "staging split");
-    __shared__ GemmSmem<GW, HL, BN, UNIT> sm;
+    __shared__ GemmSmem<BN> sm;
     int ti, sub, rg;
     // the grid covers the tile upper bound; the items of the tiles that exist are spread over the XCDs
     // as if the grid were exact, and the rest exit (otherwise the XCDs whose ranges hold the missing
@@ -376,7 +226,7 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
     if (!grp.identity) n_eff = min(n_items, R * *grp.n_tiles * (MFMA_BN / BN));
     // down over a long K: KS adjacent workgroups per item (on different XCDs), each a range of K writing
     // its own part of y
-    const int kp = GATEUP ? 0 : (int)(blockIdx.x % KS), LB = GATEUP ? (int)blockIdx.x : (int)(blockIdx.x / KS);
+    const int kp = (int)(blockIdx.x % KS), LB = (int)(blockIdx.x / KS);
     if ((LB >> 3) >= (n_eff >> 3) + ((LB & 7) < (n_eff & 7) ? 1 : 0)) return;
     work_item(LB, n_eff, R, MFMA_BN / BN, RC, ti, sub, rg);
     int e, p0, cnt;
@@ -388,23 +238,19 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    using A_ = Arr<GATEUP, GW, TM, TN, BN>;
+    using A_ = Arr<GW, TM, TN, BN>;
     const int pg = wave % A_::NPG, rw = wave / A_::NPG;  // pair group, row slot
     const int pbase = pg * TN * 32;                       // first pair of the wave within the tile
-    // the wave's row tiles: gate/up tile rt0 of both matrices, or down tiles rt0 .. rt0 + TM - 1
-    const int rt0 = GATEUP ? rg * A_::RW + rw : (rg * A_::RW + rw) * TM;
+    const int rt0 = (rg * A_::RW + rw) * TM;  // the wave's row tiles: rt0 .. rt0 + TM - 1
     const bool active = rt0 < W0.nrt;  // wave-uniform; inactive waves still stage and sync
 
-    if (tid < BN) {  // activation row of each staged pair: token (gate/up) or pair (down)
-        const int p = p0 + min(tid, cnt - 1);
-        sm.src[tid] = (GATEUP && !grp.identity) ? grp.pair_tok[p] : p;
-    }
+    if (tid < BN) sm.src[tid] = p0 + min(tid, cnt - 1);  // activation row of each staged pair
     __syncthreads();
 
     const int H = in.KH;
     const int KB = in.K / 32;
     // this workgroup's half-units [h0, h1): whole super-blocks (an even count), the last part the rest
-    const int HP = ((H + KS - 1) / KS + 1) & ~1, h0 = GATEUP ? 0 : kp * HP, h1 = GATEUP ? H : min(H, h0 + HP);
+    const int HP = ((H + KS - 1) / KS + 1) & ~1, h0 = kp * HP, h1 = min(H, h0 + HP);
     // Source rows ascend within a tile (an expert's pairs are in token order; down rows are
     // consecutive pairs), so the workgroup's buffers are based at its first source row in 64 bits
     // and every per-lane offset is relative to it: below 2^32 whenever n_tok rows of the activation
@@ -423,17 +269,9 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
     const uint32_t srow = (uint32_t)(sm.src[64 * min(sj, BN / 64 - 1) + lane] - (int)src0);
     const uint32_t peoff = srow * (uint32_t)(H * 4);
     const uint32_t xoff = Q4K ? srow * (uint32_t)(in.KU * 48) : 0u;
-    const uint32_t rxoff = UNIT ? srow * (uint32_t)(H * HB * 4) : 0u;
-    const uint8_t* qsrc = reinterpret_cast<const uint8_t*>(UNIT ? in.q16 : in.hl) + src0 * (size_t)(H * GB);
-    const uint8_t* pesrc = reinterpret_cast<const uint8_t*>(UNIT ? in.pu : in.pe) + src0 * (size_t)(H * 4);
-    const uint8_t* xmsrc = reinterpret_cast<const uint8_t*>(UNIT ? in.xu : in.xm) + src0 * (size_t)(in.KU * 48);
-    const uint8_t* rxsrc = UNIT ? reinterpret_cast<const uint8_t*>(in.rx) + src0 * (size_t)(H * HB * 4) : nullptr;
-    const uint8_t* rdsrc = nullptr;
-    if constexpr (UNIT)
-        if (active) {
-            const QMat& W = g ? W1 : W0;
-            rdsrc = W.mn + (size_t)e * W.mn_es + (size_t)rt0 * W.nkb * MN_SB + MN_RD + n * 4;
-        }
+    const uint8_t* qsrc = reinterpret_cast<const uint8_t*>(in.hl) + src0 * (size_t)(H * GB);
+    const uint8_t* pesrc = reinterpret_cast<const uint8_t*>(in.pe) + src0 * (size_t)(H * 4);
+    const uint8_t* xmsrc = reinterpret_cast<const uint8_t*>(in.xm) + src0 * (size_t)(in.KU * 48);
     auto stage = [&](int h) {
         St& S = sm.st[h & 1];
         const uint8_t* base = qsrc + (size_t)h * GB;
@@ -444,16 +282,6 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                 const uint8_t* xb = xmsrc + (size_t)(h >> 1) * 48;
                 if (wave < BN / 64)
                     for (int pc = 0; pc < 3; ++pc) dma16(xb + xoff + pc * 16, S.xm + pc * (BN * 8) + 64 * sj * 8);
-            }
-        }
-        if constexpr (UNIT) {
-            // the super-block's weight-unit ratios of the wave's own rows (lanes 0-31 gate, 32-63 up)
-            if (!(h & 1) && active) dma4(rdsrc + (size_t)(h >> 1) * MN_SB, sm.rd + wave * 64);
-            // unit ratios of the half-unit's blocks, [block][pair]
-            if (wave < BN / 64) {
-                const uint8_t* rb = rxsrc + (size_t)h * (HB * 4) + rxoff;
-#pragma unroll
-                for (int j = 0; j < HB; ++j) dma4(rb + 4 * j, sm.rx[h & 1] + j * BN + 64 * sj);
             }
         }
         if (wave < BN / 64) dma4(pesrc + (size_t)h * 4 + peoff, S.pe + 64 * sj);
@@ -468,11 +296,11 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
     uint32_t qo[TM], so[TM], mo[TM], xo[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-        const QMat& W = (GATEUP && i == 1) ? W1 : W0;
+        const QMat& W = W0;
         qbase[i] = W.qs + (size_t)e * W.qs_es;
         sbase[i] = W.sc + (size_t)e * W.sc_es;
         xbase[i] = W.ex ? W.ex + (size_t)e * W.ex_es : nullptr;
-        const int rt = min(GATEUP ? rt0 : rt0 + i, W.nrt - 1);
+        const int rt = min(rt0 + i, W.nrt - 1);
         mbase[i] = Q4K ? W.mn + (size_t)e * W.mn_es + (size_t)rt * W.nkb * MN_SB : nullptr;
         qo[i] = WRaw<TYPE>::qoff(W, rt, n, g);
         so[i] = WRaw<TYPE>::soff(W, rt, n);
@@ -480,9 +308,8 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
         xo[i] = WRaw<TYPE>::xoff(W, rt, n, g);
     }
 
-    // Q4_0 / Q5_0 / Q8_0 down: two accumulator sets, acc for even 32-blocks and acc2 for odd ones, each in
-    // its own unit (down only: with gate/up's two weight tiles per wave the second set spills, 394 -> 702 us)
-    constexpr bool DUAL = !SUPER && !GATEUP;
+    // Q4_0 / Q5_0 / Q8_0: two accumulator sets, acc for even 32-blocks and acc2 for odd ones, each in its own unit
+    constexpr bool DUAL = !SUPER;
     constexpr int TM2 = DUAL ? TM : 1, TN2 = DUAL ? TN : 1;
     v16f acc[TM][TN], acc2[TM2][TN2];
 #pragma unroll
@@ -503,7 +330,7 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         hdr[i] = make_uint4(0, 0, 0, 0);
-        dl[i] = RESCALE ? 1.0f : 0.0f;
+        dl[i] = 1.0f;
         dz[i] = false;
     }
 #pragma unroll
@@ -515,8 +342,8 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                                    min(HB, KB - h0 * HB));
     stage(h0);
 
-    // LDS byte offset of this lane's A chunk (hi/lo hl, sub-block j of the half-unit, K-half m) in pair tile 0
-    auto boff = [&](int hl, int j, int m) { return n * PB + (((16 * hl + 4 * j + 2 * g + m) ^ (n % CPP)) << 4); };
+    // LDS byte offset of this lane's A chunk (sub-block j of the half-unit, K-half m) in pair tile 0
+    auto boff = [&](int j, int m) { return n * PB + (((4 * j + 2 * g + m) ^ (n % CPP)) << 4); };
 
     auto half = [&](int h, auto parity, WRaw<TYPE>(&cur)[TM], WRaw<TYPE>(&nxt)[TM]) {
         constexpr bool ODD = decltype(parity)::value;
@@ -533,26 +360,7 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
         if (!active) return;
         const uint8_t* sa = sm.st[ODD].q + pg * TN * 32 * PB;
         if constexpr (SUPER) {
-            if constexpr (UNIT) {
-                if (!ODD) {  // into the super-block's weight units (rows 8 ii + 4 g .. of the wave's tiles)
-                    const float* rd = sm.rd + wave * 64 + 4 * g;
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) {
-                        hdr[i] = cur[i].cs;
-#pragma unroll
-                        for (int ii = 0; ii < 4; ++ii) {
-                            const float4 v = *reinterpret_cast<const float4*>(rd + 32 * i + 8 * ii);
-#pragma unroll
-                            for (int t = 0; t < TN; ++t) {
-                                acc[i][t][4 * ii] *= v.x;
-                                acc[i][t][4 * ii + 1] *= v.y;
-                                acc[i][t][4 * ii + 2] *= v.z;
-                                acc[i][t][4 * ii + 3] *= v.w;
-                            }
-                        }
-                    }
-                }
-            } else if (!ODD) {
+            if (!ODD) {
 #pragma unroll
                 for (int i = 0; i < TM; ++i) {
                     float d;
@@ -563,61 +371,47 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                         hdr[i] = cur[i].cs;  // the super-block's operand scales, for both halves
                         d = f16_to_f32(cur[i].hd & 0xFFFFu);
                     }
-                    if constexpr (RESCALE) {
-                        dz[i] = d == 0.0f;
-                        const float u = dz[i] ? 1.0f : d;  // the unit the min table divides by
-                        const float ratio = dl[i] * __builtin_amdgcn_rcpf(u);  // ~1 ulp
-                        dl[i] = u;
+                    dz[i] = d == 0.0f;
+                    const float u = dz[i] ? 1.0f : d;  // the unit the min table divides by
+                    const float ratio = dl[i] * __builtin_amdgcn_rcpf(u);  // ~1 ulp
+                    dl[i] = u;
 #pragma unroll
-                        for (int t = 0; t < TN; ++t)
+                    for (int t = 0; t < TN; ++t)
 #pragma unroll
-                            for (int r = 0; r < 16; ++r) acc[i][t][r] *= ratio;
-                    } else {
-                        (void)d;
-                    }
+                        for (int r = 0; r < 16; ++r) acc[i][t][r] *= ratio;
                 }
             }
             if constexpr (Q4K) if (ODD) {
                 // min term, once per super-block: acc += sum_j (dx_j sum q_j) (-dmin m_j / unit) on bf16
-                // 3-piece splits (the activation side in xm, the weight side from the min table); six of
-                // the nine piece products (all above 2^-24 relative) in three MFMAs, (MFMA, lane half) ->
-                // (activation piece, weight piece): (0,0) h.h (0,1) m.h (1,0) h.m (1,1) l.h (2,0) h.l (2,1) m.m.
-                // The down projection drops the third (h.l and m.m, ~2^-16 relative each): its hi-only
-                // activations already carry 2^-12, and nothing downstream re-quantizes.
+                // 3-piece splits (the activation side in xm, the weight side from the min table), four of
+                // the nine piece products in two MFMAs, (MFMA, lane half) -> (activation piece, weight
+                // piece): (0,0) h.h (0,1) m.h (1,0) h.m (1,1) l.h.  (h.l and m.m are ~2^-16 relative
+                // each: the hi-only activations already carry 2^-12, and nothing downstream re-quantizes.)
                 const uint16_t* xm = sm.st[1].xm + pbase * 8;
 #pragma unroll
                 for (int i = 0; i < TM; ++i) {
-                    const uint4 w1 = g ? cur[i].mn[0] : cur[i].mn[1], w2 = g ? cur[i].mn[1] : cur[i].mn[2];
-                    const b8 wm[3] = {__builtin_bit_cast(b8, cur[i].mn[0]), __builtin_bit_cast(b8, w1),
-                                      __builtin_bit_cast(b8, w2)};
+                    const uint4 w1 = g ? cur[i].mn[0] : cur[i].mn[1];
+                    const b8 wm[2] = {__builtin_bit_cast(b8, cur[i].mn[0]), __builtin_bit_cast(b8, w1)};
 #pragma unroll
                     for (int t = 0; t < TN; ++t) {
                         const int pr = 32 * t + n;
                         const b8 x0 = *reinterpret_cast<const b8*>(xm + (g ? 1 : 0) * BN * 8 + pr * 8);
                         const b8 x1 = *reinterpret_cast<const b8*>(xm + (g ? 2 : 0) * BN * 8 + pr * 8);
-                        if constexpr (UNIT) {
-                            acc[i][t] = mfma16b(wm[0], x0, acc[i][t]);
-                            acc[i][t] = mfma16b(wm[1], x1, acc[i][t]);
-                            acc[i][t] = mfma16b(wm[2], x0, acc[i][t]);
-                        } else {
-                            acc[i][t] = mfma16b(x0, wm[0], acc[i][t]);
-                            acc[i][t] = mfma16b(x1, wm[1], acc[i][t]);
-                        }
+                        acc[i][t] = mfma16b(x0, wm[0], acc[i][t]);
+                        acc[i][t] = mfma16b(x1, wm[1], acc[i][t]);
                     }
                 }
             }
             // 8 K-steps of 16 per half-unit (sub-block jj = st / 2, K-half m = st % 2), software
             // pipelined: while step st's 2 * TN * TM MFMAs run, the activation operands of step st + 1
             // are read from LDS and its weights converted (the schedule is pinned below)
-            h8 av[2][TN][HL];
+            h8 av[2][TN];
             h8 wv[2][TM];
             h2v c1[TM], c0[TM];
-            auto read_av = [&](int st, h8(&dst)[TN][HL]) {
+            auto read_av = [&](int st, h8(&dst)[TN]) {
 #pragma unroll
                 for (int t = 0; t < TN; ++t)
-#pragma unroll
-                    for (int hl = 0; hl < HL; ++hl)
-                        dst[t][hl] = *reinterpret_cast<const h8*>(sa + t * 32 * PB + boff(hl, st >> 1, st & 1));
+                    dst[t] = *reinterpret_cast<const h8*>(sa + t * 32 * PB + boff(st >> 1, st & 1));
             };
             auto convert = [&](int st, h8(&dst)[TM]) {
                 const int jj = st >> 1, m = st & 1;
@@ -629,7 +423,7 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                             // constants exact; the result rounds once, exact up to |sc * (q6 - 32)| <= 2048)
                             const int k = 8 * ODD + 2 * jj + g;
                             const uint32_t wsc = k < 4 ? hdr[i].x : (k < 8 ? hdr[i].y : (k < 12 ? hdr[i].z : hdr[i].w));
-                            const float scf = RESCALE && dz[i] ? 0.0f : (float)(int8_t)(uint8_t)(wsc >> (8 * (k & 3)));
+                            const float scf = dz[i] ? 0.0f : (float)(int8_t)(uint8_t)(wsc >> (8 * (k & 3)));
                             c1[i] = splat(scf * 0.25f);
                             c0[i] = splat(scf * -288.0f);
                         } else {
@@ -665,22 +459,8 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                     }
                 }
             };
-            // block-unit form: the lane's pair's unit ratio of a block, read from LDS one step ahead
-            float rxv[UNIT ? TN : 1];
-            const float* rxs = nullptr;
-            if constexpr (UNIT) rxs = sm.rx[ODD] + pbase + n;
-            auto read_rx1 = [&](int jj, int t) { rxv[t] = rxs[jj * BN + 32 * t]; };
-            auto read_rx = [&](int jj) {
-#pragma unroll
-                for (int t = 0; t < TN; ++t) read_rx1(jj, t);
-            };
-            auto rescale = [&](int i, int t) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][t][r] *= rxv[t];
-            };
             read_av(0, av[0]);
             convert(0, wv[0]);
-            if constexpr (UNIT) read_rx(0);
 #pragma unroll
             for (int st = 0; st < 2 * HB; ++st) {
                 const int b = st & 1;
@@ -689,95 +469,17 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                 // scheduling barriers), so their latency hides behind 2 * TN * TM MFMAs
                 if (st + 1 < 2 * HB) read_av(st + 1, av[b ^ 1]);
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (UNIT && TN == 2 && TM == 2) {
-                    // tiles k = (t, i) in order (0,0) (0,1) (1,0) (1,1); tile k's rescale into block jj's
-                    // units must fall between its last MFMA of block jj - 1 and its first of block jj:
-                    // pair tile 0's two go in block jj - 1's second step, after their own MFMAs there,
-                    // and pair tile 1's two in block jj's first step, before theirs, so every step
-                    // carries two rescales beside its four MFMAs (a half-unit's first block has its
-                    // ratios staged only at its own first step and takes all four there)
-                    const int jj = st >> 1;
-                    if (b == 0) {
-                        if (jj == 0) {
-                            rescale(0, 0);
-                            acc[0][0] = mfma16(wv[b][0], av[b][0][0], acc[0][0]);
-                            rescale(1, 0);
-                            acc[1][0] = mfma16(wv[b][1], av[b][0][0], acc[1][0]);
-                        } else {
-                            acc[0][0] = mfma16(wv[b][0], av[b][0][0], acc[0][0]);
-                            acc[1][0] = mfma16(wv[b][1], av[b][0][0], acc[1][0]);
-                        }
-                        rescale(0, 1);
-                        acc[0][1] = mfma16(wv[b][0], av[b][1][0], acc[0][1]);
-                        rescale(1, 1);
-                        acc[1][1] = mfma16(wv[b][1], av[b][1][0], acc[1][1]);
-                        if (jj + 1 < HB) read_rx1(jj + 1, 0);
-                        if (jj == 0) {
 #pragma unroll
-                            for (int k = 0; k < 4; ++k) {
-                                __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
-                                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                            }
-                        } else {
-                            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-                    } else {
-                        acc[0][0] = mfma16(wv[b][0], av[b][0][0], acc[0][0]);
-                        acc[1][0] = mfma16(wv[b][1], av[b][0][0], acc[1][0]);
-                        acc[0][1] = mfma16(wv[b][0], av[b][1][0], acc[0][1]);
-                        acc[1][1] = mfma16(wv[b][1], av[b][1][0], acc[1][1]);
-                        if (jj + 1 < HB) {
-                            rescale(0, 0);
-                            rescale(1, 0);
-                            read_rx1(jj + 1, 1);
-                            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
-                } else if (UNIT && b == 0) {
-                    // a block's first step: each tile moves into the block's units right before its
-                    // MFMA, so the MFMAs of the tiles before it run while the multiplies issue
+                for (int t = 0; t < TN; ++t)
 #pragma unroll
-                    for (int t = 0; t < TN; ++t)
-#pragma unroll
-                        for (int i = 0; i < TM; ++i) {
-                            rescale(i, t);
-                            acc[i][t] = mfma16(wv[b][i], av[b][t][0], acc[i][t]);
-                        }
-#pragma unroll
-                    for (int k = 0; k < TN * TM; ++k) {
-                        __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);  // VALU: one tile's rescale
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA: its product
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                } else {
-#pragma unroll
-                    for (int hl = 0; hl < HL; ++hl)
-#pragma unroll
-                        for (int t = 0; t < TN; ++t)
-#pragma unroll
-                            for (int i = 0; i < TM; ++i)
-                                acc[i][t] = UNIT ? mfma16(wv[b][i], av[b][t][hl], acc[i][t])
-                                                 : mfma16(av[b][t][hl], wv[b][i], acc[i][t]);
-                }
-                if (UNIT && !(TN == 2 && TM == 2) && b == 1 && st + 1 < 2 * HB) read_rx((st + 1) >> 1);
+                    for (int i = 0; i < TM; ++i) acc[i][t] = mfma16(av[b][t], wv[b][i], acc[i][t]);
                 if (st + 1 < 2 * HB) {
                     convert(st + 1, wv[b ^ 1]);  // VALU work spread between the MFMAs
-                    if (!UNIT || (b == 1 && !(TN == 2 && TM == 2)))
 #pragma unroll
-                        for (int k = 0; k < HL * TN * TM; ++k) {
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-                            __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
-                        }
+                    for (int k = 0; k < TN * TM; ++k) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+                        __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);  // VALU
+                    }
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -818,7 +520,7 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                 }
 #pragma unroll
                 for (int m = 0; m < 2; ++m) {
-                    h8 wv[TM], av[TN][HL];
+                    h8 wv[TM], av[TN];
 #pragma unroll
                     for (int i = 0; i < TM; ++i) {
                         if constexpr (TYPE == T_Q5_0) {
@@ -833,103 +535,18 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                     }
 #pragma unroll
                     for (int t = 0; t < TN; ++t)
-#pragma unroll
-                        for (int hl = 0; hl < HL; ++hl)
-                            av[t][hl] = *reinterpret_cast<const h8*>(sa + t * 32 * PB + boff(hl, j, m));
-#pragma unroll
-                    for (int hl = 0; hl < HL; ++hl)
-#pragma unroll
-                        for (int t = 0; t < TN; ++t)
-#pragma unroll
-                            for (int i = 0; i < TM; ++i) A[i][t] = mfma16(av[t][hl], wv[i], A[i][t]);
-                }
-            };
-            static_assert(HB % 2 == 0, "block pairs");
-            if constexpr (DUAL) {  // K % 128 == 0: every half-unit holds HB full blocks
-#pragma unroll
-                for (int j = 0; j < HB; j += 2) {
-                    block(j, acc, dl);
-                    block(j + 1, acc2, dl2);
-                }
-            } else if constexpr (!Q4K) {
-                // software pipelined as the Q4_K path: step st = (block st / 2, K-half st % 2); the next
-                // step's LDS reads and weight conversion go out around this step's MFMAs. At a block's
-                // first step each tile is rescaled into the block's unit right before its own hi MFMA,
-                // so the MFMAs of the tiles before it run while the multiplies issue.
-                h8 av[2][TN][HL];
-                h8 wv[2][TM];
-                h2v c1[TM], c0[TM];
-                float ratio[TM];
-                auto scales = [&](int j) {
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) {
-                        const float d = f16_to_f32(cur[i].d[j]);
-                        const bool z = d == 0.0f;
-                        const float u = z ? 1.0f : d;
-                        ratio[i] = dl[i] * __builtin_amdgcn_rcpf(u);  // ~1 ulp; units only need consistency
-                        dl[i] = u;
-                        c1[i] = splat(z ? 0.0f : k1);
-                        c0[i] = splat(z ? 0.0f : k0);
-                    }
-                };
-                auto read_av = [&](int st, h8(&dst)[TN][HL]) {
+                        av[t] = *reinterpret_cast<const h8*>(sa + t * 32 * PB + boff(j, m));
 #pragma unroll
                     for (int t = 0; t < TN; ++t)
 #pragma unroll
-                        for (int hl = 0; hl < HL; ++hl)
-                            dst[t][hl] = *reinterpret_cast<const h8*>(sa + t * 32 * PB + boff(hl, st >> 1, st & 1));
-                };
-                auto convert = [&](int st, h8(&dst)[TM]) {
-#pragma unroll
-                    for (int i = 0; i < TM; ++i) {
-                        const uint4 raw = cur[i].q[st >> 1];
-                        dst[i] = (st & 1) ? cvt8(raw.z, raw.w, mask, flip, c1[i], c0[i])
-                                          : cvt8(raw.x, raw.y, mask, flip, c1[i], c0[i]);
-                    }
-                };
-                scales(0);
-                read_av(0, av[0]);
-                convert(0, wv[0]);
-#pragma unroll
-                for (int st = 0; st < 2 * HB; ++st) {
-                    const int b = st & 1;
-                    if (st + 1 < 2 * HB) read_av(st + 1, av[b ^ 1]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if ((st & 1) == 0) {
-#pragma unroll
-                        for (int t = 0; t < TN; ++t)
-#pragma unroll
-                            for (int i = 0; i < TM; ++i) {
-#pragma unroll
-                                for (int r = 0; r < 16; ++r) acc[i][t][r] *= ratio[i];
-                                acc[i][t] = mfma16(av[b][t][0], wv[b][i], acc[i][t]);
-                            }
-#pragma unroll
-                        for (int hl = 1; hl < HL; ++hl)
-#pragma unroll
-                            for (int t = 0; t < TN; ++t)
-#pragma unroll
-                                for (int i = 0; i < TM; ++i) acc[i][t] = mfma16(av[b][t][hl], wv[b][i], acc[i][t]);
-#pragma unroll
-                        for (int k = 0; k < TN * TM; ++k) {
-                            __builtin_amdgcn_sched_group_barrier(0x002, 16, 0);  // VALU: one tile's rescale
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA: its hi product
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-                    } else {
-#pragma unroll
-                        for (int hl = 0; hl < HL; ++hl)
-#pragma unroll
-                            for (int t = 0; t < TN; ++t)
-#pragma unroll
-                                for (int i = 0; i < TM; ++i) acc[i][t] = mfma16(av[b][t][hl], wv[b][i], acc[i][t]);
-                    }
-                    if (st + 1 < 2 * HB) {
-                        if (!((st + 1) & 1)) scales((st + 1) >> 1);  // the next block's unit and operand constants
-                        convert(st + 1, wv[b ^ 1]);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
+                        for (int i = 0; i < TM; ++i) A[i][t] = mfma16(av[t], wv[i], A[i][t]);
                 }
+            };
+            static_assert(HB % 2 == 0, "block pairs");
+#pragma unroll
+            for (int j = 0; j < HB; j += 2) {  // K % 128 == 0: every half-unit holds HB full blocks
+                block(j, acc, dl);
+                block(j + 1, acc2, dl2);
             }
         }
     };
@@ -940,67 +557,8 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
     }
 
     // ------------------------------------------------------------ epilogue
-    if constexpr (UNIT) {
-        if (!active) return;
-        // Lane (n, g) holds pair 32 t + n and rows 8 (r / 4) + 4 g + r % 4 of the wave's gate and up tiles: back
-        // to natural units, h = act(gate) * up, and h's block of 32 rows (row tile rt0) split over the lanes of
-        // both halves.
-        const float* pe = sm.st[(h1 - 1) & 1].pe + pbase + n;
-        const float* ug = reinterpret_cast<const float*>(W0.mn + (size_t)e * W0.mn_es + ((size_t)rt0 * W0.nkb + W0.nkb - 1) * MN_SB + MN_U) + 4 * g;
-        const float* uu = reinterpret_cast<const float*>(W1.mn + (size_t)e * W1.mn_es + ((size_t)rt0 * W1.nkb + W1.nkb - 1) * MN_SB + MN_U) + 4 * g;
-#pragma unroll
-        for (int t = 0; t < TN; ++t) {
-            const float pv = pe[32 * t];
-            float v[16];
-#pragma unroll
-            for (int ii = 0; ii < 4; ++ii) {
-                const float4 a = *reinterpret_cast<const float4*>(ug + 8 * ii), b = *reinterpret_cast<const float4*>(uu + 8 * ii);
-                const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    v[4 * ii + c] = gated(acc[0][t][4 * ii + c] * (pv * av[c]), acc[1][t][4 * ii + c] * (pv * bv[c]), W0.act);
-            }
-            const int pr = pbase + 32 * t + n;
-            const size_t p = (size_t)(p0 + pr);
-            const bool valid = pr < cnt;
-            if (hf && valid) {
-                float* fd = hf + p * (size_t)hf_ld + rt0 * 32 + 4 * g;
-#pragma unroll
-                for (int ii = 0; ii < 4; ++ii)
-                    *reinterpret_cast<float4*>(fd + 8 * ii) = make_float4(v[4 * ii], v[4 * ii + 1], v[4 * ii + 2], v[4 * ii + 3]);
-            }
-            if (!hq.q) continue;
-            // Q8_0 of the block (quantize_row_q8_0): both halves' lanes hold the same scale and sum
-            float amax = 0.0f;
-#pragma unroll
-            for (int c = 0; c < 16; ++c) amax = fmaxf(amax, __builtin_fabsf(v[c]));
-            amax = fmaxf(amax, __shfl_xor(amax, 32));
-            const float d = amax / 127.0f;
-            const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
-            int s = 0;
-            uint32_t w[4];
-#pragma unroll
-            for (int c = 0; c < 16; ++c) {
-                float r = round_away(v[c] * id);
-                r = fminf(fmaxf(r, -127.0f), 127.0f);
-                const int q = (int)r;
-                s += q;
-                if ((c & 3) == 0) w[c >> 2] = 0;
-                w[c >> 2] |= ((uint32_t)q & 0xFFu) << (8 * (c & 3));
-            }
-            s += __shfl_xor(s, 32);
-            // word ii of half g is rows 8 ii + 4 g ..: exchange so half g stores rows 16 g .. 16 g + 15
-            const auto x0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
-            const auto x1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
-            if (valid) {
-                *reinterpret_cast<uint4*>(hq.q + p * (size_t)hq.K + rt0 * 32 + 16 * g) = make_uint4(x0[0], x0[1], x1[0], x1[1]);
-                if (g == 0)
-                    hq.s[p * (size_t)(hq.K / 32) + rt0] = make_float2(f16_to_f32(f32_to_f16_trunc(d)), (float)s);
-            }
-        }
-        return;
-    }
-    if (active) {  // back to natural units: the row's unit (RESCALE) and the token's exponent
+    if (!active) return;
+    {  // back to natural units: the row's unit and the token's exponent
         const float* pe = sm.st[(h1 - 1) & 1].pe + pbase;
 #pragma unroll
         for (int t = 0; t < TN; ++t)
@@ -1019,82 +577,17 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
                     }
             }
     }
-    if constexpr (GATEUP && !UNIT) {
-        // h = SiLU(g) * u in registers, written transposed to LDS: [pair][row of the workgroup]
-        constexpr int HLD = A_::RW * 32 + 4;              // h row stride (floats)
-        float* hs = reinterpret_cast<float*>(&sm.st[0]);  // [128 pairs][HLD], over both stage buffers
-        static_assert((size_t)BN * HLD * 4 <= 2 * sizeof(St), "epilogue buffer");
-        __syncthreads();  // every wave is done with the stage buffers
-        if (active) {
 #pragma unroll
-            for (int t = 0; t < TN; ++t)
+    for (int i = 0; i < TM; ++i) {
+        const int rt = rt0 + i;
+        if (rt >= W0.nrt) continue;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float gv = acc[0][t][r], uv = acc[1][t][r];
-                    const int pr = pbase + 32 * t + 8 * (r >> 2) + 4 * g + (r & 3);
-                    hs[pr * HLD + rw * 32 + n] = gated(gv, uv, W0.act);  // SwiGLU / GELU
-                }
-        }
-        __syncthreads();
-        // Q8_0 of h (quantize_row_q8_0 over the down projection's K = these rows), one thread per
-        // (pair, 32-row block = gate/up row tile)
-        for (int it = tid; it < A_::RW * BN; it += NTH) {
-            const int pr = it % BN, b = it / BN;
-            const int blk = rg * A_::RW + b;
-            if (pr >= cnt || blk >= W0.nrt) continue;
-            const size_t p = (size_t)(p0 + pr);
-            const float* hv = hs + pr * HLD + b * 32;
-            float v[32];
+        for (int t = 0; t < TN; ++t)
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const float4 f = *reinterpret_cast<const float4*>(hv + 4 * c);
-                v[4 * c] = f.x;
-                v[4 * c + 1] = f.y;
-                v[4 * c + 2] = f.z;
-                v[4 * c + 3] = f.w;
+            for (int r = 0; r < 16; ++r) {
+                const int pr = pbase + 32 * t + 8 * (r >> 2) + 4 * g + (r & 3);
+                if (pr < cnt) y[(size_t)kp * ystride + (size_t)(p0 + pr) * W0.rows + rt * 32 + n] = acc[i][t][r];
             }
-            if (hf) {
-                float* fd = hf + p * (size_t)hf_ld + blk * 32;
-#pragma unroll
-                for (int c = 0; c < 8; ++c)
-                    *reinterpret_cast<float4*>(fd + 4 * c) = make_float4(v[4 * c], v[4 * c + 1], v[4 * c + 2], v[4 * c + 3]);
-            }
-            if (!hq.q) continue;
-            float amax = 0.0f;
-#pragma unroll
-            for (int c = 0; c < 32; ++c) amax = fmaxf(amax, __builtin_fabsf(v[c]));
-            const float d = amax / 127.0f;
-            const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
-            int s = 0;
-            uint32_t w[8];
-#pragma unroll
-            for (int c = 0; c < 32; ++c) {
-                float r = round_away(v[c] * id);
-                r = fminf(fmaxf(r, -127.0f), 127.0f);
-                const int q = (int)r;
-                s += q;
-                if ((c & 3) == 0) w[c >> 2] = 0;
-                w[c >> 2] |= ((uint32_t)q & 0xFFu) << (8 * (c & 3));
-            }
-            uint4* qd = reinterpret_cast<uint4*>(hq.q + p * (size_t)hq.K + blk * 32);
-            qd[0] = make_uint4(w[0], w[1], w[2], w[3]);
-            qd[1] = make_uint4(w[4], w[5], w[6], w[7]);
-            hq.s[p * (size_t)(hq.K / 32) + blk] = make_float2(f16_to_f32(f32_to_f16_trunc(d)), (float)s);
-        }
-    } else if constexpr (!GATEUP) {
-        if (!active) return;
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            const int rt = rt0 + i;
-            if (rt >= W0.nrt) continue;
-#pragma unroll
-            for (int t = 0; t < TN; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int pr = pbase + 32 * t + 8 * (r >> 2) + 4 * g + (r & 3);
-                    if (pr < cnt) y[(size_t)kp * ystride + (size_t)(p0 + pr) * W0.rows + rt * 32 + n] = acc[i][t][r];
-                }
-        }
     }
 }
 
@@ -1106,8 +599,7 @@ k_wgemm(QMat W0, QMat W1, ActH in, Groups grp, int R, int n_items, int RC, ActQ8
 // Also the GEMM's A-operand scale of each sub-block J (fp16, exact): the weight fragment holds 1024 + v
 // with v = q for Q5_K and Q4_K low nibbles, v = 16 q for Q4_K high nibbles, and s1 (1024 + v) - 1024 s1 =
 // sc_J q in one fused fp16 fma, with s1 = sc_J (sc_J / 16 for high nibbles), zero where d is zero.
-// Converting the 6-bit scales in the kernel cost ~90 VALU instructions per super-block and wave of the
-// gate/up GEMM.
+// Converting the 6-bit scales in the kernel cost ~90 VALU instructions per super-block and wave.
 __global__ void __launch_bounds__(256) k_min_table(QMat m, uint8_t* mn) {
     const size_t n = (size_t)m.n_mats * m.nrt * m.nkb * 32;
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -1139,14 +631,6 @@ __global__ void __launch_bounds__(256) k_min_table(QMat m, uint8_t* mn) {
     for (int c = 0; c < 3; ++c)
         *reinterpret_cast<uint4*>(base + c * 512) = make_uint4(pw[c][0], pw[c][1], pw[c][2], pw[c][3]);
     *reinterpret_cast<uint4*>(base + MN_CS) = make_uint4(cw[0], cw[1], cw[2], cw[3]);
-    float up = 1.0f;  // the previous super-block's unit (1 before the first)
-    if (t % m.nkb) {
-        const float dp = f16_to_f32(*reinterpret_cast<const uint32_t*>(m.sc + ((t - 1) * 32 + row) * 16) & 0xFFFFu);
-        up = dp == 0.0f ? 1.0f : dp;
-    }
-    float* ru = reinterpret_cast<float*>(mn + t * MN_SB + MN_RD) + row;
-    ru[0] = up / u;
-    ru[(MN_U - MN_RD) / 4] = u;
 }
 
 void launch_min_table(const QMat& m, uint8_t* mn, hipStream_t st) {
@@ -1154,52 +638,12 @@ void launch_min_table(const QMat& m, uint8_t* mn, hipStream_t st) {
     hipLaunchKernelGGL(k_min_table, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m, mn);
 }
 
-// Workgroup shape: waves, row tiles and pair tiles per wave, pairs per
-// workgroup (BN) and workgroups per CU (WGS; the registers are budgeted for
-// WGS * GW / 4 waves per SIMD).  Gate/up stages 64 pairs (hi and lo, 72 KB of
-// LDS) and the hi-only down GEMM 128 pairs (78 KB), so two workgroups share a
-// CU and one's staging waits overlap the other's matrix-core work.
-#ifndef JX_GEMM_GU_GW
-#define JX_GEMM_GU_GW 4
-#endif
-#ifndef JX_GEMM_GU_TN
-#define JX_GEMM_GU_TN 2
-#endif
-#ifndef JX_GEMM_GU_WGS
-#define JX_GEMM_GU_WGS 2
-#endif
-#ifndef JX_GEMM_GU_BN
-#define JX_GEMM_GU_BN 64
-#endif
-#ifndef JX_DOWN_GW
-#define JX_DOWN_GW 4
-#endif
-#ifndef JX_DOWN_TM
-#define JX_DOWN_TM 1
-#endif
-#ifndef JX_DOWN_TN
-#define JX_DOWN_TN 4
-#endif
-#ifndef JX_DOWN_WGS
-#define JX_DOWN_WGS 2
-#endif
-// Row groups per band of the workgroup order (0: all of them).  Gate/up: 8
-// (with the XCD-balanced item mapping, Qwen3-shaped 2048 tokens 384 -> 354 us,
-// the other shapes unchanged; 2 and 16 slower); down: 4 (2 and 8 slower).
-#ifndef JX_GEMM_GU_RC
-#define JX_GEMM_GU_RC 8
-#endif
-#ifndef JX_DOWN_RC
-#define JX_DOWN_RC 4
-#endif
-template <int TYPE, bool GATEUP>
+// Workgroup shape: waves, row tiles and pair tiles per wave, pairs per workgroup (BN) and waves per SIMD
+// the registers are budgeted for.  78 KB of LDS per workgroup, so two share a CU and one's staging waits
+// overlap the other's matrix-core work.  RC row groups per band of the workgroup order (2 and 8 slower).
+template <int TYPE>
 struct Shape {
-    static constexpr int GW = GATEUP ? JX_GEMM_GU_GW : JX_DOWN_GW;
-    static constexpr int TM = GATEUP ? 2 : JX_DOWN_TM;
-    static constexpr int TN = GATEUP ? JX_GEMM_GU_TN : JX_DOWN_TN;
-    static constexpr int WPE = (GATEUP ? JX_GEMM_GU_WGS : JX_DOWN_WGS) * GW / 4;
-    static constexpr int BN = GATEUP ? JX_GEMM_GU_BN : MFMA_BN;
-    static constexpr int RC = GATEUP ? JX_GEMM_GU_RC : JX_DOWN_RC;
+    static constexpr int GW = 4, TM = 1, TN = 4, WPE = 2, BN = MFMA_BN, RC = 4;
 };
 
 // Down over fewer pairs per expert (batched decode, where fp32-activation downs have no GEMV form on the
@@ -1212,48 +656,27 @@ struct Shape {
 template <int TYPE>
 struct ShapeSmallDown {
     static constexpr int WPE = TYPE == T_Q6_K ? 4 : TYPE == T_Q5_0 ? 2 : 3;
-    static constexpr int GW = 4, TM = 1, TN = 2, BN = 64, RC = JX_DOWN_RC;
+    static constexpr int GW = 4, TM = 1, TN = 2, BN = 64, RC = 4;
 };
 
-template <int TYPE, bool GATEUP, typename S = Shape<TYPE, GATEUP>>
-static void launch_t(const QMat& w0, const QMat& w1, const ActH& in, const Groups& grp, int tiles_ub, const ActQ8& hq,
-                     float* hf, int hf_ld, float* y, hipStream_t st, int KS = 1, size_t ystride = 0) {
-    constexpr int rows_per_wg = Arr<GATEUP, S::GW, S::TM, S::TN, S::BN>::WROWS;  // row tiles of each matrix per workgroup
-    const int R = (w0.nrt + rows_per_wg - 1) / rows_per_wg;
+template <int TYPE, typename S>
+static void launch_t(const QMat& dn, const ActH& in, const Groups& grp, int tiles_ub, float* y, hipStream_t st, int KS,
+                     size_t ystride) {
+    constexpr int rows_per_wg = Arr<S::GW, S::TM, S::TN, S::BN>::WROWS;  // row tiles per workgroup
+    const int R = (dn.nrt + rows_per_wg - 1) / rows_per_wg;
     const int n_items = R * tiles_ub * (MFMA_BN / S::BN);
     if (n_items <= 0) return;
-    const int RC = S::RC > 0 ? std::min(S::RC, R) : R;
-    const int grid = n_items * KS;
-    hipLaunchKernelGGL((k_wgemm<TYPE, GATEUP, S::GW, S::TM, S::TN, S::WPE, S::BN>), dim3(grid), dim3(S::GW * 64), 0, st,
-                       w0, w1, in, grp, R, n_items, RC, hq, hf, hf_ld, y, KS, ystride);
+    hipLaunchKernelGGL((k_wgemm<TYPE, S::GW, S::TM, S::TN, S::WPE, S::BN>), dim3(n_items * KS), dim3(S::GW * 64), 0, st,
+                       dn, in, grp, R, n_items, std::min(S::RC, R), y, KS, ystride);
 }
-
-void launch_mfma_gateup(const QMat& g, const QMat& u, const ActH& xin, const Groups& grp, int tiles_ub,
-                        const ActQ8& hq, float* hf, hipStream_t st) {
-    const int hf_ld = ((g.rows + 255) / 256) * 256;
-    // Q4_K reads the block-unit form, the others the hi/lo form (the caller allocates the forms its
-    // matrices need; a missing one is a caller bug, and nothing is launched on null pointers)
-    const bool unit = g.type == T_Q4_K || g.type == T_Q5_K;
-    if (unit ? !(xin.q16 && xin.rx && xin.pu && xin.xu) : !(xin.hl && xin.pe)) return;
-    switch (g.type) {
-        case T_Q4_0: launch_t<T_Q4_0, true>(g, u, xin, grp, tiles_ub, hq, hf, hf_ld, nullptr, st); break;
-        case T_Q8_0: launch_t<T_Q8_0, true>(g, u, xin, grp, tiles_ub, hq, hf, hf_ld, nullptr, st); break;
-        case T_Q4_K: launch_t<T_Q4_K, true>(g, u, xin, grp, tiles_ub, hq, hf, hf_ld, nullptr, st); break;
-        case T_Q5_K: launch_t<T_Q5_K, true>(g, u, xin, grp, tiles_ub, hq, hf, hf_ld, nullptr, st); break;
-        default: break;  // Q5_0 / Q6_K gate/up: GEMV only (gemm_gateup_ok)
-    }
-}
-
-bool gemm_gateup_ok(int type) { return type == T_Q4_0 || type == T_Q8_0 || type == T_Q4_K || type == T_Q5_K; }
 
 int mfma_down_ksplit(int K) { return K >= MFMA_DOWN_KSPLIT_MIN_K ? 2 : 1; }
 
 template <int TYPE>
 static void down_t(const QMat& dn, const ActH& hin, const Groups& grp, int tiles_ub, float* y, hipStream_t st, int KS,
                    size_t ystride, bool small) {
-    const ActQ8 none{};
-    if (small) launch_t<TYPE, false, ShapeSmallDown<TYPE>>(dn, dn, hin, grp, tiles_ub, none, nullptr, 0, y, st, KS, ystride);
-    else launch_t<TYPE, false>(dn, dn, hin, grp, tiles_ub, none, nullptr, 0, y, st, KS, ystride);
+    if (small) launch_t<TYPE, ShapeSmallDown<TYPE>>(dn, hin, grp, tiles_ub, y, st, KS, ystride);
+    else launch_t<TYPE, Shape<TYPE>>(dn, hin, grp, tiles_ub, y, st, KS, ystride);
 }
 
 void launch_mfma_down(const QMat& dn, const ActH& hin, const Groups& grp, int tiles_ub, float* y, hipStream_t st,

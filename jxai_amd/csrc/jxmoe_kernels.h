@@ -22,8 +22,7 @@ namespace jx {
 //         sc  [e][rt][sb][32 rows][16 B] = the 16 int8 sub-block scales
 //         ex  [e][rt][sb][32] fp16 d
 // Byte totals of qs+sc(+ex) equal the GGUF tensor (18/34/144/22/176/210 B per block).
-// QMat::mn bytes per (row tile, super-block); offsets of the scales, the unit ratios and the units
-constexpr int MN_SB = 2304, MN_CS = 1536, MN_RD = 2048, MN_U = 2176;
+constexpr int MN_SB = 2048, MN_CS = 1536;  // QMat::mn bytes per (row tile, super-block); scales offset
 
 struct QMat {
     int type = 0;
@@ -44,14 +43,23 @@ struct QMat {
     const uint8_t* ex = nullptr;
     size_t ex_es = 0;
     const uint8_t* pad_ex = nullptr;
-    // Q4_K / Q5_K table for the matrix-core GEMMs (launch_min_table; null for other types
-    // and for matrices only the GEMVs read): per (expert, row tile, super-block) MN_SB
+    // Q4_K / Q5_K table for the down GEMM (launch_min_table; null for other types
+    // and for matrices it does not read): per (expert, row tile, super-block) MN_SB
     // bytes, 3 x [32 rows][16 B] = the bf16 pieces (hi, mid, lo) of -dmin * m_j / u for
     // the 8 sub-blocks j, u = d (1 where d is zero), then at MN_CS [32 rows][16 B] = the
-    // fp16 A-operand scales s1 of the 8 sub-blocks, at MN_RD [32 rows] fp32 u(s-1) / u(s) of super-block s
-    // (u(-1) = 1) and at MN_U [32 rows] fp32 u(s).
+    // fp16 operand scales s1 of the 8 sub-blocks.
     const uint8_t* mn = nullptr;
     size_t mn_es = 0;  // per-expert stride (bytes)
+    // FP6 form for the gate/up GEMM (launch_g6_tables; Q4_0 / Q4_K / Q5_K gate and up matrices): per (expert,
+    // row tile, 32-block) 1024 B = [32 rows][16 B] code words 0..3, [32 rows][8 B] code words 4, 5, [32 rows][8 B]
+    // the block scale's bf16 pieces (hi | mid << 16, lo).  Code of value v (q - 8 / q / q - 16): sign << 5 | |v|,
+    // element i at bit 6 i.
+    const uint8_t* g6 = nullptr;
+    size_t g6_es = 0;
+    // Q4_K / Q5_K beside it: per (expert, row tile, super-block) G6M_SB bytes = 3 x [32 rows][16 B], the bf16
+    // pieces (hi, mid, lo) of the 8 sub-blocks' factors of dx * sum(q): -dmin m_j (Q5_K: + 16 d sc_j).
+    const uint8_t* g6m = nullptr;
+    size_t g6m_es = 0;
     // Gated activation applied to this matrix's outputs when it is the gate of
     // a gate/up pair (ACT_SILU or ACT_GELU_TANH); unused otherwise.
     int act = 0;
@@ -61,6 +69,8 @@ struct QMat {
     int valid_rows = 0;
 };
 constexpr size_t QMAT_PAD = 8192;
+constexpr int G6M_SB = 1536;
+inline bool g6_type(int t) { return t == T_Q4_0 || t == T_Q4_K || t == T_Q5_K; }
 
 // Q8_0 activations on the device: q [rows][K] int8, s [rows][K/32] = (fp16-truncated
 // scale as fp32, sum of the 32 quants as fp32).
@@ -82,22 +92,18 @@ struct ActQ8 {
 //   xm [rows][KU][3][8]  per 256-element unit: bf16 pieces (hi, mid, lo) of
 //                        dx * sum(q) (fp32 rows: the block sum) times 2^-E for its
 //                        8 blocks (Q4_K min term)
-// and, for the Q4_K gate/up GEMM, the block-unit form (each form is written
-// where its pointers are set):
-//   q16 [rows][K]        the quants q as fp16 (exact)
-//   rx [rows][K/32]      u(b-1) / u(b) per 32-block b, where the unit u(b) is the
-//                        block's scale dx, the previous unit where dx is zero, and
-//                        1 before the first nonzero scale (rx = 1 for block 0)
-//   pu [rows][KH]        u of the last block of each half-unit
-//   xu [rows][KU][3][8]  as xm, of dx * sum(q) / u(8s + 3) for super-block s
+// and, for the FP6 gate/up GEMM (each form is written where its pointers are set):
+//   q6 [rows][KH][256 B]  the quant is sign * (16 a + b): the a's (part 0) and the b's (part 1) as 32 FP6
+//                        codes (sign << 5 | digit, element i at bit 6 i) and the block scale's bf16 pieces,
+//                        dx = p0 + p1: (p, p, p, 0) with p = p0 in part 0 and p1 in part 1.  Per half-unit:
+//                        [4 blocks][2 parts][16 B] code words 0..3, [4][2][8 B] words 4, 5, [4][2][8 B] pieces
+//   x6 [rows][KU][3][8]  bf16 pieces (hi, mid, lo) of dx * sum(q) of the 8 blocks of each 256 (Q4_K / Q5_K)
 struct ActH {
     uint16_t* hl = nullptr;
     float* pe = nullptr;
     uint16_t* xm = nullptr;
-    uint16_t* q16 = nullptr;
-    float* rx = nullptr;
-    float* pu = nullptr;
-    uint16_t* xu = nullptr;
+    uint8_t* q6 = nullptr;
+    uint16_t* x6 = nullptr;
     int K = 0;
     int KH = 0;  // K / 128
     int KU = 0;  // ceil(K / 256)
@@ -253,9 +259,13 @@ bool gemv_down_f16_fits(int type, int K);
 void launch_gemv_down_f16(const QMat& dn, const ActH& hh, const Groups& grp, int slots, float* y, hipStream_t st);
 // Prefill regime: matrix-core grouped GEMMs over the dispatch tile table.
 // gate/up writes SwiGLU(h) as Q8_0 (hq.q != null; the down GEMM takes it after
-// launch_q8_to_acth) and/or fp32 (hf != null).
-void launch_mfma_gateup(const QMat& g, const QMat& u, const ActH& xin, const Groups& grp, int tiles_ub,
+// launch_q8_to_acth) and/or fp32 (hf != null).  Q8_0 weights read x's Q8_0 form xq, the
+// others its FP6 form xin.
+void launch_mfma_gateup(const QMat& g, const QMat& u, const ActH& xin, const ActQ8& xq, const Groups& grp, int tiles_ub,
                         const ActQ8& hq, float* hf, hipStream_t st);
+// Fill m.g6 (n_mats * nrt * cols / 32 * 1024 bytes) and, K-quants, m.g6m (n_mats * nrt * nkb * G6M_SB bytes;
+// null otherwise) from a repacked matrix of a g6_type (cols % 32 == 0).
+void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, hipStream_t st);
 // KS > 1: the K range split over KS workgroups per item (whole super-blocks each), part q of the
 // output at y + q * ystride (the combine adds the parts in order).  small: few pairs per expert (the
 // 64-pair tile form at more workgroups per CU).
@@ -271,8 +281,8 @@ constexpr int MFMA_DOWN_SMALL_MAX_PPE = 256;
 // 155 -> 133 us; at K 768 - 1408 the per-workgroup overhead makes it slower).
 constexpr int MFMA_DOWN_KSPLIT_MIN_K = 8192;
 int mfma_down_ksplit(int K);
-// Weight types the matrix-core gate/up GEMM takes (Q5_0 has no Q8_0-activation form; Q6_K's sc * q
-// operand is not exact in fp16, and gate/up products must be: h is re-quantized).
+// Weight types the matrix-core gate/up GEMM takes (Q5_0 has no Q8_0-activation form, and Q6_K's 16-element
+// sub-blocks no exact 32-block product; gate/up products must be exact: h is re-quantized).
 bool gemm_gateup_ok(int type);
 // Fill m.mn (m.n_mats * m.nrt * m.nkb * MN_SB bytes) from a repacked Q4_K or Q5_K matrix.
 void launch_min_table(const QMat& m, uint8_t* mn, hipStream_t st);
@@ -366,9 +376,10 @@ void launch_quantize_q8(const float* x, int rows, int K, ActQ8 out, hipStream_t 
 // dst[r][0 .. kpad) = x[r][0 .. n) then zeros, for rows r (x rows of n floats).
 void launch_copy_pad(const float* x, int n, int kpad, float* dst, hipStream_t st, int rows = 1);
 
-// Matrix-core form of existing Q8_0 activations (int8 quants + (scale, sum)).
-// lo = false writes only the fp16 hi halves (the down GEMM's operand).
-void launch_q8_to_acth(const ActQ8& in, int rows, ActH out, hipStream_t st, bool lo = true);
+// Matrix-core form of existing Q8_0 activations (int8 quants + (scale, sum)), the down GEMM's operand.
+void launch_q8_to_acth(const ActQ8& in, int rows, ActH out, hipStream_t st);
+// Their FP6 form (out.q6, and out.x6 unless null), the gate/up GEMM's operand.
+void launch_q8_to_q6(const ActQ8& in, int rows, ActH out, hipStream_t st);
 // Matrix-core form (hi only) of fp32 activation rows [rows][ld] (out.K % 128 == 0, columns up to
 // out.K zero-padded).
 void launch_f32_to_acth(const float* h, int ld, int rows, ActH out, hipStream_t st);

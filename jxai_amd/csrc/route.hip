@@ -25,13 +25,10 @@ __device__ __forceinline__ int quant_block(float v, int l32, bool ok, const ActQ
     return q;
 }
 
-// Matrix-core form (ActH) of one activation row from its Q8_0 quants q[K] and
-// (scale, sum) per 32-block, written by the NTH threads of one block.  One
-// exponent per row: E = exponent(max block scale of the row) - 7, so every
+// Matrix-core form (ActH) of Q8_0 rows, the down GEMM's operand: one
+// exponent per row, E = exponent(max block scale of the row) - 7, so every
 // dx * q * 2^-E (exact in fp32: an 11-bit scale times |q| <= 127) is below
-// 2^15 and splits into fp16 hi + lo exactly (a block whose scale is 2^21
-// times smaller than the row's largest loses bits of lo in fp16's subnormal
-// range: at most 2^-25 absolute, 2^-40 of the row's largest value).  The Q4_K
+// 2^15 and rounds to fp16 once.  The K-quant
 // min-term values dx * sum(q) are stored times 2^-E as well; pe holds 2^E
 // for every half-unit of the row.
 // Row exponent of the matrix-core form from the row's largest block scale M.
@@ -51,80 +48,60 @@ __device__ __forceinline__ void store_pieces3(uint16_t* xm, float X) {
     xm[16] = (uint16_t)(__float_as_uint(r2) >> 16);
 }
 
-// Unit of the block-unit form after block b of a row with block scales
-// sc[0..]: the last nonzero scale at or before b, 1 if there is none.
-__device__ __forceinline__ float block_unit(const float2* sc, int b) {
-    for (; b >= 0; --b) {
-        const float d = sc[b].x;
-        if (d != 0.0f) return d;
+// The FP6 form of one 32-block (ActH::q6, and its min-term pieces ActH::x6): quants w[8] (four signed bytes a
+// word) of block b with (scale, sum) sb.
+__device__ __forceinline__ void write_q6_block(const uint32_t (&w)[8], float2 sb, const ActH& o, size_t row, int b) {
+    uint32_t hi[6] = {0, 0, 0, 0, 0, 0}, lo[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        const int q = (int)(int8_t)(w[i >> 2] >> (8 * (i & 3)));
+        const uint32_t m = (uint32_t)(q < 0 ? -q : q), s = q < 0 ? 32u : 0u;
+        const uint32_t a = s | (m >> 4), c = s | (m & 15u);
+        const int at = (6 * i) / 32, sh = (6 * i) % 32;
+        hi[at] |= a << sh;
+        lo[at] |= c << sh;
+        if (sh > 26) {
+            hi[at + 1] |= a >> (32 - sh);
+            lo[at + 1] |= c >> (32 - sh);
+        }
     }
-    return 1.0f;
+    const uint32_t p0 = __float_as_uint(sb.x) >> 16;                                           // 8 of the 11 bits
+    const uint32_t p1 = __float_as_uint(sb.x - __uint_as_float(p0 << 16)) >> 16;               // the rest, exact
+    uint8_t* d = o.q6 + row * (size_t)o.K * 2 + (b >> 2) * 256;
+    const int j = b & 3;
+    *reinterpret_cast<uint4*>(d + j * 32) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+    *reinterpret_cast<uint4*>(d + j * 32 + 16) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    *reinterpret_cast<uint4*>(d + 128 + j * 16) = make_uint4(hi[4], hi[5], lo[4], lo[5]);
+    *reinterpret_cast<uint4*>(d + 192 + j * 16) = make_uint4(p0 | p0 << 16, p0, p1 | p1 << 16, p1);
+    if (o.x6) store_pieces3(o.x6 + row * (size_t)o.KU * 24 + (b / 8) * 24 + (b % 8), sb.x * sb.y);  // product exact
 }
 
-// Elements 8c .. 8c+7 of one row (all in one 32-block): for the hi/lo form
-// one 16-byte store each of hi and lo, plus the row's pe entry and the
-// block's min-term pieces when the chunk opens them; for the block-unit form
-// the chunk's 8 quants as fp16, plus the block's unit ratio and min-term
-// pieces and the half-unit's unit when the chunk opens them.
-// qq: the chunk's 8 quants, sb: its block's (scale, sum), sr: the row's
-// (scale, sum) of every block.
-__device__ __forceinline__ void acth_chunk_v(uint2 qq, float2 sb, const float2* sr, int K, const ActH& o, size_t row,
-                                             int c, int E, bool lo) {
+// Elements 8c .. 8c+7 of one row (all in one 32-block): one 16-byte store, plus the row's pe entry
+// and the block's min-term pieces when the chunk opens them.
+// qq: the chunk's 8 quants, sb: its block's (scale, sum).
+__device__ __forceinline__ void acth_chunk_v(uint2 qq, float2 sb, int K, const ActH& o, size_t row, int c, int E) {
     const int KH = K / 128;
     const int i = 8 * c, b = i >> 5, hh = i >> 7;
-    if (o.q16) {
-        // a block whose fp16 scale is zero (an underflow leaves nonzero quants) contributes nothing:
-        // its quants are written as zeros, since the block keeps the previous block's unit
-        if (sb.x == 0.0f) qq = make_uint2(0u, 0u);
-        uint32_t w[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const uint32_t word = u < 2 ? qq.x : qq.y;
-            const _Float16 h0 = (_Float16)(float)(int8_t)(word >> (16 * (u & 1)));
-            const _Float16 h1 = (_Float16)(float)(int8_t)(word >> (16 * (u & 1) + 8));
-            w[u] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-        }
-        *reinterpret_cast<uint4*>(o.q16 + row * (size_t)K + i) = make_uint4(w[0], w[1], w[2], w[3]);
-        if ((i & 31) == 0) {
-            const int KB = K / 32;
-            o.rx[row * (size_t)KB + b] = (b > 0 && sb.x != 0.0f) ? block_unit(sr, b - 1) / sb.x : 1.0f;
-            const float uref = block_unit(sr, min((b & ~7) + 3, KB - 1));
-            store_pieces3(o.xu + row * (size_t)o.KU * 24 + (b / 8) * 24 + (b % 8), sb.x * sb.y / uref);
-        }
-        if ((i & 127) == 0) o.pu[row * (size_t)KH + hh] = block_unit(sr, 4 * hh + 3);
-    }
-    if (!o.hl) return;
     const float dn = __uint_as_float((uint32_t)(127 - E) << 23), up = __uint_as_float((uint32_t)(127 + E) << 23);
     const float s = sb.x * dn;  // exact: power-of-two scaling
-    uint32_t hw[4], lw[4];
+    uint32_t hw[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const uint32_t word = u < 2 ? qq.x : qq.y;
         const int q0 = (int)(int8_t)(word >> (16 * (u & 1))), q1 = (int)(int8_t)(word >> (16 * (u & 1) + 8));
-        const float v0 = s * (float)q0, v1 = s * (float)q1;  // exact: 11-bit scale x |q| <= 127
-        const _Float16 h0 = (_Float16)v0, h1 = (_Float16)v1;
-        const _Float16 l0 = (_Float16)(v0 - (float)h0), l1 = (_Float16)(v1 - (float)h1);
+        const _Float16 h0 = (_Float16)(s * (float)q0), h1 = (_Float16)(s * (float)q1);  // products exact
         hw[u] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-        lw[u] = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
     }
-    uint16_t* hl = o.hl + row * (size_t)KH * 256 + hh * 256 + (i & 127);
-    *reinterpret_cast<uint4*>(hl) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-    if (lo) *reinterpret_cast<uint4*>(hl + 128) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+    *reinterpret_cast<uint4*>(o.hl + row * (size_t)KH * 256 + hh * 256 + (i & 127)) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
     if ((i & 127) == 0) o.pe[row * (size_t)KH + hh] = up;
     if ((i & 31) == 0)  // exact: 11-bit scale x |sum| < 2^12, times 2^-E
         store_pieces3(o.xm + row * (size_t)o.KU * 24 + (b / 8) * 24 + (b % 8), sb.x * sb.y * dn);
 }
 
-__device__ __forceinline__ void acth_chunk(const int8_t* q, const float2* sc, int K, const ActH& o, size_t row, int c,
-                                           int E, bool lo) {
-    acth_chunk_v(*reinterpret_cast<const uint2*>(q + 8 * c), sc[c >> 2], sc, K, o, row, c, E, lo);
-}
-
 // One row by one wave (all 64 lanes): the row exponent from a wave maximum of
 // the block scales, then four chunks per lane per pass with every load issued
 // before the first store.
-__device__ void write_acth_row(const int8_t* q, const float2* sc, int K, const ActH& o, size_t row, int lane,
-                               bool lo = true) {
+__device__ void write_acth_row(const int8_t* q, const float2* sc, int K, const ActH& o, size_t row, int lane) {
     const int KB = K / 32;
     float M = 0.0f;
     for (int b = lane; b < KB; b += 64) M = fmaxf(M, sc[b].x);
@@ -144,7 +121,7 @@ __device__ void write_acth_row(const int8_t* q, const float2* sc, int K, const A
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (c0 + u * 64 < nc) acth_chunk_v(qq[u], sb[u], sc, K, o, row, c0 + u * 64, E, lo);
+            if (c0 + u * 64 < nc) acth_chunk_v(qq[u], sb[u], K, o, row, c0 + u * 64, E);
     }
 }
 
@@ -193,8 +170,7 @@ constexpr int RT_TMAX = JX_RT_TMAX;
 constexpr size_t RT_LDS_TARGET = JX_RT_LDS_KB * 1024;  // two blocks per CU
 
 static size_t route_lds(int T, int d, int E) {
-    return (size_t)T * 16 * rs_stride(d) * sizeof(float) + (size_t)T * d + (size_t)T * (d / 32) * sizeof(float2) +
-           (size_t)T * E * sizeof(float);
+    return ((size_t)T * 16 * rs_stride(d) + (size_t)T * E) * sizeof(float);
 }
 
 struct RouteShape {
@@ -223,15 +199,12 @@ __global__ void __launch_bounds__(RT_THREADS) k_route(RouteArgs a, int nsplit, i
     extern __shared__ __align__(16) float lds[];
     __shared__ int sel[T][MAX_K];
     __shared__ float shl[T];
-    __shared__ float rmax[T];
     const int d = a.d, E = a.E, S = rs_stride(d), RS = 16 * S, KB = d / 32;
     const int split = blockIdx.x % nsplit;
     const int t0 = (blockIdx.x / nsplit) * T, nt = min(T, a.n - t0);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x;
     float* xs = lds;                                       // [T][16][S] chain-major rows
-    int8_t* qs = reinterpret_cast<int8_t*>(xs + T * RS);   // [T][d] quants
-    float2* ss = reinterpret_cast<float2*>(qs + T * d);    // [T][KB] (scale, sum)
-    float* lg = reinterpret_cast<float*>(ss + T * KB);     // [T][E] logits
+    float* lg = xs + T * RS;                               // [T][E] logits
     // every selection slot holds a valid expert even if NaN logits break the ranking
     for (int i = tid; i < T * MAX_K; i += RT_THREADS) sel[i / MAX_K][i % MAX_K] = i % MAX_K;
 
@@ -293,26 +266,7 @@ __global__ void __launch_bounds__(RT_THREADS) k_route(RouteArgs a, int nsplit, i
             gq[0] = w0;
             gq[1] = w1;
             a.xq.s[(size_t)(t0 + t) * KB + b] = sv;
-            uint4* lq = reinterpret_cast<uint4*>(qs + t * d + 32 * b);
-            lq[0] = w0;
-            lq[1] = w1;
-            ss[t * KB + b] = sv;
-        }
-        __syncthreads();
-        if (a.xh.hl || a.xh.q16) {  // matrix-core forms (hi/lo: one exponent per row from its largest block scale)
-            for (int t = wave; t < nt; t += RT_THREADS / 64) {
-                float M = 0.0f;
-                for (int b = lane; b < KB; b += 64) M = fmaxf(M, ss[t * KB + b].x);
-#pragma unroll
-                for (int off = 32; off >= 1; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-                if (lane == 0) rmax[t] = M;
-            }
-            __syncthreads();
-            const int cpr = d / 8;
-            for (int c = tid; c < nt * cpr; c += RT_THREADS) {
-                const int t = c / cpr;
-                acth_chunk(qs + t * d, ss + t * KB, d, a.xh, (size_t)(t0 + t), c - t * cpr, acth_exponent(rmax[t]), true);
-            }
+            if (a.xh.q6) write_q6_block(w, sv, a.xh, (size_t)(t0 + t), b);
         }
     }
 
@@ -611,15 +565,15 @@ void launch_route(const RouteArgs& a, hipStream_t st) {
 }
 
 // Matrix-core form of Q8_0 activations already in global memory, one wave per row.
-__global__ void __launch_bounds__(256) k_q8_to_acth(ActQ8 in, int rows, ActH out, int lo) {
+__global__ void __launch_bounds__(256) k_q8_to_acth(ActQ8 in, int rows, ActH out) {
     const size_t row = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= (size_t)rows) return;  // wave-uniform
-    write_acth_row(in.q + row * in.K, in.s + row * (in.K / 32), in.K, out, row, threadIdx.x & 63, lo != 0);
+    write_acth_row(in.q + row * in.K, in.s + row * (in.K / 32), in.K, out, row, threadIdx.x & 63);
 }
 
 __device__ __forceinline__ uint32_t comp4(const uint4& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
 
-// The hi-only form (the down GEMM's operand, no block-unit form) of Q8_0 rows, one wave per row:
+// The same, one wave per row:
 // every quant and scale load of the row is in flight before the first conversion (16 quants per lane
 // and chunk, NC chunks per lane), and the row exponent comes from the scales already loaded.  The
 // values are those of acth_chunk_v: fp16(dx * 2^-E * q), 2^E per half-unit, the min-term pieces of
@@ -669,9 +623,9 @@ __global__ void __launch_bounds__(256) k_q8_to_acth_hi(ActQ8 in, int rows, ActH 
     }
 }
 
-void launch_q8_to_acth(const ActQ8& in, int rows, ActH out, hipStream_t st, bool lo) {
+void launch_q8_to_acth(const ActQ8& in, int rows, ActH out, hipStream_t st) {
     const int nc = (in.K / 16 + 63) / 64;
-    if (!lo && !out.q16 && in.K % 128 == 0 && nc <= 16) {
+    if (in.K % 128 == 0 && nc <= 16) {
         const dim3 grid((rows + 3) / 4);
         if (nc <= 1) hipLaunchKernelGGL(k_q8_to_acth_hi<1>, grid, dim3(256), 0, st, in, rows, out);
         else if (nc <= 2) hipLaunchKernelGGL(k_q8_to_acth_hi<2>, grid, dim3(256), 0, st, in, rows, out);
@@ -680,7 +634,22 @@ void launch_q8_to_acth(const ActQ8& in, int rows, ActH out, hipStream_t st, bool
         else hipLaunchKernelGGL(k_q8_to_acth_hi<16>, grid, dim3(256), 0, st, in, rows, out);
         return;
     }
-    hipLaunchKernelGGL(k_q8_to_acth, dim3((rows + 3) / 4), dim3(256), 0, st, in, rows, out, lo ? 1 : 0);
+    hipLaunchKernelGGL(k_q8_to_acth, dim3((rows + 3) / 4), dim3(256), 0, st, in, rows, out);
+}
+
+// The FP6 form of Q8_0 rows already in global memory, one thread per 32-block.
+__global__ void __launch_bounds__(256) k_q8_to_q6(ActQ8 in, int rows, ActH out) {
+    const int KB = in.K / 32;
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, row = i / KB;
+    if (row >= (size_t)rows) return;
+    const uint4 a = ld16(in.q + i * 32), b = ld16(in.q + i * 32 + 16);
+    const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    write_q6_block(w, in.s[i], out, row, (int)(i - row * KB));
+}
+
+void launch_q8_to_q6(const ActQ8& in, int rows, ActH out, hipStream_t st) {
+    const size_t n = (size_t)rows * (in.K / 32);
+    hipLaunchKernelGGL(k_q8_to_q6, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, in, rows, out);
 }
 
 // Matrix-core form (fp16 hi only) of fp32 activation rows h [rows][ld], out.K

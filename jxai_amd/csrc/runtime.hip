@@ -125,18 +125,21 @@ struct DevMat {
     uint8_t* qs = nullptr;
     uint8_t* sc = nullptr;
     uint8_t* ex = nullptr;  // Q5_0 / Q5_K high bits, Q6_K d
-    uint8_t* mn = nullptr;  // Q4_K / Q5_K min-term table (matrix-core GEMMs)
+    uint8_t* mn = nullptr;   // Q4_K / Q5_K min-term table (down GEMM)
+    uint8_t* g6 = nullptr;   // FP6 form and its min-term pieces (gate/up GEMM)
+    uint8_t* g6m = nullptr;
     void release() {
-        for (uint8_t* p : {qs, sc, ex, mn})
+        for (uint8_t* p : {qs, sc, ex, mn, g6, g6m})
             if (p) (void)hipFree(p);
-        qs = sc = ex = mn = nullptr;
+        qs = sc = ex = mn = g6 = g6m = nullptr;
     }
 };
 
 // Upload n_mats [rows][cols] block matrices and repack them on the device;
-// with `gemm`, Q4_K / Q5_K matrices also get the matrix-core GEMMs' min-term table.
+// `gemm` names the matrix-core GEMM that will read it: its tables are built beside the matrix.
+enum class Gemm { none, gateup, down };
 int upload_matrix(int type, int n_mats, int rows, int cols, const void* host, DevMat& out, hipStream_t st,
-                  bool gemm = false) {
+                  Gemm gemm = Gemm::none) {
     if (!expert_type_ok(type))
         return fail(JX_ERR_UNSUPPORTED, "expert weight type must be Q4_0, Q5_0, Q8_0, Q4_K, Q5_K or Q6_K");
     if (rows % jx::ROWS_PER_TILE != 0) return fail(JX_ERR_UNSUPPORTED, "matrix rows must be a multiple of 32");
@@ -187,7 +190,21 @@ int upload_matrix(int type, int n_mats, int rows, int cols, const void* host, De
         jx::launch_repack(raw, m, out.qs, out.sc, out.ex, st);
         e = hipGetLastError();
     }
-    if (e == hipSuccess && gemm && (type == jx::T_Q4_K || type == jx::T_Q5_K)) {
+    if (e == hipSuccess && gemm == Gemm::gateup && jx::g6_type(type) && q8_activation(type, cols) && cols % 128 == 0) {
+        m.g6_es = (size_t)rows * cols;
+        e = hipMalloc(&out.g6, m.g6_es * n_mats);
+        if (e == hipSuccess && jx::is_kquant(type)) {
+            m.g6m_es = (size_t)m.nrt * m.nkb * jx::G6M_SB;
+            e = hipMalloc(&out.g6m, m.g6m_es * n_mats);
+        }
+        if (e == hipSuccess) {
+            m.g6 = out.g6;
+            m.g6m = out.g6m;
+            jx::launch_g6_tables(m, out.g6, out.g6m, st);
+            e = hipGetLastError();
+        }
+    }
+    if (e == hipSuccess && gemm == Gemm::down && (type == jx::T_Q4_K || type == jx::T_Q5_K)) {
         m.mn_es = (size_t)m.nrt * m.nkb * jx::MN_SB;
         e = hipMalloc(&out.mn, m.mn_es * n_mats);
         if (e == hipSuccess) {
@@ -211,32 +228,34 @@ int dalloc(T*& p, size_t n) {
     return JX_OK;
 }
 
-// Matrix-core activation buffers for `rows` rows of K: the hi/lo form, the
-// block-unit form (the Q4_K gate/up input), or both.
+// Matrix-core activation buffers for `rows` rows of K: the hi form (the down GEMM's input),
+// or the FP6 form (gate/up), with its min-term pieces for K-quant weights.
 struct DevActH {
     jx::ActH a;
     void release() {
-        for (void* p : {(void*)a.hl, (void*)a.pe, (void*)a.xm, (void*)a.q16, (void*)a.rx, (void*)a.pu, (void*)a.xu})
+        for (void* p : {(void*)a.hl, (void*)a.pe, (void*)a.xm, (void*)a.q6, (void*)a.x6})
             if (p) (void)hipFree(p);
         a = jx::ActH{};
     }
-    int alloc(size_t rows, int K, bool hilo = true, bool unit = false) {
+    void shape(int K) {
         release();
         a.K = K;
         a.KH = K / 128;
         a.KU = (K + 255) / 256;
+    }
+    int alloc_hi(size_t rows, int K) {
+        shape(K);
         if (K % 128 != 0) return JX_OK;  // the matrix-core path is not used for this shape
-        if (hilo) {
-            HIPCHK(hipMalloc(&a.hl, rows * a.KH * 256 * sizeof(uint16_t)));
-            HIPCHK(hipMalloc(&a.pe, rows * a.KH * sizeof(float)));
-            HIPCHK(hipMalloc(&a.xm, rows * a.KU * 24 * sizeof(uint16_t)));
-        }
-        if (unit) {
-            HIPCHK(hipMalloc(&a.q16, rows * (size_t)K * sizeof(uint16_t)));
-            HIPCHK(hipMalloc(&a.rx, rows * (size_t)(K / 32) * sizeof(float)));
-            HIPCHK(hipMalloc(&a.pu, rows * a.KH * sizeof(float)));
-            HIPCHK(hipMalloc(&a.xu, rows * a.KU * 24 * sizeof(uint16_t)));
-        }
+        HIPCHK(hipMalloc(&a.hl, rows * a.KH * 256 * sizeof(uint16_t)));
+        HIPCHK(hipMalloc(&a.pe, rows * a.KH * sizeof(float)));
+        HIPCHK(hipMalloc(&a.xm, rows * a.KU * 24 * sizeof(uint16_t)));
+        return JX_OK;
+    }
+    int alloc_fp6(size_t rows, int K, bool q6, bool min) {
+        shape(K);
+        if (K % 128 != 0) return JX_OK;
+        if (q6) HIPCHK(hipMalloc(&a.q6, rows * (size_t)K * 2));
+        if (min) HIPCHK(hipMalloc(&a.x6, rows * a.KU * 24 * sizeof(uint16_t)));
         return JX_OK;
     }
 };
@@ -381,16 +400,15 @@ int ensure_workspace(jx_moe_layer* L, int n) {
     // h's matrix-core form: K = d_ff, or for fp32 h of a K-quant d_ff padded to whole super-blocks
     const int hK = down_h_k(L->down.m.type, L->F, L->down_f32);
     const int hKs = L->shared ? down_h_k(L->sdown.m.type, L->Fs, L->sdown_f32) : 0;
-    // x's forms for the gate/up GEMMs: block-unit for Q4_K / Q5_K, hi/lo for Q4_0 / Q8_0 (routed and shared)
-    auto unit_t = [](int t) { return t == jx::T_Q4_K || t == jx::T_Q5_K; };
-    auto hilo_t = [](int t) { return t == jx::T_Q4_0 || t == jx::T_Q8_0; };
-    const bool xunit = unit_t(L->gate.m.type) || (L->shared && unit_t(L->sgate.m.type));
-    const bool xhilo = hilo_t(L->gate.m.type) || (L->shared && hilo_t(L->sgate.m.type));
-    if ((r = L->xh.alloc((size_t)cap, L->d, xhilo, xunit)) != JX_OK || (r = L->hh.alloc(nk, hK)) != JX_OK) {
+    // x's FP6 form where a gate/up GEMM reads it (routed or shared; Q8_0 weights read the quants themselves)
+    auto any_gu = [&](auto pred) { return pred(L->gate.m) || (L->shared && pred(L->sgate.m)); };
+    const bool x6 = any_gu([](const jx::QMat& m) { return m.g6 != nullptr; });
+    const bool xmin = any_gu([](const jx::QMat& m) { return m.g6m != nullptr; });
+    if ((r = L->xh.alloc_fp6((size_t)cap, L->d, x6, xmin)) != JX_OK || (r = L->hh.alloc_hi(nk, hK)) != JX_OK) {
         L->cap = 0;
         return r;
     }
-    if (L->shared && (r = L->hhs.alloc((size_t)cap, hKs)) != JX_OK) {
+    if (L->shared && (r = L->hhs.alloc_hi((size_t)cap, hKs)) != JX_OK) {
         L->cap = 0;
         return r;
     }
@@ -569,17 +587,17 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     bool mfma = (size_t)nk >= (size_t)min_ppe * E;
     if (flags & JX_FWD_FORCE_GEMV) mfma = false;
     if (flags & JX_FWD_FORCE_MFMA) mfma = true;
-    // The matrix-core GEMMs stage K in 128-element half-units; their Q4_K / Q5_K matrices carry the min
-    // table.  Gate/up takes the GEMM only with a Q8_0 form of x and a type whose products stay exact
-    // there (gemm_gateup_ok); otherwise it runs on the GEMVs (the multi-token form at prefill sizes)
-    // and the down projection still decides for itself.
-    auto ready = [](const DevMat& M) {
-        return !(M.m.type == jx::T_Q4_K || M.m.type == jx::T_Q5_K) || M.m.mn != nullptr;
-    };
+    // The matrix-core GEMMs stage K in 128-element half-units and read the tables built at upload (gate/up: the
+    // FP6 form, Q8_0 matrices as they are; down: Q4_K / Q5_K the min table).  Gate/up takes the GEMM only with
+    // a Q8_0 form of x and a type whose products stay exact there (gemm_gateup_ok); otherwise it runs on
+    // the GEMVs (the multi-token form at prefill sizes) and the down projection still decides for itself.
     auto gu_gemm = [&](const DevMat& G, const DevMat& U, bool f32) {
-        return !f32 && jx::gemm_gateup_ok(G.m.type) && d % 128 == 0 && ready(G) && ready(U);
+        return !f32 && jx::gemm_gateup_ok(G.m.type) && d % 128 == 0 && (G.m.type == jx::T_Q8_0 || (G.m.g6 && U.m.g6));
     };
-    auto dn_gemm = [&](const DevMat& D, int f, bool f32) { return down_h_k(D.m.type, f, f32) % 128 == 0 && ready(D); };
+    auto dn_gemm = [&](const DevMat& D, int f, bool f32) {
+        return down_h_k(D.m.type, f, f32) % 128 == 0 &&
+               (!(D.m.type == jx::T_Q4_K || D.m.type == jx::T_Q5_K) || D.m.mn != nullptr);
+    };
     const bool mfma_gu = mfma && gu_gemm(L->gate, L->up, L->gu_f32);
     const bool dn_shape = dn_gemm(L->down, L->F, L->down_f32);
     const bool smfma = L->shared && n >= L->smfma_min && !(flags & JX_FWD_FORCE_GEMV);
@@ -700,7 +718,7 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
         }
         if (mfma_gu || smfma_gu) {
             Launch l(L, "to_matrix_form", st);
-            jx::launch_q8_to_acth(L->xq, n, L->xh.a, st);
+            if (L->xh.a.q6) jx::launch_q8_to_q6(L->xq, n, L->xh.a, st);
         }
     } else {
         Launch l(L, "route", st);
@@ -761,7 +779,7 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     auto shared_gateup = [&](hipStream_t ss) {
         if (smfma_gu) {
             Launch l(L, "shared_gateup_mfma", ss);
-            jx::launch_mfma_gateup(L->sgate.m, L->sup.m, L->xh.a, sg, st_ub, L->sdown_f32 ? jx::ActQ8{} : L->hqs,
+            jx::launch_mfma_gateup(L->sgate.m, L->sup.m, L->xh.a, L->xq, sg, st_ub, L->sdown_f32 ? jx::ActQ8{} : L->hqs,
                                    L->sdown_f32 ? L->hfs : nullptr, ss);
         } else {
             Launch l(L, "shared_gateup_gemv", ss);
@@ -775,7 +793,7 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
             if (L->sdown_f32)
                 jx::launch_f32_to_acth(L->hfs, (int)fspad, n, L->hhs.a, ss);
             else
-                jx::launch_q8_to_acth(L->hqs, n, L->hhs.a, ss, false);
+                jx::launch_q8_to_acth(L->hqs, n, L->hhs.a, ss);
             jx::launch_mfma_down(L->sdown.m, L->hhs.a, sg, st_ub, L->ysh, ss);
         } else if (sh_ksplit) {
             // the dense shared down's long K in parts, each block a routed block's share of units (the
@@ -836,7 +854,7 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     const float* gxf = L->gu_f32 ? L->xf : nullptr;
     if (mfma_gu) {
         Launch l(L, "gateup_mfma", st);
-        jx::launch_mfma_gateup(L->gate.m, L->up.m, L->xh.a, grp, tiles_ub, L->down_f32 ? jx::ActQ8{} : L->hq,
+        jx::launch_mfma_gateup(L->gate.m, L->up.m, L->xh.a, L->xq, grp, tiles_ub, L->down_f32 ? jx::ActQ8{} : L->hq,
                                L->down_f32 ? L->hf : nullptr, st);
     } else if (small_logits) {
         jx::Groups lg = grp;
@@ -878,7 +896,7 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
             if (L->down_f32)
                 jx::launch_f32_to_acth(L->hf, (int)fpad, nk, L->hh.a, st);
             else
-                jx::launch_q8_to_acth(L->hq, nk, L->hh.a, st, false);
+                jx::launch_q8_to_acth(L->hq, nk, L->hh.a, st);
         }
         // fp32 h at a few tokens per expert: the multi-token down on the fp16 matrix cores where built
         if (!mfma && L->down_f32 && jx::gemv_down_f16_fits(L->down.m.type, L->hh.a.K)) {
@@ -1074,18 +1092,18 @@ int jx_moe_layer_create(const jx_moe_layer_desc* D, jx_moe_layer** out) {
         if (hipMemcpy(L->bias, D->router_bias, E * 4, hipMemcpyHostToDevice) != hipSuccess)
             return bail(fail(JX_ERR_HIP, "router bias upload"));
     }
-    if ((r = upload_matrix(D->gate_type, L->E, L->F, L->d, D->gate_exps, L->gate, st, true)) != JX_OK) return bail(r);
+    if ((r = upload_matrix(D->gate_type, L->E, L->F, L->d, D->gate_exps, L->gate, st, Gemm::gateup)) != JX_OK) return bail(r);
     L->gate.m.act = D->activation;
-    if ((r = upload_matrix(D->up_type, L->E, L->F, L->d, D->up_exps, L->up, st, true)) != JX_OK) return bail(r);
-    if ((r = upload_matrix(D->down_type, L->E, L->d, L->F, D->down_exps, L->down, st, true)) != JX_OK) return bail(r);
+    if ((r = upload_matrix(D->up_type, L->E, L->F, L->d, D->up_exps, L->up, st, Gemm::gateup)) != JX_OK) return bail(r);
+    if ((r = upload_matrix(D->down_type, L->E, L->d, L->F, D->down_exps, L->down, st, Gemm::down)) != JX_OK) return bail(r);
     if (L->shared) {
-        if ((r = upload_matrix(D->sh_gate_type, 1, L->Fs, L->d, D->sh_gate, L->sgate, st, true)) != JX_OK) return bail(r);
+        if ((r = upload_matrix(D->sh_gate_type, 1, L->Fs, L->d, D->sh_gate, L->sgate, st, Gemm::gateup)) != JX_OK) return bail(r);
         // The shared expert is always SwiGLU: src/transformer.cpp:2741-2745 calls matmul_swiglu_quant_f32
         // without hp_.use_gelu (default false, include/quant.h:361); GELU-tanh reaches only the routed
         // experts (2721-2724).
         L->sgate.m.act = jx::ACT_SILU;
-        if ((r = upload_matrix(D->sh_up_type, 1, L->Fs, L->d, D->sh_up, L->sup, st, true)) != JX_OK) return bail(r);
-        if ((r = upload_matrix(D->sh_down_type, 1, L->d, L->Fs, D->sh_down, L->sdown, st, true)) != JX_OK) return bail(r);
+        if ((r = upload_matrix(D->sh_up_type, 1, L->Fs, L->d, D->sh_up, L->sup, st, Gemm::gateup)) != JX_OK) return bail(r);
+        if ((r = upload_matrix(D->sh_down_type, 1, L->d, L->Fs, D->sh_down, L->sdown, st, Gemm::down)) != JX_OK) return bail(r);
         if (D->sh_gate_inp) {
             if ((r = dalloc(L->shgate, d)) != JX_OK) return bail(r);
             if (hipMemcpy(L->shgate, D->sh_gate_inp, d * 4, hipMemcpyHostToDevice) != hipSuccess)
