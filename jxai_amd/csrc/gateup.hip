@@ -9,16 +9,16 @@
 //   acc = fma(S, P, acc), 16 per lane
 // so the VALU does nothing but the accumulation: no operand is converted and no
 // accumulator rescaled.  Forms of S:
-//   Q4_0, Q4_K, Q5_K  v_mfma_scale_f32_32x32x64_f8f6f4 on FP6 (e2m3) operands.  FP6 holds
-//        0..15 with a sign exactly in units of 1/8 (the code's low bits are the value),
-//        and -16.  The weight q (Q4_0: q - 8, Q5_K: q - 16) is one digit; the Q8_0 quant
-//        is sign * (16 a + b), two digits, its lanes' block scales 2^4 and 1.  K = 64 of the
-//        instruction is the block's 32 weights twice, against the a's and the b's.
-//        |S| < 2^17: exact in fp32.
+//   Q4_0, Q4_K, Q5_K  v_mfma_scale_f32_32x32x64_f8f6f4.  A: the weight q (Q4_0: q - 8, Q5_K: q - 16)
+//        is one FP6 e2m3 digit (0..15 with a sign are the codes themselves in units of 1/8; -16 is a code
+//        too).  B: the Q8_0 quant is 16 a + b with |a|, |b| <= 8, two BF6 e3m2 digits (3 significant bits; 16 a
+//        is a shift of the exponent).  A lane half holds 16 elements: its a's, then its b's, against its
+//        weights twice (three register copies per 32 weights instead of loading them in both halves:
+//        Mixtral-shaped 2048 tokens gate/up 1336 -> 1194 us).  |S| < 2^17: exact in fp32.
 //   Q8_0  v_mfma_i32_32x32x32_i8 on the quants as they are, converted to fp32 for the fma
 //        (|S| < 2^19).  (FP6 would need two weight digits and a second MFMA.)
-// P is exact up to one rounding: bf16 pieces of the scales (FP6 form: d or d * sc_j, 3
-// pieces; dx, 2 pieces) or the fp16 scales themselves (Q8_0).  The Q4_K / Q5_K min term
+// P is exact up to one rounding: the fp16 scales themselves (dx; Q4_0 and Q8_0 d), d * sc_j as an exact
+// fp16 hi + lo pair.  The Q4_K / Q5_K min term
 // -dmin * sum_j m_j * (dx_j * sum q_j) (Q5_K: plus 16 d sc_j for the offset) is three bf16
 // MFMAs on 3-piece splits once per super-block, straight into acc.  Only the fp32 rounding of
 // the accumulation differs from the reference; it matters, because h = SiLU(g) * u is
@@ -49,7 +49,7 @@ namespace {
 
 typedef int v6i __attribute__((ext_vector_type(6)));
 typedef int v2i __attribute__((ext_vector_type(2)));
-typedef short s4 __attribute__((ext_vector_type(4)));
+typedef int v3i __attribute__((ext_vector_type(3)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 
 enum : int { GU_F6 = 0, GU_F6_MIN = 1, GU_I8 = 2 };
@@ -87,11 +87,11 @@ __device__ __forceinline__ v6i join6(v4i a, v2i b) {
     return __builtin_shufflevector(a, __builtin_shufflevector(b, b, 0, 1, -1, -1), 0, 1, 2, 3, 4, 5);
 }
 
-// 32 x 32 sums of 32 FP6 products of each lane half (element blocks scaled by 2^(sa - 127), 2^(sb - 127)).
-__device__ __forceinline__ v16f mfma_fp6(v6i a, v6i b, int sa, int sb) {
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(__builtin_shufflevector(a, a, 0, 1, 2, 3, 4, 5, -1, -1),
+// 32 x 32 integer sums of 32 weights (16 FP6 codes a lane half) x Q8_0 quants (their BF6 digits).
+__device__ __forceinline__ v16f mfma_fp6(v3i a, v6i b, int sa, int sb) {
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(__builtin_shufflevector(a, a, 0, 1, 2, 0, 1, 2, -1, -1),
                                                            __builtin_shufflevector(b, b, 0, 1, 2, 3, 4, 5, -1, -1), v16f{},
-                                                           2, 2, 0, sa, 0, sb);
+                                                           2, 3, 0, sa, 0, sb);
 }
 
 // Keeps a uniform address in scalar registers, so loads take it with a 32-bit lane offset (the compiler
@@ -111,6 +111,11 @@ template <typename T>
 __device__ __forceinline__ T gload(gbyte* p) {
     return *reinterpret_cast<const __attribute__((address_space(1))) T*>(p);
 }
+template <>
+__device__ __forceinline__ v3i gload<v3i>(gbyte* p) {
+    const __attribute__((address_space(1))) int* w = reinterpret_cast<const __attribute__((address_space(1))) int*>(p);
+    return v3i{w[0], w[1], w[2]};
+}
 // 64 lanes x 16 bytes from src + off (per lane) into LDS at byte `lds` (wave-uniform), lane i at lds + 16 i.  In
 // asm because the compiler, which counts the builtin as a flat access, then waits for every load in flight
 // before it uses any.  It has no result registers; the waits are the kernel's own (vmcnt counts in order, so the
@@ -126,12 +131,8 @@ __device__ __forceinline__ void dma16v(const uint8_t* src, uint32_t lds) {
 // The weight ring: one 32-block of a row tile.
 template <int KIND>
 struct Wt {
-    v6i w;  // row n's FP6 codes
-    v2i p;  // its scale's bf16 pieces
-    __device__ __forceinline__ void load(gbyte* q, gbyte*, uint32_t o0, uint32_t o1) {
-        w = join6(gload<v4i>(q + o0), gload<v2i>(q + 512 + o1));
-        p = gload<v2i>(q + 768 + o1);
-    }
+    v3i w;  // FP6 codes of elements 16g .. 16g+15 of row n's block
+    __device__ __forceinline__ void load(gbyte* q, gbyte*, uint32_t o0, uint32_t) { w = gload<v3i>(q + o0); }
 };
 template <>
 struct Wt<GU_I8> {
@@ -143,7 +144,8 @@ struct Wt<GU_I8> {
     }
 };
 
-// VGPRs 256 of 256 at two waves per SIMD: acc 64, two (S, P) sets 64, the weight ring 64 (FP6), operands 16.
+// Registers at two waves per SIMD (256): acc 64, two (S, P) sets 64, the weight ring 24 and its scales 16 (FP6),
+// operands 16 and the doubled weight codes 12.
 template <int KIND>
 __global__ void __launch_bounds__(GU_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ8 hq, float* hf, int hf_ld) {
@@ -202,7 +204,8 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const QMat& W = i ? W1 : W0;
-        wb[i] = (I8 ? W.qs + (size_t)e * W.qs_es : W.g6 + (size_t)e * W.g6_es) + (size_t)rt0 * KB * 1024;
+        wb[i] = I8 ? W.qs + (size_t)e * W.qs_es + (size_t)rt0 * KB * 1024
+                   : W.g6 + (size_t)e * W.g6_es + (size_t)rt0 * H * G6_HU;
         wsb[i] = W.sc + (size_t)e * W.sc_es + (size_t)rt0 * KB * 64;
         wmb[i] = MIN ? W.g6m + (size_t)e * W.g6m_es + (size_t)rt0 * in.KU * G6M_SB : nullptr;
     }
@@ -252,12 +255,18 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
     // pieces, or the scale)
     const uint32_t lb0 = (uint32_t)(n * PB + ((g ^ (n % CPP)) << 4));
     const uint32_t lb1 = I8 ? (uint32_t)n * 16 : (uint32_t)(n * PB + ((8 ^ (n % CPP)) << 4) + 8 * g);
-    const uint32_t lo0 = (uint32_t)(I8 ? lane : n) * 16, lo1 = (uint32_t)n * (I8 ? 2 : 8);
+    v4i wsc[2][2];  // FP6: row n's scales of a half-unit's blocks (fp16 hi | lo << 16), by its parity
+    const uint32_t lo0 = (uint32_t)lane * (I8 ? 16 : 12), lo1 = (uint32_t)n * (I8 ? 2 : 16);
     auto load = [&](int h, int j, uint32_t o0, uint32_t o1) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-            ring[j][i].load(scalar(wb[i] + (size_t)(uint32_t)h * (HB * 1024) + j * 1024),
+            ring[j][i].load(scalar(wb[i] + (size_t)(uint32_t)h * (I8 ? HB * 1024 : G6_HU) + j * (I8 ? 1024 : 768)),
                             I8 ? scalar(wsb[i] + (size_t)(uint32_t)h * (HB * 64) + j * 64) : nullptr, o0, o1);
+    };
+    auto load_scales = [&](int h, int odd, uint32_t o1) {
+        if constexpr (!I8)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) wsc[odd][i] = gload<v4i>(scalar(wb[i] + (size_t)(uint32_t)h * G6_HU + 3072) + o1);
     };
     // acc of tile (i, t) takes the sums of set c
     auto fold = [&](int i, int t, int c) {
@@ -266,11 +275,13 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
             acc[i][t][r] = __builtin_fmaf(I8 ? (float)Si[c][r] : S[c][r], P[c][r], acc[i][t][r]);
         asm volatile("" : "+v"(acc[i][t]));  // here, not where acc is next read: (S, P) stay two sets
     };
-    const int sa = 130, sbx = g ? 130 : 134;  // 2^3 takes the codes' 1/8 away; the a digits count 16
+    const int sa = 130, sb = 131;  // 2^3, 2^4: the codes' units
     const uint32_t gmask = g ? 0u : 0xFFFFu;
 
     stage(0, 0);
     asm volatile("" ::: "memory");
+    load_scales(0, 0, lo1);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < HB; ++j) {
         load(0, j, lo0, lo1);
@@ -278,9 +289,9 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
     }
 
     auto half = [&](int h, bool odd) {
-        // this half-unit's DMAs are older than the ring loads (Q8_0 16, FP6 24); the other waves' reads of the other stage are done
+        // this half-unit's DMAs are older than the ring loads (Q8_0 16, FP6 10); the other waves' reads of the other stage are done
         if constexpr (I8) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(24) lgkmcnt(0)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (h + 1 < H) stage(h + 1, odd ? 0 : 1);
@@ -289,6 +300,8 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
         const St& cur = sm.st[odd ? 1 : 0];
         const int hn = min(h + 1, H - 1);
         const uint32_t o0 = here(lo0), o1 = here(lo1);
+        load_scales(hn, odd ? 0 : 1, o1);
+        __builtin_amdgcn_sched_barrier(0);
         // operand B of pair tile t, block j
         v6i bf[2];
         v2i bp[2];
@@ -323,9 +336,11 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
                     P[c] = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(h4, v2i{(int)(uint32_t)ring[j][i].d, 0}),
                                                                __builtin_bit_cast(h4, v2i{(int)dx, 0}), v16f{}, 0, 0, 0);
                 } else {
-                    S[c] = mfma_fp6(ring[j][i].w, bf[t], sa, sbx);
-                    P[c] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(s4, ring[j][i].p),
-                                                                   __builtin_bit_cast(s4, bp[t]), v16f{}, 0, 0, 0);
+                    // (hi, lo) of blocks j & ~1 and j | 1 against (dx, dx) in the block's place, zero in the other
+                    const v4i ws = wsc[odd ? 1 : 0][i];
+                    S[c] = mfma_fp6(ring[j][i].w, bf[t], sa, sb);
+                    P[c] = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(h4, j < 2 ? v2i{ws[0], ws[1]} : v2i{ws[2], ws[3]}),
+                                                               __builtin_bit_cast(h4, bp[t]), v16f{}, 0, 0, 0);
                 }
                 if (j > 0 || k > 0) fold((k + 3) & 1, ((k + 3) & 3) >> 1, c ^ 1);  // the tile before
                 if (i == 1 && j + 1 < HB) read_b(t, j + 1);
@@ -418,8 +433,9 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
 }
 
 // The FP6 weight form of a repacked Q4_0 / Q4_K / Q5_K matrix (QMat::g6), one thread per (expert, row tile,
-// 32-block, row): the block's 32 codes, element i at bit 6 i, then the scale's bf16 pieces.
-__global__ void __launch_bounds__(256) k_g6_table(QMat m, int KB, uint8_t* out) {
+// 32-block, row).  A scale d * sc_j past fp16 sets *over (d above 1000: no model's; such a matrix then has no
+// FP6 form).
+__global__ void __launch_bounds__(256) k_g6_table(QMat m, int KB, uint8_t* out, int* over) {
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (size_t)m.n_mats * m.nrt * KB * 32) return;
     const size_t t = idx / 32;  // (e * nrt + rt) * KB + b
@@ -454,20 +470,27 @@ __global__ void __launch_bounds__(256) k_g6_table(QMat m, int KB, uint8_t* out) 
         scale = f16_to_f32(hd.x & 0xFFFFu) * (float)sc;  // exact: 11 x 6 bits
     }
     const int off = m.type == T_Q4_0 ? 8 : m.type == T_Q5_K ? 16 : 0;
-    uint32_t c[6] = {0, 0, 0, 0, 0, 0};
+    uint32_t c[6] = {0, 0, 0, 0, 0, 0};  // two parts of 16 codes
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
         const int v = (int)((lo[i >> 2] >> (8 * (i & 3))) & 0xFFu) - off;
         const uint32_t code = v < 0 ? 32u | (uint32_t)-v : (uint32_t)v;
-        c[(6 * i) / 32] |= code << ((6 * i) % 32);
-        if ((6 * i) % 32 > 26) c[(6 * i) / 32 + 1] |= code >> (32 - (6 * i) % 32);
+        const int at = (6 * i) / 32, sh = (6 * i) % 32;
+        c[at] |= code << sh;
+        if (sh > 26) c[at + 1] |= code >> (32 - sh);
     }
-    uint16_t p0, p1, p2;
-    split3(scale, p0, p1, p2);
-    uint8_t* o = out + t * 1024 + row * 16;
-    *reinterpret_cast<uint4*>(o) = make_uint4(c[0], c[1], c[2], c[3]);
-    *reinterpret_cast<uint2*>(o + 512 - row * 8) = make_uint2(c[4], c[5]);
-    *reinterpret_cast<uint2*>(o + 768 - row * 8) = make_uint2((uint32_t)p0 | (uint32_t)p1 << 16, p2);
+    const _Float16 h = (_Float16)scale;
+    if (!(__builtin_fabsf((float)h) < __builtin_inff())) atomicOr(over, 1);
+    const _Float16 l = (_Float16)(scale - (float)h);  // exact: scale is a multiple of 2^-24 of 17 bits at most
+    uint8_t* o = out + (er * (KB / HB) + b / HB) * (size_t)G6_HU;
+    uint32_t* oc = reinterpret_cast<uint32_t*>(o + (b % HB) * 768 + row * 12);
+#pragma unroll
+    for (int w = 0; w < 3; ++w) {
+        oc[w] = c[w];
+        oc[96 + w] = c[3 + w];
+    }
+    *reinterpret_cast<uint32_t*>(o + 3072 + row * 16 + (b % HB) * 4) =
+        (uint32_t)__builtin_bit_cast(uint16_t, h) | (uint32_t)__builtin_bit_cast(uint16_t, l) << 16;
 }
 
 // The min-term pieces of a repacked Q4_K / Q5_K matrix (QMat::g6m), one thread per (expert, row tile,
@@ -510,10 +533,10 @@ void launch_kind(const QMat& g, const QMat& u, const GuIn& in, const Groups& grp
 
 bool gemm_gateup_ok(int type) { return type == T_Q8_0 || g6_type(type); }
 
-void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, hipStream_t st) {
+void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, int* over, hipStream_t st) {
     const int KB = m.cols / 32;
     const size_t n = (size_t)m.n_mats * m.nrt * KB * 32;
-    hipLaunchKernelGGL(k_g6_table, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m, KB, g6);
+    hipLaunchKernelGGL(k_g6_table, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m, KB, g6, over);
     if (!g6m) return;
     const size_t ns = (size_t)m.n_mats * m.nrt * m.nkb * 32;
     hipLaunchKernelGGL(k_g6_min_table, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, st, m, g6m);

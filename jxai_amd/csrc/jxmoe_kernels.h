@@ -51,9 +51,9 @@ struct QMat {
     const uint8_t* mn = nullptr;
     size_t mn_es = 0;  // per-expert stride (bytes)
     // FP6 form for the gate/up GEMM (launch_g6_tables; Q4_0 / Q4_K / Q5_K gate and up matrices): per (expert,
-    // row tile, 32-block) 1024 B = [32 rows][16 B] code words 0..3, [32 rows][8 B] code words 4, 5, [32 rows][8 B]
-    // the block scale's bf16 pieces (hi | mid << 16, lo).  Code of value v (q - 8 / q / q - 16): sign << 5 | |v|,
-    // element i at bit 6 i.
+    // row tile, half-unit of 128 columns) G6_HU bytes = [4 blocks][2 parts of 16 elements][32 rows][12 B] codes,
+    // then [32 rows][4 blocks] scales d (* sc_j) as fp16 hi | lo << 16.  Code of value v (q - 8 / q / q - 16):
+    // sign << 5 | |v|, element i of a part at bit 6 i.
     const uint8_t* g6 = nullptr;
     size_t g6_es = 0;
     // Q4_K / Q5_K beside it: per (expert, row tile, super-block) G6M_SB bytes = 3 x [32 rows][16 B], the bf16
@@ -69,7 +69,7 @@ struct QMat {
     int valid_rows = 0;
 };
 constexpr size_t QMAT_PAD = 8192;
-constexpr int G6M_SB = 1536;
+constexpr int G6_HU = 3584, G6M_SB = 1536;
 inline bool g6_type(int t) { return t == T_Q4_0 || t == T_Q4_K || t == T_Q5_K; }
 
 // Q8_0 activations on the device: q [rows][K] int8, s [rows][K/32] = (fp16-truncated
@@ -93,10 +93,11 @@ struct ActQ8 {
 //                        dx * sum(q) (fp32 rows: the block sum) times 2^-E for its
 //                        8 blocks (Q4_K min term)
 // and, for the FP6 gate/up GEMM (each form is written where its pointers are set):
-//   q6 [rows][KH][256 B]  the quant is sign * (16 a + b): the a's (part 0) and the b's (part 1) as 32 FP6
-//                        codes (sign << 5 | digit, element i at bit 6 i) and the block scale's bf16 pieces,
-//                        dx = p0 + p1: (p, p, p, 0) with p = p0 in part 0 and p1 in part 1.  Per half-unit:
-//                        [4 blocks][2 parts][16 B] code words 0..3, [4][2][8 B] words 4, 5, [4][2][8 B] pieces
+//   q6 [rows][KH][256 B]  the quant is 16 a + b, |a|, |b| <= 8: per block and part of 16 elements the codes
+//                        of 16 a, then of b, as BF6 (e3m2) in units of 1/16, code i at bit 6 i, and the block
+//                        scale's fp16 dx.  Per half-unit: [4 blocks][2 parts][16 B] code words 0..3,
+//                        [4][2][8 B] words 4, 5, [4][2][8 B] (dx, dx, 0, 0) in part 0 of even blocks, (0, 0, dx, dx)
+//                        of odd ones, zeros in part 1
 //   x6 [rows][KU][3][8]  bf16 pieces (hi, mid, lo) of dx * sum(q) of the 8 blocks of each 256 (Q4_K / Q5_K)
 struct ActH {
     uint16_t* hl = nullptr;
@@ -263,9 +264,10 @@ void launch_gemv_down_f16(const QMat& dn, const ActH& hh, const Groups& grp, int
 // others its FP6 form xin.
 void launch_mfma_gateup(const QMat& g, const QMat& u, const ActH& xin, const ActQ8& xq, const Groups& grp, int tiles_ub,
                         const ActQ8& hq, float* hf, hipStream_t st);
-// Fill m.g6 (n_mats * nrt * cols / 32 * 1024 bytes) and, K-quants, m.g6m (n_mats * nrt * nkb * G6M_SB bytes;
-// null otherwise) from a repacked matrix of a g6_type (cols % 32 == 0).
-void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, hipStream_t st);
+// Fill m.g6 (n_mats * nrt * cols / 128 * G6_HU bytes) and, K-quants, m.g6m (n_mats * nrt * nkb * G6M_SB bytes;
+// null otherwise) from a repacked matrix of a g6_type (cols % 128 == 0).  *over is set where a scale passes
+// fp16: the form is then not usable.
+void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, int* over, hipStream_t st);
 // KS > 1: the K range split over KS workgroups per item (whole super-blocks each), part q of the
 // output at y + q * ystride (the combine adds the parts in order).  small: few pairs per expert (the
 // 64-pair tile form at more workgroups per CU).

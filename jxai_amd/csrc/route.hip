@@ -48,31 +48,34 @@ __device__ __forceinline__ void store_pieces3(uint16_t* xm, float X) {
     xm[16] = (uint16_t)(__float_as_uint(r2) >> 16);
 }
 
-// The FP6 form of one 32-block (ActH::q6, and its min-term pieces ActH::x6): quants w[8] (four signed bytes a
+// The BF6 form of one 32-block (ActH::q6, and its min-term pieces ActH::x6): quants w[8] (four signed bytes a
 // word) of block b with (scale, sum) sb.
 __device__ __forceinline__ void write_q6_block(const uint32_t (&w)[8], float2 sb, const ActH& o, size_t row, int b) {
-    uint32_t hi[6] = {0, 0, 0, 0, 0, 0}, lo[6] = {0, 0, 0, 0, 0, 0};
+    uint32_t c[2][6] = {};
 #pragma unroll
     for (int i = 0; i < 32; ++i) {
         const int q = (int)(int8_t)(w[i >> 2] >> (8 * (i & 3)));
-        const uint32_t m = (uint32_t)(q < 0 ? -q : q), s = q < 0 ? 32u : 0u;
-        const uint32_t a = s | (m >> 4), c = s | (m & 15u);
-        const int at = (6 * i) / 32, sh = (6 * i) % 32;
-        hi[at] |= a << sh;
-        lo[at] |= c << sh;
-        if (sh > 26) {
-            hi[at + 1] |= a >> (32 - sh);
-            lo[at + 1] |= c >> (32 - sh);
+        const int a = (q + 8) >> 4, l = q - 16 * a;
+        const uint32_t ma = (uint32_t)(a < 0 ? -a : a), ml = (uint32_t)(l < 0 ? -l : l);
+        // |b| is its own code; 16 |a| = 16, 32, 48, 64 .. 128 units: 12, 16, 18, 20 .. 24
+        const uint32_t ca = (a < 0 ? 32u : 0u) | (ma >= 4 ? 16 + ma : ma >= 2 ? 12 + 2 * ma : 12 * ma);
+        const uint32_t cl = (l < 0 ? 32u : 0u) | ml;
+        uint32_t* d = c[i >> 4];
+        const int ba = 6 * (i & 15), bl = 96 + ba;
+        d[ba / 32] |= ca << (ba % 32);
+        d[bl / 32] |= cl << (bl % 32);
+        if (ba % 32 > 26) {
+            d[ba / 32 + 1] |= ca >> (32 - ba % 32);
+            d[bl / 32 + 1] |= cl >> (32 - bl % 32);
         }
     }
-    const uint32_t p0 = __float_as_uint(sb.x) >> 16;                                           // 8 of the 11 bits
-    const uint32_t p1 = __float_as_uint(sb.x - __uint_as_float(p0 << 16)) >> 16;               // the rest, exact
+    const uint32_t dx = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)sb.x) * 0x00010001u;  // exact: an fp16 widened
     uint8_t* d = o.q6 + row * (size_t)o.K * 2 + (b >> 2) * 256;
     const int j = b & 3;
-    *reinterpret_cast<uint4*>(d + j * 32) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-    *reinterpret_cast<uint4*>(d + j * 32 + 16) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-    *reinterpret_cast<uint4*>(d + 128 + j * 16) = make_uint4(hi[4], hi[5], lo[4], lo[5]);
-    *reinterpret_cast<uint4*>(d + 192 + j * 16) = make_uint4(p0 | p0 << 16, p0, p1 | p1 << 16, p1);
+    *reinterpret_cast<uint4*>(d + j * 32) = make_uint4(c[0][0], c[0][1], c[0][2], c[0][3]);
+    *reinterpret_cast<uint4*>(d + j * 32 + 16) = make_uint4(c[1][0], c[1][1], c[1][2], c[1][3]);
+    *reinterpret_cast<uint4*>(d + 128 + j * 16) = make_uint4(c[0][4], c[0][5], c[1][4], c[1][5]);
+    *reinterpret_cast<uint4*>(d + 192 + j * 16) = make_uint4(j & 1 ? 0u : dx, j & 1 ? dx : 0u, 0u, 0u);
     if (o.x6) store_pieces3(o.x6 + row * (size_t)o.KU * 24 + (b / 8) * 24 + (b % 8), sb.x * sb.y);  // product exact
 }
 

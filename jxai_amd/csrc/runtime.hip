@@ -191,18 +191,30 @@ int upload_matrix(int type, int n_mats, int rows, int cols, const void* host, De
         e = hipGetLastError();
     }
     if (e == hipSuccess && gemm == Gemm::gateup && jx::g6_type(type) && q8_activation(type, cols) && cols % 128 == 0) {
-        m.g6_es = (size_t)rows * cols;
+        int* over = nullptr;
+        int host_over = 0;
+        m.g6_es = (size_t)m.nrt * (cols / 128) * jx::G6_HU;
         e = hipMalloc(&out.g6, m.g6_es * n_mats);
+        if (e == hipSuccess) e = hipMalloc(&over, sizeof(int));
+        if (e == hipSuccess) e = hipMemsetAsync(over, 0, sizeof(int), st);
         if (e == hipSuccess && jx::is_kquant(type)) {
             m.g6m_es = (size_t)m.nrt * m.nkb * jx::G6M_SB;
             e = hipMalloc(&out.g6m, m.g6m_es * n_mats);
         }
         if (e == hipSuccess) {
-            m.g6 = out.g6;
-            m.g6m = out.g6m;
-            jx::launch_g6_tables(m, out.g6, out.g6m, st);
+            jx::launch_g6_tables(m, out.g6, out.g6m, over, st);
             e = hipGetLastError();
         }
+        if (e == hipSuccess) e = hipMemcpyAsync(&host_over, over, sizeof(int), hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        (void)hipFree(over);
+        if (e == hipSuccess && host_over) {  // a scale past fp16: gate/up stays on the GEMVs
+            (void)hipFree(out.g6);
+            (void)hipFree(out.g6m);
+            out.g6 = out.g6m = nullptr;
+        }
+        m.g6 = out.g6;
+        m.g6m = out.g6m;
     }
     if (e == hipSuccess && gemm == Gemm::down && (type == jx::T_Q4_K || type == jx::T_Q5_K)) {
         m.mn_es = (size_t)m.nrt * m.nkb * jx::MN_SB;
