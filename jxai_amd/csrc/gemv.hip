@@ -903,6 +903,73 @@ k_gemv_down(QMat D, ActQ8 hq, const float* hf, int hf_ld, Groups grp, float* y, 
     }
 }
 
+// One token through up to three matrices of one format (k_gemv_down's row tiles, unit split and sums), x
+// quantized by every block for itself while its first two weight units are in flight.  The Q8_0 of x costs a
+// block 16 KB from L2 (4096 columns) inside the latency of its weights; a launch of its own for it and one
+// per matrix cost four latencies in a row: q / k / v of 4096 columns (Q4_K, 4096 + 2 x 1024 rows)
+// 20.0 -> 9.8 us.
+struct QkvArgs {
+    QMat W[3];     // unused ones: nrt 0
+    float* out[3];
+    const float* x;
+    int K;
+};
+template <int TYPE, int WAVES>
+__global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(GEMV_WAVES_PER_SIMD(1))))
+k_gemv_qkv(QkvArgs a) {
+    extern __shared__ __align__(16) int8_t smem[];
+    __shared__ float red[WAVES][32];
+    int rt = blockIdx.x;
+    QMat W = a.W[0];
+    float* out = a.out[0];
+#pragma unroll
+    for (int i = 1; i < 3; ++i)
+        if (rt >= W.nrt) {  // block-uniform
+            rt -= W.nrt;
+            W = a.W[i];
+            out = a.out[i];
+        }
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m = lane & 31, h = lane >> 5;
+    const int K = a.K;
+    float2* xs = reinterpret_cast<float2*>(smem + K);
+    const ActLds A{smem, xs, nullptr, K};
+    float acc[1] = {0.0f};
+    kloop<TYPE, 1>(
+        W, W, 0, rt, wave, n_units<TYPE>(W.nkb), WAVES, m, h,
+        [&] {
+            constexpr int HW = 2 * WAVES, XPER = 8;  // half-waves; 32-blocks each has in flight
+            const int KB = K / 32;
+            for (int b0 = 2 * wave + h; b0 - h < KB; b0 += XPER * HW) {  // wave-uniform
+                float v[XPER];
+#pragma unroll
+                for (int q = 0; q < XPER; ++q) v[q] = b0 + q * HW < KB ? a.x[(b0 + q * HW) * 32 + m] : 0.0f;
+#pragma unroll
+                for (int q = 0; q < XPER; ++q) {
+                    const int b = b0 + q * HW;
+                    float2 sv;
+                    const int8_t x8 = (int8_t)q8_block_vals(v[q], sv);
+                    if (b < KB) {
+                        smem[b * 32 + m] = x8;
+                        if (m == 0) xs[b] = sv;
+                    }
+                }
+            }
+            __syncthreads();
+        },
+        [&](const typename Fmt<TYPE>::Raw& c, const typename Fmt<TYPE>::Raw&, int u) {
+            unit_accum<TYPE, 1>(c, A, u, h, 1, W.nkb, acc);
+        });
+    acc[0] += __shfl_xor(acc[0], 32, 64);
+    if (h == 0) red[wave][m] = acc[0];
+    __syncthreads();
+    if (wave == 0 && h == 0) {
+        float s = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) s += red[w][m];
+        if (!W.valid_rows || rt * 32 + m < W.valid_rows) out[rt * 32 + m] = s;  // (padding rows are not written)
+    }
+}
+
 // ---------------------------------------------------------------- several tokens per expert
 // Multi-token GEMV on the matrix cores: one v_mfma_i32_32x32x32_i8 per 32-element block gives the
 // exact integer block sums of up to MX_NT tokens against the 32 rows of a tile.  Operand B is the
@@ -1883,6 +1950,32 @@ bool launch_gemv_gateup(const QMat& g, const QMat& u, const ActQ8& xq, const Gro
             if (xf) return gateup_t<T_Q5_0>(g, u, xq, xf, xf_ld, grp, slots, tb, hq, hf, st, t, sh);
             return false;
         default: return false;
+    }
+}
+
+template <int TYPE>
+static void qkv_t(const QkvArgs& a, hipStream_t st) {
+    const size_t lds = act_lds_bytes(1, a.K, false);
+    lds_optin(k_gemv_qkv<TYPE, DOWN_WAVES>, lds);
+    hipLaunchKernelGGL((k_gemv_qkv<TYPE, DOWN_WAVES>), dim3(a.W[0].nrt + a.W[1].nrt + a.W[2].nrt), dim3(DOWN_WAVES * 64),
+                       lds, st, a);
+}
+
+void launch_gemv_qkv(const QMat* const* W, float* const* out, int n, const float* x, int K, hipStream_t st) {
+    QkvArgs a{};
+    for (int i = 0; i < n; ++i) {
+        a.W[i] = *W[i];
+        a.out[i] = out[i];
+    }
+    a.x = x;
+    a.K = K;
+    switch (W[0]->type) {
+        case T_Q4_0: qkv_t<T_Q4_0>(a, st); break;
+        case T_Q8_0: qkv_t<T_Q8_0>(a, st); break;
+        case T_Q4_K: qkv_t<T_Q4_K>(a, st); break;
+        case T_Q5_K: qkv_t<T_Q5_K>(a, st); break;
+        case T_Q6_K: qkv_t<T_Q6_K>(a, st); break;
+        default: break;  // Q5_0 has no Q8_0-activation form
     }
 }
 

@@ -258,6 +258,9 @@ bool launch_gemv_down(const QMat& dn, const ActQ8& hq, const float* hf, int hf_l
 // k_f32_to_acth), a few tokens per expert; built for Q4_K and Q5_0 where the staged tokens fit the LDS.
 bool gemv_down_f16_fits(int type, int K);
 void launch_gemv_down_f16(const QMat& dn, const ActH& hh, const Groups& grp, int slots, float* y, hipStream_t st);
+// One token x[K] through n <= 3 matrices of one format with a Q8_0-activation form (K % 32 == 0), out[i] = W[i] x,
+// in one launch that quantizes x itself.
+void launch_gemv_qkv(const QMat* const* W, float* const* out, int n, const float* x, int K, hipStream_t st);
 // Prefill regime: matrix-core grouped GEMMs over the dispatch tile table.
 // gate/up writes SwiGLU(h) as Q8_0 (hq.q != null; the down GEMM takes it after
 // launch_q8_to_acth) and/or fp32 (hf != null).  Q8_0 weights read x's Q8_0 form xq, the

@@ -1454,7 +1454,23 @@ int jx_matmul_qkv_quant_f32_dev(jx_qmatrix* Wq, jx_qmatrix* Wk, jx_qmatrix* Wv, 
     bool need_f32 = false;
     for (int i = 0; i < 3; ++i)
         if (Ws[i] && !(quantized && q8_activation(Ws[i]->type, cols))) need_f32 = true;
-    if (quantized) jx::launch_quantize_q8(x_dev, 1, cols, first->xq, st);
+    if (kpad > (size_t)jx::gemv_max_k(false, 1, need_f32))
+        return fail(JX_ERR_UNSUPPORTED, "cols exceeds the GEMV's staged activation capacity");
+    // the Q8_0-form matrices: one launch per format among them
+    bool done[3] = {};
+    for (int i = 0; i < 3; ++i) {
+        if (!Ws[i] || done[i] || !quantized || !q8_activation(Ws[i]->type, cols)) continue;
+        const jx::QMat* w[3];
+        float* o[3];
+        int n = 0;
+        for (int k = i; k < 3; ++k)
+            if (Ws[k] && Ws[k]->type == Ws[i]->type) {
+                w[n] = &Ws[k]->w.m;
+                o[n++] = outs[k];
+                done[k] = true;
+            }
+        jx::launch_gemv_qkv(w, o, n, x_dev, cols, st);
+    }
     if (need_f32) jx::launch_copy_pad(x_dev, cols, (int)kpad, first->xf, st);
     for (int i = 0; i < 3; ++i) {
         if (!Ws[i]) continue;
