@@ -208,6 +208,10 @@ void chain_rows(const float* rows, int nrows, int d, float* out);
 void launch_dispatch(const int* ids, int nk, int E, int top_k, const DispatchOut& o, hipStream_t st,
                      int cold_max = 0);
 
+// The routing of a forward into the caller's device buffers (null ones are not written).
+void launch_copy_routing(const int* ids, const float* w, const int* counts, int* ids_out, float* w_out, int* counts_out,
+                         int nk, int E, hipStream_t st);
+
 // A dense shared expert's blocks appended to a routed multi-token GEMV launch (k_gemv_mxt): its own
 // matrices and outputs over groups of 16 tokens, so its few long-lived blocks run among the routed
 // ones instead of beside them from a second stream.  Gate/up: g and u, h into hq (and fp32 hf when its

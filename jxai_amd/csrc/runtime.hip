@@ -1282,11 +1282,17 @@ int jx_moe_forward(jx_moe_layer* L, const float* x, int32_t n_tok, float* out, i
     }
     L->last_n = n_tok;
     const size_t nk = (size_t)n_tok * L->k;
-    const hipMemcpyKind k2 = dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-    if (!dev) HIPCHK(hipMemcpyAsync(out, L->out, xd * 4, hipMemcpyDeviceToHost, st));
-    if (topk_ids) HIPCHK(hipMemcpyAsync(topk_ids, L->ids, nk * 4, k2, st));
-    if (topk_w) HIPCHK(hipMemcpyAsync(topk_w, L->probs, nk * 4, k2, st));
-    if (expert_counts) HIPCHK(hipMemcpyAsync(expert_counts, L->counts, (size_t)L->E * 4, k2, st));
+    if (dev) {
+        if (topk_ids || topk_w || expert_counts) {
+            jx::launch_copy_routing(L->ids, L->probs, L->counts, topk_ids, topk_w, expert_counts, (int)nk, L->E, st);
+            HIPCHK(hipGetLastError());
+        }
+    } else {
+        HIPCHK(hipMemcpyAsync(out, L->out, xd * 4, hipMemcpyDeviceToHost, st));
+        if (topk_ids) HIPCHK(hipMemcpyAsync(topk_ids, L->ids, nk * 4, hipMemcpyDeviceToHost, st));
+        if (topk_w) HIPCHK(hipMemcpyAsync(topk_w, L->probs, nk * 4, hipMemcpyDeviceToHost, st));
+        if (expert_counts) HIPCHK(hipMemcpyAsync(expert_counts, L->counts, (size_t)L->E * 4, hipMemcpyDeviceToHost, st));
+    }
     if (!(flags & JX_FWD_ASYNC)) {
         HIPCHK(hipStreamSynchronize(st));
         if (L->prof.on && (r = resolve_profile(L)) != JX_OK) return r;
