@@ -47,6 +47,7 @@ namespace jx {
 
 namespace {
 
+typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v6i __attribute__((ext_vector_type(6)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v3i __attribute__((ext_vector_type(3)));
@@ -56,7 +57,7 @@ enum : int { GU_F6 = 0, GU_F6_MIN = 1, GU_I8 = 2 };
 
 constexpr int GU_BN = 64;     // pairs per workgroup
 constexpr int GU_WAVES = 4;   // row-tile slots
-constexpr int GU_RC = 8;      // row groups per band (work_item)
+constexpr int GU_RC = 8, DN_RC = 4;  // row groups per band (work_item)
 
 // One staged half-unit of GU_BN activation rows.
 template <int KIND>
@@ -87,11 +88,23 @@ __device__ __forceinline__ v6i join6(v4i a, v2i b) {
     return __builtin_shufflevector(a, __builtin_shufflevector(b, b, 0, 1, -1, -1), 0, 1, 2, 3, 4, 5);
 }
 
-// 32 x 32 integer sums of 32 weights (16 FP6 codes a lane half) x Q8_0 quants (their BF6 digits).
-__device__ __forceinline__ v16f mfma_fp6(v3i a, v6i b, int sa, int sb) {
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(__builtin_shufflevector(a, a, 0, 1, 2, 0, 1, 2, -1, -1),
-                                                           __builtin_shufflevector(b, b, 0, 1, 2, 3, 4, 5, -1, -1), v16f{},
-                                                           2, 3, 0, sa, 0, sb);
+// 32 x 32 integer sums of 32 weights (16 FP6 codes a lane half) x Q8_0 quants (their BF6 digits), into
+// [row][pair] (WROW) or [pair][row] of the result layout.  The scales take the codes' units (1/8, 1/16) away.
+template <bool WROW>
+__device__ __forceinline__ v16f mfma_fp6(v3i w, v6i x, int sw, int sx) {
+    const v8i w8 = __builtin_shufflevector(w, w, 0, 1, 2, 0, 1, 2, -1, -1);
+    const v8i x8 = __builtin_shufflevector(x, x, 0, 1, 2, 3, 4, 5, -1, -1);
+    if constexpr (WROW) return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w8, x8, v16f{}, 2, 3, 0, sw, 0, sx);
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x8, w8, v16f{}, 3, 2, 0, sx, 0, sw);
+}
+template <bool WROW>
+__device__ __forceinline__ v16f mfma_scales(h4 w, h4 x) {
+    return WROW ? __builtin_amdgcn_mfma_f32_32x32x8f16(w, x, v16f{}, 0, 0, 0)
+                : __builtin_amdgcn_mfma_f32_32x32x8f16(x, w, v16f{}, 0, 0, 0);
+}
+template <bool WROW>
+__device__ __forceinline__ v16f mfma_min(b8 w, b8 x, v16f c) {
+    return WROW ? mfma16b(w, x, c) : mfma16b(x, w, c);
 }
 
 // Keeps a uniform address in scalar registers, so loads take it with a 32-bit lane offset (the compiler
@@ -128,6 +141,17 @@ __device__ __forceinline__ void dma16v(const uint8_t* src, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
 }
 
+// What it writes.
+struct BgOut {
+    ActQ8 hq;           // gate/up: h as Q8_0 (null q: not written),
+    ActH h6;            //   in the FP6 form's activation operand (null q6: not written),
+    float* hf;          //   or in fp32, rows of hf_ld floats (null: not written)
+    int hf_ld;
+    float* y;           // down: y[pair][rows], part k of KS along K at y + k * ystride
+    int KS;
+    size_t ystride;
+};
+
 // The weight ring: one 32-block of a row tile.
 template <int KIND>
 struct Wt {
@@ -146,9 +170,9 @@ struct Wt<GU_I8> {
 
 // Registers at two waves per SIMD (256): acc 64, two (S, P) sets 64, the weight ring 24 and its scales 16 (FP6),
 // operands 16 and the doubled weight codes 12.
-template <int KIND>
+template <int KIND, bool GATEUP>
 __global__ void __launch_bounds__(GU_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ8 hq, float* hf, int hf_ld) {
+k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut o) {
     constexpr bool I8 = KIND == GU_I8, MIN = KIND == GU_F6_MIN;
     using St = GuStage<KIND>;
     constexpr int PB = St::PB, CPP = PB / 16, PPI = 64 / CPP;  // row bytes, chunks, rows per DMA
@@ -159,7 +183,8 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
     // the grid were exact, and the rest exit
     int n_eff = n_items;
     if (!grp.identity) n_eff = min(n_items, R * *grp.n_tiles * (MFMA_BN / GU_BN));
-    const int LB = (int)blockIdx.x;
+    // down over a long K: KS adjacent workgroups per item (on different XCDs), each a range of K
+    const int kp = GATEUP ? 0 : (int)(blockIdx.x % o.KS), LB = GATEUP ? (int)blockIdx.x : (int)(blockIdx.x / o.KS);
     if ((LB >> 3) >= (n_eff >> 3) + ((LB & 7) < (n_eff & 7) ? 1 : 0)) return;
     work_item(LB, n_eff, R, MFMA_BN / GU_BN, RC, ti, sub, rg);
     int e, p0, cnt;
@@ -172,17 +197,20 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // a wave past the matrix repeats the last row tile and drops its results
-    const bool active = rg * GU_WAVES + wave < W0.nrt;
-    const int rt0 = min(rg * GU_WAVES + wave, W0.nrt - 1);
+    // a row tile past the matrix repeats the last one, its results are dropped
+    const int slot = rg * GU_WAVES + wave;
+    const bool active = (GATEUP ? slot : 2 * slot) < W0.nrt;
+    const int rt0 = min(GATEUP ? slot : 2 * slot, W0.nrt - 1);  // gate/up: of both matrices; down: and the next one
 
     if (tid < GU_BN) {
         const int p = p0 + min(tid, cnt - 1);
-        sm.src[tid] = grp.identity ? p : grp.pair_tok[p];
+        sm.src[tid] = !GATEUP || grp.identity ? p : grp.pair_tok[p];
     }
     __syncthreads();
 
     const int KB = in.K / 32, H = in.K / 128;
+    // this workgroup's half-units [h0, h1): whole super-blocks, the last part the rest
+    const int HP = GATEUP ? H : ((H + o.KS - 1) / o.KS + 1) & ~1, h0 = kp * HP, h1 = min(H, h0 + HP);
     // an expert's pairs are in token order, so the buffers are based at the first source row in 64 bits and
     // per-lane offsets stay below 2^32 (jx_moe_forward refuses larger batches)
     const size_t src0 = (size_t)(uint32_t)__builtin_amdgcn_readfirstlane(sm.src[0]);
@@ -203,11 +231,12 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
     const uint8_t* wmb[2];  // their min-term pieces
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const QMat& W = i ? W1 : W0;
-        wb[i] = I8 ? W.qs + (size_t)e * W.qs_es + (size_t)rt0 * KB * 1024
-                   : W.g6 + (size_t)e * W.g6_es + (size_t)rt0 * H * G6_HU;
-        wsb[i] = W.sc + (size_t)e * W.sc_es + (size_t)rt0 * KB * 64;
-        wmb[i] = MIN ? W.g6m + (size_t)e * W.g6m_es + (size_t)rt0 * in.KU * G6M_SB : nullptr;
+        const QMat& W = GATEUP && i ? W1 : W0;
+        const int rt = GATEUP ? rt0 : min(rt0 + i, W.nrt - 1);
+        wb[i] = I8 ? W.qs + (size_t)e * W.qs_es + (size_t)rt * KB * 1024
+                   : W.g6 + (size_t)e * W.g6_es + (size_t)rt * H * G6_HU;
+        wsb[i] = W.sc + (size_t)e * W.sc_es + (size_t)rt * KB * 64;
+        wmb[i] = MIN ? W.g6m + (size_t)e * W.g6m_es + (size_t)rt * in.KU * G6M_SB : nullptr;
     }
     const uint8_t* wlo = MIN ? (g ? wmb[1] : wmb[0]) + 1024 + n * 16 : nullptr;
 
@@ -278,13 +307,14 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
     const int sa = 130, sb = 131;  // 2^3, 2^4: the codes' units
     const uint32_t gmask = g ? 0u : 0xFFFFu;
 
-    stage(0, 0);
+    if (h0 >= h1) return;  // (workgroup-uniform; more parts than super-blocks: never launched)
+    stage(h0, 0);
     asm volatile("" ::: "memory");
-    load_scales(0, 0, lo1);
+    load_scales(h0, 0, lo1);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < HB; ++j) {
-        load(0, j, lo0, lo1);
+        load(h0, j, lo0, lo1);
         __builtin_amdgcn_sched_barrier(0);  // in the ring's order: the loop waits by count
     }
 
@@ -294,11 +324,11 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
         else asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (h + 1 < H) stage(h + 1, odd ? 0 : 1);
+        if (h + 1 < h1) stage(h + 1, odd ? 0 : 1);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
         const St& cur = sm.st[odd ? 1 : 0];
-        const int hn = min(h + 1, H - 1);
+        const int hn = min(h + 1, h1 - 1);
         const uint32_t o0 = here(lo0), o1 = here(lo1);
         load_scales(hn, odd ? 0 : 1, o1);
         __builtin_amdgcn_sched_barrier(0);
@@ -331,16 +361,17 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
                 const int i = k & 1, t = k >> 1, c = k & 1;
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (I8) {
-                    Si[c] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[j][i].w, bi[t], v16i{}, 0, 0, 0);
+                    Si[c] = GATEUP ? __builtin_amdgcn_mfma_i32_32x32x32_i8(ring[j][i].w, bi[t], v16i{}, 0, 0, 0)
+                                   : __builtin_amdgcn_mfma_i32_32x32x32_i8(bi[t], ring[j][i].w, v16i{}, 0, 0, 0);
                     const uint32_t dx = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)__int_as_float(bd[t])) & gmask;
-                    P[c] = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(h4, v2i{(int)(uint32_t)ring[j][i].d, 0}),
-                                                               __builtin_bit_cast(h4, v2i{(int)dx, 0}), v16f{}, 0, 0, 0);
+                    P[c] = mfma_scales<GATEUP>(__builtin_bit_cast(h4, v2i{(int)(uint32_t)ring[j][i].d, 0}),
+                                              __builtin_bit_cast(h4, v2i{(int)dx, 0}));
                 } else {
                     // (hi, lo) of blocks j & ~1 and j | 1 against (dx, dx) in the block's place, zero in the other
                     const v4i ws = wsc[odd ? 1 : 0][i];
-                    S[c] = mfma_fp6(ring[j][i].w, bf[t], sa, sb);
-                    P[c] = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(h4, j < 2 ? v2i{ws[0], ws[1]} : v2i{ws[2], ws[3]}),
-                                                               __builtin_bit_cast(h4, bp[t]), v16f{}, 0, 0, 0);
+                    S[c] = mfma_fp6<GATEUP>(ring[j][i].w, bf[t], sa, sb);
+                    P[c] = mfma_scales<GATEUP>(__builtin_bit_cast(h4, j < 2 ? v2i{ws[0], ws[1]} : v2i{ws[2], ws[3]}),
+                                              __builtin_bit_cast(h4, bp[t]));
                 }
                 if (j > 0 || k > 0) fold((k + 3) & 1, ((k + 3) & 3) >> 1, c ^ 1);  // the tile before
                 if (i == 1 && j + 1 < HB) read_b(t, j + 1);
@@ -373,19 +404,35 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
                     const b8 w2 = *reinterpret_cast<const b8*>(wm + (g ? i * 1024 + 512 : 2048 + i * 512));
 #pragma unroll
                     for (int t = 0; t < 2; ++t) {
-                        acc[i][t] = mfma16b(w0, x0[t], acc[i][t]);
-                        acc[i][t] = mfma16b(w1, x1[t], acc[i][t]);
-                        acc[i][t] = mfma16b(w2, x0[t], acc[i][t]);
+                        acc[i][t] = mfma_min<GATEUP>(w0, x0[t], acc[i][t]);
+                        acc[i][t] = mfma_min<GATEUP>(w1, x1[t], acc[i][t]);
+                        acc[i][t] = mfma_min<GATEUP>(w2, x0[t], acc[i][t]);
                     }
                 }
             }
         }
     };
-    for (int h = 0; h < H; h += 2) {
+    for (int h = h0; h < h1; h += 2) {
         half(h, false);
-        if (h + 1 < H) half(h + 1, true);
+        if (h + 1 < h1) half(h + 1, true);
     }
 
+    if constexpr (!GATEUP) {
+        // lane (n, g) holds row n of a row tile and, in register r, pair 8 (r / 4) + 4 g + r % 4 of a pair tile
+        float* y = o.y + (size_t)kp * o.ystride + (size_t)p0 * W0.rows;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            if (2 * slot + i >= W0.nrt) return;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int pr = 32 * t + 8 * (r >> 2) + 4 * g + (r & 3);
+                    if (pr < cnt) y[(size_t)pr * W0.rows + (2 * slot + i) * 32 + n] = acc[i][t][r];
+                }
+        }
+        return;
+    }
     // h = act(gate) * up, and h's block of 32 rows (row tile rt0) split over lanes n and n + 32
     if (!active) return;
 #pragma unroll
@@ -396,13 +443,13 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
         const int pr = 32 * t + n;
         const size_t p = (size_t)(p0 + pr);
         const bool valid = pr < cnt;
-        if (hf && valid) {
-            float* fd = hf + p * (size_t)hf_ld + rt0 * 32 + 4 * g;
+        if (o.hf && valid) {
+            float* fd = o.hf + p * (size_t)o.hf_ld + rt0 * 32 + 4 * g;
 #pragma unroll
             for (int ii = 0; ii < 4; ++ii)
                 *reinterpret_cast<float4*>(fd + 8 * ii) = make_float4(v[4 * ii], v[4 * ii + 1], v[4 * ii + 2], v[4 * ii + 3]);
         }
-        if (!hq.q) continue;
+        if (!o.hq.q && !o.h6.q6) continue;
         // Q8_0 of the block (quantize_row_q8_0): both halves' lanes hold the same scale and sum
         float amax = 0.0f;
 #pragma unroll
@@ -425,9 +472,15 @@ k_gateup(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, ActQ
         // word ii of half g is rows 8 ii + 4 g ..: exchange so half g stores rows 16 g .. 16 g + 15
         const auto x0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
         const auto x1 = __builtin_amdgcn_permlane32_swap(w[1], w[3], false, false);
-        if (valid) {
-            *reinterpret_cast<uint4*>(hq.q + p * (size_t)hq.K + rt0 * 32 + 16 * g) = make_uint4(x0[0], x0[1], x1[0], x1[1]);
-            if (g == 0) hq.s[p * (size_t)(hq.K / 32) + rt0] = make_float2(f16_to_f32(f32_to_f16_trunc(d)), (float)s);
+        if (!valid) continue;
+        const float2 sv = make_float2(f16_to_f32(f32_to_f16_trunc(d)), (float)s);
+        if (o.hq.q) {
+            *reinterpret_cast<uint4*>(o.hq.q + p * (size_t)o.hq.K + rt0 * 32 + 16 * g) = make_uint4(x0[0], x0[1], x1[0], x1[1]);
+            if (g == 0) o.hq.s[p * (size_t)(o.hq.K / 32) + rt0] = sv;
+        }
+        if (o.h6.q6) {
+            const uint32_t w4[4] = {x0[0], x0[1], x1[0], x1[1]};
+            write_q6_part(w4, sv, o.h6, p, rt0, g);
         }
     }
 }
@@ -519,19 +572,44 @@ __global__ void __launch_bounds__(256) k_g6_min_table(QMat m, uint8_t* out) {
         *reinterpret_cast<uint4*>(out + t * G6M_SB + c * 512 + row * 16) = make_uint4(pw[c][0], pw[c][1], pw[c][2], pw[c][3]);
 }
 
-template <int KIND>
-void launch_kind(const QMat& g, const QMat& u, const GuIn& in, const Groups& grp, int tiles_ub, const ActQ8& hq,
-                 float* hf, hipStream_t st) {
-    const int R = (g.nrt + GU_WAVES - 1) / GU_WAVES;
+// Workgroups of an item list over row groups of `slots` row-tile slots.
+template <int KIND, bool GATEUP>
+void launch_kind(const QMat& w0, const QMat& w1, const GuIn& in, const Groups& grp, int tiles_ub, const BgOut& o,
+                 hipStream_t st) {
+    const int slots = GATEUP ? w0.nrt : (w0.nrt + 1) / 2;
+    const int R = (slots + GU_WAVES - 1) / GU_WAVES;
     const int n_items = R * tiles_ub * (MFMA_BN / GU_BN);
     if (n_items <= 0) return;
-    hipLaunchKernelGGL(k_gateup<KIND>, dim3(n_items), dim3(GU_WAVES * 64), 0, st, g, u, in, grp, R, n_items,
-                       std::min(GU_RC, R), hq, hf, ((g.rows + 255) / 256) * 256);
+    hipLaunchKernelGGL((k_bgemm<KIND, GATEUP>), dim3(n_items * (GATEUP ? 1 : o.KS)), dim3(GU_WAVES * 64), 0, st, w0, w1, in,
+                       grp, R, n_items, std::min(GATEUP ? GU_RC : DN_RC, R), o);
+}
+
+// The launch of a matrix (pair)'s format over x's forms; false: a form is missing (a caller bug: nothing is
+// launched on null pointers).
+template <bool GATEUP>
+bool launch_form(const QMat& w0, const QMat& w1, const ActH& x6, const ActQ8& xq, const Groups& grp, int tiles_ub,
+                 const BgOut& o, hipStream_t st) {
+    GuIn in{x6.q6, nullptr, reinterpret_cast<const uint8_t*>(x6.x6), w0.cols, (w0.cols + 255) / 256};
+    if (w0.type == T_Q8_0) {
+        if (!xq.q || !xq.s) return false;
+        in.q = reinterpret_cast<const uint8_t*>(xq.q);
+        in.s = reinterpret_cast<const uint8_t*>(xq.s);
+        launch_kind<GU_I8, GATEUP>(w0, w1, in, grp, tiles_ub, o, st);
+        return true;
+    }
+    if (!w0.g6 || !w1.g6 || !in.q) return false;
+    if (w0.type == T_Q4_0) {
+        launch_kind<GU_F6, GATEUP>(w0, w1, in, grp, tiles_ub, o, st);
+        return true;
+    }
+    if (!w0.g6m || !w1.g6m || !in.xm) return false;
+    launch_kind<GU_F6_MIN, GATEUP>(w0, w1, in, grp, tiles_ub, o, st);
+    return true;
 }
 
 }  // namespace
 
-bool gemm_gateup_ok(int type) { return type == T_Q8_0 || g6_type(type); }
+bool gemm_block_ok(int type) { return type == T_Q8_0 || g6_type(type); }
 
 void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, int* over, hipStream_t st) {
     const int KB = m.cols / 32;
@@ -543,19 +621,13 @@ void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, int* over, hipSt
 }
 
 void launch_mfma_gateup(const QMat& g, const QMat& u, const ActH& xin, const ActQ8& xq, const Groups& grp, int tiles_ub,
-                        const ActQ8& hq, float* hf, hipStream_t st) {
-    GuIn in{xin.q6, nullptr, reinterpret_cast<const uint8_t*>(xin.x6), g.cols, (g.cols + 255) / 256};
-    if (g.type == T_Q8_0) {
-        in.q = reinterpret_cast<const uint8_t*>(xq.q);
-        in.s = reinterpret_cast<const uint8_t*>(xq.s);
-        launch_kind<GU_I8>(g, u, in, grp, tiles_ub, hq, hf, st);
-        return;
-    }
-    // the caller allocates the forms its matrices need; a missing one is a caller bug, and nothing is launched
-    // on null pointers
-    if (!g.g6 || !u.g6 || !in.q) return;
-    if (g.type == T_Q4_0) launch_kind<GU_F6>(g, u, in, grp, tiles_ub, hq, hf, st);
-    else if (g.g6m && u.g6m && in.xm) launch_kind<GU_F6_MIN>(g, u, in, grp, tiles_ub, hq, hf, st);
+                        const ActQ8& hq, const ActH& h6, float* hf, hipStream_t st) {
+    (void)launch_form<true>(g, u, xin, xq, grp, tiles_ub, BgOut{hq, h6, hf, ((g.rows + 255) / 256) * 256, nullptr, 1, 0}, st);
+}
+
+void launch_mfma_down_block(const QMat& dn, const ActH& h6, const ActQ8& hq, const Groups& grp, int tiles_ub, float* y,
+                            hipStream_t st, int KS, size_t ystride) {
+    (void)launch_form<false>(dn, dn, h6, hq, grp, tiles_ub, BgOut{ActQ8{}, ActH{}, nullptr, 0, y, KS, ystride}, st);
 }
 
 }  // namespace jx

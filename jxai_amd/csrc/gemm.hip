@@ -670,6 +670,10 @@ static void launch_t(const QMat& dn, const ActH& in, const Groups& grp, int tile
                        dn, in, grp, R, n_items, std::min(S::RC, R), y, KS, ystride);
 }
 
+bool gemm_f16_ok(const QMat& m) {
+    return m.type == T_Q5_0 || m.type == T_Q6_K || ((m.type == T_Q4_K || m.type == T_Q5_K) && m.mn);
+}
+
 int mfma_down_ksplit(int K) { return K >= MFMA_DOWN_KSPLIT_MIN_K ? 2 : 1; }
 
 template <int TYPE>
@@ -682,8 +686,6 @@ static void down_t(const QMat& dn, const ActH& hin, const Groups& grp, int tiles
 void launch_mfma_down(const QMat& dn, const ActH& hin, const Groups& grp, int tiles_ub, float* y, hipStream_t st,
                       int KS, size_t ystride, bool small) {
     switch (dn.type) {
-        case T_Q4_0: down_t<T_Q4_0>(dn, hin, grp, tiles_ub, y, st, KS, ystride, small); break;
-        case T_Q8_0: down_t<T_Q8_0>(dn, hin, grp, tiles_ub, y, st, KS, ystride, small); break;
         case T_Q4_K: down_t<T_Q4_K>(dn, hin, grp, tiles_ub, y, st, KS, ystride, small); break;
         case T_Q5_0: down_t<T_Q5_0>(dn, hin, grp, tiles_ub, y, st, KS, ystride, small); break;
         case T_Q5_K: down_t<T_Q5_K>(dn, hin, grp, tiles_ub, y, st, KS, ystride, small); break;

@@ -41,6 +41,41 @@ __device__ __forceinline__ void split3(float v, uint16_t& h, uint16_t& m, uint16
     l = (uint16_t)(__float_as_uint(r2) >> 16);
 }
 
+// Exact bf16 (hi, mid, lo) pieces of an fp32 value (truncation keeps each
+// remainder exact) at xm[0], xm[8], xm[16].
+__device__ __forceinline__ void store_pieces3(uint16_t* xm, float X) { split3(X, xm[0], xm[8], xm[16]); }
+
+// The BF6 form (ActH::q6, and the block's min-term pieces ActH::x6) of part `part` (16 quants, four signed bytes
+// a word) of block b with (scale, sum) sb.
+__device__ __forceinline__ void write_q6_part(const uint32_t (&w)[4], float2 sb, const ActH& o, size_t row, int b, int part) {
+    uint32_t c[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int q = (int)(int8_t)(w[i >> 2] >> (8 * (i & 3)));
+        const int a = (q + 8) >> 4, l = q - 16 * a;
+        const uint32_t ma = (uint32_t)(a < 0 ? -a : a), ml = (uint32_t)(l < 0 ? -l : l);
+        // |b| is its own code; 16 |a| = 16, 32, 48, 64 .. 128 units: 12, 16, 18, 20 .. 24
+        const uint32_t ca = (a < 0 ? 32u : 0u) | (ma >= 4 ? 16 + ma : ma >= 2 ? 12 + 2 * ma : 12 * ma);
+        const uint32_t cl = (l < 0 ? 32u : 0u) | ml;
+        const int ba = 6 * i, bl = 96 + ba;
+        c[ba / 32] |= ca << (ba % 32);
+        c[bl / 32] |= cl << (bl % 32);
+        if (ba % 32 > 26) {
+            c[ba / 32 + 1] |= ca >> (32 - ba % 32);
+            c[bl / 32 + 1] |= cl >> (32 - bl % 32);
+        }
+    }
+    // exact: sb.x is an fp16 widened
+    const uint32_t dx = part ? 0u : (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)sb.x) * 0x00010001u;
+    const int j = b & 3;
+    uint8_t* d = o.q6 + row * (size_t)o.K * 2 + (b >> 2) * 256;
+    *reinterpret_cast<uint4*>(d + j * 32 + part * 16) = make_uint4(c[0], c[1], c[2], c[3]);
+    *reinterpret_cast<uint2*>(d + 128 + j * 16 + part * 8) = make_uint2(c[4], c[5]);
+    *reinterpret_cast<uint2*>(d + 192 + j * 16 + part * 8) = make_uint2(j & 1 ? 0u : dx, j & 1 ? dx : 0u);
+    if (o.x6 && part == 0)
+        store_pieces3(o.x6 + row * (size_t)o.KU * 24 + (b / 8) * 24 + (b % 8), sb.x * sb.y);  // product exact
+}
+
 // (scale, min) j of a Q4_K header in registers (get_scale_min_k4,
 // src/quant.cpp:1107-1115).
 __device__ __forceinline__ void hdr_scale_min(const uint4& hd, int j, int& sc, int& mn) {

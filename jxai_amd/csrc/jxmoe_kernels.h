@@ -258,25 +258,27 @@ int gemv_max_k(bool gateup, int tb, bool f32);
 bool launch_gemv_down(const QMat& dn, const ActQ8& hq, const float* hf, int hf_ld, const Groups& grp,
                       int slots, int tb, float* y, hipStream_t st, const CombineOut& comb = CombineOut{},
                       SharedPart* sh = nullptr);
+// One token x[K] through n <= 3 matrices of one format with a Q8_0-activation form (K % 32 == 0), out[i] = W[i] x,
+// in one launch that quantizes x itself.
+void launch_gemv_qkv(const QMat* const* W, float* const* out, int n, const float* x, int K, hipStream_t st);
 // Decode regime, fp32 h (no Q8_0 form): the down projection on fp16 matrix cores over h's hi form (hh,
 // k_f32_to_acth), a few tokens per expert; built for Q4_K and Q5_0 where the staged tokens fit the LDS.
 bool gemv_down_f16_fits(int type, int K);
 void launch_gemv_down_f16(const QMat& dn, const ActH& hh, const Groups& grp, int slots, float* y, hipStream_t st);
-// One token x[K] through n <= 3 matrices of one format with a Q8_0-activation form (K % 32 == 0), out[i] = W[i] x,
-// in one launch that quantizes x itself.
-void launch_gemv_qkv(const QMat* const* W, float* const* out, int n, const float* x, int K, hipStream_t st);
 // Prefill regime: matrix-core grouped GEMMs over the dispatch tile table.
-// gate/up writes SwiGLU(h) as Q8_0 (hq.q != null; the down GEMM takes it after
-// launch_q8_to_acth) and/or fp32 (hf != null).  Q8_0 weights read x's Q8_0 form xq, the
-// others its FP6 form xin.
+// gate/up writes SwiGLU(h) as Q8_0 (hq.q != null), in the BF6 form (h6.q6 != null) and/or fp32 (hf != null).
+// Q8_0 weights read the activations' Q8_0 form (xq, hq), the others their BF6 form (xin, h6).
 void launch_mfma_gateup(const QMat& g, const QMat& u, const ActH& xin, const ActQ8& xq, const Groups& grp, int tiles_ub,
-                        const ActQ8& hq, float* hf, hipStream_t st);
+                        const ActQ8& hq, const ActH& h6, float* hf, hipStream_t st);
+// Down on the same GEMM.  KS > 1: the K range split over KS workgroups per item (whole super-blocks each), part q of
+// the output at y + q * ystride (the combine adds the parts in order).
+void launch_mfma_down_block(const QMat& dn, const ActH& h6, const ActQ8& hq, const Groups& grp, int tiles_ub, float* y,
+                            hipStream_t st, int KS = 1, size_t ystride = 0);
 // Fill m.g6 (n_mats * nrt * cols / 128 * G6_HU bytes) and, K-quants, m.g6m (n_mats * nrt * nkb * G6M_SB bytes;
 // null otherwise) from a repacked matrix of a g6_type (cols % 128 == 0).  *over is set where a scale passes
 // fp16: the form is then not usable.
 void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, int* over, hipStream_t st);
-// KS > 1: the K range split over KS workgroups per item (whole super-blocks each), part q of the
-// output at y + q * ystride (the combine adds the parts in order).  small: few pairs per expert (the
+// The fp16 down GEMM, KS as above.  small: few pairs per expert (the
 // 64-pair tile form at more workgroups per CU).
 void launch_mfma_down(const QMat& dn, const ActH& hin, const Groups& grp, int tiles_ub, float* y, hipStream_t st,
                       int KS = 1, size_t ystride = 0, bool small = false);
@@ -290,9 +292,11 @@ constexpr int MFMA_DOWN_SMALL_MAX_PPE = 256;
 // 155 -> 133 us; at K 768 - 1408 the per-workgroup overhead makes it slower).
 constexpr int MFMA_DOWN_KSPLIT_MIN_K = 8192;
 int mfma_down_ksplit(int K);
-// Weight types the matrix-core gate/up GEMM takes (Q5_0 has no Q8_0-activation form, and Q6_K's 16-element
-// sub-blocks no exact 32-block product; gate/up products must be exact: h is re-quantized).
-bool gemm_gateup_ok(int type);
+// Weight types the block GEMM takes (Q5_0 has no Q8_0-activation form, and Q6_K's 16-element sub-blocks no
+// product per 32-block).
+bool gemm_block_ok(int type);
+// Whether the fp16 down GEMM is built for a matrix: Q5_0, Q6_K, and Q4_K / Q5_K with their min table.
+bool gemm_f16_ok(const QMat& m);
 // Fill m.mn (m.n_mats * m.nrt * m.nkb * MN_SB bytes) from a repacked Q4_K or Q5_K matrix.
 void launch_min_table(const QMat& m, uint8_t* mn, hipStream_t st);
 

@@ -5,6 +5,7 @@
 
 #include "jxmoe_device.h"
 #include "jxmoe_dispatch.h"
+#include "jxmoe_gemm.h"
 #include "jxmoe_kernels.h"
 
 namespace jx {
@@ -34,49 +35,6 @@ __device__ __forceinline__ int quant_block(float v, int l32, bool ok, const ActQ
 // Row exponent of the matrix-core form from the row's largest block scale M.
 __device__ __forceinline__ int acth_exponent(float M) {
     return (M > 0.0f) ? (int)((__float_as_uint(M) >> 23) & 0xFF) - 127 - 7 : 0;
-}
-
-// Exact bf16 (hi, mid, lo) pieces of an fp32 value (truncation keeps each
-// remainder exact) at xm[0], xm[8], xm[16].
-__device__ __forceinline__ void store_pieces3(uint16_t* xm, float X) {
-    const uint32_t bh = __float_as_uint(X) & 0xFFFF0000u;
-    const float r1 = X - __uint_as_float(bh);
-    const uint32_t bm = __float_as_uint(r1) & 0xFFFF0000u;
-    const float r2 = r1 - __uint_as_float(bm);
-    xm[0] = (uint16_t)(bh >> 16);
-    xm[8] = (uint16_t)(bm >> 16);
-    xm[16] = (uint16_t)(__float_as_uint(r2) >> 16);
-}
-
-// The BF6 form of one 32-block (ActH::q6, and its min-term pieces ActH::x6): quants w[8] (four signed bytes a
-// word) of block b with (scale, sum) sb.
-__device__ __forceinline__ void write_q6_block(const uint32_t (&w)[8], float2 sb, const ActH& o, size_t row, int b) {
-    uint32_t c[2][6] = {};
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-        const int q = (int)(int8_t)(w[i >> 2] >> (8 * (i & 3)));
-        const int a = (q + 8) >> 4, l = q - 16 * a;
-        const uint32_t ma = (uint32_t)(a < 0 ? -a : a), ml = (uint32_t)(l < 0 ? -l : l);
-        // |b| is its own code; 16 |a| = 16, 32, 48, 64 .. 128 units: 12, 16, 18, 20 .. 24
-        const uint32_t ca = (a < 0 ? 32u : 0u) | (ma >= 4 ? 16 + ma : ma >= 2 ? 12 + 2 * ma : 12 * ma);
-        const uint32_t cl = (l < 0 ? 32u : 0u) | ml;
-        uint32_t* d = c[i >> 4];
-        const int ba = 6 * (i & 15), bl = 96 + ba;
-        d[ba / 32] |= ca << (ba % 32);
-        d[bl / 32] |= cl << (bl % 32);
-        if (ba % 32 > 26) {
-            d[ba / 32 + 1] |= ca >> (32 - ba % 32);
-            d[bl / 32 + 1] |= cl >> (32 - bl % 32);
-        }
-    }
-    const uint32_t dx = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)sb.x) * 0x00010001u;  // exact: an fp16 widened
-    uint8_t* d = o.q6 + row * (size_t)o.K * 2 + (b >> 2) * 256;
-    const int j = b & 3;
-    *reinterpret_cast<uint4*>(d + j * 32) = make_uint4(c[0][0], c[0][1], c[0][2], c[0][3]);
-    *reinterpret_cast<uint4*>(d + j * 32 + 16) = make_uint4(c[1][0], c[1][1], c[1][2], c[1][3]);
-    *reinterpret_cast<uint4*>(d + 128 + j * 16) = make_uint4(c[0][4], c[0][5], c[1][4], c[1][5]);
-    *reinterpret_cast<uint4*>(d + 192 + j * 16) = make_uint4(j & 1 ? 0u : dx, j & 1 ? dx : 0u, 0u, 0u);
-    if (o.x6) store_pieces3(o.x6 + row * (size_t)o.KU * 24 + (b / 8) * 24 + (b % 8), sb.x * sb.y);  // product exact
 }
 
 // Elements 8c .. 8c+7 of one row (all in one 32-block): one 16-byte store, plus the row's pe entry
@@ -269,7 +227,11 @@ __global__ void __launch_bounds__(RT_THREADS) k_route(RouteArgs a, int nsplit, i
             gq[0] = w0;
             gq[1] = w1;
             a.xq.s[(size_t)(t0 + t) * KB + b] = sv;
-            if (a.xh.q6) write_q6_block(w, sv, a.xh, (size_t)(t0 + t), b);
+            if (a.xh.q6)
+                for (int part = 0; part < 2; ++part) {
+                    const uint32_t w4[4] = {w[4 * part], w[4 * part + 1], w[4 * part + 2], w[4 * part + 3]};
+                    write_q6_part(w4, sv, a.xh, (size_t)(t0 + t), b, part);
+                }
         }
     }
 
@@ -529,25 +491,6 @@ void launch_route(const RouteArgs& a, hipStream_t st) {
             (void)hipFuncSetAttribute(reinterpret_cast<const void*>(q), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       (int)lq);
         hipLaunchKernelGGL(q, dim3((a.n + T - 1) / T), dim3(RT_THREADS), lq, st, a, 1, 0);
-// The routing into the caller's device buffers (each may be null), in one launch: three device-to-device copies
-// of a few KB cost a launch and its hand-over each.  Qwen3-shaped 37 tokens, residual form, routing kept: per
-// step 119.0 -> 115.3 us.
-__global__ void __launch_bounds__(256) k_copy_routing(const int* ids, const float* w, const int* counts, int* ids_out,
-                                                      float* w_out, int* counts_out, int nk, int E) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < nk) {
-        if (ids_out) ids_out[i] = ids[i];
-        if (w_out) w_out[i] = w[i];
-    }
-    if (counts_out && i < E) counts_out[i] = counts[i];
-}
-
-void launch_copy_routing(const int* ids, const float* w, const int* counts, int* ids_out, float* w_out, int* counts_out,
-                         int nk, int E, hipStream_t st) {
-    hipLaunchKernelGGL(k_copy_routing, dim3((std::max(nk, E) + 255) / 256), dim3(256), 0, st, ids, w, counts, ids_out, w_out,
-                       counts_out, nk, E);
-}
-
         const int R = a.E + (a.shgate ? 1 : 0), RS = (R + RT_GROUPS - 1) / RT_GROUPS;
         const size_t lr = (size_t)2 * RR_TC * 16 * rs_stride(a.d) * sizeof(float);
         // tokens per block: about 512 blocks in all, in whole LDS chunks, at most RR_TPB
@@ -584,6 +527,25 @@ void launch_copy_routing(const int* ids, const float* w, const int* counts, int*
         default: go(k_route<1>); break;
     }
     if (r.RS > 1) launch_route_topk(a, st);
+}
+
+// The routing into the caller's device buffers (each may be null), in one launch: three device-to-device copies
+// of a few KB cost a launch and its hand-over each.  Qwen3-shaped 37 tokens, residual form, routing kept: per
+// step 119.0 -> 115.3 us.
+__global__ void __launch_bounds__(256) k_copy_routing(const int* ids, const float* w, const int* counts, int* ids_out,
+                                                      float* w_out, int* counts_out, int nk, int E) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < nk) {
+        if (ids_out) ids_out[i] = ids[i];
+        if (w_out) w_out[i] = w[i];
+    }
+    if (counts_out && i < E) counts_out[i] = counts[i];
+}
+
+void launch_copy_routing(const int* ids, const float* w, const int* counts, int* ids_out, float* w_out, int* counts_out,
+                         int nk, int E, hipStream_t st) {
+    hipLaunchKernelGGL(k_copy_routing, dim3((std::max(nk, E) + 255) / 256), dim3(256), 0, st, ids, w, counts, ids_out, w_out,
+                       counts_out, nk, E);
 }
 
 // Matrix-core form of Q8_0 activations already in global memory, one wave per row.
@@ -659,18 +621,18 @@ void launch_q8_to_acth(const ActQ8& in, int rows, ActH out, hipStream_t st) {
     hipLaunchKernelGGL(k_q8_to_acth, dim3((rows + 3) / 4), dim3(256), 0, st, in, rows, out);
 }
 
-// The FP6 form of Q8_0 rows already in global memory, one thread per 32-block.
+// The BF6 form of Q8_0 rows already in global memory, one thread per half 32-block.
 __global__ void __launch_bounds__(256) k_q8_to_q6(ActQ8 in, int rows, ActH out) {
-    const int KB = in.K / 32;
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, row = i / KB;
+    const int KP = in.K / 16;
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, row = i / KP;
     if (row >= (size_t)rows) return;
-    const uint4 a = ld16(in.q + i * 32), b = ld16(in.q + i * 32 + 16);
-    const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    write_q6_block(w, in.s[i], out, row, (int)(i - row * KB));
+    const uint4 a = ld16(in.q + i * 16);
+    const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+    write_q6_part(w, in.s[i / 2], out, row, (int)(i - row * KP) / 2, (int)(i & 1));
 }
 
 void launch_q8_to_q6(const ActQ8& in, int rows, ActH out, hipStream_t st) {
-    const size_t n = (size_t)rows * (in.K / 32);
+    const size_t n = (size_t)rows * (in.K / 16);
     hipLaunchKernelGGL(k_q8_to_q6, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, in, rows, out);
 }
 

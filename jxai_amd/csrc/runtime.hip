@@ -125,8 +125,8 @@ struct DevMat {
     uint8_t* qs = nullptr;
     uint8_t* sc = nullptr;
     uint8_t* ex = nullptr;  // Q5_0 / Q5_K high bits, Q6_K d
-    uint8_t* mn = nullptr;   // Q4_K / Q5_K min-term table (down GEMM)
-    uint8_t* g6 = nullptr;   // FP6 form and its min-term pieces (gate/up GEMM)
+    uint8_t* mn = nullptr;   // Q4_K / Q5_K min-term table (fp16 down GEMM)
+    uint8_t* g6 = nullptr;   // FP6 form and its min-term pieces (block GEMM)
     uint8_t* g6m = nullptr;
     void release() {
         for (uint8_t* p : {qs, sc, ex, mn, g6, g6m})
@@ -190,7 +190,8 @@ int upload_matrix(int type, int n_mats, int rows, int cols, const void* host, De
         jx::launch_repack(raw, m, out.qs, out.sc, out.ex, st);
         e = hipGetLastError();
     }
-    if (e == hipSuccess && gemm == Gemm::gateup && jx::g6_type(type) && q8_activation(type, cols) && cols % 128 == 0) {
+    // (a down projection without a Q8_0 form of h, or without the FP6 form, runs on the fp16 GEMM)
+    if (e == hipSuccess && gemm != Gemm::none && jx::g6_type(type) && q8_activation(type, cols) && cols % 128 == 0) {
         int* over = nullptr;
         int host_over = 0;
         m.g6_es = (size_t)m.nrt * (cols / 128) * jx::G6_HU;
@@ -208,7 +209,7 @@ int upload_matrix(int type, int n_mats, int rows, int cols, const void* host, De
         if (e == hipSuccess) e = hipMemcpyAsync(&host_over, over, sizeof(int), hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
         (void)hipFree(over);
-        if (e == hipSuccess && host_over) {  // a scale past fp16: gate/up stays on the GEMVs
+        if (e == hipSuccess && host_over) {  // a scale past fp16: no FP6 form
             (void)hipFree(out.g6);
             (void)hipFree(out.g6m);
             out.g6 = out.g6m = nullptr;
@@ -216,7 +217,7 @@ int upload_matrix(int type, int n_mats, int rows, int cols, const void* host, De
         m.g6 = out.g6;
         m.g6m = out.g6m;
     }
-    if (e == hipSuccess && gemm == Gemm::down && (type == jx::T_Q4_K || type == jx::T_Q5_K)) {
+    if (e == hipSuccess && gemm == Gemm::down && !m.g6 && (type == jx::T_Q4_K || type == jx::T_Q5_K)) {
         m.mn_es = (size_t)m.nrt * m.nkb * jx::MN_SB;
         e = hipMalloc(&out.mn, m.mn_es * n_mats);
         if (e == hipSuccess) {
@@ -240,8 +241,8 @@ int dalloc(T*& p, size_t n) {
     return JX_OK;
 }
 
-// Matrix-core activation buffers for `rows` rows of K: the hi form (the down GEMM's input),
-// or the FP6 form (gate/up), with its min-term pieces for K-quant weights.
+// Matrix-core activation buffers for `rows` rows of K: the fp16 form (fp16 down GEMM),
+// or the BF6 form (block GEMM), with its min-term pieces for K-quant weights.
 struct DevActH {
     jx::ActH a;
     void release() {
@@ -380,6 +381,12 @@ namespace {
 // whole super-blocks (the fp32 rows are stored padded that far).
 int down_h_k(int type, int f, bool f32) { return f32 && jx::is_kquant(type) ? (f + 255) / 256 * 256 : f; }
 
+// Whether a projection over K columns runs on the block GEMM: Q8_0 activations, a half-unit's multiple of
+// columns, and a format it takes in the form built at upload (Q8_0: the matrix as it is).
+bool block_gemm(const DevMat& D, int K, bool f32) {
+    return !f32 && K % 128 == 0 && jx::gemm_block_ok(D.m.type) && (D.m.type == jx::T_Q8_0 || D.m.g6);
+}
+
 int ensure_workspace(jx_moe_layer* L, int n) {
     if (n <= L->cap) return JX_OK;
     // captured graphs hold the old buffer addresses
@@ -416,11 +423,15 @@ int ensure_workspace(jx_moe_layer* L, int n) {
     auto any_gu = [&](auto pred) { return pred(L->gate.m) || (L->shared && pred(L->sgate.m)); };
     const bool x6 = any_gu([](const jx::QMat& m) { return m.g6 != nullptr; });
     const bool xmin = any_gu([](const jx::QMat& m) { return m.g6m != nullptr; });
-    if ((r = L->xh.alloc_fp6((size_t)cap, L->d, x6, xmin)) != JX_OK || (r = L->hh.alloc_hi(nk, hK)) != JX_OK) {
+    auto alloc_h = [](DevActH& h, size_t rows, const DevMat& D, int K, bool f32) {
+        return block_gemm(D, K, f32) ? h.alloc_fp6(rows, K, D.m.g6 != nullptr, D.m.g6m != nullptr) : h.alloc_hi(rows, K);
+    };
+    if ((r = L->xh.alloc_fp6((size_t)cap, L->d, x6, xmin)) != JX_OK ||
+        (r = alloc_h(L->hh, nk, L->down, hK, L->down_f32)) != JX_OK) {
         L->cap = 0;
         return r;
     }
-    if (L->shared && (r = L->hhs.alloc_hi((size_t)cap, hKs)) != JX_OK) {
+    if (L->shared && (r = alloc_h(L->hhs, (size_t)cap, L->sdown, hKs, L->sdown_f32)) != JX_OK) {
         L->cap = 0;
         return r;
     }
@@ -593,23 +604,21 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
         xdev = L->xn;
     }
     const int nk = n * k;
+    const int hK = down_h_k(L->down.m.type, L->F, L->down_f32);
     const int min_ppe = L->gate.m.type == jx::T_Q8_0                 ? MFMA_MIN_PAIRS_PER_EXPERT_Q8
                         : (size_t)d * L->F >= LARGE_EXPERT_ELEMS ? MFMA_MIN_PAIRS_PER_EXPERT_Q4_LARGE
                                                                  : MFMA_MIN_PAIRS_PER_EXPERT_Q4;
     bool mfma = (size_t)nk >= (size_t)min_ppe * E;
     if (flags & JX_FWD_FORCE_GEMV) mfma = false;
     if (flags & JX_FWD_FORCE_MFMA) mfma = true;
-    // The matrix-core GEMMs stage K in 128-element half-units and read the tables built at upload (gate/up: the
-    // FP6 form, Q8_0 matrices as they are; down: Q4_K / Q5_K the min table).  Gate/up takes the GEMM only with
-    // a Q8_0 form of x and a type whose products stay exact there (gemm_gateup_ok); otherwise it runs on
-    // the GEMVs (the multi-token form at prefill sizes) and the down projection still decides for itself.
-    auto gu_gemm = [&](const DevMat& G, const DevMat& U, bool f32) {
-        return !f32 && jx::gemm_gateup_ok(G.m.type) && d % 128 == 0 && (G.m.type == jx::T_Q8_0 || (G.m.g6 && U.m.g6));
-    };
+    // Gate/up takes the block GEMM (its products are exact: h is re-quantized) or the GEMVs (the multi-token
+    // form at prefill sizes); down the block GEMM, or for fp32 h, Q6_K and Q5_0 the fp16 one.
+    auto gu_gemm = [&](const DevMat& G, const DevMat& U, bool f32) { return block_gemm(G, d, f32) && block_gemm(U, d, f32); };
     auto dn_gemm = [&](const DevMat& D, int f, bool f32) {
-        return down_h_k(D.m.type, f, f32) % 128 == 0 &&
-               (!(D.m.type == jx::T_Q4_K || D.m.type == jx::T_Q5_K) || D.m.mn != nullptr);
+        return block_gemm(D, f, f32) || (down_h_k(D.m.type, f, f32) % 128 == 0 && jx::gemm_f16_ok(D.m));
     };
+    const bool dn_block = block_gemm(L->down, L->F, L->down_f32);
+    const bool sdn_block = L->shared && block_gemm(L->sdown, L->Fs, L->sdown_f32);
     const bool mfma_gu = mfma && gu_gemm(L->gate, L->up, L->gu_f32);
     const bool dn_shape = dn_gemm(L->down, L->F, L->down_f32);
     const bool smfma = L->shared && n >= L->smfma_min && !(flags & JX_FWD_FORCE_GEMV);
@@ -791,7 +800,9 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     auto shared_gateup = [&](hipStream_t ss) {
         if (smfma_gu) {
             Launch l(L, "shared_gateup_mfma", ss);
-            jx::launch_mfma_gateup(L->sgate.m, L->sup.m, L->xh.a, L->xq, sg, st_ub, L->sdown_f32 ? jx::ActQ8{} : L->hqs,
+            const bool h6 = smfma_dn && sdn_block && L->sdown.m.g6;  // h straight into its down's operand form
+            jx::launch_mfma_gateup(L->sgate.m, L->sup.m, L->xh.a, L->xq, sg, st_ub,
+                                   L->sdown_f32 || h6 ? jx::ActQ8{} : L->hqs, h6 ? L->hhs.a : jx::ActH{},
                                    L->sdown_f32 ? L->hfs : nullptr, ss);
         } else {
             Launch l(L, "shared_gateup_gemv", ss);
@@ -802,11 +813,16 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     auto shared_down = [&](hipStream_t ss) {
         if (smfma_dn) {
             Launch l(L, "shared_down", ss);
-            if (L->sdown_f32)
-                jx::launch_f32_to_acth(L->hfs, (int)fspad, n, L->hhs.a, ss);
-            else
-                jx::launch_q8_to_acth(L->hqs, n, L->hhs.a, ss);
-            jx::launch_mfma_down(L->sdown.m, L->hhs.a, sg, st_ub, L->ysh, ss);
+            if (sdn_block) {
+                if (L->sdown.m.g6 && !smfma_gu) jx::launch_q8_to_q6(L->hqs, n, L->hhs.a, ss);
+                jx::launch_mfma_down_block(L->sdown.m, L->hhs.a, L->hqs, sg, st_ub, L->ysh, ss);
+            } else {
+                if (L->sdown_f32)
+                    jx::launch_f32_to_acth(L->hfs, (int)fspad, n, L->hhs.a, ss);
+                else
+                    jx::launch_q8_to_acth(L->hqs, n, L->hhs.a, ss);
+                jx::launch_mfma_down(L->sdown.m, L->hhs.a, sg, st_ub, L->ysh, ss);
+            }
         } else if (sh_ksplit) {
             // the dense shared down's long K in parts, each block a routed block's share of units (the
             // combine adds the parts), so it is done before the routed gate/up that the routed down
@@ -843,7 +859,7 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     // the tile table; the GEMV blocks of the others exit at once.
     const bool hybrid = mfma && mfma_gu && mfma_down && !L->shared && dispatch_later && E >= HYBRID_MIN_E &&
                         !L->gu_f32 && !L->down_f32 && !(flags & JX_FWD_FORCE_MFMA) &&
-                        jx::mfma_down_ksplit(L->hh.a.K) == 1 && L->cold_pairs > 0;
+                        jx::mfma_down_ksplit(hK) == 1 && L->cold_pairs > 0;
     if (dispatch_later) {
         Launch l(L, "dispatch", st);
         jx::launch_dispatch(L->ids, nk, E, k, dout, st, hybrid ? L->cold_pairs : 0);
@@ -866,7 +882,9 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     const float* gxf = L->gu_f32 ? L->xf : nullptr;
     if (mfma_gu) {
         Launch l(L, "gateup_mfma", st);
-        jx::launch_mfma_gateup(L->gate.m, L->up.m, L->xh.a, L->xq, grp, tiles_ub, L->down_f32 ? jx::ActQ8{} : L->hq,
+        const bool h6 = mfma_down && dn_block && L->down.m.g6;  // h straight into its down's operand form
+        jx::launch_mfma_gateup(L->gate.m, L->up.m, L->xh.a, L->xq, grp, tiles_ub,
+                               L->down_f32 || h6 ? jx::ActQ8{} : L->hq, h6 ? L->hh.a : jx::ActH{},
                                L->down_f32 ? L->hf : nullptr, st);
     } else if (small_logits) {
         jx::Groups lg = grp;
@@ -903,10 +921,12 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
 
     int ks = 1;  // parts of the down GEMM's K (the combine adds them)
     if (mfma_down) {
-        {
+        if (dn_block ? L->down.m.g6 && !mfma_gu : true) {
             Launch l(L, "h_to_matrix_form", st);
             if (L->down_f32)
                 jx::launch_f32_to_acth(L->hf, (int)fpad, nk, L->hh.a, st);
+            else if (dn_block)
+                jx::launch_q8_to_q6(L->hq, nk, L->hh.a, st);
             else
                 jx::launch_q8_to_acth(L->hq, nk, L->hh.a, st);
         }
@@ -916,8 +936,11 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
             jx::launch_gemv_down_f16(L->down.m, L->hh.a, grp, slots, L->y, st);
         } else {
             Launch l(L, "down_mfma", st);
-            ks = jx::mfma_down_ksplit(L->hh.a.K);
-            jx::launch_mfma_down(L->down.m, L->hh.a, grp, tiles_ub, L->y, st, ks, L->ystride,
+            ks = jx::mfma_down_ksplit(hK);
+            if (dn_block)
+                jx::launch_mfma_down_block(L->down.m, L->hh.a, L->hq, grp, tiles_ub, L->y, st, ks, L->ystride);
+            else
+                jx::launch_mfma_down(L->down.m, L->hh.a, grp, tiles_ub, L->y, st, ks, L->ystride,
                                  nk <= jx::MFMA_DOWN_SMALL_MAX_PPE * E);
         }
     } else {
@@ -1479,8 +1502,8 @@ int jx_matmul_qkv_quant_f32_dev(jx_qmatrix* Wq, jx_qmatrix* Wk, jx_qmatrix* Wv, 
     }
     if (need_f32) jx::launch_copy_pad(x_dev, cols, (int)kpad, first->xf, st);
     for (int i = 0; i < 3; ++i) {
-        if (!Ws[i]) continue;
-        const int r = dev_gemv(Ws[i], quantized && q8_activation(Ws[i]->type, cols), first->xq, first->xf, outs[i], st);
+        if (!Ws[i] || done[i]) continue;
+        const int r = dev_gemv(Ws[i], false, first->xq, first->xf, outs[i], st);
         if (r != JX_OK) return r;
     }
     HIPCHK(hipGetLastError());
