@@ -107,14 +107,6 @@ __device__ __forceinline__ v16f mfma_min(b8 w, b8 x, v16f c) {
     return WROW ? mfma16b(w, x, c) : mfma16b(x, w, c);
 }
 
-// Keeps a uniform address in scalar registers, so loads take it with a 32-bit lane offset (the compiler
-// would otherwise add the lane offsets first and hold 64-bit vector addresses).
-typedef const __attribute__((address_space(1))) uint8_t gbyte;
-__device__ __forceinline__ gbyte* scalar(const uint8_t* p) {
-    gbyte* g = (gbyte*)p;
-    asm("" : "+s"(g));
-    return g;
-}
 // The lane offset beside it: redefined where it is used, so its widening stays in the load's own block.
 __device__ __forceinline__ uint32_t here(uint32_t v) {
     asm volatile("" : "+v"(v));
@@ -129,18 +121,6 @@ __device__ __forceinline__ v3i gload<v3i>(gbyte* p) {
     const __attribute__((address_space(1))) int* w = reinterpret_cast<const __attribute__((address_space(1))) int*>(p);
     return v3i{w[0], w[1], w[2]};
 }
-// 64 lanes x 16 bytes from src + off (per lane) into LDS at byte `lds` (wave-uniform), lane i at lds + 16 i.  In
-// asm because the compiler, which counts the builtin as a flat access, then waits for every load in flight
-// before it uses any.  It has no result registers; the waits are the kernel's own (vmcnt counts in order, so the
-// compiler's counted waits for the weights only get stricter).  Nothing else in the kernel uses m0.
-__device__ __forceinline__ void dma16g(gbyte* src, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(src) : "memory");
-}
-// The same from per-lane addresses.
-__device__ __forceinline__ void dma16v(const uint8_t* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
-}
-
 // What it writes.
 struct BgOut {
     ActQ8 hq;           // gate/up: h as Q8_0 (null q: not written),
@@ -244,12 +224,12 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)&sm;
     auto stage = [&](int h, int buf) {
         const uint32_t S = lds0 + buf * (uint32_t)sizeof(St);
-        gbyte* base = scalar(qsrc + (size_t)h * PB);
+        gbyte* base = dma_base(qsrc + (size_t)h * PB);
 #pragma unroll
         for (int k = 0; k < PER; ++k) dma16g(base, soff[k], S + (wave * PER + k) * 1024);
         if constexpr (I8) {
             if (wave == 0) {
-                gbyte* b = scalar(xsrc + (size_t)h * (HB * 8));
+                gbyte* b = dma_base(xsrc + (size_t)h * (HB * 8));
                 dma16g(b, xoff, S + offsetof(St, sx));
                 dma16g(b + 16, xoff, S + offsetof(St, sx) + GU_BN * 16);
             }
@@ -258,12 +238,12 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
             if (h & 1) {  // the super-block's min-term pieces, used at the end of its second half
                 const uint32_t sb = (uint32_t)(h >> 1) * G6M_SB;
                 const uint32_t d = S + offsetof(St, wm) + wave * 3072;
-                gbyte *m0 = scalar(wmb[0] + sb), *m1 = scalar(wmb[1] + sb);
+                gbyte *m0 = dma_base(wmb[0] + sb), *m1 = dma_base(wmb[1] + sb);
                 dma16g(m0, (uint32_t)lane * 16, d);
                 dma16g(m1, (uint32_t)lane * 16, d + 1024);
                 dma16v(wlo + sb, d + 2048);
                 if (wave == 0) {
-                    gbyte* b = scalar(xsrc + (size_t)(h >> 1) * 48);
+                    gbyte* b = dma_base(xsrc + (size_t)(h >> 1) * 48);
 #pragma unroll
                     for (int pc = 0; pc < 3; ++pc) dma16g(b + pc * 16, xoff, S + offsetof(St, xm) + pc * (GU_BN * 16));
                 }

@@ -21,6 +21,43 @@ __device__ __forceinline__ void dma4(const void* src, void* base) {
     __builtin_amdgcn_global_load_lds(src, (lds_ptr)base, 4, 0, 0);
 }
 
+// Keeps a uniform address in scalar registers, so loads take it with a 32-bit lane offset (the compiler
+// would otherwise add the lane offsets first and hold 64-bit vector addresses).
+typedef const __attribute__((address_space(1))) uint8_t gbyte;
+__device__ __forceinline__ gbyte* scalar(const uint8_t* p) {
+    gbyte* g = (gbyte*)p;
+    asm("" : "+s"(g));
+    return g;
+}
+// The same as the base of dma16g: past the wait states that a vector-memory read of a scalar register needs after a
+// vector instruction wrote it, which the compiler does not count into asm.
+__device__ __forceinline__ gbyte* dma_base(const uint8_t* p) {
+    gbyte* g = (gbyte*)p;
+    asm("s_nop 4" : "+s"(g));
+    return g;
+}
+// A wave-uniform address that the compiler computed in vector registers (a 64-bit product), in scalar ones.  (The
+// asm keeps the compiler from dropping the readfirstlane of a value it knows to be uniform.)
+__device__ __forceinline__ const uint8_t* uniform_ptr(const void* p) {
+    uint32_t lo = (uint32_t)(uint64_t)p, hi = (uint32_t)((uint64_t)p >> 32);
+    asm("s_nop 1" : "+v"(lo), "+v"(hi));
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    hi = __builtin_amdgcn_readfirstlane(hi);
+    return reinterpret_cast<const uint8_t*>((uint64_t)hi << 32 | lo);
+}
+
+// 64 lanes x 16 bytes from src (dma_base) + off (per lane) into LDS at byte `lds` (wave-uniform), lane i at lds + 16 i.  In
+// asm because the compiler, which counts the builtin as a flat access, then waits for every load in flight
+// before it uses any.  It has no result registers; the waits are the kernel's own (vmcnt counts in order, so the
+// compiler's counted waits for the weights only get stricter).  A kernel that uses it uses m0 for nothing else.
+__device__ __forceinline__ void dma16g(gbyte* src, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(src) : "memory");
+}
+// The same from per-lane addresses.
+__device__ __forceinline__ void dma16v(const uint8_t* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+
 __device__ __forceinline__ v16f mfma16(h8 a, h8 b, v16f c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }

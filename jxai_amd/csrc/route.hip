@@ -154,7 +154,7 @@ static RouteShape route_shape(const RouteArgs& a) {
     return r;
 }
 
-// rpb = 0: only steps 1-2 (the quantized and matrix-core forms of x), for k_route_rows.
+// rpb = 0: only steps 1-2 (the quantized and matrix-core forms of x), for k_route_mfma.
 template <int T>
 __global__ void __launch_bounds__(RT_THREADS) k_route(RouteArgs a, int nsplit, int rpb) {
     extern __shared__ __align__(16) float lds[];
@@ -343,110 +343,107 @@ __global__ void __launch_bounds__(RT_THREADS) k_route(RouteArgs a, int nsplit, i
     }
 }
 
-// Router logits for many tokens against a router of more than 16 rows with
-// d <= 2048 (d / 64 in 8, 16, 24, 32): a block owns 16 rows and tpb tokens.  Lane j
-// of a row's 16-lane group keeps its whole vec_dot_f32 chain of router values
-// in registers (read once), and the tokens stream through LDS four at a time,
-// chain-major, the next chunk's loads in flight while the current one is
-// consumed.  Router traffic is one read per block instead of one per 4 tokens.
-// Same chain order and reduction as k_route (src/quant.cpp:2756-2778).
-#ifndef JX_RR_TPB
-#define JX_RR_TPB 32
-#endif
-#ifndef JX_RR_TC
-#define JX_RR_TC 4
-#endif
-constexpr int RR_TPB = JX_RR_TPB;  // tokens per block, at most (fewer keep small batches spread)
-constexpr int RR_TC = JX_RR_TC;    // tokens per LDS chunk
+// Router logits for many tokens against a router of more than 16 rows, on the matrix cores: a step of a
+// vec_dot_f32 chain (src/quant.cpp:2756-2778) for 64 tokens x 16 rows is one v_mfma_f32_16x16x1_4b_f32, an
+// inner length of 1, so each result is one fused multiply-add rounded once: the chains' own arithmetic, in
+// their order, at twice the vector unit's rate and from one operand register a side.  (Register-resident
+// router rows against tokens from LDS, a 16-byte LDS read per four multiply-adds, were LDS-bound.)  A block
+// owns 64 tokens and 16 rows, wave q the chains 4q .. 4q + 3 (a row's elements 16 i + 4q ..: one 16-byte LDS read
+// of each operand per step).  Chunks of 4 steps come by DMA, three in flight (16-byte pieces XOR-swizzled by row
+// against bank conflicts).
+// Qwen3-shaped 2048 tokens (128 x 2048): 46 -> 24 us.
+constexpr int RM_T = 64, RM_R = 16, RM_C = 64, RM_NB = 4;  // tokens, rows, floats per chunk, buffers
 
-template <int M4>  // d / 64 float4 chain steps per lane
-__global__ void __launch_bounds__(RT_THREADS) k_route_rows(RouteArgs a, int nsplit, int tpb) {
-    extern __shared__ __align__(16) float xs[];  // [2][RR_TC][16][S]
-    constexpr int d = 64 * M4, C4 = d / 4, S = rs_stride(d), RS = 16 * S, Sg = chain_stride_of(d);
-    constexpr int PER = (RR_TC * C4 + RT_THREADS - 1) / RT_THREADS;  // float4 per thread per chunk
-    const int split = blockIdx.x % nsplit, t0 = (blockIdx.x / nsplit) * tpb;
-    const int tend = min(a.n, t0 + tpb);
-    const int tid = threadIdx.x, grp = tid >> 4, j = tid & 15;
-    const int E = a.E, R = E + (a.shgate ? 1 : 0);
-    const int r = split * RT_GROUPS + grp;
-    const bool live = r < R;
-    float4 w[M4];
-    {
-        const float* wr = a.router_cm + (size_t)min(r, R - 1) * 16 * Sg + j * Sg;
+__global__ void __launch_bounds__(RT_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_route_mfma(RouteArgs a) {
+    __shared__ __align__(16) float lds[RM_NB][RM_T + RM_R][RM_C];  // row r, piece c at piece c ^ (r % 16)
+    const int tid = threadIdx.x, lane = tid & 63, q = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int t0 = (int)blockIdx.y * RM_T, r0 = (int)blockIdx.x * RM_R;  // the row splits of a token block in a row
+    const int d = a.d, E = a.E, R = E + (a.shgate ? 1 : 0), nc = d / RM_C;
+    // a wave's DMAs of a chunk: tokens 16 q .. 16 q + 15 and rows 4 q .. 4 q + 3 (past the last: repeated, dropped below)
+    const int l4 = lane >> 4, c16 = lane & 15;
+    uint32_t xoff[4];
 #pragma unroll
-        for (int i = 0; i < M4; ++i) w[i] = *reinterpret_cast<const float4*>(wr + 4 * i);
+    for (int u = 0; u < 4; ++u) {
+        const int r = 16 * q + 4 * u + l4;
+        xoff[u] = (uint32_t)(min(t0 + r, a.n - 1) - t0) * (uint32_t)(d * 4) + (uint32_t)((c16 ^ (r & 15)) << 4);
     }
-    // chunk staging: RR_TC tokens x d floats; float4 c of token t holds chains 4(c%4)..4(c%4)+3 at step c/4
-    float4 v[PER];
-    auto issue = [&](int c0) {
-        const int last = min(RR_TC, tend - c0) * C4 - 1;
+    const int rw = 4 * q + l4, rr = min(r0 + rw, R - 1);
+    const uint8_t* wsrc = reinterpret_cast<const uint8_t*>(rr < E ? a.router + (size_t)rr * d : a.shgate) + ((c16 ^ rw) << 4);
+    const uint8_t* xsrc = uniform_ptr(a.x + (size_t)t0 * d);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)&lds[0][0][0];
+    auto stage = [&](int c) {  // 5 DMAs, also past the last chunk (a buffer nothing reads any more)
+        const uint32_t b = lds0 + (uint32_t)(c % RM_NB) * (uint32_t)sizeof(lds[0]);
+        const size_t o = (size_t)min(c, nc - 1) * (RM_C * 4);
+        gbyte* base = dma_base(xsrc + o);
 #pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int i = min(u * RT_THREADS + tid, last);
-            v[u] = *reinterpret_cast<const float4*>(a.x + (size_t)c0 * d + 4 * i);
-        }
+        for (int u = 0; u < 4; ++u) dma16g(base, xoff[u], b + (16 * q + 4 * u) * (RM_C * 4));
+        dma16v(wsrc + o, b + (RM_T + 4 * q) * (RM_C * 4));
     };
-    auto store = [&](int c0, float* buf) {
-        const int last = min(RR_TC, tend - c0) * C4 - 1;
+    v16f acc[4];
 #pragma unroll
-        for (int u = 0; u < PER; ++u) {
-            const int i = min(u * RT_THREADS + tid, last);  // clamped duplicates store the same values
-            const int t = i / C4, c = i % C4;
-            float* dst = buf + t * RS + 4 * (c & 3) * S + (c >> 2);
-            dst[0] = v[u].x;
-            dst[S] = v[u].y;
-            dst[2 * S] = v[u].z;
-            dst[3 * S] = v[u].w;
+    for (int k = 0; k < 4; ++k) acc[k] = v16f{};
+    for (int c = 0; c < RM_NB - 1; ++c) stage(c);
+    for (int c = 0; c < nc; ++c) {
+        // chunk c is in (two younger ones are not), and every wave has read chunk c - 1
+        asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)" ::: "memory");
+        static_assert(RM_NB == 4, "two chunks of 5 DMAs younger than the one waited for");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        stage(c + RM_NB - 1);
+        const float(*buf)[RM_C] = lds[c % RM_NB];
+#pragma unroll
+        for (int i = 0; i < RM_C / 16; ++i) {
+            const int at = ((4 * i + q) ^ c16) * 4;  // both rows are lane % 16 modulo 16
+            const float4 x4 = *reinterpret_cast<const float4*>(&buf[lane][at]);
+            const float4 w4 = *reinterpret_cast<const float4*>(&buf[RM_T + c16][at]);
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x1f32(x4.x, w4.x, acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x1f32(x4.y, w4.y, acc[1], 0, 0, 0);
+            acc[2] = __builtin_amdgcn_mfma_f32_16x16x1f32(x4.z, w4.z, acc[2], 0, 0, 0);
+            acc[3] = __builtin_amdgcn_mfma_f32_16x16x1f32(x4.w, w4.w, acc[3], 0, 0, 0);
         }
-    };
-    issue(t0);
-    store(t0, xs);
-    int buf = 0;
-    for (int c0 = t0; c0 < tend; c0 += RR_TC) {
-        const int nt = min(RR_TC, tend - c0);
-        if (c0 + RR_TC < tend) issue(c0 + RR_TC);  // block-uniform
-        __syncthreads();  // chunk c0 staged; the other buffer's readers are done
-        const float* xb = xs + buf * RR_TC * RS;
-        if (live) {
-            const float* xr[RR_TC];
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the buffers are reused: no DMA may still land
+    // acc0[j] + acc1[j] (chains j and j + 8: waves 0 and 2, 1 and 3), then their sum from j = 0 on
+    __syncthreads();
+    float* red = &lds[0][0][0];  // [2 waves][4 chains][16][64]
+    static_assert(2 * 4 * 16 * 64 <= RM_NB * (RM_T + RM_R) * RM_C, "the chains' sums fit the staging buffers");
+    if (q >= 2)
 #pragma unroll
-            for (int t = 0; t < RR_TC; ++t) xr[t] = xb + min(t, nt - 1) * RS + j * S;
-            float acc[RR_TC];
+        for (int k = 0; k < 4; ++k)
 #pragma unroll
-            for (int t = 0; t < RR_TC; ++t) acc[t] = 0.0f;
+            for (int v = 0; v < 16; ++v) red[(((q - 2) * 4 + k) * 16 + v) * 64 + lane] = acc[k][v];
+    __syncthreads();
+    float sum[16];
+    if (q < 2) {
 #pragma unroll
-            for (int i = 0; i < M4; ++i) {
+        for (int v = 0; v < 16; ++v) {
 #pragma unroll
-                for (int t = 0; t < RR_TC; ++t) {
-                    const float4 x4 = *reinterpret_cast<const float4*>(xr[t] + 4 * i);
-                    acc[t] = __builtin_fmaf(w[i].x, x4.x, acc[t]);
-                    acc[t] = __builtin_fmaf(w[i].y, x4.y, acc[t]);
-                    acc[t] = __builtin_fmaf(w[i].z, x4.z, acc[t]);
-                    acc[t] = __builtin_fmaf(w[i].w, x4.w, acc[t]);
-                }
-            }
-            float sums[RR_TC];
+            for (int k = 0; k < 4; ++k) acc[k][v] += red[((q * 4 + k) * 16 + v) * 64 + lane];
+            sum[v] = 0.0f;
+            if (q == 0)
 #pragma unroll
-            for (int t = 0; t < RR_TC; ++t) {
-                const float hi = __shfl_down(acc[t], 8, 16);
-                const float vv = acc[t] + hi;  // acc0[j] + acc1[j] for j < 8
-                float sum = 0.0f;
-#pragma unroll
-                for (int q = 0; q < 8; ++q) sum += __shfl(vv, q, 16);
-                sums[t] = sum;
-            }
-#pragma unroll
-            for (int t = 0; t < RR_TC; ++t) {
-                const float sum = sums[t];
-                if (j == 0 && t < nt) {
-                    const size_t tok = (size_t)(c0 + t);
-                    if (r < E) a.logits[tok * E + r] = a.bias ? sum + a.bias[r] : sum;
-                    else a.shscale[tok] = sum;  // raw shared-gate logit; k_route_topk applies the sigmoid
-                }
-            }
+                for (int k = 0; k < 4; ++k) sum[v] += acc[k][v];
         }
-        if (c0 + RR_TC < tend) store(c0 + RR_TC, xs + (buf ^ 1) * RR_TC * RS);
-        buf ^= 1;
+    }
+    __syncthreads();
+    if (q == 0)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) red[v * 64 + lane] = sum[v];
+    __syncthreads();
+    if (q != 1) return;
+    const int r = r0 + (lane & 15);
+    if (r >= R) return;
+    const float bias = r < E && a.bias ? a.bias[r] : 0.0f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {  // result of tokens 16 (v / 4) + 4 (lane / 16) + v % 4, row lane % 16
+        float s = red[v * 64 + lane];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s += acc[k][v];
+        const int tok = t0 + 16 * (v >> 2) + 4 * (lane >> 4) + (v & 3);
+        if (tok >= a.n) continue;
+        if (r < E) a.logits[(size_t)tok * E + r] = a.bias ? s + bias : s;
+        else a.shscale[tok] = s;  // raw shared-gate logit; k_route_topk applies the sigmoid
     }
 }
 
@@ -469,45 +466,24 @@ static void launch_route_topk(const RouteArgs& a, hipStream_t st) {
     else hipLaunchKernelGGL(k_route_topk<MAX_E / 64>, grid, dim3(256), 0, st, a);
 }
 
-static bool route_rows_fits(const RouteArgs& a) {
-    const int R = a.E + (a.shgate ? 1 : 0);
-    const int m4 = a.d / 64;
-// below ~512 tokens the split k_route (one token per block, router from L2) measured faster
-#ifndef JX_RR_MIN_N
-#define JX_RR_MIN_N 512
-#endif
-    // (F16 / BF16 routers: two chain columns per lane would not fit the register-resident rows)
-    return R > RT_GROUPS && a.d % 64 == 0 && (m4 == 8 || m4 == 16 || m4 == 24 || m4 == 32) && a.n >= JX_RR_MIN_N &&
-           !a.chain8;
+// The matrix-core router: more than 16 rows (fewer leave most of a result's 16 columns empty) in the fp32 chain
+// order (F16 / BF16 rows have another), whole chunks, and from 512 tokens on (below, the split
+// k_route, one token per block, fills more CUs).
+static bool route_mfma_fits(const RouteArgs& a) {
+    return a.E + (a.shgate ? 1 : 0) > RT_GROUPS && a.d % RM_C == 0 && a.n >= 512 && a.n <= 65535 * RM_T && !a.chain8;
 }
 
 void launch_route(const RouteArgs& a, hipStream_t st) {
-    if (route_rows_fits(a)) {
-        // quantized / matrix-core forms of x, then the logits with register-resident router rows, then top-k
-        const int T = a.n >= 256 ? 4 : 1;
+    if (route_mfma_fits(a)) {
+        // quantized / matrix-core forms of x, then the logits, then top-k
+        const int T = route_lds(4, a.d, a.E) <= RT_LDS_TARGET ? 4 : route_lds(2, a.d, a.E) <= RT_LDS_TARGET ? 2 : 1;
         const size_t lq = route_lds(T, a.d, a.E);
-        auto q = T == 4 ? k_route<4> : k_route<1>;
+        auto forms = T == 4 ? k_route<4> : T == 2 ? k_route<2> : k_route<1>;
         if (lq > 65536)
-            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(q), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)lq);
-        hipLaunchKernelGGL(q, dim3((a.n + T - 1) / T), dim3(RT_THREADS), lq, st, a, 1, 0);
-        const int R = a.E + (a.shgate ? 1 : 0), RS = (R + RT_GROUPS - 1) / RT_GROUPS;
-        const size_t lr = (size_t)2 * RR_TC * 16 * rs_stride(a.d) * sizeof(float);
-        // tokens per block: about 512 blocks in all, in whole LDS chunks, at most RR_TPB
-        const int tpb = std::min(RR_TPB, std::max(RR_TC, ((a.n * RS + 511) / 512 + RR_TC - 1) / RR_TC * RR_TC));
-        const dim3 grid(RS * ((a.n + tpb - 1) / tpb));
-        auto go = [&](auto kern) {
-            if (lr > 65536)
-                (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lr);
-            hipLaunchKernelGGL(kern, grid, dim3(RT_THREADS), lr, st, a, RS, tpb);
-        };
-        switch (a.d / 64) {
-            case 8: go(k_route_rows<8>); break;
-            case 16: go(k_route_rows<16>); break;
-            case 24: go(k_route_rows<24>); break;
-            default: go(k_route_rows<32>); break;
-        }
+            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(forms), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lq);
+        hipLaunchKernelGGL(forms, dim3((a.n + T - 1) / T), dim3(RT_THREADS), lq, st, a, 1, 0);
+        const int R = a.E + (a.shgate ? 1 : 0), RS = (R + RM_R - 1) / RM_R;
+        hipLaunchKernelGGL(k_route_mfma, dim3(RS, (a.n + RM_T - 1) / RM_T), dim3(RT_THREADS), 0, st, a);
         launch_route_topk(a, st);
         return;
     }

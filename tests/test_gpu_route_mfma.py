@@ -1,0 +1,30 @@
+"""Router logits on the matrix cores (more than 16 rows, many tokens): bit-exact, at the edges of its blocks."""
+import numpy as np
+import pytest
+
+from jxai_amd import formats as F
+from jxai_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+# rows: one more than a block's 16, a ragged last block with the shared gate's row, several full ones; tokens: 64 a
+# block; d: fewer chunks than buffers and more (64 floats a chunk)
+@pytest.mark.parametrize("E,shared,d", [(17, False, 128), (24, True, 704), (64, False, 2304)])
+@pytest.mark.parametrize("n", [512, 575, 641])
+def test_router_logits_bitexact(port, E, shared, d, n):
+    from jxai_amd import moe
+    moe.init(0)
+    print(f"[gpu] router E={E} shared={shared} d={d} n={n}", flush=True)
+    cfg = synth.LayerConfig(f"rm_{E}_{d}", d, E, 4, 256, F.Q4_0, d_ff_shared=256 if shared else 0, shared_gate=shared)
+    lw = synth.make_layer(cfg)
+    x = synth.make_tokens(cfg, n)
+    x[3] = 0.0
+    x[5] *= np.float32(1e-30)  # subnormal products
+    L = moe.MoELayer.from_weights(lw)
+    _, ids, w, _ = L.forward(x)
+    lg_o, ids_o, w_o = port.route(lw, x)
+    assert np.array_equal(L.last_logits(n).view(np.uint32), lg_o.view(np.uint32))
+    assert np.array_equal(ids, ids_o)
+    np.testing.assert_allclose(w, w_o, rtol=2e-6, atol=0)
+    L.close()
