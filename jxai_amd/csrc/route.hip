@@ -877,20 +877,18 @@ void launch_route_small(const RouteArgs& a, const DispatchOut& o, hipStream_t st
 // offset, MFMA tile offset and active-list slot, then writes the positions of
 // its (token, slot) pairs in flat order -- a stable counting sort, so tokens
 // keep their order inside each expert.
-//  - histogram: four ids per thread per 16-byte load; up to 16 experts by
-//    wave ballots (LDS atomics on so few bins would serialize), else LDS atomics;
-//  - positions: rounds of up to 4 x DP_U x 256 ids, each wave a contiguous quarter:
-//    one pass records the matches as a 64-bit mask per lane (4 ids x DP_U loads),
+//  - ids: rounds of 4 x U x 256 ids, each wave a contiguous quarter; a lane's U 16-byte loads of a round are all
+//    in flight at once (loaded one by one, their latencies were most of the kernel: 16384 ids over 128 experts
+//    20 -> 15 us), and a batch of one round keeps them in registers for both passes;
+//  - histogram: up to 16 experts by packed per-thread counters (LDS atomics on so few bins would serialize), else
+//    LDS atomics;
+//  - positions: the matches as a 64-bit mask per lane (4 ids x U loads),
 //    one barrier exchanges the wave totals, and the writes follow the masks
 //    in flat order (lane prefixes from three ballots of the per-lane count).
 constexpr int DISPATCH_THREADS = 256;
 constexpr int DP_U = 16;  // 16-byte id loads per lane per round, at most
 
-__device__ __forceinline__ int4 load_ids4(const int* ids, int f, int nk) {
-    if (f + 3 < nk) return *reinterpret_cast<const int4*>(ids + f);  // ids 16-byte aligned, f % 4 == 0
-    return make_int4(f < nk ? ids[f] : -1, f + 1 < nk ? ids[f + 1] : -1, f + 2 < nk ? ids[f + 2] : -1, -1);
-}
-
+template <int U>
 __global__ void __launch_bounds__(DISPATCH_THREADS)
 k_dispatch(const int* ids, int nk, int E, int top_k, DispatchOut o, int cold_max) {
     extern __shared__ int hist[];
@@ -898,8 +896,24 @@ k_dispatch(const int* ids, int nk, int E, int top_k, DispatchOut o, int cold_max
     __shared__ int wtot[2][DISPATCH_THREADS / 64];
     const int e = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int NW = DISPATCH_THREADS / 64;
+    constexpr int NW = DISPATCH_THREADS / 64, ROUND = NW * 256 * U;
     for (int i = tid; i < E; i += DISPATCH_THREADS) hist[i] = 0;
+    // a round's ids, -1 past the last: group f (4 ids) by one load where it is whole, the last partial one from `tail`
+    const int whole = nk & ~3;
+    int4 v[U];
+    const int4 tail = make_int4(whole < nk ? ids[whole] : -1, whole + 1 < nk ? ids[whole + 1] : -1,
+                                whole + 2 < nk ? ids[whole + 2] : -1, -1);
+    auto load = [&](int r0) {
+        const int f0 = r0 + wave * 256 * U + 4 * lane;
+        if (whole > 0)  // block-uniform
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = *reinterpret_cast<const int4*>(ids + min(f0 + 256 * u, whole - 4));
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int f = f0 + 256 * u;
+            if (f >= whole) v[u] = f == whole ? tail : make_int4(-1, -1, -1, -1);
+        }
+    };
     __syncthreads();
     if (E <= 16) {
         // per-thread 8-bit counters (experts 0-7 in lo, 8-15 in hi), flushed before any can reach 256
@@ -919,25 +933,35 @@ k_dispatch(const int* ids, int nk, int E, int top_k, DispatchOut o, int cold_max
             lo += id >= 0 && id < 8 ? one : 0ull;
             hi += id >= 8 ? one : 0ull;
         };
-        for (int base = wave * 256; base < nk; base += DISPATCH_THREADS * 4) {  // wave-uniform
-            const int4 v = load_ids4(ids, base + 4 * lane, nk);
-            count(v.x);
-            count(v.y);
-            count(v.z);
-            count(v.w);
-            if (++since == 63) {  // 63 * 4 = 252 per counter at most
+        for (int r0 = 0; r0 < nk; r0 += ROUND) {
+            load(r0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                count(v[u].x);
+                count(v[u].y);
+                count(v[u].z);
+                count(v[u].w);
+            }
+            since += U;
+            if (since + U > 63) {  // 63 * 4 = 252 per counter at most
                 flush();
                 since = 0;
             }
         }
         flush();
     } else {
-        for (int f = 4 * tid; f < nk; f += 4 * DISPATCH_THREADS) {
-            const int4 v = load_ids4(ids, f, nk);
-            atomicAdd(&hist[v.x], 1);
-            if (v.y >= 0) atomicAdd(&hist[v.y], 1);
-            if (v.z >= 0) atomicAdd(&hist[v.z], 1);
-            if (v.w >= 0) atomicAdd(&hist[v.w], 1);
+        auto count = [&](int id) {
+            if (id >= 0) atomicAdd(&hist[id], 1);
+        };
+        for (int r0 = 0; r0 < nk; r0 += ROUND) {
+            load(r0);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                count(v[u].x);
+                count(v[u].y);
+                count(v[u].z);
+                count(v[u].w);
+            }
         }
     }
     __syncthreads();
@@ -986,19 +1010,15 @@ k_dispatch(const int* ids, int nk, int E, int top_k, DispatchOut o, int cold_max
         o.tiles[toff + i] = make_int4(e, off + i * MFMA_BN, min(MFMA_BN, cnt - i * MFMA_BN), 0);
     if (cnt == 0) return;  // block-uniform
     const uint64_t lt_mask = (1ull << lane) - 1ull;
-    // loads per lane and round: up to DP_U, fewer when the pairs fit, so every wave takes a share
-    const int U = min(DP_U, (nk + NW * 256 - 1) / (NW * 256));
     int run = off;
-    for (int r0 = 0, par = 0; r0 < nk; r0 += NW * 256 * U, par ^= 1) {
+    for (int r0 = 0, par = 0; r0 < nk; r0 += ROUND, par ^= 1) {
         const int wbase = r0 + wave * 256 * U;
+        if (nk > ROUND) load(r0);  // (a single round's ids are still here)
         uint64_t bits = 0;  // bit 4u + c: id wbase + 256u + 4 lane + c is expert e
 #pragma unroll
-        for (int u = 0; u < DP_U; ++u) {
-            if (u < U) {  // uniform
-                const int4 v = load_ids4(ids, wbase + 256 * u + 4 * lane, nk);
-                const uint32_t m = (v.x == e) | (v.y == e) << 1 | (v.z == e) << 2 | (v.w == e) << 3;
-                bits |= (uint64_t)m << (4 * u);
-            }
+        for (int u = 0; u < U; ++u) {
+            const uint32_t m = (v[u].x == e) | (v[u].y == e) << 1 | (v[u].z == e) << 2 | (v[u].w == e) << 3;
+            bits |= (uint64_t)m << (4 * u);
         }
         int wt = __popcll(bits);
 #pragma unroll
@@ -1034,8 +1054,13 @@ k_dispatch(const int* ids, int nk, int E, int top_k, DispatchOut o, int cold_max
 }
 
 void launch_dispatch(const int* ids, int nk, int E, int top_k, const DispatchOut& o, hipStream_t st, int cold_max) {
-    hipLaunchKernelGGL(k_dispatch, dim3(E), dim3(DISPATCH_THREADS), (size_t)E * sizeof(int), st, ids, nk, E, top_k, o,
-                       cold_max);
+    // loads per lane and round: the fewest (1, 4 or 16) that take the pairs in one
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(E), dim3(DISPATCH_THREADS), (size_t)E * sizeof(int), st, ids, nk, E, top_k, o, cold_max);
+    };
+    if (nk <= DISPATCH_THREADS * 4) go(k_dispatch<1>);
+    else if (nk <= DISPATCH_THREADS * 16) go(k_dispatch<4>);
+    else go(k_dispatch<DP_U>);
 }
 
 // sum_i x[i] * x[i] over one row in vec_dot_f32's order (src/quant.cpp:2756-2778;
