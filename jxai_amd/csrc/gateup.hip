@@ -132,6 +132,11 @@ struct BgOut {
     size_t ystride;
 };
 
+template <int N>
+struct Tiles {
+    static constexpr int value = N;
+};
+
 // The weight ring: one 32-block of a row tile.
 template <int KIND>
 struct Wt {
@@ -148,9 +153,15 @@ struct Wt<GU_I8> {
     }
 };
 
+// PARTS: a workgroup with at most 32 pairs (an expert's last part, or all of them at a few pairs per expert) stages and
+// multiplies one pair tile.  The second loop costs the FP6 kernels register copies (Mixtral-shaped 512 tokens 684 ->
+// 697 us per step), so they take it where the average expert has fewer than BG_FEW pairs (Qwen1.5-shaped 200 tokens
+// 229 -> 210 us, DeepSeek-V2-Lite-shaped 130 tokens 213 -> 208 us, 13 and 12 pairs; Mixtral-shaped 150 tokens, 37
+// pairs, 370 -> 376 us); the int8 kernel always (Qwen3-shaped 64 / 600 / 2048 tokens 125 / 246 / 404 -> 107 / 232 /
+// 393 us).
 // Registers at two waves per SIMD (256): acc 64, two (S, P) sets 64, the weight ring 24 and its scales 16 (FP6),
 // operands 16 and the doubled weight codes 12.
-template <int KIND, bool GATEUP>
+template <int KIND, bool GATEUP, bool PARTS>
 __global__ void __launch_bounds__(GU_WAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut o) {
     constexpr bool I8 = KIND == GU_I8, MIN = KIND == GU_F6_MIN;
@@ -226,7 +237,9 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
         const uint32_t S = lds0 + buf * (uint32_t)sizeof(St);
         gbyte* base = dma_base(qsrc + (size_t)h * PB);
 #pragma unroll
-        for (int k = 0; k < PER; ++k) dma16g(base, soff[k], S + (wave * PER + k) * 1024);
+        for (int k = 0; k < PER; ++k)
+            if (!PARTS || wave * PER * PPI < cnt)  // (the wave's rows are in use)
+                dma16g(base, soff[k], S + (wave * PER + k) * 1024);
         if constexpr (I8) {
             if (wave == 0) {
                 gbyte* b = dma_base(xsrc + (size_t)h * (HB * 8));
@@ -298,7 +311,8 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
         __builtin_amdgcn_sched_barrier(0);  // in the ring's order: the loop waits by count
     }
 
-    auto half = [&](int h, bool odd) {
+    auto half = [&](int h, bool odd, auto tiles) __attribute__((always_inline)) {
+        constexpr int NT = decltype(tiles)::value;  // pair tiles in use
         // this half-unit's DMAs are older than the ring loads (Q8_0 16, FP6 10); the other waves' reads of the other stage are done
         if constexpr (I8) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
         else asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)" ::: "memory");
@@ -332,12 +346,12 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
                 bp[t] = *reinterpret_cast<const v2i*>(q + (b1 ^ ((4 + j) << 4)));
             }
         };
-        read_b(0, 0);
-        read_b(1, 0);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) read_b(t, 0);
 #pragma unroll
         for (int j = 0; j < HB; ++j) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
+            for (int k = 0; k < 2 * NT; ++k) {
                 const int i = k & 1, t = k >> 1, c = k & 1;
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (I8) {
@@ -353,7 +367,7 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
                     P[c] = mfma_scales<GATEUP>(__builtin_bit_cast(h4, j < 2 ? v2i{ws[0], ws[1]} : v2i{ws[2], ws[3]}),
                                               __builtin_bit_cast(h4, bp[t]));
                 }
-                if (j > 0 || k > 0) fold((k + 3) & 1, ((k + 3) & 3) >> 1, c ^ 1);  // the tile before
+                if (j > 0 || k > 0) fold(c ^ 1, ((k + 2 * NT - 1) % (2 * NT)) >> 1, c ^ 1);  // the tile before
                 if (i == 1 && j + 1 < HB) read_b(t, j + 1);
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
                 __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);  // VALU
@@ -363,7 +377,7 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
             __builtin_amdgcn_sched_barrier(0);
             load(hn, j, o0, o1);
         }
-        fold(1, 1, 1);
+        fold(1, NT - 1, 1);
         if constexpr (MIN) {
             if (odd) {
                 // acc += sum_j (dx_j sum q_j)(-dmin m_j): six of the nine piece products (all above 2^-24
@@ -372,7 +386,7 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
                 const uint8_t* wm = cur.wm + wave * 3072 + n * 16;
                 b8 x0[2], x1[2];
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
+                for (int t = 0; t < NT; ++t) {
                     const uint16_t* xp = cur.xm + (32 * t + n) * 8;
                     x0[t] = *reinterpret_cast<const b8*>(xp + (g ? 1 : 0) * GU_BN * 8);
                     x1[t] = *reinterpret_cast<const b8*>(xp + (g ? 2 : 0) * GU_BN * 8);
@@ -383,7 +397,7 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
                     const b8 w1 = *reinterpret_cast<const b8*>(wm + i * 1024 + (g ? 0 : 512));
                     const b8 w2 = *reinterpret_cast<const b8*>(wm + (g ? i * 1024 + 512 : 2048 + i * 512));
 #pragma unroll
-                    for (int t = 0; t < 2; ++t) {
+                    for (int t = 0; t < NT; ++t) {
                         acc[i][t] = mfma_min<GATEUP>(w0, x0[t], acc[i][t]);
                         acc[i][t] = mfma_min<GATEUP>(w1, x1[t], acc[i][t]);
                         acc[i][t] = mfma_min<GATEUP>(w2, x0[t], acc[i][t]);
@@ -392,10 +406,14 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
             }
         }
     };
-    for (int h = h0; h < h1; h += 2) {
-        half(h, false);
-        if (h + 1 < h1) half(h + 1, true);
-    }
+    auto run = [&](auto tiles) __attribute__((always_inline)) {
+        for (int h = h0; h < h1; h += 2) {
+            half(h, false, tiles);
+            if (h + 1 < h1) half(h + 1, true, tiles);
+        }
+    };
+    if (!PARTS || cnt > 32) run(Tiles<2>{});
+    else run(Tiles<1>{});
 
     if constexpr (!GATEUP) {
         // lane (n, g) holds row n of a row tile and, in register r, pair 8 (r / 4) + 4 g + r % 4 of a pair tile
@@ -407,6 +425,7 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
             for (int t = 0; t < 2; ++t)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
+                    if (32 * t >= cnt) break;
                     const int pr = 32 * t + 8 * (r >> 2) + 4 * g + (r & 3);
                     if (pr < cnt) y[(size_t)pr * W0.rows + (2 * slot + i) * 32 + n] = acc[i][t][r];
                 }
@@ -417,6 +436,7 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
     if (!active) return;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
+        if (32 * t >= cnt) return;
         float v[16];
 #pragma unroll
         for (int c = 0; c < 16; ++c) v[c] = gated(acc[0][t][c], acc[1][t][c], W0.act);
@@ -555,35 +575,39 @@ __global__ void __launch_bounds__(256) k_g6_min_table(QMat m, uint8_t* out) {
 // Workgroups of an item list over row groups of `slots` row-tile slots.
 template <int KIND, bool GATEUP>
 void launch_kind(const QMat& w0, const QMat& w1, const GuIn& in, const Groups& grp, int tiles_ub, const BgOut& o,
-                 hipStream_t st) {
+                 bool few, hipStream_t st) {
     const int slots = GATEUP ? w0.nrt : (w0.nrt + 1) / 2;
     const int R = (slots + GU_WAVES - 1) / GU_WAVES;
     const int n_items = R * tiles_ub * (MFMA_BN / GU_BN);
     if (n_items <= 0) return;
-    hipLaunchKernelGGL((k_bgemm<KIND, GATEUP>), dim3(n_items * (GATEUP ? 1 : o.KS)), dim3(GU_WAVES * 64), 0, st, w0, w1, in,
-                       grp, R, n_items, std::min(GATEUP ? GU_RC : DN_RC, R), o);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(n_items * (GATEUP ? 1 : o.KS)), dim3(GU_WAVES * 64), 0, st, w0, w1, in, grp, R, n_items,
+                           std::min(GATEUP ? GU_RC : DN_RC, R), o);
+    };
+    if (KIND == GU_I8 || few) go(k_bgemm<KIND, GATEUP, true>);
+    else if constexpr (KIND != GU_I8) go(k_bgemm<KIND, GATEUP, false>);
 }
 
 // The launch of a matrix (pair)'s format over x's forms; false: a form is missing (a caller bug: nothing is
 // launched on null pointers).
 template <bool GATEUP>
 bool launch_form(const QMat& w0, const QMat& w1, const ActH& x6, const ActQ8& xq, const Groups& grp, int tiles_ub,
-                 const BgOut& o, hipStream_t st) {
+                 const BgOut& o, bool few, hipStream_t st) {
     GuIn in{x6.q6, nullptr, reinterpret_cast<const uint8_t*>(x6.x6), w0.cols, (w0.cols + 255) / 256};
     if (w0.type == T_Q8_0) {
         if (!xq.q || !xq.s) return false;
         in.q = reinterpret_cast<const uint8_t*>(xq.q);
         in.s = reinterpret_cast<const uint8_t*>(xq.s);
-        launch_kind<GU_I8, GATEUP>(w0, w1, in, grp, tiles_ub, o, st);
+        launch_kind<GU_I8, GATEUP>(w0, w1, in, grp, tiles_ub, o, few, st);
         return true;
     }
     if (!w0.g6 || !w1.g6 || !in.q) return false;
     if (w0.type == T_Q4_0) {
-        launch_kind<GU_F6, GATEUP>(w0, w1, in, grp, tiles_ub, o, st);
+        launch_kind<GU_F6, GATEUP>(w0, w1, in, grp, tiles_ub, o, few, st);
         return true;
     }
     if (!w0.g6m || !w1.g6m || !in.xm) return false;
-    launch_kind<GU_F6_MIN, GATEUP>(w0, w1, in, grp, tiles_ub, o, st);
+    launch_kind<GU_F6_MIN, GATEUP>(w0, w1, in, grp, tiles_ub, o, few, st);
     return true;
 }
 
@@ -601,13 +625,13 @@ void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, int* over, hipSt
 }
 
 void launch_mfma_gateup(const QMat& g, const QMat& u, const ActH& xin, const ActQ8& xq, const Groups& grp, int tiles_ub,
-                        const ActQ8& hq, const ActH& h6, float* hf, hipStream_t st) {
-    (void)launch_form<true>(g, u, xin, xq, grp, tiles_ub, BgOut{hq, h6, hf, ((g.rows + 255) / 256) * 256, nullptr, 1, 0}, st);
+                        const ActQ8& hq, const ActH& h6, float* hf, hipStream_t st, bool few) {
+    (void)launch_form<true>(g, u, xin, xq, grp, tiles_ub, BgOut{hq, h6, hf, ((g.rows + 255) / 256) * 256, nullptr, 1, 0}, few, st);
 }
 
 void launch_mfma_down_block(const QMat& dn, const ActH& h6, const ActQ8& hq, const Groups& grp, int tiles_ub, float* y,
-                            hipStream_t st, int KS, size_t ystride) {
-    (void)launch_form<false>(dn, dn, h6, hq, grp, tiles_ub, BgOut{ActQ8{}, ActH{}, nullptr, 0, y, KS, ystride}, st);
+                            hipStream_t st, int KS, size_t ystride, bool few) {
+    (void)launch_form<false>(dn, dn, h6, hq, grp, tiles_ub, BgOut{ActQ8{}, ActH{}, nullptr, 0, y, KS, ystride}, few, st);
 }
 
 }  // namespace jx

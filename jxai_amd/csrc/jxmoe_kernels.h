@@ -269,11 +269,13 @@ void launch_gemv_down_f16(const QMat& dn, const ActH& hh, const Groups& grp, int
 // gate/up writes SwiGLU(h) as Q8_0 (hq.q != null), in the BF6 form (h6.q6 != null) and/or fp32 (hf != null).
 // Q8_0 weights read the activations' Q8_0 form (xq, hq), the others their BF6 form (xin, h6).
 void launch_mfma_gateup(const QMat& g, const QMat& u, const ActH& xin, const ActQ8& xq, const Groups& grp, int tiles_ub,
-                        const ActQ8& hq, const ActH& h6, float* hf, hipStream_t st);
+                        const ActQ8& hq, const ActH& h6, float* hf, hipStream_t st, bool few = false);
 // Down on the same GEMM.  KS > 1: the K range split over KS workgroups per item (whole super-blocks each), part q of
 // the output at y + q * ystride (the combine adds the parts in order).
 void launch_mfma_down_block(const QMat& dn, const ActH& h6, const ActQ8& hq, const Groups& grp, int tiles_ub, float* y,
-                            hipStream_t st, int KS = 1, size_t ystride = 0);
+                            hipStream_t st, int KS = 1, size_t ystride = 0, bool few = false);
+// `few`: the average expert has fewer than BG_FEW pairs, most of its parts one pair tile.
+constexpr int BG_FEW = 24;
 // Fill m.g6 (n_mats * nrt * cols / 128 * G6_HU bytes) and, K-quants, m.g6m (n_mats * nrt * nkb * G6M_SB bytes;
 // null otherwise) from a repacked matrix of a g6_type (cols % 128 == 0).  *over is set where a scale passes
 // fp16: the form is then not usable.

@@ -554,14 +554,13 @@ constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q4 = 12;
 constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q4_LARGE = 16;
 constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q8 = 4;
 constexpr size_t LARGE_EXPERT_ELEMS = (size_t)1 << 25;  // d * d_ff per matrix
-// The cold experts' GEMVs beside the GEMMs: layers of at least HYBRID_MIN_E experts, experts under
-// COLD_PAIRS pairs (JX_COLD_PAIRS overrides it, 0 turns the split off: A/B measurement).  Measured on
-// the Qwen3-shaped 2048-token step with Zipf routing (61 / 76 / 86 / 93 experts under 16 / 32 / 48 / 64
-// pairs): 624 us without the split, 600 / 609 / 621 / 637 us with these thresholds.  The GEMMs are
-// matrix-core bound on the head experts (the largest holds 1902 pairs), and the GEMV blocks share the
-// CUs with them.
+// The cold experts' GEMVs beside the GEMMs (JX_COLD_PAIRS=n: layers of at least HYBRID_MIN_E experts, experts under n
+// pairs; 0, the default: none).  Beside the fp16 GEMMs 16 was the faster setting; the block GEMM multiplies a part
+// of at most 32 pairs as one pair tile, and the GEMV blocks then cost the CUs more than they save.  Qwen3-shaped
+// with Zipf routing, 0 / 16: 64 tokens 107 / 120 us, 200 174 / 172, 600 232 / 231, 2048 393 / 395 (GEMV blocks on
+// the side stream).
 constexpr int HYBRID_MIN_E = 32;
-constexpr int COLD_PAIRS = 16;
+constexpr int COLD_PAIRS = 0;
 
 // Whether a call takes the fused one-token launch (k_decode1), apart from stream capture: one token in
 // the GEMV regime, Q8_0 activations on both sides, a shared expert (if any) in the routed formats, a
@@ -885,7 +884,7 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
         const bool h6 = mfma_down && dn_block && L->down.m.g6;  // h straight into its down's operand form
         jx::launch_mfma_gateup(L->gate.m, L->up.m, L->xh.a, L->xq, grp, tiles_ub,
                                L->down_f32 || h6 ? jx::ActQ8{} : L->hq, h6 ? L->hh.a : jx::ActH{},
-                               L->down_f32 ? L->hf : nullptr, st);
+                               L->down_f32 ? L->hf : nullptr, st, nk < jx::BG_FEW * E);
     } else if (small_logits) {
         jx::Groups lg = grp;
         lg.logits = L->logits;
@@ -938,7 +937,8 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
             Launch l(L, "down_mfma", st);
             ks = jx::mfma_down_ksplit(hK);
             if (dn_block)
-                jx::launch_mfma_down_block(L->down.m, L->hh.a, L->hq, grp, tiles_ub, L->y, st, ks, L->ystride);
+                jx::launch_mfma_down_block(L->down.m, L->hh.a, L->hq, grp, tiles_ub, L->y, st, ks, L->ystride,
+                                           nk < jx::BG_FEW * E);
             else
                 jx::launch_mfma_down(L->down.m, L->hh.a, grp, tiles_ub, L->y, st, ks, L->ystride,
                                  nk <= jx::MFMA_DOWN_SMALL_MAX_PPE * E);
