@@ -139,12 +139,10 @@ constexpr int MAX_SLOTS_DEC = 16;  // routed slots (top_k) of the fused one-toke
 
 constexpr int MFMA_BN = 128;  // pairs per matrix-core GEMM tile
 // shared expert on the matrix cores from this many tokens (one dense expert fills few GEMM
-// workgroups below that: 44 gate/up and 16 down workgroups for a 5632 x 2048 expert at 64 tokens).
-// The 16-token matrix-core GEMV in one group per 16 tokens is faster up to 256 tokens for the formats
-// it runs at 3 waves per SIMD (Qwen1.5-shaped, Q4_0: 64 tokens 233 -> 177 us per step), up to 64 for
-// Q4_K / Q6_K (2 waves per SIMD; DeepSeek-V2-Lite-shaped).
-constexpr int MFMA_MIN_SHARED_TOKENS = 256;
-constexpr int MFMA_MIN_SHARED_TOKENS_KQ = 64;  // Q4_K / Q6_K shared experts
+// workgroups below that: 44 gate/up workgroups for a 5632 x 2048 expert at 64 tokens; the 16-token GEMV runs in one
+// group per 16 tokens).  Per step with 64 / 128 / 256: Qwen1.5-shaped 96 tokens 191 / 182 / 183 us, 190 tokens 201 /
+// 201 / 208, 250 tokens 204 / 204 / 226; DeepSeek-V2-Lite-shaped 70 tokens 195 / 169 / 170, 130 tokens 201 / 201 / 210.
+constexpr int MFMA_MIN_SHARED_TOKENS = 128;
 
 // The weighted combine folded into the down GEMV (few-token decode with at most two
 // contributions per output element: top_k <= 2 and no shared expert): out [n][d] is

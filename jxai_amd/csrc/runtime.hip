@@ -546,13 +546,19 @@ int resolve_profile(jx_moe_layer* L) {
 
 // Regime: the matrix-core GEMMs once the average expert sees this many (token, slot) pairs.  The
 // multi-token GEMV (int8 matrix cores, 16 tokens per weight pass) streams an expert's weights once
-// per 16 tokens, the GEMM once per 64-pair tile computing the whole tile.  Forced-GEMV vs forced-GEMM
-// sweeps on MI355X put the crossover at 3-4 pairs for the Q8_0 layer (Qwen3-shaped), ~11 for the
-// small 4-bit experts (DeepSeek-V2-Lite-, Qwen1.5-shaped) and ~15 for large ones (Mixtral-shaped,
-// 14336 x 4096 per matrix, whose GEMV streams near its best rate).
-constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q4 = 12;
-constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q4_LARGE = 16;
-constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q8 = 4;
+// per 16 tokens, the GEMM once per 64-pair tile.  Forced-GEMV against forced-GEMM steps (us):
+//   Q8_0 (Qwen3-shaped): 8 / 12 / 16 / 24 / 32 / 64 tokens (0.5 / 0.75 / 1 / 1.5 / 2 / 4 pairs) 53 / 65 / 71 / 91 / 101 / 167
+//   against 58 / 59 / 62 / 67 / 73 / 107
+//   Q4_0 (Qwen1.5-shaped): 64 / 96 / 128 / 176 tokens (4 / 6 / 9 / 12 pairs) 127 / 183 / 187 / 222 against 153 / 181 / 184 / 206
+//   small K-quant experts (DeepSeek-V2-Lite-shaped): 96 / 128 tokens (9 / 12 pairs) 184 / 208 against 192 / 194
+//   large experts (Mixtral-shaped, 14336 x 4096 per matrix, whose GEMV streams near its best rate): 64 / 96 tokens
+//   (16 / 24 pairs) 318 / 405 against 320 / 344
+// Large Q8_0 experts and batches under 12 tokens keep 4 pairs.
+constexpr int MFMA_MIN_PAIRS_PER_EXPERT_KQ = 12;
+constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q4_0 = 7;
+constexpr int MFMA_MIN_PAIRS_PER_EXPERT_LARGE = 16;
+constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q8 = 1, MFMA_MIN_TOKENS_Q8 = 12;
+constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q8_LARGE = 4;
 constexpr size_t LARGE_EXPERT_ELEMS = (size_t)1 << 25;  // d * d_ff per matrix
 // The cold experts' GEMVs beside the GEMMs (JX_COLD_PAIRS=n: layers of at least HYBRID_MIN_E experts, experts under n
 // pairs; 0, the default: none).  Beside the fp16 GEMMs 16 was the faster setting; the block GEMM multiplies a part
@@ -604,9 +610,12 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     }
     const int nk = n * k;
     const int hK = down_h_k(L->down.m.type, L->F, L->down_f32);
-    const int min_ppe = L->gate.m.type == jx::T_Q8_0                 ? MFMA_MIN_PAIRS_PER_EXPERT_Q8
-                        : (size_t)d * L->F >= LARGE_EXPERT_ELEMS ? MFMA_MIN_PAIRS_PER_EXPERT_Q4_LARGE
-                                                                 : MFMA_MIN_PAIRS_PER_EXPERT_Q4;
+    const bool large = (size_t)d * L->F >= LARGE_EXPERT_ELEMS;
+    const int min_ppe = L->gate.m.type == jx::T_Q8_0
+                            ? (large || n < MFMA_MIN_TOKENS_Q8 ? MFMA_MIN_PAIRS_PER_EXPERT_Q8_LARGE : MFMA_MIN_PAIRS_PER_EXPERT_Q8)
+                        : large                            ? MFMA_MIN_PAIRS_PER_EXPERT_LARGE
+                        : L->gate.m.type == jx::T_Q4_0     ? MFMA_MIN_PAIRS_PER_EXPERT_Q4_0
+                                                           : MFMA_MIN_PAIRS_PER_EXPERT_KQ;
     bool mfma = (size_t)nk >= (size_t)min_ppe * E;
     if (flags & JX_FWD_FORCE_GEMV) mfma = false;
     if (flags & JX_FWD_FORCE_MFMA) mfma = true;
@@ -639,7 +648,6 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     // (Qwen1.5-shaped 16 / 32 tokens 127 / 164 -> 112 / 131 us, DeepSeek-V2-Lite-shaped 12 / 16 tokens
     // 127 / 137 -> 117 / 116 us against the VALU form; Mixtral-shaped 4 tokens 144 us VALU, 154 us MFMA)
     const bool q8w = L->gate.m.type == jx::T_Q8_0;
-    const bool large = (size_t)d * L->F >= LARGE_EXPERT_ELEMS;
     auto gemv_tb = [&](int tokens_per_expert_x2) {  // twice the average tokens per expert
         return n == 1 ? 1 : (tokens_per_expert_x2 >= (q8w ? 1 : large ? 3 : 2) ? 16 : 4);
     };
@@ -1188,9 +1196,7 @@ int jx_moe_layer_create(const jx_moe_layer_desc* D, jx_moe_layer** out) {
     L->cold_pairs = COLD_PAIRS;
     if (const char* f = std::getenv("JX_SH_KSPLIT")) L->sh_ksplit = std::strcmp(f, "0") != 0;
     if (const char* f = std::getenv("JX_COLD_PAIRS")) L->cold_pairs = std::max(0, std::atoi(f));
-    L->smfma_min = (L->shared && (L->sgate.m.type == jx::T_Q4_K || L->sgate.m.type == jx::T_Q6_K))
-                       ? jx::MFMA_MIN_SHARED_TOKENS_KQ
-                       : jx::MFMA_MIN_SHARED_TOKENS;
+    L->smfma_min = jx::MFMA_MIN_SHARED_TOKENS;
     if (const char* f = std::getenv("JX_SMFMA_MIN")) L->smfma_min = std::max(1, std::atoi(f));
     if ((r = dalloc(L->dsync, 1)) != JX_OK) return bail(r);
     if ((r = dalloc(L->hw, (size_t)L->k * L->F / 4)) != JX_OK) return bail(r);

@@ -41,6 +41,24 @@ def test_gateup_tile_edges(moe, port, fmt, d, ff):
     L.close()
 
 
+# the largest batch of the GEMVs and the smallest of the GEMMs: 7 pairs per expert (Q4_0), 12 (K-quants), 12 tokens (Q8_0)
+@pytest.mark.parametrize("fmt,n", [(F.Q4_0, 28), (F.Q4_K, 48), (F.Q8_0, 12)])
+def test_regime_edge(moe, port, fmt, n):
+    """Either side of the line the layer's own choice is that regime's result bit for bit, and the oracle's."""
+    cfg = synth.LayerConfig(f"edge_{fmt}", 512, 8, 2, 1280, fmt)
+    lw = synth.make_layer(cfg)
+    L = moe.MoELayer.from_weights(lw)
+    for m, regime in ((n - 1, "gemv"), (n, "mfma")):
+        print(f"[gpu] regime edge {fmt} n={m}", flush=True)
+        x = synth.make_tokens(cfg, m)
+        out, ids, _, _ = L.forward(x)
+        assert np.array_equal(out, L.forward(x, regime=regime)[0])
+        want, ids_o, _, _ = port.moe_forward(lw, x)
+        assert np.array_equal(ids, ids_o)
+        assert (np.abs(out - want).max(axis=1) <= 1e-3 * np.abs(want).max(axis=1)).all()  # d_ff past 1024: the layer bar
+    L.close()
+
+
 @pytest.mark.parametrize("fmt", [F.Q4_0, F.Q8_0, F.Q4_K, F.Q5_K, F.Q6_K])
 @pytest.mark.parametrize("cols,rows", [(256, (8, 33, 1)), (4352, (160, 32, 64))])
 def test_projection_launch(moe, port, fmt, cols, rows):
