@@ -24,8 +24,8 @@ the device-pointer asynchronous path (the one timed) is checked bit for bit
 against the host-pointer path.  Kernel durations for the rooflines come from a
 second pass with HIP events around every launch.  The prefill roofline is the
 fraction of the dense int8 peak (the path's products are int8 x int8 block
-sums); the GEMMs run v_mfma_f32_32x32x16_f16 on exact integer-valued operands,
-so the fraction of the fp16 peak is reported beside it.
+sums; the GEMM forms them exactly on FP6 operands, and the scales' products on fp16
+ones); the rate as a fraction of the fp16 peak is reported beside it.
 The reference's CPU path (its own quant.cpp/tier.cpp built in oracle/_ref,
 AVX2 dot order) is timed on a bounded token sample on the host cores.
 """
@@ -136,12 +136,6 @@ def copy_calibration():
         b.copy_(a)
     torch.cuda.synchronize()
     print(f"[bench] copied {nbytes} bytes x3", file=sys.stderr, flush=True)
-
-
-def issued_per_algorithmic(cfg):
-    """Matrix-core flops the gate/up GEMM issues per algorithmic flop: Q4_K one fp16 MFMA per
-    16 of K plus the min term's three per 256 of K (19 / 16); Q4_0 / Q8_0 hi and lo (2)."""
-    return 19 / 16 if cfg.wtype == F.Q4_K else 2.0
 
 
 def algorithmic(cfg, n, counts):
@@ -344,10 +338,9 @@ def main():
     gu_avg = gu_ms / max(gu_n, 1) / 1e3
     gu_rate = a_pre["gateup_ops"] / gu_avg / 1e12
     traffic, traffic_note = measured_traffic("gateup_mfma", n)
-    # the fraction of the int8 peak (the path's arithmetic is int8 x int8 block sums); the GEMM issues
-    # v_mfma_f32_32x32x16_f16 on exact integer-valued operands, so its fraction of the fp16 peak and of
-    # the issued matrix-core work are reported beside it
-    pre_roof = {"bound": "mfma", "kernel": "k_wgemm<Q4_K, gate+up> (fp16 matrix-core grouped GEMM + SwiGLU)",
+    # the fraction of the int8 peak (the path's arithmetic is int8 x int8 block sums); the rate as a fraction of
+    # the fp16 peak is reported beside it
+    pre_roof = {"bound": "mfma", "kernel": "k_bgemm<FP6, gate+up> (matrix-core grouped GEMM on exact block products + SwiGLU)",
                 "achieved": gu_rate, "peak": INT8_PEAK_TOPS, "unit": "TFLOP/s",
                 "ops": "algorithmic int8 ops (2 per multiply-accumulate, 2*n*k*2*d*F per launch) per second in "
                        "units of 1e12, against the dense int8 peak of 5.0 POP/s",
@@ -355,7 +348,6 @@ def main():
                 "traffic": traffic, "traffic_note": traffic_note,
                 "avg_launch_us": gu_avg * 1e6,
                 "fp16_peak_frac": gu_rate / FP16_PEAK_TFLOPS,
-                "issued_fp16_frac": issued_per_algorithmic(cfg) * gu_rate / FP16_PEAK_TFLOPS,
                 "layer_int8_frac": a_pre["ops"] / s_pre / 1e12 / INT8_PEAK_TOPS}
 
     nd = args.decode_tokens
@@ -455,7 +447,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f16 MFMA on exact integer operands, f32 accumulate (decode: int8 dot, i32)",
+        "dtype": "MFMA on exact integer operands (block sums exact, scale products f16 hi + lo), f32 accumulate (decode: int8 dot, i32)",
         "data": "synthetic: seeded SplitMix64 Q4_K weights and N(0,1) activations of the layer shape",
         "config": {"workload": f"{cfg.describe}, prefill {n} tokens", "d_model": cfg.d_model,
                    "n_experts": cfg.n_experts, "top_k": cfg.top_k, "d_ff": cfg.d_ff,
