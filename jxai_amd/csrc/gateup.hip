@@ -1,4 +1,4 @@
-// Prefill gate/up: grouped GEMM on the matrix cores, one exact product per 32-block.
+// Prefill gate/up, and the down over a Q8_0 h: grouped GEMM on the matrix cores, one exact product per 32-block.
 //
 // The reference's dots (vec_dot_{q4_0,q8_0,q4_K,q5_K}_q8_0, src/quant.cpp:3307-3730)
 // sum each 32-element block exactly in integers and scale it by (weight scale x

@@ -288,8 +288,9 @@ void launch_mfma_down(const QMat& dn, const ActH& hin, const Groups& grp, int ti
 // 512 per expert, 566 us in the 128-pair form against 590 in the small one).
 constexpr int MFMA_DOWN_SMALL_MAX_PPE = 256;
 // K-split of the down GEMM for a K of K: two parts from MFMA_DOWN_KSPLIT_MIN_K on (twice the
-// workgroups, finer rounds; measured Mixtral-shaped, K 14336: 2048 tokens 634 -> 575 us, 256 tokens
-// 155 -> 133 us; at K 768 - 1408 the per-workgroup overhead makes it slower).
+// workgroups, finer rounds; measured per step on the block GEMM, Mixtral-shaped, K 14336: 300 / 512 / 1024 / 2048
+// tokens 505 / 690 / 1093 / 1997 -> 488 / 669 / 1064 / 1954 us; at K 768 - 1408 the per-workgroup overhead makes it
+// slower).
 constexpr int MFMA_DOWN_KSPLIT_MIN_K = 8192;
 int mfma_down_ksplit(int K);
 // Weight types the block GEMM takes (Q5_0 has no Q8_0-activation form, and Q6_K's 16-element sub-blocks no
