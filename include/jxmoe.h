@@ -206,8 +206,10 @@ int jx_matmul_swiglu_quant_f32(jx_qmatrix* Wg, jx_qmatrix* Wu, const float* x, f
  * matrix's workspace is used) must not overlap.
  *   jx_matmul_quant_f32_dev:     matmul_quant_f32 (src/quant.cpp:3895-3922)
  *   jx_matmul_qkv_quant_f32_dev: matmul_qkv_quant_f32 (src/quant.cpp:3924-3968):
- *     x quantized once when the given matrices hold >= 8 rows together; any of
- *     Wq, Wk, Wv may be NULL; they share cols. */
+ *     x takes its Q8_0 form when the given matrices hold >= 8 rows together; any of
+ *     Wq, Wk, Wv may be NULL; they share cols.
+ * Outputs may overlap x (every product then uses x as it was before the call);
+ * where outputs overlap each other, the later of q, k, v stands. */
 int jx_matmul_quant_f32_dev(jx_qmatrix* W, const float* x_dev, float* out_dev, void* stream);
 int jx_matmul_qkv_quant_f32_dev(jx_qmatrix* Wq, jx_qmatrix* Wk, jx_qmatrix* Wv, const float* x_dev, float* q_dev,
                                 float* k_dev, float* v_dev, void* stream);

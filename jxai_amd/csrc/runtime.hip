@@ -1491,26 +1491,41 @@ int jx_matmul_qkv_quant_f32_dev(jx_qmatrix* Wq, jx_qmatrix* Wk, jx_qmatrix* Wv, 
         if (Ws[i] && !(quantized && q8_activation(Ws[i]->type, cols))) need_f32 = true;
     if (kpad > (size_t)jx::gemv_max_k(false, 1, need_f32))
         return fail(JX_ERR_UNSUPPORTED, "cols exceeds the GEMV's staged activation capacity");
-    // the Q8_0-form matrices: one launch per format among them
+    // The one-launch form reads x in every block while others store their rows, and a later launch reads it after
+    // an earlier one's stores.  Where an output shares memory with x, all of them read the workspace's copy; where
+    // outputs share memory with each other, each matrix takes its own launch, in the order q, k, v.
+    auto share = [](const float* a, size_t n, const float* b, size_t m) {
+        const uintptr_t ua = reinterpret_cast<uintptr_t>(a), ub = reinterpret_cast<uintptr_t>(b);
+        return ua < ub + m * sizeof(float) && ub < ua + n * sizeof(float);
+    };
+    bool x_shared = false, outs_shared = false;
+    for (int i = 0; i < 3; ++i) {
+        if (!Ws[i]) continue;
+        x_shared |= share(x_dev, (size_t)cols, outs[i], (size_t)Ws[i]->rows);
+        for (int k = i + 1; k < 3; ++k)
+            if (Ws[k]) outs_shared |= share(outs[i], (size_t)Ws[i]->rows, outs[k], (size_t)Ws[k]->rows);
+    }
+    if (need_f32 || x_shared) jx::launch_copy_pad(x_dev, cols, (int)kpad, first->xf, st);
+    const float* x = x_shared ? first->xf : x_dev;
     bool done[3] = {};
     for (int i = 0; i < 3; ++i) {
-        if (!Ws[i] || done[i] || !quantized || !q8_activation(Ws[i]->type, cols)) continue;
+        if (!Ws[i] || done[i]) continue;
+        if (!(quantized && q8_activation(Ws[i]->type, cols))) {
+            const int r = dev_gemv(Ws[i], false, first->xq, first->xf, outs[i], st);
+            if (r != JX_OK) return r;
+            continue;
+        }
+        // the Q8_0-form matrices: one launch per format among them
         const jx::QMat* w[3];
         float* o[3];
         int n = 0;
-        for (int k = i; k < 3; ++k)
+        for (int k = i; k < (outs_shared ? i + 1 : 3); ++k)
             if (Ws[k] && Ws[k]->type == Ws[i]->type) {
                 w[n] = &Ws[k]->w.m;
                 o[n++] = outs[k];
                 done[k] = true;
             }
-        jx::launch_gemv_qkv(w, o, n, x_dev, cols, st);
-    }
-    if (need_f32) jx::launch_copy_pad(x_dev, cols, (int)kpad, first->xf, st);
-    for (int i = 0; i < 3; ++i) {
-        if (!Ws[i] || done[i]) continue;
-        const int r = dev_gemv(Ws[i], false, first->xq, first->xf, outs[i], st);
-        if (r != JX_OK) return r;
+        jx::launch_gemv_qkv(w, o, n, x, cols, st);
     }
     HIPCHK(hipGetLastError());
     return JX_OK;

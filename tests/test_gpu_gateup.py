@@ -83,3 +83,38 @@ def test_projection_launch(moe, port, fmt, cols, rows):
         assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
     for q in qm:
         q.close()
+
+
+# the projections on one format and on mixed ones (Q5_0 takes fp32 activations)
+@pytest.mark.parametrize("fmts", [(F.Q4_K, F.Q4_K, F.Q4_K), (F.Q4_0, F.Q8_0, F.Q4_0), (F.Q8_0, F.Q5_0, F.Q6_K)])
+@pytest.mark.parametrize("at", [0, 100, 4000])
+def test_projection_outputs_over_x(moe, fmts, at):
+    """An output that shares memory with x (its start, its middle, its end) changes nothing: every product uses x
+    as it was before the call.  Where k and v share memory, v stands."""
+    cols, rows = 4096, (2048, 96, 320)
+    print(f"[gpu] projection over x {fmts} at {at}", flush=True)
+    x = synth.normal_f32(synth.sub_seed("qkvo", "x"), cols, 1.0)
+    qm = [moe.QMatrix(f, synth.quant_matrix(synth.sub_seed("qkvo", f"{i}"), f, r, cols), r, cols)
+          for i, (f, r) in enumerate(zip(fmts, rows))]
+    buf = moe.DeviceBuffer(4 * (cols + 8192))
+    sep = [moe.DeviceBuffer(r * 4) for r in rows]
+
+    def call(ptrs):
+        buf.upload(x)
+        assert moe.lib().jx_matmul_qkv_quant_f32_dev(*[q.handle for q in qm], buf.ptr, *ptrs, None) == 0
+        moe.lib().jx_device_synchronize()
+
+    call([b.ptr for b in sep])
+    want = [b.download(np.empty(r, np.float32)) for b, r in zip(sep, rows)]
+    for over in range(3):
+        for b in sep:
+            b.upload(np.zeros(b.nbytes // 4, np.float32))
+        call([buf.ptr.value + 4 * at if i == over else b.ptr for i, b in enumerate(sep)])
+        whole = buf.download(np.empty(cols + 8192, np.float32))
+        for i, (b, r) in enumerate(zip(sep, rows)):
+            got = whole[at:at + r] if i == over else b.download(np.empty(r, np.float32))
+            assert np.array_equal(got, want[i]), (over, i)
+    call([sep[0].ptr, sep[2].ptr, sep[2].ptr])
+    assert np.array_equal(sep[2].download(np.empty(rows[2], np.float32)), want[2])
+    for q in qm:
+        q.close()
