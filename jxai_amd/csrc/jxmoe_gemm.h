@@ -82,7 +82,7 @@ __device__ __forceinline__ void split3(float v, uint16_t& h, uint16_t& m, uint16
 // remainder exact) at xm[0], xm[8], xm[16].
 __device__ __forceinline__ void store_pieces3(uint16_t* xm, float X) { split3(X, xm[0], xm[8], xm[16]); }
 
-// The BF6 form (ActH::q6, and the block's min-term pieces ActH::x6) of part `part` (16 quants, four signed bytes
+// The BF6 form (ActH::q6) of part `part` (16 quants, four signed bytes
 // a word) of block b with (scale, sum) sb.
 __device__ __forceinline__ void write_q6_part(const uint32_t (&w)[4], float2 sb, const ActH& o, size_t row, int b, int part) {
     uint32_t c[6] = {0, 0, 0, 0, 0, 0};
@@ -109,8 +109,11 @@ __device__ __forceinline__ void write_q6_part(const uint32_t (&w)[4], float2 sb,
     *reinterpret_cast<uint4*>(d + j * 32 + part * 16) = make_uint4(c[0], c[1], c[2], c[3]);
     *reinterpret_cast<uint2*>(d + 128 + j * 16 + part * 8) = make_uint2(c[4], c[5]);
     *reinterpret_cast<uint2*>(d + 192 + j * 16 + part * 8) = make_uint2(j & 1 ? 0u : dx, j & 1 ? dx : 0u);
-    if (o.x6 && part == 0)
-        store_pieces3(o.x6 + row * (size_t)o.KU * 24 + (b / 8) * 24 + (b % 8), sb.x * sb.y);  // product exact
+}
+
+// The min-term pieces (ActH::xp) of block b of a row with (scale, sum) sv.
+__device__ __forceinline__ void q8_pieces(float2 sv, const ActH& o, size_t row, int b) {
+    store_pieces3(o.xp + row * (size_t)o.KU * 24 + (b / 8) * 24 + b % 8, sv.x * sv.y);  // product exact
 }
 
 // (scale, min) j of a Q4_K header in registers (get_scale_min_k4,

@@ -50,16 +50,17 @@ struct QMat {
     // fp16 operand scales s1 of the 8 sub-blocks.
     const uint8_t* mn = nullptr;
     size_t mn_es = 0;  // per-expert stride (bytes)
-    // FP6 form for the gate/up GEMM (launch_g6_tables; Q4_0 / Q4_K / Q5_K gate and up matrices): per (expert,
-    // row tile, half-unit of 128 columns) G6_HU bytes = [4 blocks][2 parts of 16 elements][32 rows][12 B] codes,
-    // then [32 rows][4 blocks] scales d (* sc_j) as fp16 hi | lo << 16.  Code of value v (q - 8 / q / q - 16):
-    // sign << 5 | |v|, element i of a part at bit 6 i.
+    // Q4_K / Q5_K table for the block GEMM (launch_block_table): per (expert, row tile, super-block) BT_SB bytes =
+    // 2 half-units x [32 rows][4 sub-blocks] scales d * sc_j as fp16 hi | lo << 16, then at BT_MIN 2 x [32 rows][16 B], the
+    // bf16 pieces (hi, lo) of the 8 sub-blocks' factors -dmin m_j of dx * sum(q).
+    const uint8_t* bt = nullptr;
+    size_t bt_es = 0;
+    // Q4_0 / Q4_K, where device memory is plentiful: the quants as FP6 codes for the block GEMM (launch_g6_codes), per
+    // (expert, row tile, half-unit of 128 columns) [4 blocks][2 parts of 16 elements][32 rows][12 B], then for Q4_0
+    // [32 rows][4 blocks] scales d (fp16 in 32 bits).  Code of value v (q - 8 / q): sign << 5 | |v|, element i of a part
+    // at bit 6 i.
     const uint8_t* g6 = nullptr;
     size_t g6_es = 0;
-    // Q4_K / Q5_K beside it: per (expert, row tile, super-block) G6M_SB bytes = 3 x [32 rows][16 B], the bf16
-    // pieces (hi, mid, lo) of the 8 sub-blocks' factors of dx * sum(q): -dmin m_j (Q5_K: + 16 d sc_j).
-    const uint8_t* g6m = nullptr;
-    size_t g6m_es = 0;
     // Gated activation applied to this matrix's outputs when it is the gate of
     // a gate/up pair (ACT_SILU or ACT_GELU_TANH); unused otherwise.
     int act = 0;
@@ -69,8 +70,8 @@ struct QMat {
     int valid_rows = 0;
 };
 constexpr size_t QMAT_PAD = 8192;
-constexpr int G6_HU = 3584, G6M_SB = 1536;
-inline bool g6_type(int t) { return t == T_Q4_0 || t == T_Q4_K || t == T_Q5_K; }
+constexpr int BT_SB = 2048, BT_MIN = 1024;
+constexpr int g6_half_unit(int type) { return type == T_Q4_0 ? 3584 : 3072; }
 
 // Q8_0 activations on the device: q [rows][K] int8, s [rows][K/32] = (fp16-truncated
 // scale as fp32, sum of the 32 quants as fp32).
@@ -92,19 +93,20 @@ struct ActQ8 {
 //   xm [rows][KU][3][8]  per 256-element unit: bf16 pieces (hi, mid, lo) of
 //                        dx * sum(q) (fp32 rows: the block sum) times 2^-E for its
 //                        8 blocks (Q4_K min term)
-// and, for the FP6 gate/up GEMM (each form is written where its pointers are set):
+// and, for the block GEMM (each form is written where its pointer is set):
 //   q6 [rows][KH][256 B]  the quant is 16 a + b, |a|, |b| <= 8: per block and part of 16 elements the codes
 //                        of 16 a, then of b, as BF6 (e3m2) in units of 1/16, code i at bit 6 i, and the block
 //                        scale's fp16 dx.  Per half-unit: [4 blocks][2 parts][16 B] code words 0..3,
 //                        [4][2][8 B] words 4, 5, [4][2][8 B] (dx, dx, 0, 0) in part 0 of even blocks, (0, 0, dx, dx)
 //                        of odd ones, zeros in part 1
-//   x6 [rows][KU][3][8]  bf16 pieces (hi, mid, lo) of dx * sum(q) of the 8 blocks of each 256 (Q4_K / Q5_K)
+//   xp [rows][KU][3][8]  bf16 pieces (hi, mid, lo) of dx * sum(q) of the 8 blocks of each 256 (K-quants'
+//                        min term)
 struct ActH {
     uint16_t* hl = nullptr;
     float* pe = nullptr;
     uint16_t* xm = nullptr;
     uint8_t* q6 = nullptr;
-    uint16_t* x6 = nullptr;
+    uint16_t* xp = nullptr;
     int K = 0;
     int KH = 0;  // K / 128
     int KU = 0;  // ceil(K / 256)
@@ -264,20 +266,22 @@ void launch_gemv_qkv(const QMat* const* W, float* const* out, int n, const float
 bool gemv_down_f16_fits(int type, int K);
 void launch_gemv_down_f16(const QMat& dn, const ActH& hh, const Groups& grp, int slots, float* y, hipStream_t st);
 // Prefill regime: matrix-core grouped GEMMs over the dispatch tile table.
-// gate/up writes SwiGLU(h) as Q8_0 (hq.q != null), in the BF6 form (h6.q6 != null) and/or fp32 (hf != null).
-// Q8_0 weights read the activations' Q8_0 form (xq, hq), the others their BF6 form (xin, h6).
-void launch_mfma_gateup(const QMat& g, const QMat& u, const ActH& xin, const ActQ8& xq, const Groups& grp, int tiles_ub,
-                        const ActQ8& hq, const ActH& h6, float* hf, hipStream_t st, bool few = false);
+// The block GEMM over Q8_0 activations: from the matrices' codes where they have them (x's ActH::q6), else from their
+// blocks (xq); Q4_K / Q5_K with the min-term pieces (ActH::xp).  Both give the same bits.
+// Gate/up writes SwiGLU(h) as Q8_0 (hq.q != null), in its block-GEMM forms (hh.q6, hh.xp) and/or fp32 (hf != null).
+void launch_mfma_gateup(const QMat& g, const QMat& u, const ActQ8& xq, const ActH& xh, const Groups& grp, int tiles_ub,
+                        const ActQ8& hq, const ActH& hh, float* hf, hipStream_t st, bool few = false);
 // Down on the same GEMM.  KS > 1: the K range split over KS workgroups per item (whole super-blocks each), part q of
 // the output at y + q * ystride (the combine adds the parts in order).
-void launch_mfma_down_block(const QMat& dn, const ActH& h6, const ActQ8& hq, const Groups& grp, int tiles_ub, float* y,
+void launch_mfma_down_block(const QMat& dn, const ActQ8& hq, const ActH& hh, const Groups& grp, int tiles_ub, float* y,
                             hipStream_t st, int KS = 1, size_t ystride = 0, bool few = false);
 // `few`: the average expert has fewer than BG_FEW pairs, most of its parts one pair tile.
 constexpr int BG_FEW = 24;
-// Fill m.g6 (n_mats * nrt * cols / 128 * G6_HU bytes) and, K-quants, m.g6m (n_mats * nrt * nkb * G6M_SB bytes;
-// null otherwise) from a repacked matrix of a g6_type (cols % 128 == 0).  *over is set where a scale passes
-// fp16: the form is then not usable.
-void launch_g6_tables(const QMat& m, uint8_t* g6, uint8_t* g6m, int* over, hipStream_t st);
+// Fill m.bt (n_mats * nrt * nkb * BT_SB bytes) from a repacked Q4_K / Q5_K matrix (cols % 256 == 0).  *over is set
+// where a scale passes fp16: the table is then not usable.
+void launch_block_table(const QMat& m, uint8_t* bt, int* over, hipStream_t st);
+// Fill m.g6 (n_mats * nrt * cols / 128 * g6_half_unit bytes) from a repacked Q4_0 / Q4_K matrix (cols % 128 == 0).
+void launch_g6_codes(const QMat& m, uint8_t* g6, hipStream_t st);
 // The fp16 down GEMM, KS as above.  small: few pairs per expert (the
 // 64-pair tile form at more workgroups per CU).
 void launch_mfma_down(const QMat& dn, const ActH& hin, const Groups& grp, int tiles_ub, float* y, hipStream_t st,
@@ -293,9 +297,9 @@ constexpr int MFMA_DOWN_SMALL_MAX_PPE = 256;
 // slower).
 constexpr int MFMA_DOWN_KSPLIT_MIN_K = 8192;
 int mfma_down_ksplit(int K);
-// Weight types the block GEMM takes (Q5_0 has no Q8_0-activation form, and Q6_K's 16-element sub-blocks no
-// product per 32-block).
-bool gemm_block_ok(int type);
+// Whether the block GEMM takes a matrix: Q4_0, Q8_0, and Q4_K / Q5_K with their table (Q5_0 has no Q8_0-activation form,
+// and Q6_K's 16-element sub-blocks no product per 32-block).
+bool gemm_block_ok(const QMat& m);
 // Whether the fp16 down GEMM is built for a matrix: Q5_0, Q6_K, and Q4_K / Q5_K with their min table.
 bool gemm_f16_ok(const QMat& m);
 // Fill m.mn (m.n_mats * m.nrt * m.nkb * MN_SB bytes) from a repacked Q4_K or Q5_K matrix.
@@ -392,8 +396,8 @@ void launch_copy_pad(const float* x, int n, int kpad, float* dst, hipStream_t st
 
 // Matrix-core form of existing Q8_0 activations (int8 quants + (scale, sum)), the down GEMM's operand.
 void launch_q8_to_acth(const ActQ8& in, int rows, ActH out, hipStream_t st);
-// Their FP6 form (out.q6, and out.x6 unless null), the gate/up GEMM's operand.
-void launch_q8_to_q6(const ActQ8& in, int rows, ActH out, hipStream_t st);
+// The block GEMM's forms (out.q6, out.xp where set) of existing Q8_0 activations.
+void launch_q8_to_block(const ActQ8& in, int rows, const ActH& out, hipStream_t st);
 // Matrix-core form (hi only) of fp32 activation rows [rows][ld] (out.K % 128 == 0, columns up to
 // out.K zero-padded).
 void launch_f32_to_acth(const float* h, int ld, int rows, ActH out, hipStream_t st);

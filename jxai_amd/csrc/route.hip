@@ -232,6 +232,7 @@ __global__ void __launch_bounds__(RT_THREADS) k_route(RouteArgs a, int nsplit, i
                     const uint32_t w4[4] = {w[4 * part], w[4 * part + 1], w[4 * part + 2], w[4 * part + 3]};
                     write_q6_part(w4, sv, a.xh, (size_t)(t0 + t), b, part);
                 }
+            if (a.xh.xp) q8_pieces(sv, a.xh, (size_t)(t0 + t), b);
         }
     }
 
@@ -597,19 +598,24 @@ void launch_q8_to_acth(const ActQ8& in, int rows, ActH out, hipStream_t st) {
     hipLaunchKernelGGL(k_q8_to_acth, dim3((rows + 3) / 4), dim3(256), 0, st, in, rows, out);
 }
 
-// The BF6 form of Q8_0 rows already in global memory, one thread per half 32-block.
-__global__ void __launch_bounds__(256) k_q8_to_q6(ActQ8 in, int rows, ActH out) {
+// The block GEMM's forms of Q8_0 rows already in global memory, one thread per half 32-block.
+__global__ void __launch_bounds__(256) k_q8_to_block(ActQ8 in, int rows, ActH out) {
     const int KP = in.K / 16;
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, row = i / KP;
     if (row >= (size_t)rows) return;
-    const uint4 a = ld16(in.q + i * 16);
-    const uint32_t w[4] = {a.x, a.y, a.z, a.w};
-    write_q6_part(w, in.s[i / 2], out, row, (int)(i - row * KP) / 2, (int)(i & 1));
+    const float2 sv = in.s[i / 2];
+    const int b = (int)(i - row * KP) / 2, part = (int)(i & 1);
+    if (out.q6) {
+        const uint4 a = ld16(in.q + i * 16);
+        const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+        write_q6_part(w, sv, out, row, b, part);
+    }
+    if (out.xp && part == 0) q8_pieces(sv, out, row, b);
 }
 
-void launch_q8_to_q6(const ActQ8& in, int rows, ActH out, hipStream_t st) {
+void launch_q8_to_block(const ActQ8& in, int rows, const ActH& out, hipStream_t st) {
     const size_t n = (size_t)rows * (in.K / 16);
-    hipLaunchKernelGGL(k_q8_to_q6, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, in, rows, out);
+    hipLaunchKernelGGL(k_q8_to_block, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, in, rows, out);
 }
 
 // Matrix-core form (fp16 hi only) of fp32 activation rows h [rows][ld], out.K

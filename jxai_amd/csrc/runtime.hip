@@ -126,20 +126,90 @@ struct DevMat {
     uint8_t* sc = nullptr;
     uint8_t* ex = nullptr;  // Q5_0 / Q5_K high bits, Q6_K d
     uint8_t* mn = nullptr;   // Q4_K / Q5_K min-term table (fp16 down GEMM)
-    uint8_t* g6 = nullptr;   // FP6 form and its min-term pieces (block GEMM)
-    uint8_t* g6m = nullptr;
+    uint8_t* bt = nullptr;   // Q4_K / Q5_K scale and min-term table, FP6 codes (block GEMM)
+    uint8_t* g6 = nullptr;
     void release() {
-        for (uint8_t* p : {qs, sc, ex, mn, g6, g6m})
+        for (uint8_t* p : {qs, sc, ex, mn, bt, g6})
             if (p) (void)hipFree(p);
-        qs = sc = ex = mn = g6 = g6m = nullptr;
+        qs = sc = ex = mn = bt = g6 = nullptr;
     }
 };
 
-// Upload n_mats [rows][cols] block matrices and repack them on the device;
-// `gemm` names the matrix-core GEMM that will read it: its tables are built beside the matrix.
 enum class Gemm { none, gateup, down };
+
+// What a matrix-core GEMM reads beside an uploaded matrix, all of it for speed only: where the device has no memory left
+// for a part, the matrix goes without.
+//   Q4_K / Q5_K: the block GEMM's table over Q8_0 activations; otherwise (fp32 h, or a scale past fp16) the fp16 GEMM's
+//   for a down.  0.25 B per weight each; without one the projection takes the GEMVs.
+//   Q4_0 / Q4_K with Q8_0 activations: FP6 codes, 0.88 / 0.75 B per weight.  The block GEMM gives the same bits without
+//   them from the blocks themselves (gateup.hip), so they are built only while CODES_FREE of the device stays free
+//   behind them: models of more layers than that keep the memory for their weights and caches.
+constexpr double CODES_FREE = 0.75;
+hipError_t build_gemm_tables(DevMat& out, Gemm gemm, bool q8, bool codes, hipStream_t st) {
+    jx::QMat& m = out.m;
+    auto alloc = [](uint8_t*& p, size_t bytes) {
+        hipError_t e = hipMalloc(&p, bytes);
+        if (e == hipErrorOutOfMemory) {
+            p = nullptr;
+            (void)hipGetLastError();
+            e = hipSuccess;
+        }
+        return e;
+    };
+    hipError_t e = hipSuccess;
+    const bool kq = m.type == jx::T_Q4_K || m.type == jx::T_Q5_K;
+    if (kq && q8) {
+        int* over = nullptr;
+        int host_over = 0;
+        m.bt_es = (size_t)m.nrt * m.nkb * jx::BT_SB;
+        if ((e = alloc(out.bt, m.bt_es * m.n_mats)) != hipSuccess) return e;
+        if (out.bt) {
+            if ((e = hipMalloc(&over, sizeof(int))) != hipSuccess) return e;
+            e = hipMemsetAsync(over, 0, sizeof(int), st);
+            if (e == hipSuccess) {
+                jx::launch_block_table(m, out.bt, over, st);
+                e = hipGetLastError();
+            }
+            if (e == hipSuccess) e = hipMemcpyAsync(&host_over, over, sizeof(int), hipMemcpyDeviceToHost, st);
+            if (e == hipSuccess) e = hipStreamSynchronize(st);
+            (void)hipFree(over);
+            if (e != hipSuccess) return e;
+            if (host_over) {
+                (void)hipFree(out.bt);
+                out.bt = nullptr;
+            }
+        }
+        m.bt = out.bt;
+    }
+    if (kq && gemm == Gemm::down && !m.bt) {
+        m.mn_es = (size_t)m.nrt * m.nkb * jx::MN_SB;
+        if ((e = alloc(out.mn, m.mn_es * m.n_mats)) != hipSuccess) return e;
+        if (out.mn) {
+            jx::launch_min_table(m, out.mn, st);
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+        }
+        m.mn = out.mn;
+    }
+    if (codes && q8 && m.cols % 128 == 0 && (m.type == jx::T_Q4_0 || (m.type == jx::T_Q4_K && m.bt))) {
+        size_t left = 0, total = 0;
+        m.g6_es = (size_t)m.nrt * (m.cols / 128) * jx::g6_half_unit(m.type);
+        if ((e = hipMemGetInfo(&left, &total)) != hipSuccess) return e;
+        if ((double)left >= (double)(m.g6_es * m.n_mats) + CODES_FREE * (double)total) {
+            if ((e = alloc(out.g6, m.g6_es * m.n_mats)) != hipSuccess) return e;
+            if (out.g6) {
+                jx::launch_g6_codes(m, out.g6, st);
+                if ((e = hipGetLastError()) != hipSuccess) return e;
+            }
+        }
+        m.g6 = out.g6;
+    }
+    return hipStreamSynchronize(st);
+}
+
+// Upload n_mats [rows][cols] block matrices and repack them on the device;
+// `gemm` names the matrix-core GEMM that will read it: what that needs is built beside the matrix (`codes`: FP6 codes too).
 int upload_matrix(int type, int n_mats, int rows, int cols, const void* host, DevMat& out, hipStream_t st,
-                  Gemm gemm = Gemm::none) {
+                  Gemm gemm = Gemm::none, bool codes = false) {
     if (!expert_type_ok(type))
         return fail(JX_ERR_UNSUPPORTED, "expert weight type must be Q4_0, Q5_0, Q8_0, Q4_K, Q5_K or Q6_K");
     if (rows % jx::ROWS_PER_TILE != 0) return fail(JX_ERR_UNSUPPORTED, "matrix rows must be a multiple of 32");
@@ -165,7 +235,7 @@ int upload_matrix(int type, int n_mats, int rows, int cols, const void* host, De
     m.qs_es = units * qs_u;
     m.sc_es = units * sc_u;
     m.ex_es = units * ex_u;
-    // the GEMMs address one expert's matrix with 32-bit offsets (the GEMM table: 4x the headers)
+    // the GEMMs address one expert's matrix with 32-bit offsets (the fp16 GEMM's table: 4x the headers)
     if (m.qs_es >= ((size_t)1 << 32) || m.sc_es * 4 >= ((size_t)1 << 32))
         return fail(JX_ERR_UNSUPPORTED, "one expert matrix exceeds 4 GiB");
     const size_t raw_bytes = (size_t)n_mats * rows * row_bytes(type, cols);
@@ -190,44 +260,9 @@ int upload_matrix(int type, int n_mats, int rows, int cols, const void* host, De
         jx::launch_repack(raw, m, out.qs, out.sc, out.ex, st);
         e = hipGetLastError();
     }
-    // (a down projection without a Q8_0 form of h, or without the FP6 form, runs on the fp16 GEMM)
-    if (e == hipSuccess && gemm != Gemm::none && jx::g6_type(type) && q8_activation(type, cols) && cols % 128 == 0) {
-        int* over = nullptr;
-        int host_over = 0;
-        m.g6_es = (size_t)m.nrt * (cols / 128) * jx::G6_HU;
-        e = hipMalloc(&out.g6, m.g6_es * n_mats);
-        if (e == hipSuccess) e = hipMalloc(&over, sizeof(int));
-        if (e == hipSuccess) e = hipMemsetAsync(over, 0, sizeof(int), st);
-        if (e == hipSuccess && jx::is_kquant(type)) {
-            m.g6m_es = (size_t)m.nrt * m.nkb * jx::G6M_SB;
-            e = hipMalloc(&out.g6m, m.g6m_es * n_mats);
-        }
-        if (e == hipSuccess) {
-            jx::launch_g6_tables(m, out.g6, out.g6m, over, st);
-            e = hipGetLastError();
-        }
-        if (e == hipSuccess) e = hipMemcpyAsync(&host_over, over, sizeof(int), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        (void)hipFree(over);
-        if (e == hipSuccess && host_over) {  // a scale past fp16: no FP6 form
-            (void)hipFree(out.g6);
-            (void)hipFree(out.g6m);
-            out.g6 = out.g6m = nullptr;
-        }
-        m.g6 = out.g6;
-        m.g6m = out.g6m;
-    }
-    if (e == hipSuccess && gemm == Gemm::down && !m.g6 && (type == jx::T_Q4_K || type == jx::T_Q5_K)) {
-        m.mn_es = (size_t)m.nrt * m.nkb * jx::MN_SB;
-        e = hipMalloc(&out.mn, m.mn_es * n_mats);
-        if (e == hipSuccess) {
-            m.mn = out.mn;
-            jx::launch_min_table(m, out.mn, st);
-            e = hipGetLastError();
-        }
-    }
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     (void)hipFree(raw);
+    if (e == hipSuccess && gemm != Gemm::none) e = build_gemm_tables(out, gemm, q8_activation(type, cols), codes, st);
     if (e != hipSuccess) return fail(JX_ERR_HIP, std::string("weight upload: ") + hipGetErrorString(e));
     return JX_OK;
 }
@@ -242,11 +277,11 @@ int dalloc(T*& p, size_t n) {
 }
 
 // Matrix-core activation buffers for `rows` rows of K: the fp16 form (fp16 down GEMM),
-// or the BF6 form (block GEMM), with its min-term pieces for K-quant weights.
+// or the block GEMM's forms: codes for weights with FP6 codes, min-term pieces for K-quants.
 struct DevActH {
     jx::ActH a;
     void release() {
-        for (void* p : {(void*)a.hl, (void*)a.pe, (void*)a.xm, (void*)a.q6, (void*)a.x6})
+        for (void* p : {(void*)a.hl, (void*)a.pe, (void*)a.xm, (void*)a.q6, (void*)a.xp})
             if (p) (void)hipFree(p);
         a = jx::ActH{};
     }
@@ -264,11 +299,10 @@ struct DevActH {
         HIPCHK(hipMalloc(&a.xm, rows * a.KU * 24 * sizeof(uint16_t)));
         return JX_OK;
     }
-    int alloc_fp6(size_t rows, int K, bool q6, bool min) {
+    int alloc_block(size_t rows, int K, bool codes, bool pieces) {
         shape(K);
-        if (K % 128 != 0) return JX_OK;
-        if (q6) HIPCHK(hipMalloc(&a.q6, rows * (size_t)K * 2));
-        if (min) HIPCHK(hipMalloc(&a.x6, rows * a.KU * 24 * sizeof(uint16_t)));
+        if (codes) HIPCHK(hipMalloc(&a.q6, rows * (size_t)K * 2));
+        if (pieces) HIPCHK(hipMalloc(&a.xp, rows * a.KU * 24 * sizeof(uint16_t)));
         return JX_OK;
     }
 };
@@ -382,10 +416,8 @@ namespace {
 int down_h_k(int type, int f, bool f32) { return f32 && jx::is_kquant(type) ? (f + 255) / 256 * 256 : f; }
 
 // Whether a projection over K columns runs on the block GEMM: Q8_0 activations, a half-unit's multiple of
-// columns, and a format it takes in the form built at upload (Q8_0: the matrix as it is).
-bool block_gemm(const DevMat& D, int K, bool f32) {
-    return !f32 && K % 128 == 0 && jx::gemm_block_ok(D.m.type) && (D.m.type == jx::T_Q8_0 || D.m.g6);
-}
+// columns, and a matrix it takes.
+bool block_gemm(const DevMat& D, int K, bool f32) { return !f32 && K % 128 == 0 && jx::gemm_block_ok(D.m); }
 
 int ensure_workspace(jx_moe_layer* L, int n) {
     if (n <= L->cap) return JX_OK;
@@ -419,14 +451,13 @@ int ensure_workspace(jx_moe_layer* L, int n) {
     // h's matrix-core form: K = d_ff, or for fp32 h of a K-quant d_ff padded to whole super-blocks
     const int hK = down_h_k(L->down.m.type, L->F, L->down_f32);
     const int hKs = L->shared ? down_h_k(L->sdown.m.type, L->Fs, L->sdown_f32) : 0;
-    // x's FP6 form where a gate/up GEMM reads it (routed or shared; Q8_0 weights read the quants themselves)
-    auto any_gu = [&](auto pred) { return pred(L->gate.m) || (L->shared && pred(L->sgate.m)); };
-    const bool x6 = any_gu([](const jx::QMat& m) { return m.g6 != nullptr; });
-    const bool xmin = any_gu([](const jx::QMat& m) { return m.g6m != nullptr; });
+    // x's forms that a gate/up GEMM reads (routed or shared)
+    const bool x6 = (L->gate.m.g6 && L->up.m.g6) || (L->shared && L->sgate.m.g6 && L->sup.m.g6);
+    const bool xmin = L->gate.m.bt || (L->shared && L->sgate.m.bt);
     auto alloc_h = [](DevActH& h, size_t rows, const DevMat& D, int K, bool f32) {
-        return block_gemm(D, K, f32) ? h.alloc_fp6(rows, K, D.m.g6 != nullptr, D.m.g6m != nullptr) : h.alloc_hi(rows, K);
+        return block_gemm(D, K, f32) ? h.alloc_block(rows, K, D.m.g6 != nullptr, D.m.bt != nullptr) : h.alloc_hi(rows, K);
     };
-    if ((r = L->xh.alloc_fp6((size_t)cap, L->d, x6, xmin)) != JX_OK ||
+    if ((r = L->xh.alloc_block((size_t)cap, L->d, x6, xmin)) != JX_OK ||
         (r = alloc_h(L->hh, nk, L->down, hK, L->down_f32)) != JX_OK) {
         L->cap = 0;
         return r;
@@ -744,9 +775,9 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
             Launch l(L, "route_dispatch", st);
             jx::launch_route_small(ra, dout, st);
         }
-        if (mfma_gu || smfma_gu) {
+        if ((mfma_gu || smfma_gu) && (L->xh.a.q6 || L->xh.a.xp)) {
             Launch l(L, "to_matrix_form", st);
-            if (L->xh.a.q6) jx::launch_q8_to_q6(L->xq, n, L->xh.a, st);
+            jx::launch_q8_to_block(L->xq, n, L->xh.a, st);
         }
     } else {
         Launch l(L, "route", st);
@@ -807,10 +838,9 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     auto shared_gateup = [&](hipStream_t ss) {
         if (smfma_gu) {
             Launch l(L, "shared_gateup_mfma", ss);
-            const bool h6 = smfma_dn && sdn_block && L->sdown.m.g6;  // h straight into its down's operand form
-            jx::launch_mfma_gateup(L->sgate.m, L->sup.m, L->xh.a, L->xq, sg, st_ub,
-                                   L->sdown_f32 || h6 ? jx::ActQ8{} : L->hqs, h6 ? L->hhs.a : jx::ActH{},
-                                   L->sdown_f32 ? L->hfs : nullptr, ss);
+            const jx::ActH hh = smfma_dn && sdn_block ? L->hhs.a : jx::ActH{};  // h straight into its down's forms
+            jx::launch_mfma_gateup(L->sgate.m, L->sup.m, L->xq, L->xh.a, sg, st_ub,
+                                   L->sdown_f32 || hh.q6 ? jx::ActQ8{} : L->hqs, hh, L->sdown_f32 ? L->hfs : nullptr, ss);
         } else {
             Launch l(L, "shared_gateup_gemv", ss);
             jx::launch_gemv_gateup(L->sgate.m, L->sup.m, L->xq, sg, sslots, tbs, L->hqs, L->sdown_f32 ? L->hfs : nullptr, ss,
@@ -821,8 +851,8 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
         if (smfma_dn) {
             Launch l(L, "shared_down", ss);
             if (sdn_block) {
-                if (L->sdown.m.g6 && !smfma_gu) jx::launch_q8_to_q6(L->hqs, n, L->hhs.a, ss);
-                jx::launch_mfma_down_block(L->sdown.m, L->hhs.a, L->hqs, sg, st_ub, L->ysh, ss);
+                if ((L->hhs.a.q6 || L->hhs.a.xp) && !smfma_gu) jx::launch_q8_to_block(L->hqs, n, L->hhs.a, ss);
+                jx::launch_mfma_down_block(L->sdown.m, L->hqs, L->hhs.a, sg, st_ub, L->ysh, ss);
             } else {
                 if (L->sdown_f32)
                     jx::launch_f32_to_acth(L->hfs, (int)fspad, n, L->hhs.a, ss);
@@ -889,10 +919,10 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     const float* gxf = L->gu_f32 ? L->xf : nullptr;
     if (mfma_gu) {
         Launch l(L, "gateup_mfma", st);
-        const bool h6 = mfma_down && dn_block && L->down.m.g6;  // h straight into its down's operand form
-        jx::launch_mfma_gateup(L->gate.m, L->up.m, L->xh.a, L->xq, grp, tiles_ub,
-                               L->down_f32 || h6 ? jx::ActQ8{} : L->hq, h6 ? L->hh.a : jx::ActH{},
-                               L->down_f32 ? L->hf : nullptr, st, nk < jx::BG_FEW * E);
+        const jx::ActH hh = mfma_down && dn_block ? L->hh.a : jx::ActH{};  // h straight into its down's forms
+        jx::launch_mfma_gateup(L->gate.m, L->up.m, L->xq, L->xh.a, grp, tiles_ub,
+                               L->down_f32 || hh.q6 ? jx::ActQ8{} : L->hq, hh, L->down_f32 ? L->hf : nullptr, st,
+                               nk < jx::BG_FEW * E);
     } else if (small_logits) {
         jx::Groups lg = grp;
         lg.logits = L->logits;
@@ -928,12 +958,12 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
 
     int ks = 1;  // parts of the down GEMM's K (the combine adds them)
     if (mfma_down) {
-        if (dn_block ? L->down.m.g6 && !mfma_gu : true) {
+        if (dn_block ? (L->hh.a.q6 || L->hh.a.xp) && !mfma_gu : true) {
             Launch l(L, "h_to_matrix_form", st);
             if (L->down_f32)
                 jx::launch_f32_to_acth(L->hf, (int)fpad, nk, L->hh.a, st);
             else if (dn_block)
-                jx::launch_q8_to_q6(L->hq, nk, L->hh.a, st);
+                jx::launch_q8_to_block(L->hq, nk, L->hh.a, st);
             else
                 jx::launch_q8_to_acth(L->hq, nk, L->hh.a, st);
         }
@@ -945,7 +975,7 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
             Launch l(L, "down_mfma", st);
             ks = jx::mfma_down_ksplit(hK);
             if (dn_block)
-                jx::launch_mfma_down_block(L->down.m, L->hh.a, L->hq, grp, tiles_ub, L->y, st, ks, L->ystride,
+                jx::launch_mfma_down_block(L->down.m, L->hq, L->hh.a, grp, tiles_ub, L->y, st, ks, L->ystride,
                                            nk < jx::BG_FEW * E);
             else
                 jx::launch_mfma_down(L->down.m, L->hh.a, grp, tiles_ub, L->y, st, ks, L->ystride,
@@ -1135,18 +1165,20 @@ int jx_moe_layer_create(const jx_moe_layer_desc* D, jx_moe_layer** out) {
         if (hipMemcpy(L->bias, D->router_bias, E * 4, hipMemcpyHostToDevice) != hipSuccess)
             return bail(fail(JX_ERR_HIP, "router bias upload"));
     }
-    if ((r = upload_matrix(D->gate_type, L->E, L->F, L->d, D->gate_exps, L->gate, st, Gemm::gateup)) != JX_OK) return bail(r);
+    bool codes = true;  // JX_GEMM_CODES=0: no FP6 codes beside the weights (the same results, slower prompts)
+    if (const char* f = std::getenv("JX_GEMM_CODES")) codes = std::strcmp(f, "0") != 0;
+    if ((r = upload_matrix(D->gate_type, L->E, L->F, L->d, D->gate_exps, L->gate, st, Gemm::gateup, codes)) != JX_OK) return bail(r);
     L->gate.m.act = D->activation;
-    if ((r = upload_matrix(D->up_type, L->E, L->F, L->d, D->up_exps, L->up, st, Gemm::gateup)) != JX_OK) return bail(r);
-    if ((r = upload_matrix(D->down_type, L->E, L->d, L->F, D->down_exps, L->down, st, Gemm::down)) != JX_OK) return bail(r);
+    if ((r = upload_matrix(D->up_type, L->E, L->F, L->d, D->up_exps, L->up, st, Gemm::gateup, codes)) != JX_OK) return bail(r);
+    if ((r = upload_matrix(D->down_type, L->E, L->d, L->F, D->down_exps, L->down, st, Gemm::down, codes)) != JX_OK) return bail(r);
     if (L->shared) {
-        if ((r = upload_matrix(D->sh_gate_type, 1, L->Fs, L->d, D->sh_gate, L->sgate, st, Gemm::gateup)) != JX_OK) return bail(r);
+        if ((r = upload_matrix(D->sh_gate_type, 1, L->Fs, L->d, D->sh_gate, L->sgate, st, Gemm::gateup, codes)) != JX_OK) return bail(r);
         // The shared expert is always SwiGLU: src/transformer.cpp:2741-2745 calls matmul_swiglu_quant_f32
         // without hp_.use_gelu (default false, include/quant.h:361); GELU-tanh reaches only the routed
         // experts (2721-2724).
         L->sgate.m.act = jx::ACT_SILU;
-        if ((r = upload_matrix(D->sh_up_type, 1, L->Fs, L->d, D->sh_up, L->sup, st, Gemm::gateup)) != JX_OK) return bail(r);
-        if ((r = upload_matrix(D->sh_down_type, 1, L->d, L->Fs, D->sh_down, L->sdown, st, Gemm::down)) != JX_OK) return bail(r);
+        if ((r = upload_matrix(D->sh_up_type, 1, L->Fs, L->d, D->sh_up, L->sup, st, Gemm::gateup, codes)) != JX_OK) return bail(r);
+        if ((r = upload_matrix(D->sh_down_type, 1, L->d, L->Fs, D->sh_down, L->sdown, st, Gemm::down, codes)) != JX_OK) return bail(r);
         if (D->sh_gate_inp) {
             if ((r = dalloc(L->shgate, d)) != JX_OK) return bail(r);
             if (hipMemcpy(L->shgate, D->sh_gate_inp, d * 4, hipMemcpyHostToDevice) != hipSuccess)
