@@ -117,7 +117,8 @@ void jx_moe_layer_destroy(jx_moe_layer* layer);
 /* The MoE block for n_tok tokens (replaces src/transformer.cpp:2589-2757 for
  * one token at a time; tokens are independent, so a batch is the per-token
  * block applied to each row):
- *   x           [n_tok][d] fp32 post-ffn_norm activations
+ *   x           [n_tok][d] fp32 post-ffn_norm activations (device pointers: any alignment of fp32,
+ *               16 bytes for the fastest router at 512 tokens and more)
  *   out         [n_tok][d] fp32 moe_accum (the residual add stays with the caller)
  *   topk_ids    [n_tok][k] int32 selected experts, descending logit   (or NULL)
  *   topk_w      [n_tok][k] fp32 softmax weights over the k             (or NULL)

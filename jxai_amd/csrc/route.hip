@@ -469,9 +469,10 @@ static void launch_route_topk(const RouteArgs& a, hipStream_t st) {
 
 // The matrix-core router: more than 16 rows (fewer leave most of a result's 16 columns empty) in the fp32 chain
 // order (F16 / BF16 rows have another), whole chunks, and from 512 tokens on (below, the split
-// k_route, one token per block, fills more CUs).
+// k_route, one token per block, fills more CUs).  x comes by 16-byte DMA, so a caller's x off that alignment stays with
+// k_route's ordinary loads.
 static bool route_mfma_fits(const RouteArgs& a) {
-    return a.E + (a.shgate ? 1 : 0) > RT_GROUPS && a.d % RM_C == 0 && a.n >= 512 && a.n <= 65535 * RM_T && !a.chain8;
+    return reinterpret_cast<uintptr_t>(a.x) % 16 == 0 && a.E + (a.shgate ? 1 : 0) > RT_GROUPS && a.d % RM_C == 0 && a.n >= 512 && a.n <= 65535 * RM_T && !a.chain8;
 }
 
 void launch_route(const RouteArgs& a, hipStream_t st) {

@@ -28,3 +28,28 @@ def test_router_logits_bitexact(port, E, shared, d, n):
     assert np.array_equal(ids, ids_o)
     np.testing.assert_allclose(w, w_o, rtol=2e-6, atol=0)
     L.close()
+
+
+@pytest.mark.parametrize("n", [130, 512, 600])
+def test_router_unaligned_x(port, n):
+    """A caller's x on the alignment of a float only: the same logits and outputs, bit for bit."""
+    from jxai_amd import moe
+    moe.init(0)
+    cfg = synth.LayerConfig("rm_off", 256, 24, 4, 256, F.Q4_0)
+    lw = synth.make_layer(cfg)
+    L = moe.MoELayer.from_weights(lw)
+    x = synth.make_tokens(cfg, n)
+    got = []
+    for at in (0, 1, 2, 4):  # floats
+        print(f"[gpu] router x off by {4 * at} bytes n={n}", flush=True)
+        xb = moe.DeviceBuffer(x.nbytes + 64).upload(np.concatenate([np.zeros(at, np.float32), x.reshape(-1)]))
+        xb.ptr = type(xb.ptr)(xb.ptr.value + 4 * at)
+        out = moe.DeviceBuffer(x.nbytes)
+        L.forward_device(xb, n, out)
+        xb.ptr = type(xb.ptr)(xb.ptr.value - 4 * at)
+        got.append((L.last_logits(n), out.download(np.empty_like(x))))
+    assert np.array_equal(got[0][0].view(np.uint32), port.route(lw, x)[0].view(np.uint32))
+    for logits, out in got[1:]:
+        assert np.array_equal(logits.view(np.uint32), got[0][0].view(np.uint32))
+        assert np.array_equal(out, got[0][1])
+    L.close()
