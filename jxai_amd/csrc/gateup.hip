@@ -638,8 +638,7 @@ void launch_t(const QMat& w0, const QMat& w1, const GuIn& in, const Groups& grp,
                        w1, in, grp, R, n_items, std::min(GATEUP ? Rg::GU_RC : Rg::DN_RC, R), o);
 }
 
-// The launch of a matrix (pair)'s format over x's forms; false: a form is missing (a caller bug: nothing is
-// launched on null pointers).
+// The launch of a matrix (pair)'s format over x's forms; false: a form is missing and nothing was launched.
 template <bool GATEUP>
 bool launch_form(const QMat& w0, const QMat& w1, const ActQ8& xq, const ActH& xh, const Groups& grp, int tiles_ub,
                  const BgOut& o, bool few, hipStream_t st) {
@@ -683,14 +682,14 @@ void launch_g6_codes(const QMat& m, uint8_t* g6, hipStream_t st) {
     hipLaunchKernelGGL(k_g6_codes, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, m, KB, g6);
 }
 
-void launch_mfma_gateup(const QMat& g, const QMat& u, const ActQ8& xq, const ActH& xh, const Groups& grp, int tiles_ub,
+bool launch_mfma_gateup(const QMat& g, const QMat& u, const ActQ8& xq, const ActH& xh, const Groups& grp, int tiles_ub,
                         const ActQ8& hq, const ActH& hh, float* hf, hipStream_t st, bool few) {
-    (void)launch_form<true>(g, u, xq, xh, grp, tiles_ub, BgOut{hq, hh, hf, ((g.rows + 255) / 256) * 256, nullptr, 1, 0}, few, st);
+    return launch_form<true>(g, u, xq, xh, grp, tiles_ub, BgOut{hq, hh, hf, ((g.rows + 255) / 256) * 256, nullptr, 1, 0}, few, st);
 }
 
-void launch_mfma_down_block(const QMat& dn, const ActQ8& hq, const ActH& hh, const Groups& grp, int tiles_ub, float* y,
+bool launch_mfma_down_block(const QMat& dn, const ActQ8& hq, const ActH& hh, const Groups& grp, int tiles_ub, float* y,
                             hipStream_t st, int KS, size_t ystride, bool few) {
-    (void)launch_form<false>(dn, dn, hq, hh, grp, tiles_ub, BgOut{ActQ8{}, ActH{}, nullptr, 0, y, KS, ystride}, few, st);
+    return launch_form<false>(dn, dn, hq, hh, grp, tiles_ub, BgOut{ActQ8{}, ActH{}, nullptr, 0, y, KS, ystride}, few, st);
 }
 
 }  // namespace jx

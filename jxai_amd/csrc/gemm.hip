@@ -683,15 +683,16 @@ static void down_t(const QMat& dn, const ActH& hin, const Groups& grp, int tiles
     else launch_t<TYPE, Shape<TYPE>>(dn, hin, grp, tiles_ub, y, st, KS, ystride);
 }
 
-void launch_mfma_down(const QMat& dn, const ActH& hin, const Groups& grp, int tiles_ub, float* y, hipStream_t st,
+bool launch_mfma_down(const QMat& dn, const ActH& hin, const Groups& grp, int tiles_ub, float* y, hipStream_t st,
                       int KS, size_t ystride, bool small) {
+    if (!gemm_f16_ok(dn) || !hin.hl || !hin.pe || !hin.xm) return false;
     switch (dn.type) {
         case T_Q4_K: down_t<T_Q4_K>(dn, hin, grp, tiles_ub, y, st, KS, ystride, small); break;
         case T_Q5_0: down_t<T_Q5_0>(dn, hin, grp, tiles_ub, y, st, KS, ystride, small); break;
         case T_Q5_K: down_t<T_Q5_K>(dn, hin, grp, tiles_ub, y, st, KS, ystride, small); break;
-        case T_Q6_K: down_t<T_Q6_K>(dn, hin, grp, tiles_ub, y, st, KS, ystride, small); break;
-        default: break;
+        default: down_t<T_Q6_K>(dn, hin, grp, tiles_ub, y, st, KS, ystride, small); break;
     }
+    return true;
 }
 
 }  // namespace jx

@@ -7,6 +7,11 @@
 
 namespace jx {
 
+enum : int { T_F32 = 0, T_Q4_0 = 2, T_Q5_0 = 6, T_Q8_0 = 8, T_Q4_K = 12, T_Q5_K = 13, T_Q6_K = 14 };
+
+// Super-block formats (256 elements per K-unit, Q4_K-style header for Q4_K and Q5_K).
+__host__ __device__ constexpr bool is_kquant(int t) { return t == T_Q4_K || t == T_Q5_K || t == T_Q6_K; }
+
 // One projection (gate, up or down) of every expert, repacked in HBM into
 // tiles of 32 rows so a wave's 32 lanes read 32 rows' 16-byte chunks of the
 // same K-block as one contiguous 512-byte run:
@@ -268,12 +273,13 @@ void launch_gemv_down_f16(const QMat& dn, const ActH& hh, const Groups& grp, int
 // Prefill regime: matrix-core grouped GEMMs over the dispatch tile table.
 // The block GEMM over Q8_0 activations: from the matrices' codes where they have them (x's ActH::q6), else from their
 // blocks (xq); Q4_K / Q5_K with the min-term pieces (ActH::xp).  Both give the same bits.
+// These launches return false, with nothing launched, where a matrix or its activations lack the form they read.
 // Gate/up writes SwiGLU(h) as Q8_0 (hq.q != null), in its block-GEMM forms (hh.q6, hh.xp) and/or fp32 (hf != null).
-void launch_mfma_gateup(const QMat& g, const QMat& u, const ActQ8& xq, const ActH& xh, const Groups& grp, int tiles_ub,
+bool launch_mfma_gateup(const QMat& g, const QMat& u, const ActQ8& xq, const ActH& xh, const Groups& grp, int tiles_ub,
                         const ActQ8& hq, const ActH& hh, float* hf, hipStream_t st, bool few = false);
 // Down on the same GEMM.  KS > 1: the K range split over KS workgroups per item (whole super-blocks each), part q of
 // the output at y + q * ystride (the combine adds the parts in order).
-void launch_mfma_down_block(const QMat& dn, const ActQ8& hq, const ActH& hh, const Groups& grp, int tiles_ub, float* y,
+bool launch_mfma_down_block(const QMat& dn, const ActQ8& hq, const ActH& hh, const Groups& grp, int tiles_ub, float* y,
                             hipStream_t st, int KS = 1, size_t ystride = 0, bool few = false);
 // `few`: the average expert has fewer than BG_FEW pairs, most of its parts one pair tile.
 constexpr int BG_FEW = 24;
@@ -284,7 +290,7 @@ void launch_block_table(const QMat& m, uint8_t* bt, int* over, hipStream_t st);
 void launch_g6_codes(const QMat& m, uint8_t* g6, hipStream_t st);
 // The fp16 down GEMM, KS as above.  small: few pairs per expert (the
 // 64-pair tile form at more workgroups per CU).
-void launch_mfma_down(const QMat& dn, const ActH& hin, const Groups& grp, int tiles_ub, float* y, hipStream_t st,
+bool launch_mfma_down(const QMat& dn, const ActH& hin, const Groups& grp, int tiles_ub, float* y, hipStream_t st,
                       int KS = 1, size_t ystride = 0, bool small = false);
 // Down GEMM in the small form up to this many (token, slot) pairs per expert on average (measured:
 // Mixtral-shaped 512 tokens, 128 per expert, 239 -> 202 us; Qwen3-shaped 2048 tokens with Zipf-skewed

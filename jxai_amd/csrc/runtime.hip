@@ -835,12 +835,13 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     // measured per step, weights from HBM: 48 / 64 tokens 133.6 / 138.8 -> 127.2 / 137.3 us.  Two parts
     // (DeepSeek-V2-Lite-shaped 2816 against 1408) measured slower: 32 tokens 132.5 -> 135.7 us.
     const bool sh_ksplit = L->shared && !smfma_dn && tbs == 16 && !L->sdown_f32 && L->shparts_cap >= 4 && L->sh_ksplit;
+    bool launched = true;  // a GEMM launch without its operands' forms launches nothing and clears it
     auto shared_gateup = [&](hipStream_t ss) {
         if (smfma_gu) {
             Launch l(L, "shared_gateup_mfma", ss);
             const jx::ActH hh = smfma_dn && sdn_block ? L->hhs.a : jx::ActH{};  // h straight into its down's forms
-            jx::launch_mfma_gateup(L->sgate.m, L->sup.m, L->xq, L->xh.a, sg, st_ub,
-                                   L->sdown_f32 || hh.q6 ? jx::ActQ8{} : L->hqs, hh, L->sdown_f32 ? L->hfs : nullptr, ss);
+            launched &= jx::launch_mfma_gateup(L->sgate.m, L->sup.m, L->xq, L->xh.a, sg, st_ub,
+                                               L->sdown_f32 || hh.q6 ? jx::ActQ8{} : L->hqs, hh, L->sdown_f32 ? L->hfs : nullptr, ss);
         } else {
             Launch l(L, "shared_gateup_gemv", ss);
             jx::launch_gemv_gateup(L->sgate.m, L->sup.m, L->xq, sg, sslots, tbs, L->hqs, L->sdown_f32 ? L->hfs : nullptr, ss,
@@ -852,13 +853,13 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
             Launch l(L, "shared_down", ss);
             if (sdn_block) {
                 if ((L->hhs.a.q6 || L->hhs.a.xp) && !smfma_gu) jx::launch_q8_to_block(L->hqs, n, L->hhs.a, ss);
-                jx::launch_mfma_down_block(L->sdown.m, L->hqs, L->hhs.a, sg, st_ub, L->ysh, ss);
+                launched &= jx::launch_mfma_down_block(L->sdown.m, L->hqs, L->hhs.a, sg, st_ub, L->ysh, ss);
             } else {
                 if (L->sdown_f32)
                     jx::launch_f32_to_acth(L->hfs, (int)fspad, n, L->hhs.a, ss);
                 else
                     jx::launch_q8_to_acth(L->hqs, n, L->hhs.a, ss);
-                jx::launch_mfma_down(L->sdown.m, L->hhs.a, sg, st_ub, L->ysh, ss);
+                launched &= jx::launch_mfma_down(L->sdown.m, L->hhs.a, sg, st_ub, L->ysh, ss);
             }
         } else if (sh_ksplit) {
             // the dense shared down's long K in parts, each block a routed block's share of units (the
@@ -920,9 +921,9 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     if (mfma_gu) {
         Launch l(L, "gateup_mfma", st);
         const jx::ActH hh = mfma_down && dn_block ? L->hh.a : jx::ActH{};  // h straight into its down's forms
-        jx::launch_mfma_gateup(L->gate.m, L->up.m, L->xq, L->xh.a, grp, tiles_ub,
-                               L->down_f32 || hh.q6 ? jx::ActQ8{} : L->hq, hh, L->down_f32 ? L->hf : nullptr, st,
-                               nk < jx::BG_FEW * E);
+        launched &= jx::launch_mfma_gateup(L->gate.m, L->up.m, L->xq, L->xh.a, grp, tiles_ub,
+                                           L->down_f32 || hh.q6 ? jx::ActQ8{} : L->hq, hh, L->down_f32 ? L->hf : nullptr,
+                                           st, nk < jx::BG_FEW * E);
     } else if (small_logits) {
         jx::Groups lg = grp;
         lg.logits = L->logits;
@@ -975,11 +976,11 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
             Launch l(L, "down_mfma", st);
             ks = jx::mfma_down_ksplit(hK);
             if (dn_block)
-                jx::launch_mfma_down_block(L->down.m, L->hq, L->hh.a, grp, tiles_ub, L->y, st, ks, L->ystride,
-                                           nk < jx::BG_FEW * E);
+                launched &= jx::launch_mfma_down_block(L->down.m, L->hq, L->hh.a, grp, tiles_ub, L->y, st, ks, L->ystride,
+                                                       nk < jx::BG_FEW * E);
             else
-                jx::launch_mfma_down(L->down.m, L->hh.a, grp, tiles_ub, L->y, st, ks, L->ystride,
-                                 nk <= jx::MFMA_DOWN_SMALL_MAX_PPE * E);
+                launched &= jx::launch_mfma_down(L->down.m, L->hh.a, grp, tiles_ub, L->y, st, ks, L->ystride,
+                                                 nk <= jx::MFMA_DOWN_SMALL_MAX_PPE * E);
         }
     } else {
         jx::CombineOut comb;
@@ -1016,6 +1017,7 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
                            ks > 1 ? L->y + L->ystride : nullptr, shparts);
     }
     HIPCHK(hipGetLastError());
+    if (!launched) return fail(JX_ERR_HIP, "a GEMM's operands lack the form it reads; the outputs are invalid");
     return JX_OK;
 }
 

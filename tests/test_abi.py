@@ -82,3 +82,15 @@ def test_compiled_caller_without_device(jxlib, tmp_path):
     r = subprocess.run([exe, "nodevice"], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "-> 5" in r.stdout
+
+
+def test_gemm_launches_refuse_missing_forms(jxlib, tmp_path):
+    """A GEMM launch whose operands lack the form it reads reports it (and launches nothing: no GPU is needed)."""
+    from jxai_amd import _lib
+    exe = os.path.join(str(tmp_path), "launch_caller")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include",
+                    "-I", os.path.join(ROOT, "jxai_amd", "csrc"), os.path.join(ROOT, "tests", "launch_caller.cpp"),
+                    "-o", exe, _lib.LIB_PATH, "-Wl,-rpath," + os.path.dirname(_lib.LIB_PATH)], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert r.stdout.count("refused") == 24
