@@ -49,13 +49,14 @@ __device__ __forceinline__ const uint8_t* uniform_ptr(const void* p) {
 // 64 lanes x 16 bytes from src (dma_base) + off (per lane) into LDS at byte `lds` (wave-uniform), lane i at lds + 16 i.  In
 // asm because the compiler, which counts the builtin as a flat access, then waits for every load in flight
 // before it uses any.  It has no result registers; the waits are the kernel's own (vmcnt counts in order, so the
-// compiler's counted waits for the weights only get stricter).  A kernel that uses it uses m0 for nothing else.
+// compiler's counted waits for the weights only get stricter).
 __device__ __forceinline__ void dma16g(gbyte* src, uint32_t off, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(src) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(src)
+                 : "memory", "m0");
 }
 // The same from per-lane addresses.
 __device__ __forceinline__ void dma16v(const uint8_t* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }
 
 __device__ __forceinline__ v16f mfma16(h8 a, h8 b, v16f c) {

@@ -94,3 +94,17 @@ def test_gemm_launches_refuse_missing_forms(jxlib, tmp_path):
     r = subprocess.run([exe], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.count("refused") == 24
+
+
+def test_inline_asm_declares_what_it_writes():
+    """Inline asm that sets m0 says so: the compiler may keep a value of its own there."""
+    found = 0
+    csrc = os.path.join(ROOT, "jxai_amd", "csrc")
+    for f in sorted(os.listdir(csrc)):
+        if not f.endswith((".h", ".hip")):
+            continue
+        for stmt in re.findall(r"\basm\s*(?:volatile)?\s*\((.*?)\)\s*;", open(os.path.join(csrc, f)).read(), flags=re.S):
+            if re.search(r"\bm0\s*,", stmt.split("::")[0]):
+                found += 1
+                assert re.search(r':[^:]*"m0"', stmt.split("::")[-1]), (f, stmt)
+    assert found >= 2
