@@ -147,9 +147,13 @@ constexpr int MAX_SLOTS_DEC = 16;  // routed slots (top_k) of the fused one-toke
 constexpr int MFMA_BN = 128;  // pairs per matrix-core GEMM tile
 // shared expert on the matrix cores from this many tokens (one dense expert fills few GEMM
 // workgroups below that: 44 gate/up workgroups for a 5632 x 2048 expert at 64 tokens; the 16-token GEMV runs in one
-// group per 16 tokens).  Per step with 64 / 128 / 256: Qwen1.5-shaped 96 tokens 191 / 182 / 183 us, 190 tokens 201 /
-// 201 / 208, 250 tokens 204 / 204 / 226; DeepSeek-V2-Lite-shaped 70 tokens 195 / 169 / 170, 130 tokens 201 / 201 / 210.
-constexpr int MFMA_MIN_SHARED_TOKENS = 128;
+// group per 16 tokens).  Per step with 64 / 128 / 256: DeepSeek-V2-Lite-shaped (Q4_K) 70 tokens 192 / 169 / 168 us, 130 tokens
+// 199 / 201 / 210; its Q5_K form 70 tokens 218 / 179 / 179, 190 tokens 209 / 209 / 221; Qwen1.5-shaped in Q8_0 96 tokens 205 / 194 /
+// 192, 190 tokens 231 / 231 / 249.  Q4_0, whose 16-token GEMV runs at three waves per SIMD (Qwen1.5-shaped): 130 / 160 / 176 / 200
+// tokens 197 / 199 / 201 / 201 with 128, 192 / 198 / 203 / 212 with 256 (fp32 h, whose GEMV is the slow one: 130 tokens 158
+// with 128, 203 with 256).  Where only the down moves (Q6_K and Q5_0 gate/up stay on the GEMVs): Q6_K 70 / 96 / 112 tokens 190 / 201 /
+// 207 with 64, 193 / 215 / 218 with 128; Q5_0 96 tokens 460 and 477.
+constexpr int MFMA_MIN_SHARED_TOKENS = 128, MFMA_MIN_SHARED_TOKENS_Q4_0 = 160, MFMA_MIN_SHARED_TOKENS_DOWN = 64;
 
 // The weighted combine folded into the down GEMV (few-token decode with at most two
 // contributions per output element: top_k <= 2 and no shared expert): out [n][d] is

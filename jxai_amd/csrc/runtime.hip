@@ -580,13 +580,21 @@ int resolve_profile(jx_moe_layer* L) {
 // per 16 tokens, the GEMM once per 64-pair tile.  Forced-GEMV against forced-GEMM steps (us):
 //   Q8_0 (Qwen3-shaped): 8 / 12 / 16 / 24 / 32 / 64 tokens (0.5 / 0.75 / 1 / 1.5 / 2 / 4 pairs) 53 / 65 / 71 / 91 / 101 / 167
 //   against 58 / 59 / 62 / 67 / 73 / 107
-//   Q4_0 (Qwen1.5-shaped): 64 / 96 / 128 / 176 tokens (4 / 6 / 9 / 12 pairs) 127 / 183 / 187 / 222 against 153 / 181 / 184 / 206
+//   (with a Q6_K down 12 / 16 / 32 tokens 73 / 75 / 105 against 65 / 66 / 76, with a Q5_0 down 70 / 72 / 90 against 69 / 73 /
+//   83; the routing is skewed there, with uniform routing 16 / 24 / 32 / 48 tokens 101 / 118 / 123 / 142 against 114 /
+//   124 / 129 / 143)
+//   Q4_0: the line follows the gate/up workgroups (E x row groups; few pairs are one part per expert).  In one round of the
+//   chip's 512 (1408 x 2048, 32 experts, 352 workgroups) 6 / 8 / 10 / 12 pairs 88 / 92 / 94 / 130 against 65 / 66 / 66 / 66; in two
+//   (60 experts, 660) 6 / 9 / 10 pairs 106 / 114 / 143 against 124 / 130 / 131; too few for the chip (8 experts, 88)
+//   7 / 12 pairs 43 / 45 against 50 / 50.  With a shared expert of four times their size (Qwen1.5-shaped) 7 / 8.5 / 9.6 pairs
+//   182 / 186 / 210 against 180 / 180 / 200.  A Q6_K or Q5_0 down moves none of these.
 //   small K-quant experts (DeepSeek-V2-Lite-shaped): 96 / 128 tokens (9 / 12 pairs) 184 / 208 against 192 / 194
 //   large experts (Mixtral-shaped, 14336 x 4096 per matrix, whose GEMV streams near its best rate): 64 / 96 tokens
 //   (16 / 24 pairs) 318 / 405 against 320 / 344
 // Large Q8_0 experts and batches under 12 tokens keep 4 pairs.
 constexpr int MFMA_MIN_PAIRS_PER_EXPERT_KQ = 12;
-constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q4_0 = 7;
+constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q4_0 = 10, MFMA_MIN_PAIRS_PER_EXPERT_Q4_0_ROUND = 7;
+constexpr int ROUND_MIN_WGS = 128, ROUND_WGS = 512;  // two workgroups on each of 256 CUs
 constexpr int MFMA_MIN_PAIRS_PER_EXPERT_LARGE = 16;
 constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q8 = 1, MFMA_MIN_TOKENS_Q8 = 12;
 constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q8_LARGE = 4;
@@ -642,11 +650,14 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
     const int nk = n * k;
     const int hK = down_h_k(L->down.m.type, L->F, L->down_f32);
     const bool large = (size_t)d * L->F >= LARGE_EXPERT_ELEMS;
+    const int gu_wgs = E * ((L->gate.m.nrt + 3) / 4);
+    const bool one_round = gu_wgs >= ROUND_MIN_WGS && gu_wgs <= ROUND_WGS;
     const int min_ppe = L->gate.m.type == jx::T_Q8_0
                             ? (large || n < MFMA_MIN_TOKENS_Q8 ? MFMA_MIN_PAIRS_PER_EXPERT_Q8_LARGE : MFMA_MIN_PAIRS_PER_EXPERT_Q8)
                         : large                            ? MFMA_MIN_PAIRS_PER_EXPERT_LARGE
-                        : L->gate.m.type == jx::T_Q4_0     ? MFMA_MIN_PAIRS_PER_EXPERT_Q4_0
-                                                           : MFMA_MIN_PAIRS_PER_EXPERT_KQ;
+                        : L->gate.m.type != jx::T_Q4_0     ? MFMA_MIN_PAIRS_PER_EXPERT_KQ
+                        : one_round || L->shparts_cap >= 4 ? MFMA_MIN_PAIRS_PER_EXPERT_Q4_0_ROUND
+                                                           : MFMA_MIN_PAIRS_PER_EXPERT_Q4_0;
     bool mfma = (size_t)nk >= (size_t)min_ppe * E;
     if (flags & JX_FWD_FORCE_GEMV) mfma = false;
     if (flags & JX_FWD_FORCE_MFMA) mfma = true;
@@ -1230,7 +1241,10 @@ int jx_moe_layer_create(const jx_moe_layer_desc* D, jx_moe_layer** out) {
     L->cold_pairs = COLD_PAIRS;
     if (const char* f = std::getenv("JX_SH_KSPLIT")) L->sh_ksplit = std::strcmp(f, "0") != 0;
     if (const char* f = std::getenv("JX_COLD_PAIRS")) L->cold_pairs = std::max(0, std::atoi(f));
-    L->smfma_min = jx::MFMA_MIN_SHARED_TOKENS;
+    const bool sh_block = L->shared && block_gemm(L->sgate, L->d, L->sgu_f32) && block_gemm(L->sup, L->d, L->sgu_f32);
+    L->smfma_min = !sh_block                                                  ? jx::MFMA_MIN_SHARED_TOKENS_DOWN
+                   : L->sgate.m.type == jx::T_Q4_0 && !L->sdown_f32 ? jx::MFMA_MIN_SHARED_TOKENS_Q4_0
+                                                                              : jx::MFMA_MIN_SHARED_TOKENS;
     if (const char* f = std::getenv("JX_SMFMA_MIN")) L->smfma_min = std::max(1, std::atoi(f));
     if ((r = dalloc(L->dsync, 1)) != JX_OK) return bail(r);
     if ((r = dalloc(L->hw, (size_t)L->k * L->F / 4)) != JX_OK) return bail(r);

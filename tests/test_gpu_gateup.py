@@ -41,22 +41,52 @@ def test_gateup_tile_edges(moe, port, fmt, d, ff):
     L.close()
 
 
-# the largest batch of the GEMVs and the smallest of the GEMMs: 7 pairs per expert (Q4_0), 12 (K-quants), 12 tokens (Q8_0)
-@pytest.mark.parametrize("fmt,n", [(F.Q4_0, 28), (F.Q4_K, 48), (F.Q8_0, 12)])
-def test_regime_edge(moe, port, fmt, n):
+# the largest batch of the GEMVs and the smallest of the GEMMs: 10 pairs per expert (Q4_0; 7 where the gate/up workgroups
+# fill the chip once, or beside a shared expert of four times the size), 12 (K-quants), 12 tokens (Q8_0); the same with a
+# down that has no block GEMM
+@pytest.mark.parametrize("fmt,n,kw", [(F.Q4_0, 40, {}), (F.Q4_0, 28, dict(n_experts=16, top_k=4, d_ff=1024)),
+                                      (F.Q4_0, 40, dict(n_experts=64, top_k=16, d_ff=1152)),
+                                      (F.Q4_0, 28, dict(d_ff=256, d_ff_shared=1024)),
+                                      (F.Q4_0, 40, dict(down_wtype=F.Q6_K)), (F.Q4_0, 40, dict(down_wtype=F.Q5_0)),
+                                      (F.Q4_K, 48, {}), (F.Q8_0, 12, {}), (F.Q8_0, 12, dict(down_wtype=F.Q6_K))])
+def test_regime_edge(moe, port, fmt, n, kw):
     """Either side of the line the layer's own choice is that regime's result bit for bit, and the oracle's."""
-    cfg = synth.LayerConfig(f"edge_{fmt}", 512, 8, 2, 1280, fmt)
+    kw = dict(dict(n_experts=8, top_k=2, d_ff=1280), **kw)
+    cfg = synth.LayerConfig("edge_" + "_".join(str(v) for v in (fmt, *kw.values())), 512, wtype=fmt, **kw)
     lw = synth.make_layer(cfg)
     L = moe.MoELayer.from_weights(lw)
     for m, regime in ((n - 1, "gemv"), (n, "mfma")):
-        print(f"[gpu] regime edge {fmt} n={m}", flush=True)
+        print(f"[gpu] regime edge {fmt} {kw} n={m}", flush=True)
         x = synth.make_tokens(cfg, m)
         out, ids, _, _ = L.forward(x)
         assert np.array_equal(out, L.forward(x, regime=regime)[0])
         want, ids_o, _, _ = port.moe_forward(lw, x)
         assert np.array_equal(ids, ids_o)
-        assert (np.abs(out - want).max(axis=1) <= 1e-3 * np.abs(want).max(axis=1)).all()  # d_ff past 1024: the layer bar
+        # the layer bar from d_ff = 1024 on (one step of h below it: 1 / (32 sqrt(d_ff)) of a row's largest output)
+        err = np.abs(out - want).max(axis=1) / np.abs(want).max(axis=1)
+        assert err.max() <= max(1e-3, 1 / (32 * np.sqrt(cfg.d_ff))) and np.median(err) <= 1e-3
     L.close()
+
+
+@pytest.mark.parametrize("fmt,n,kw", [(F.Q4_0, 160, {}), (F.Q4_0, 128, dict(sh_down_wtype=F.Q5_0)), (F.Q4_K, 128, {}),
+                                      (F.Q8_0, 128, {}), (F.Q6_K, 64, {}), (F.Q5_0, 64, {})])
+def test_shared_regime_edge(moe, monkeypatch, fmt, n, kw):
+    """The shared expert's own line: below it the GEMVs' result, from it the GEMMs'."""
+    cfg = synth.LayerConfig(f"shedge_{fmt}_{len(kw)}", 512, 4, 2, 256, fmt, d_ff_shared=512, **kw)
+    lw = synth.make_layer(cfg)
+    layers = []
+    for line in (None, "1000000", "1"):
+        if line:
+            monkeypatch.setenv("JX_SMFMA_MIN", line)
+        layers.append(moe.MoELayer.from_weights(lw))
+    print(f"[gpu] shared regime edge {fmt} {kw} n={n}", flush=True)
+    for m, same, other in ((n - 1, 1, 2), (n, 2, 1)):
+        x = synth.make_tokens(cfg, m)
+        out = [L.forward(x)[0] for L in layers]
+        assert np.array_equal(out[0], out[same])
+        assert not np.array_equal(out[0], out[other])  # (the two round differently)
+    for L in layers:
+        L.close()
 
 
 @pytest.mark.parametrize("fmt", [F.Q4_0, F.Q8_0, F.Q4_K, F.Q5_K, F.Q6_K])
