@@ -20,7 +20,10 @@ def test_router_logits_bitexact(port, E, shared, d, n):
     lw = synth.make_layer(cfg)
     x = synth.make_tokens(cfg, n)
     x[3] = 0.0
-    x[5] *= np.float32(1e-30)  # subnormal products
+    x[5] *= np.float32(1e-37)  # subnormal products, and some that vanish
+    products = np.abs(lw.router.astype(np.float64) * x[5].astype(np.float64))
+    tiny = np.finfo(np.float32).tiny
+    assert (products < tiny).mean() > 0.9 and (products > 2.0 ** -149).mean() > 0.9
     L = moe.MoELayer.from_weights(lw)
     _, ids, w, _ = L.forward(x)
     lg_o, ids_o, w_o = port.route(lw, x)
