@@ -41,6 +41,77 @@ def test_gateup_tile_edges(moe, port, fmt, d, ff):
     L.close()
 
 
+# d: an odd number of the down's row tiles, so the last wave's second one is past the matrix; d_ff: odd numbers of its
+# half-units, and (from 8192 columns) K in two parts, for Q4_0 and Q8_0 the second an odd number of half-units.  Pairs
+# per expert as the tokens: one, either side of a pair tile, of a workgroup, and many (from 24 the FP6 forms' two-tile loop)
+@pytest.mark.parametrize("codes", ["1", "0"])
+@pytest.mark.parametrize("fmt,d,ff", [(F.Q4_0, 160, 384), (F.Q8_0, 160, 384), (F.Q4_0, 96, 8320), (F.Q8_0, 96, 8320),
+                                      (F.Q4_K, 288, 512), (F.Q5_K, 288, 512), (F.Q4_K, 32, 8448), (F.Q5_K, 32, 8448)])
+def test_down_tile_edges(moe, port, monkeypatch, fmt, d, ff, codes):
+    monkeypatch.setenv("JX_GEMM_CODES", codes)
+    cfg = synth.LayerConfig(f"dn_{fmt}_{d}_{ff}", d, 2, 2, ff, fmt)
+    lw = synth.make_layer(cfg)
+    L = moe.MoELayer.from_weights(lw)
+    for n in (1, 23, 32, 33, 65):
+        print(f"[gpu] down {fmt} d={d} ff={ff} codes={codes} n={n}", flush=True)
+        x = synth.make_tokens(cfg, n)
+        out, ids, _, _ = L.forward(x, regime="mfma")
+        want, ids_o, _, _ = port.moe_forward(lw, x)
+        assert np.array_equal(ids, ids_o)
+        # one step of h in a row's output, as test_gateup_tile_edges (K-quants with d off whole super-blocks have
+        # their gate/up on fp32 activations)
+        err = np.abs(out - want).max(axis=1) / np.abs(want).max(axis=1)
+        assert err.max() <= max(1e-3, 1 / (32 * np.sqrt(ff)))
+        assert np.median(err) <= 1e-3
+    L.close()
+
+
+def extreme_blocks(fmt, rows, cols, seed):
+    """A matrix whose 32-blocks each hold one extreme quant throughout (each sign where the format has one), or both."""
+    raw = synth.quant_matrix(seed, fmt, rows, cols).reshape(-1, F.BLOCK[fmt][1]).copy()
+    pick = synth.random_bytes(seed ^ 0x77, raw.shape[0]) % 3
+    lo, hi = (0x81, 0x7F) if fmt == F.Q8_0 else (0x00, 0xFF)
+    at = {F.Q4_0: 2, F.Q8_0: 2, F.Q4_K: 16, F.Q5_K: 16}[fmt]
+    fill = np.where(pick == 0, lo, hi).astype(np.uint8)[:, None]
+    body = np.broadcast_to(fill, (raw.shape[0], raw.shape[1] - at)).copy()
+    mixed = pick == 2
+    body[mixed, ::2] = lo
+    body[mixed, 1::2] = hi
+    raw[:, at:] = body
+    return raw.reshape(-1)
+
+
+@pytest.mark.parametrize("codes", ["1", "0"])
+@pytest.mark.parametrize("fmt", [F.Q4_0, F.Q8_0, F.Q4_K, F.Q5_K])
+def test_extreme_quants(moe, port, monkeypatch, fmt, codes):
+    """Whole blocks of the weights' largest quants against activations of +-127: the block sums of the greatest
+    magnitude (a down of one-hot columns would hide them: h is what the gate/up leaves)."""
+    monkeypatch.setenv("JX_GEMM_CODES", codes)
+    cfg = synth.LayerConfig(f"ext_{fmt}", 512, 2, 2, 1280, fmt)
+    lw = synth.make_layer(cfg)
+    lw.gate = extreme_blocks(fmt, 2 * 1280, 512, synth.sub_seed("ext", "gate"))
+    lw.up = extreme_blocks(fmt, 2 * 1280, 512, synth.sub_seed("ext", "up"))
+    lw.down = extreme_blocks(fmt, 2 * 512, 1280, synth.sub_seed("ext", "down"))
+    L = moe.MoELayer.from_weights(lw)
+    n = 70
+    print(f"[gpu] extreme quants {fmt} codes={codes}", flush=True)
+    sign = np.where(synth.random_bytes(synth.sub_seed("ext", "x"), n * 512) & 1, 1, -1).reshape(n, 512)
+    x = (sign * np.repeat(0.5 + synth.uniform01(synth.sub_seed("ext", "s"), n * 16), 32).reshape(n, 512)).astype(np.float32)
+    x[:8] = np.abs(x[:8])
+    x[8:16, ::2] = np.abs(x[8:16, ::2])
+    x[8:16, 1::2] = -np.abs(x[8:16, 1::2])
+    x *= np.float32(0.02)
+    out, ids, _, _ = L.forward(x, regime="mfma")
+    q = L.last_xq8(n).reshape(n, 16, 34)[:, :, 2:].view(np.int8)
+    assert (np.abs(q.astype(np.int32)) == 127).all()
+    want, ids_o, _, _ = port.moe_forward(lw, x)
+    assert np.array_equal(ids, ids_o)
+    err = np.abs(out - want).max(axis=1) / np.abs(want).max(axis=1)
+    # d_ff past 1024: the layer bar (a step of h against the down's extreme weights stays in proportion to the output)
+    assert err.max() <= 1e-3, err
+    L.close()
+
+
 # the largest batch of the GEMVs and the smallest of the GEMMs: 10 pairs per expert (Q4_0; 7 where the gate/up workgroups
 # fill the chip once, or beside a shared expert of four times the size), 12 (K-quants), 12 tokens (Q8_0); the same with a
 # down that has no block GEMM
