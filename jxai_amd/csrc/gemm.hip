@@ -212,7 +212,6 @@ k_wgemm(QMat W0, ActH in, Groups grp, int R, int n_items, int RC, float* y, int 
     constexpr bool Q4K = TYPE == T_Q4_K || TYPE == T_Q5_K;
     constexpr bool K6 = TYPE == T_Q6_K;
     constexpr bool SUPER = Q4K || K6;
-    constexpr int GB = 512;  // global bytes per row and half-unit (hi, lo)
     using St = Stage<BN>;
     constexpr int PB = St::PB, CPP = St::CPP, PPI = 64 / CPP;  // row bytes, chunks, rows per DMA
     constexpr int PER = BN / PPI / GW;  // 1 KB staging loads per wave and half-unit
@@ -258,23 +257,23 @@ k_wgemm(QMat W0, ActH in, Groups grp, int R, int n_items, int RC, float* y, int 
     const size_t src0 = (size_t)sm.src[0];
     // Staging: a DMA instruction moves PPI rows x PB bytes; lane l takes chunk l % CPP of row
     // PPI * slot + l / CPP, stored at chunk ((l % CPP) ^ (row % CPP)), so the operand reads of 16
-    // lanes hit 16 distinct 16-byte bank groups.  The half-unit adds h * 512, a uniform term.
+    // lanes hit 16 distinct 16-byte bank groups.  The half-unit adds h * PB, a uniform term.
     uint32_t soff[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
         const int r = PPI * (wave * PER + k) + lane / CPP;
-        soff[k] = (uint32_t)(sm.src[r] - (int)src0) * (uint32_t)(H * GB) + (uint32_t)(((lane % CPP) ^ (r % CPP)) << 4);
+        soff[k] = (uint32_t)(sm.src[r] - (int)src0) * (uint32_t)(H * PB) + (uint32_t)(((lane % CPP) ^ (r % CPP)) << 4);
     }
     const int sj = wave;  // pe / xm / rx: lane l of wave w < BN / 64 takes pair 64 * w + l
     const uint32_t srow = (uint32_t)(sm.src[64 * min(sj, BN / 64 - 1) + lane] - (int)src0);
     const uint32_t peoff = srow * (uint32_t)(H * 4);
     const uint32_t xoff = Q4K ? srow * (uint32_t)(in.KU * 48) : 0u;
-    const uint8_t* qsrc = reinterpret_cast<const uint8_t*>(in.hl) + src0 * (size_t)(H * GB);
+    const uint8_t* qsrc = reinterpret_cast<const uint8_t*>(in.hl) + src0 * (size_t)(H * PB);
     const uint8_t* pesrc = reinterpret_cast<const uint8_t*>(in.pe) + src0 * (size_t)(H * 4);
     const uint8_t* xmsrc = reinterpret_cast<const uint8_t*>(in.xm) + src0 * (size_t)(in.KU * 48);
     auto stage = [&](int h) {
         St& S = sm.st[h & 1];
-        const uint8_t* base = qsrc + (size_t)h * GB;
+        const uint8_t* base = qsrc + (size_t)h * PB;
 #pragma unroll
         for (int k = 0; k < PER; ++k) dma16(base + soff[k], S.q + (wave * PER + k) * 1024);
         if constexpr (Q4K) {

@@ -1716,7 +1716,7 @@ k_gemv_mxh(QMat W, ActH hin, Groups grp, float* y) {
             for (int q = 0; q < 4; ++q) {
                 const int i = i0 + q * NTH, t = i / c8, k = 8 * (i - t * c8);
                 v[q] = (i < NTP * c8 && t < nt)
-                           ? *reinterpret_cast<const uint4*>(hin.hl + (row0 + t) * (size_t)KH * 256 + (k >> 7) * 256 + (k & 127))
+                           ? *reinterpret_cast<const uint4*>(hin.hl + (row0 + t) * (size_t)(KH * 128) + k)
                            : make_uint4(0u, 0u, 0u, 0u);
             }
 #pragma unroll

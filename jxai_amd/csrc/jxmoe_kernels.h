@@ -86,19 +86,17 @@ struct ActQ8 {
     int K = 0;
 };
 
-// Q8_0 activations in the form the matrix-core GEMMs consume (K % 128 == 0):
-//   hl [rows][KH][256]   per 128-element half-unit: fp16 hi x128, then lo x128,
-//                        of dx * q * 2^-E (an exact split of the dequantized
-//                        value scaled into fp16 range)
-//   pe [rows][KH]        2^E of each half-unit, one E per row (the GEMMs apply
+// Activations in the forms the matrix-core GEMMs consume (K % 128 == 0).  The fp16 down GEMM's, of Q8_0 or fp32 h:
+//   hl [rows][K]         fp16 of dx * q * 2^-E (fp32 rows: h * 2^-E), rounded once
+//   pe [rows][KH]        2^E of each half-unit, one E per row (the GEMM applies
 //                        the last half-unit's): the exponent of the row's largest
-//                        block scale - 7 for Q8_0 rows (x from the router kernels,
-//                        h from k_q8_to_acth), so |dx * q| * 2^-E < 2^15; the
+//                        block scale - 7 for Q8_0 rows (k_q8_to_acth), so
+//                        |dx * q| * 2^-E < 2^15; the
 //                        exponent of max |h| - 14 for fp32 rows (k_f32_to_acth)
 //   xm [rows][KU][3][8]  per 256-element unit: bf16 pieces (hi, mid, lo) of
 //                        dx * sum(q) (fp32 rows: the block sum) times 2^-E for its
-//                        8 blocks (Q4_K min term)
-// and, for the block GEMM (each form is written where its pointer is set):
+//                        8 blocks (Q4_K / Q5_K min term)
+// and the block GEMM's, of Q8_0 x or h (each form is written where its pointer is set):
 //   q6 [rows][KH][256 B]  the quant is 16 a + b, |a|, |b| <= 8: per block and part of 16 elements the codes
 //                        of 16 a, then of b, as BF6 (e3m2) in units of 1/16, code i at bit 6 i, and the block
 //                        scale's fp16 dx.  Per half-unit: [4 blocks][2 parts][16 B] code words 0..3,

@@ -53,7 +53,7 @@ __device__ __forceinline__ void acth_chunk_v(uint2 qq, float2 sb, int K, const A
         const _Float16 h0 = (_Float16)(s * (float)q0), h1 = (_Float16)(s * (float)q1);  // products exact
         hw[u] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
     }
-    *reinterpret_cast<uint4*>(o.hl + row * (size_t)KH * 256 + hh * 256 + (i & 127)) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+    *reinterpret_cast<uint4*>(o.hl + row * (size_t)K + i) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
     if ((i & 127) == 0) o.pe[row * (size_t)KH + hh] = up;
     if ((i & 31) == 0)  // exact: 11-bit scale x |sum| < 2^12, times 2^-E
         store_pieces3(o.xm + row * (size_t)o.KU * 24 + (b / 8) * 24 + (b % 8), sb.x * sb.y * dn);
@@ -576,7 +576,7 @@ __global__ void __launch_bounds__(256) k_q8_to_acth_hi(ActQ8 in, int rows, ActH 
             const _Float16 h0 = (_Float16)(s * (float)q0), h1 = (_Float16)(s * (float)q1);  // products exact
             hw[u] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
         }
-        uint4* hl = reinterpret_cast<uint4*>(o.hl + row * (size_t)KH * 256 + hh * 256 + (e & 127));
+        uint4* hl = reinterpret_cast<uint4*>(o.hl + row * (size_t)K + e);
         hl[0] = make_uint4(hw[0], hw[1], hw[2], hw[3]);
         hl[1] = make_uint4(hw[4], hw[5], hw[6], hw[7]);
         if ((e & 127) == 0) o.pe[row * (size_t)KH + hh] = up;
@@ -658,8 +658,7 @@ __global__ void __launch_bounds__(256) k_f32_to_acth(const float* h, int ld, Act
             hw[u] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
             sum += f[2 * u] + f[2 * u + 1];
         }
-        uint16_t* hl = o.hl + row * (size_t)KH * 256 + hh * 256 + (i & 127);
-        *reinterpret_cast<uint4*>(hl) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+        *reinterpret_cast<uint4*>(o.hl + row * (size_t)K + i) = make_uint4(hw[0], hw[1], hw[2], hw[3]);
         if ((i & 127) == 0) o.pe[row * (size_t)KH + hh] = up;
         sum += __shfl_xor(sum, 1, 64);
         sum += __shfl_xor(sum, 2, 64);

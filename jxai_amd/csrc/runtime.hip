@@ -294,7 +294,7 @@ struct DevActH {
     int alloc_hi(size_t rows, int K) {
         shape(K);
         if (K % 128 != 0) return JX_OK;  // the matrix-core path is not used for this shape
-        HIPCHK(hipMalloc(&a.hl, rows * a.KH * 256 * sizeof(uint16_t)));
+        HIPCHK(hipMalloc(&a.hl, rows * K * sizeof(uint16_t)));
         HIPCHK(hipMalloc(&a.pe, rows * a.KH * sizeof(float)));
         HIPCHK(hipMalloc(&a.xm, rows * a.KU * 24 * sizeof(uint16_t)));
         return JX_OK;

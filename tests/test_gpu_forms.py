@@ -102,3 +102,24 @@ def test_scale_past_fp16(moe, port, fmt, which):
         # one step of h moves an output by 1 / (32 sqrt(d_ff)) of the row's largest; the fp16 down holds h in 11 bits
         assert err.max() <= max(1e-3, 1 / (32 * np.sqrt(cfg.d_ff))) and np.median(err) <= 1e-3
     L.close()
+
+
+def test_fp16_down_workspace(moe):
+    """The fp16 down GEMM's rows of h take 2 bytes per element, and what its kernels read is laid out by that."""
+    cfg = synth.LayerConfig("ws_q6k", 256, 2, 2, 8192, F.Q4_K, down_wtype=F.Q6_K)
+    lw = synth.make_layer(cfg)
+    L = moe.MoELayer.from_weights(lw)
+    n = 4096
+    print(f"[gpu] workspace of {n} tokens, Q6_K down", flush=True)
+    x = synth.make_tokens(cfg, n)
+    L.forward(x[:1])
+    before = free_bytes()[0]
+    L.forward(x, regime="mfma")
+    used = before - free_bytes()[0]
+    pairs = n * cfg.top_k
+    # per pair: h in Q8_0 (1 byte an element, 8 a block) and in the fp16 form (2, pieces 48 a super-block, 4 a half-unit),
+    # the down's output in two parts; per token: x three times, its Q8_0 form and codes (2 bytes) and pieces
+    h = cfg.d_ff * (1 + 8 / 32 + 2 + 48 / 256 + 4 / 128) + 2 * 4 * cfg.d_model
+    want = pairs * h + n * cfg.d_model * (3 * 4 + 1 + 8 / 32 + 2 + 48 / 256)
+    assert used <= 1.02 * want + (32 << 20), (used, want)
+    L.close()
