@@ -2,15 +2,15 @@
 // matrix cores (gate/up: gateup.hip).
 //
 // The scales ride in fp16 MFMA operands:
-//   A (weights)      Q4_K: sc_j * q  (0..945)   Q4_0: q - 8   Q8_0: q   (exact;
+//   A (weights)      Q4_K / Q5_K: sc_j * q   Q5_0: q - 16   (exact;
 //                    Q6_K: sc_j * (q - 32), rounded once)
 //   B (activations)  dx * q * 2^-E (or h * 2^-E) in fp16: relative error <= 2^-12, nothing
 //                    downstream re-quantizes
 // What is left on the VALU: the accumulator is kept in units of the current
-// weight scale d of its row (K-quants: per 256-K super-block; Q4_0 / Q5_0 / Q8_0: per
+// weight scale d of its row (K-quants: per 256-K super-block; Q5_0: per
 // 32-block; 1 where d is zero, the weight operand then zeroed) and rescaled
 // by d_prev / d_cur when the period changes; the token's exponent 2^E (one
-// per row) and the last unit are applied once at the end.  The Q4_K min term
+// per row) and the last unit are applied once at the end.  The Q4_K / Q5_K min term
 // -dmin * sum_j m_j * (dx_j * sum q_j) is two bf16 MFMAs on 3-piece
 // splits once per super-block, straight into acc.
 //
@@ -150,38 +150,34 @@ struct WRaw<T_Q6_K> {
     }
 };
 
-template <int TYPE>
-struct WRaw {  // Q4_0 / Q5_0 / Q8_0: 16 bytes per 32-block, row n's fp16 block scales (Q5_0: and fifth bits)
-    static constexpr bool Q5 = TYPE == T_Q5_0;
+template <>
+struct WRaw<T_Q5_0> {  // 16 bytes per 32-block, row n's fp16 block scales and fifth bits
     uint4 q[HB];
     uint32_t d[HB];
-    uint32_t qh[Q5 ? HB : 1];
-    __device__ static uint32_t qoff(const QMat& W, int rt, int n, int g) {
-        return TYPE != T_Q8_0 ? (uint32_t)(((size_t)rt * W.nkb * 32 + n) * 16)
-                              : (uint32_t)((((size_t)rt * W.nkb * 2 + g) * 32 + n) * 16);
+    uint32_t qh[HB];
+    __device__ static uint32_t qoff(const QMat& W, int rt, int n, int) {
+        return (uint32_t)(((size_t)rt * W.nkb * 32 + n) * 16);
     }
     __device__ static uint32_t soff(const QMat& W, int rt, int n) {
         return (uint32_t)(((size_t)rt * W.nkb * 32 + n) * 2);
     }
     __device__ static uint32_t moff(const QMat&, int, int) { return 0; }
     __device__ static uint32_t xoff(const QMat& W, int rt, int n, int) {
-        return Q5 ? (uint32_t)(((size_t)rt * W.nkb * 32 + n) * 4) : 0u;
+        return (uint32_t)(((size_t)rt * W.nkb * 32 + n) * 4);
     }
     template <int PAR>
     __device__ void load(const uint8_t* qb, const uint8_t* sb, const uint8_t*, const uint8_t* xb, uint32_t qo,
                          uint32_t so, uint32_t, uint32_t xo, int h, int nb) {
-        constexpr int QB = TYPE != T_Q8_0 ? 512 : 1024;  // bytes per 32-block of a row tile
 #pragma unroll
         for (int j = 0; j < HB; ++j) {
             if (j < nb) {
-                q[j] = ld16(qb + (size_t)(h * HB + j) * QB + qo);
+                q[j] = ld16(qb + (size_t)(h * HB + j) * 512 + qo);
                 d[j] = *reinterpret_cast<const uint16_t*>(sb + (size_t)(h * HB + j) * 64 + so);
-                if constexpr (Q5) qh[j] = *reinterpret_cast<const uint32_t*>(xb + (size_t)(h * HB + j) * 128 + xo);
+                qh[j] = *reinterpret_cast<const uint32_t*>(xb + (size_t)(h * HB + j) * 128 + xo);
             }
         }
     }
 };
-
 
 template <bool V>
 struct Parity {
@@ -307,7 +303,7 @@ k_wgemm(QMat W0, ActH in, Groups grp, int R, int n_items, int RC, float* y, int 
         xo[i] = WRaw<TYPE>::xoff(W, rt, n, g);
     }
 
-    // Q4_0 / Q5_0 / Q8_0: two accumulator sets, acc for even 32-blocks and acc2 for odd ones, each in its own unit
+    // Q5_0: two accumulator sets, acc for even 32-blocks and acc2 for odd ones, each in its own unit
     constexpr bool DUAL = !SUPER;
     constexpr int TM2 = DUAL ? TM : 1, TN2 = DUAL ? TN : 1;
     v16f acc[TM][TN], acc2[TM2][TN2];
@@ -322,8 +318,8 @@ k_wgemm(QMat W0, ActH in, Groups grp, int R, int n_items, int RC, float* y, int 
 
     WRaw<TYPE> wa[TM], wb[TM];
     uint4 hdr[TM];  // the current super-block's sub-block scales: Q6_K's 16 int8, Q4_K / Q5_K's 8 fp16 s1
-    float dl[TM];   // the unit acc is kept in for the lane's row: the current super-block's (Q4_K) or
-                    // block's (Q4_0 / Q8_0) weight scale d, 1 where d is zero
+    float dl[TM];   // the unit acc is kept in for the lane's row: the current super-block's (K-quants) or
+                    // block's (Q5_0) weight scale d, 1 where d is zero
     float dl2[TM2]; // the unit of acc2
     bool dz[TM];    // Q4_K: this super-block's d is zero (its sc * q terms vanish)
 #pragma unroll
@@ -487,17 +483,12 @@ k_wgemm(QMat W0, ActH in, Groups grp, int R, int n_items, int RC, float* y, int 
             // the block's weight scale d (unit 1 and a zeroed weight operand where d is zero), then the
             // block's MFMAs straight into it. With two sets, one set's rescale does not wait for MFMAs
             // still writing the other, and the MFMAs of one block overlap the rescale of the next.
-            // operand bytes: Q8_0 q + 128, Q4_0 the lane's nibble half in place, Q5_0 its 5-bit quants
-            // (nibble + fifth bit, built in q5w); then fp16 k1 * (1024 + byte) + k0 = the weight
-            const uint32_t mask = TYPE == T_Q4_0 ? (g ? 0xF0F0F0F0u : 0x0F0F0F0Fu) : 0xFFFFFFFFu;
-            const uint32_t flip = TYPE == T_Q8_0 ? 0x80808080u : 0u;
-            const float k1 = TYPE == T_Q4_0 && g ? 0.0625f : 1.0f;
-            const float k0 = TYPE == T_Q8_0 ? -1152.0f : (TYPE == T_Q5_0 ? -1040.0f : (g ? -72.0f : -1032.0f));
+            // operand bytes: the 5-bit quants (nibble + fifth bit, built in q5w), as fp16 (1024 + byte) - 1040
             // Q5_0: elements 16g + 8m + i are nibble half g of qs[8m + i] with fifth bit 16g + 8m + i
             // (dequantize_row_q5_0, src/quant.cpp:1585-1600)
             auto q5w = [&](const WRaw<TYPE>& w, int j, int m, uint32_t& w0, uint32_t& w1) {
                 const uint4 raw = w.q[j];
-                const uint32_t bits = (w.qh[TYPE == T_Q5_0 ? j : 0] >> (8 * (2 * g + m))) & 0xFFu;
+                const uint32_t bits = (w.qh[j] >> (8 * (2 * g + m))) & 0xFFu;
                 w0 = (((m ? raw.z : raw.x) >> (4 * g)) & 0x0F0F0F0Fu) | (spread4(bits) << 4);
                 w1 = (((m ? raw.w : raw.y) >> (4 * g)) & 0x0F0F0F0Fu) | (spread4(bits >> 4) << 4);
             };
@@ -514,23 +505,17 @@ k_wgemm(QMat W0, ActH in, Groups grp, int R, int n_items, int RC, float* y, int 
                     for (int t = 0; t < TN; ++t)
 #pragma unroll
                         for (int r = 0; r < 16; ++r) A[i][t][r] *= ratio;
-                    c1[i] = splat(z ? 0.0f : k1);
-                    c0[i] = splat(z ? 0.0f : k0);
+                    c1[i] = splat(z ? 0.0f : 1.0f);
+                    c0[i] = splat(z ? 0.0f : -1040.0f);
                 }
 #pragma unroll
                 for (int m = 0; m < 2; ++m) {
                     h8 wv[TM], av[TN];
 #pragma unroll
                     for (int i = 0; i < TM; ++i) {
-                        if constexpr (TYPE == T_Q5_0) {
-                            uint32_t w0, w1;
-                            q5w(cur[i], j, m, w0, w1);
-                            wv[i] = cvt8(w0, w1, mask, flip, c1[i], c0[i]);
-                        } else {
-                            const uint4 raw = cur[i].q[j];
-                            wv[i] = m ? cvt8(raw.z, raw.w, mask, flip, c1[i], c0[i])
-                                      : cvt8(raw.x, raw.y, mask, flip, c1[i], c0[i]);
-                        }
+                        uint32_t w0, w1;
+                        q5w(cur[i], j, m, w0, w1);
+                        wv[i] = cvt8(w0, w1, 0xFFFFFFFFu, 0u, c1[i], c0[i]);
                     }
 #pragma unroll
                     for (int t = 0; t < TN; ++t)
