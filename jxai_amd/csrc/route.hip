@@ -896,7 +896,7 @@ constexpr int DP_U = 16;  // 16-byte id loads per lane per round, at most
 
 template <int U>
 __global__ void __launch_bounds__(DISPATCH_THREADS)
-k_dispatch(const int* ids, int nk, int E, int top_k, DispatchOut o, int cold_max) {
+k_dispatch(const int* ids, int nk, int E, int top_k, DispatchOut o) {
     extern __shared__ int hist[];
     __shared__ int red[3][DISPATCH_THREADS / 64];
     __shared__ int wtot[2][DISPATCH_THREADS / 64];
@@ -971,13 +971,12 @@ k_dispatch(const int* ids, int nk, int E, int top_k, DispatchOut o, int cold_max
         }
     }
     __syncthreads();
-    // pair offset, tile offset and active index of expert e: sums over the experts before it (the tile
-    // list holds the experts of at least cold_max pairs only, when cold_max > 0: the others take the GEMVs)
+    // pair offset, tile offset and active index of expert e: sums over the experts before it
     int off = 0, toff = 0, na = 0;
     for (int i = tid; i < e; i += DISPATCH_THREADS) {
         const int c = hist[i];
         off += c;
-        toff += c >= cold_max ? (c + MFMA_BN - 1) / MFMA_BN : 0;
+        toff += (c + MFMA_BN - 1) / MFMA_BN;
         na += c > 0;
     }
 #pragma unroll
@@ -1000,7 +999,7 @@ k_dispatch(const int* ids, int nk, int E, int top_k, DispatchOut o, int cold_max
         na += red[2][w];
     }
     const int cnt = hist[e];
-    const int ntl = cnt >= cold_max ? (cnt + MFMA_BN - 1) / MFMA_BN : 0;  // this expert's tiles
+    const int ntl = (cnt + MFMA_BN - 1) / MFMA_BN;  // this expert's tiles
     if (tid == 0) {
         o.counts[e] = cnt;
         o.offs[e] = off;
@@ -1059,10 +1058,10 @@ k_dispatch(const int* ids, int nk, int E, int top_k, DispatchOut o, int cold_max
     }
 }
 
-void launch_dispatch(const int* ids, int nk, int E, int top_k, const DispatchOut& o, hipStream_t st, int cold_max) {
+void launch_dispatch(const int* ids, int nk, int E, int top_k, const DispatchOut& o, hipStream_t st) {
     // loads per lane and round: the fewest (1, 4 or 16) that take the pairs in one
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(E), dim3(DISPATCH_THREADS), (size_t)E * sizeof(int), st, ids, nk, E, top_k, o, cold_max);
+        hipLaunchKernelGGL(kern, dim3(E), dim3(DISPATCH_THREADS), (size_t)E * sizeof(int), st, ids, nk, E, top_k, o);
     };
     if (nk <= DISPATCH_THREADS * 4) go(k_dispatch<1>);
     else if (nk <= DISPATCH_THREADS * 16) go(k_dispatch<4>);

@@ -389,7 +389,6 @@ struct jx_moe_layer {
     hipStream_t last_st = nullptr;   // stream of the last forward (jx_moe_layer_status waits on it)
     uint32_t dec_epoch = 0;
     int shparts_cap = 1;  // K parts of the shared down's output the workspace holds (ysh)
-    int cold_pairs = 0;   // experts under this many pairs take the GEMVs in the matrix-core regime (0: none)
     bool sh_ksplit = true;  // JX_SH_KSPLIT=0: the standalone shared down in one part (A/B measurement)
     bool fused_decode = true;
     bool force_fused = false;  // JX_FUSED=1: also where the separate launches measured faster
@@ -599,14 +598,6 @@ constexpr int MFMA_MIN_PAIRS_PER_EXPERT_LARGE = 16;
 constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q8 = 1, MFMA_MIN_TOKENS_Q8 = 12;
 constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q8_LARGE = 4;
 constexpr size_t LARGE_EXPERT_ELEMS = (size_t)1 << 25;  // d * d_ff per matrix
-// The cold experts' GEMVs beside the GEMMs (JX_COLD_PAIRS=n: layers of at least HYBRID_MIN_E experts, experts under n
-// pairs; 0, the default: none).  Beside the fp16 GEMMs 16 was the faster setting; the block GEMM multiplies a part
-// of at most 32 pairs as one pair tile, and the GEMV blocks then cost the CUs more than they save.  Qwen3-shaped
-// with Zipf routing, 0 / 16: 64 tokens 107 / 120 us, 200 174 / 172, 600 232 / 231, 2048 393 / 395 (GEMV blocks on
-// the side stream).
-constexpr int HYBRID_MIN_E = 32;
-constexpr int COLD_PAIRS = 0;
-
 // Whether a call takes the fused one-token launch (k_decode1), apart from stream capture: one token in
 // the GEMV regime, Q8_0 activations on both sides, a shared expert (if any) in the routed formats, a
 // shape the kernel is built for, and one where it measured faster (or JX_FUSED=1).
@@ -902,31 +893,9 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
         shared_down(L->side);
         HIPCHK(hipEventRecord(L->ev_join, L->side));
     }
-    // Skewed routing over many experts in the matrix-core regime: the experts with fewer than COLD_PAIRS
-    // pairs take the multi-token GEMVs (weights streamed once per 16 tokens) on the side stream, beside
-    // the GEMMs over the others, instead of a mostly empty GEMM tile each.  The dispatch keeps them out of
-    // the tile table; the GEMV blocks of the others exit at once.
-    const bool hybrid = mfma && mfma_gu && mfma_down && !L->shared && dispatch_later && E >= HYBRID_MIN_E &&
-                        !L->gu_f32 && !L->down_f32 && !(flags & JX_FWD_FORCE_MFMA) &&
-                        jx::mfma_down_ksplit(hK) == 1 && L->cold_pairs > 0;
     if (dispatch_later) {
         Launch l(L, "dispatch", st);
-        jx::launch_dispatch(L->ids, nk, E, k, dout, st, hybrid ? L->cold_pairs : 0);
-    }
-    if (hybrid) {
-        HIPCHK(hipEventRecord(L->ev_fork, st));
-        HIPCHK(hipStreamWaitEvent(L->side, L->ev_fork, 0));
-        jx::Groups cg = grp;
-        cg.cold_max = L->cold_pairs;
-        {
-            Launch l(L, "gateup_gemv_cold", L->side);
-            jx::launch_gemv_gateup(L->gate.m, L->up.m, L->xq, cg, slots, 16, L->hq, nullptr, L->side);
-        }
-        {
-            Launch l(L, "down_gemv_cold", L->side);
-            jx::launch_gemv_down(L->down.m, L->hq, nullptr, 0, cg, slots, 16, L->y, L->side);
-        }
-        HIPCHK(hipEventRecord(L->ev_join, L->side));
+        jx::launch_dispatch(L->ids, nk, E, k, dout, st);
     }
     const float* gxf = L->gu_f32 ? L->xf : nullptr;
     if (mfma_gu) {
@@ -1020,7 +989,6 @@ int run_forward(jx_moe_layer* L, const float* xdev, int n, float* outdev, hipStr
         if (sh_gu && !joined) shared_down(st);  // (the launch took another form)
         if (joined) shparts = spd.kparts;
     }
-    if (hybrid) HIPCHK(hipStreamWaitEvent(st, L->ev_join, 0));
     if (!fold) {
         Launch l(L, "combine", st);
         jx::launch_combine(n, d, k, L->probs, L->pos_of, L->y, L->shared ? L->ysh : nullptr, L->shscale, outdev, st,
@@ -1221,8 +1189,8 @@ int jx_moe_layer_create(const jx_moe_layer_desc* D, jx_moe_layer** out) {
     }
     if ((r = ensure_workspace(L, 1)) != JX_OK) return bail(r);
     if (hipStreamCreate(&L->own) != hipSuccess) return bail(fail(JX_ERR_HIP, "stream create"));
-    // the side stream: the shared expert, or the cold experts' GEMVs beside the GEMMs
-    if ((hipStreamCreate(&L->side) != hipSuccess ||
+    // the side stream: the shared expert beside the routed gate/up
+    if (L->shared && (hipStreamCreate(&L->side) != hipSuccess ||
                       hipEventCreateWithFlags(&L->ev_fork, hipEventDisableTiming) != hipSuccess ||
                       hipEventCreateWithFlags(&L->ev_join, hipEventDisableTiming) != hipSuccess))
         return bail(fail(JX_ERR_HIP, "shared-expert stream create"));
@@ -1238,9 +1206,7 @@ int jx_moe_layer_create(const jx_moe_layer_desc* D, jx_moe_layer** out) {
     if (const char* f = std::getenv("JX_NO_FUSED")) L->fused_decode = std::strcmp(f, "0") == 0;
     if (const char* f = std::getenv("JX_FUSED")) L->force_fused = std::strcmp(f, "0") != 0;
     if (const char* f = std::getenv("JX_DECP")) L->decp_mode = std::strcmp(f, "0") != 0 ? 1 : 0;
-    L->cold_pairs = COLD_PAIRS;
     if (const char* f = std::getenv("JX_SH_KSPLIT")) L->sh_ksplit = std::strcmp(f, "0") != 0;
-    if (const char* f = std::getenv("JX_COLD_PAIRS")) L->cold_pairs = std::max(0, std::atoi(f));
     const bool sh_block = L->shared && block_gemm(L->sgate, L->d, L->sgu_f32) && block_gemm(L->sup, L->d, L->sgu_f32);
     L->smfma_min = !sh_block                                                  ? jx::MFMA_MIN_SHARED_TOKENS_DOWN
                    : L->sgate.m.type == jx::T_Q4_0 && !L->sdown_f32 ? jx::MFMA_MIN_SHARED_TOKENS_Q4_0
