@@ -577,16 +577,15 @@ int resolve_profile(jx_moe_layer* L) {
 // Regime: the matrix-core GEMMs once the average expert sees this many (token, slot) pairs.  The
 // multi-token GEMV (int8 matrix cores, 16 tokens per weight pass) streams an expert's weights once
 // per 16 tokens, the GEMM once per 64-pair tile.  Forced-GEMV against forced-GEMM steps (us):
-//   Q8_0 (Qwen3-shaped): 8 / 12 / 16 / 24 / 32 / 64 tokens (0.5 / 0.75 / 1 / 1.5 / 2 / 4 pairs) 53 / 65 / 71 / 91 / 101 / 167
-//   against 58 / 59 / 62 / 67 / 73 / 107
-//   (with a Q6_K down 12 / 16 / 32 tokens 73 / 75 / 105 against 65 / 66 / 76, with a Q5_0 down 70 / 72 / 90 against 69 / 73 /
-//   83; the routing is skewed there, with uniform routing 16 / 24 / 32 / 48 tokens 101 / 118 / 123 / 142 against 114 /
-//   124 / 129 / 143)
-//   Q4_0: the line follows the gate/up workgroups (E x row groups; few pairs are one part per expert).  In one round of the
-//   chip's 512 (1408 x 2048, 32 experts, 352 workgroups) 6 / 8 / 10 / 12 pairs 88 / 92 / 94 / 130 against 65 / 66 / 66 / 66; in two
-//   (60 experts, 660) 6 / 9 / 10 pairs 106 / 114 / 143 against 124 / 130 / 131; too few for the chip (8 experts, 88)
-//   7 / 12 pairs 43 / 45 against 50 / 50.  With a shared expert of four times their size (Qwen1.5-shaped) 7 / 8.5 / 9.6 pairs
-//   182 / 186 / 210 against 180 / 180 / 200.  A Q6_K or Q5_0 down moves none of these.
+//   Q8_0 (Qwen3-shaped, skewed routing): 8 / 12 / 16 / 24 / 32 / 64 tokens (0.5 / 0.75 / 1 / 1.5 / 2 / 4 pairs) 53 / 65 / 71 /
+//   91 / 101 / 167 against 58 / 59 / 62 / 67 / 73 / 107.  With a Q6_K down 12 / 16 / 32 tokens 73 / 75 / 105 against 65 / 66 /
+//   76, with a Q5_0 down 70 / 72 / 90 against 69 / 73 / 83.  Uniform routing, which the host cannot tell apart: 16 / 24 /
+//   32 / 48 tokens 101 / 118 / 123 / 142 against 114 / 124 / 129 / 143.
+//   Q4_0: the line follows the gate/up workgroups (E x row groups; few pairs are one part per expert).  In one round of
+//   the chip's 512 (1408 x 2048, 32 experts, 352 workgroups) 6 / 8 / 10 / 12 pairs 88 / 92 / 94 / 130 against 65 / 66 / 66 /
+//   66; in two (60 experts, 660) 6 / 9 / 10 pairs 106 / 114 / 143 against 124 / 130 / 131; too few for the chip (8 experts,
+//   88) 7 / 12 pairs 43 / 45 against 50 / 50.  With a shared expert of four times their size (Qwen1.5-shaped) 7 / 8.5 /
+//   9.6 pairs 182 / 186 / 210 against 180 / 180 / 200.  A Q6_K or Q5_0 down moves none of these.
 //   small K-quant experts (DeepSeek-V2-Lite-shaped): 96 / 128 tokens (9 / 12 pairs) 184 / 208 against 192 / 194
 //   large experts (Mixtral-shaped, 14336 x 4096 per matrix, whose GEMV streams near its best rate): 64 / 96 tokens
 //   (16 / 24 pairs) 318 / 405 against 320 / 344
@@ -598,6 +597,7 @@ constexpr int MFMA_MIN_PAIRS_PER_EXPERT_LARGE = 16;
 constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q8 = 1, MFMA_MIN_TOKENS_Q8 = 12;
 constexpr int MFMA_MIN_PAIRS_PER_EXPERT_Q8_LARGE = 4;
 constexpr size_t LARGE_EXPERT_ELEMS = (size_t)1 << 25;  // d * d_ff per matrix
+
 // Whether a call takes the fused one-token launch (k_decode1), apart from stream capture: one token in
 // the GEMV regime, Q8_0 activations on both sides, a shared expert (if any) in the routed formats, a
 // shape the kernel is built for, and one where it measured faster (or JX_FUSED=1).
@@ -1189,10 +1189,13 @@ int jx_moe_layer_create(const jx_moe_layer_desc* D, jx_moe_layer** out) {
     }
     if ((r = ensure_workspace(L, 1)) != JX_OK) return bail(r);
     if (hipStreamCreate(&L->own) != hipSuccess) return bail(fail(JX_ERR_HIP, "stream create"));
-    // the side stream: the shared expert beside the routed gate/up
-    if (L->shared && (hipStreamCreate(&L->side) != hipSuccess ||
-                      hipEventCreateWithFlags(&L->ev_fork, hipEventDisableTiming) != hipSuccess ||
-                      hipEventCreateWithFlags(&L->ev_join, hipEventDisableTiming) != hipSuccess))
+    // The side stream: the shared expert beside the routed gate/up.  Layers without one create it all the same: HIP deals
+    // streams to its few hardware queues in turn, and where layers of one and of two streams mix, a side stream can
+    // come to share the caller's queue, where nothing overlaps (DeepSeek-V2-Lite-shaped 1555 tokens after a layer
+    // without a shared expert 490 -> 504 us).
+    if (hipStreamCreate(&L->side) != hipSuccess ||
+        hipEventCreateWithFlags(&L->ev_fork, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&L->ev_join, hipEventDisableTiming) != hipSuccess)
         return bail(fail(JX_ERR_HIP, "shared-expert stream create"));
     // Graph replays pay where the forward forks the shared expert onto its second stream (the fork and
     // join become graph edges instead of event waits): measured per decode step with the host running
@@ -1264,7 +1267,7 @@ int jx_moe_forward(jx_moe_layer* L, const float* x, int32_t n_tok, float* out, i
     if ((flags & JX_FWD_FORCE_GEMV) && (flags & JX_FWD_FORCE_MFMA))
         return fail(JX_ERR_INVALID, "conflicting regime flags");
     // (token, slot) pairs are int32 indices, and the matrix-core GEMMs address a tile's activation rows
-    // with 32-bit offsets from its first row (n_tok rows of x's hi/lo form: 4 bytes per element)
+    // with 32-bit offsets from its first row (x's forms take 2 bytes per element at most; the bound is fp32 x's 4)
     if ((int64_t)n_tok * L->k > INT_MAX / 2 || (int64_t)n_tok * L->d * 4 >= ((int64_t)1 << 32))
         return fail(JX_ERR_UNSUPPORTED, "n_tok too large for one call (split the batch)");
     HIPCHK(hipSetDevice(L->device));
