@@ -24,8 +24,8 @@ the device-pointer asynchronous path (the one timed) is checked bit for bit
 against the host-pointer path.  Kernel durations for the rooflines come from a
 second pass with HIP events around every launch.  The prefill roofline is the
 fraction of the dense int8 peak (the path's products are int8 x int8 block
-sums; the GEMM forms them exactly on FP6 operands, and the scales' products on fp16
-ones); the rate as a fraction of the fp16 peak is reported beside it.
+sums; the GEMM forms them exactly on FP6 or int8 operands, and the scales' products on fp16
+ones); the rate as a fraction of the fp16 peak and the matrix cores' issued share are reported beside it.
 The reference's CPU path (its own quant.cpp/tier.cpp built in oracle/_ref,
 AVX2 dot order) is timed on a bounded token sample on the host cores.
 """
@@ -136,6 +136,14 @@ def copy_calibration():
         b.copy_(a)
     torch.cuda.synchronize()
     print(f"[bench] copied {nbytes} bytes x3", file=sys.stderr, flush=True)
+
+
+def issued_matrix_frac(cfg, ops, seconds):
+    """Share of the matrix cores' cycles (1024 SIMDs at 2.4 GHz) that the gate/up GEMM's instructions take at their
+    nominal rates, from its algorithmic ops: per 32 x 32 x 32 tile 32 cycles for the block sums, 32 for the scale
+    product and, K-quants, 3 x 32 per 8 blocks for the min term.  Work done for padding is not counted."""
+    cycles = 64 + (12 if cfg.wtype in (F.Q4_K, F.Q5_K) else 0)
+    return ops / (2 * 32 ** 3) * cycles / (1024 * 2.4e9 * seconds)
 
 
 def algorithmic(cfg, n, counts):
@@ -340,7 +348,7 @@ def main():
     traffic, traffic_note = measured_traffic("gateup_mfma", n)
     # the fraction of the int8 peak (the path's arithmetic is int8 x int8 block sums); the rate as a fraction of
     # the fp16 peak is reported beside it
-    pre_roof = {"bound": "mfma", "kernel": "k_bgemm<FP6, gate+up> (matrix-core grouped GEMM on exact block products + SwiGLU)",
+    pre_roof = {"bound": "mfma", "kernel": "k_bgemm<Q4_K, FP6 codes, gate+up> (matrix-core grouped GEMM on exact block products + SwiGLU)",
                 "achieved": gu_rate, "peak": INT8_PEAK_TOPS, "unit": "TFLOP/s",
                 "ops": "algorithmic int8 ops (2 per multiply-accumulate, 2*n*k*2*d*F per launch) per second in "
                        "units of 1e12, against the dense int8 peak of 5.0 POP/s",
@@ -348,6 +356,7 @@ def main():
                 "traffic": traffic, "traffic_note": traffic_note,
                 "avg_launch_us": gu_avg * 1e6,
                 "fp16_peak_frac": gu_rate / FP16_PEAK_TFLOPS,
+                "issued_matrix_frac": issued_matrix_frac(cfg, a_pre["gateup_ops"], gu_avg),
                 "layer_int8_frac": a_pre["ops"] / s_pre / 1e12 / INT8_PEAK_TOPS}
 
     nd = args.decode_tokens

@@ -307,7 +307,8 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
     const uint32_t lb1 = F6 ? (uint32_t)(n * PB + ((8 ^ (n % CPP)) << 4) + 8 * g) : (uint32_t)n * 16;
     const int sh = 4 - 4 * g;  // Q4_0: the lane's nibble to the upper half of its byte
     // this lane's offsets in a load of quants (and fifth bits), of scales
-    const uint32_t lo0 = F6 ? (uint32_t)lane * 12 : (uint32_t)(TYPE == T_Q4_0 ? n : lane) * 16, lo1 = (uint32_t)n * (Rg::QUAD ? 16 : 2);
+    const uint32_t lo0 = F6 ? (uint32_t)lane * 12 : (uint32_t)(TYPE == T_Q4_0 ? n : lane) * 16;
+    const uint32_t lo1 = (uint32_t)n * (Rg::QUAD ? 16 : 2);
     auto load = [&](int h, int j, uint32_t o0, uint32_t o1) {  // j: of the ring
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -403,7 +404,8 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
                 if constexpr (!F6) {
                     if (t == 0) wv[i] = unpack<TYPE>(ring[Rg::PAIR ? j >> 1 : j][i], fifth[odd ? 1 : 0][i], j, odd, sh);
                     if (i == 0) {  // (dx, dx) in the block's place of its pair, as FP6 rows hold it
-                        const int dx = (int)(__builtin_bit_cast(uint16_t, (_Float16)__int_as_float(bd[t])) & gmask) * (KQ ? 0x10001 : 1);
+                        const uint32_t d16 = __builtin_bit_cast(uint16_t, (_Float16)__int_as_float(bd[t])) & gmask;
+                        const int dx = (int)(d16 * (KQ ? 0x10001u : 1u));
                         bp[t] = KQ && (j & 1) ? v2i{0, dx} : v2i{dx, 0};
                     }
                     S[c] = mfma_i8<GATEUP>(wv[i], bi[t]);
@@ -550,7 +552,8 @@ __device__ __forceinline__ float nearest_bf16(float v) { return __uint_as_float(
 
 // The table of a repacked Q4_K / Q5_K matrix (QMat::bt), one thread per (expert, row tile, super-block, row): the 8
 // sub-blocks' d * sc_j as an exact fp16 hi + lo pair, and -dmin * m_j as an exact bf16 hi + lo pair (both products have 17
-// bits: past the 8 of the nearest bf16 an integer of magnitude 2^8 at most is left).  A scale past fp16 sets *over (d above 1000: no model's; such a matrix then has no table).
+// bits: past the 8 of the nearest bf16 an integer of magnitude 2^8 at most is left).  A scale past fp16 sets *over (d above
+// 1000: no model's; such a matrix then has no table).
 __global__ void __launch_bounds__(256) k_block_table(QMat m, uint8_t* out, int* over) {
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (size_t)m.n_mats * m.nrt * m.nkb * 32) return;
@@ -583,7 +586,8 @@ __global__ void __launch_bounds__(256) k_block_table(QMat m, uint8_t* out, int* 
         *reinterpret_cast<uint4*>(o + BT_MIN + c * 512) = make_uint4(pw[c][0], pw[c][1], pw[c][2], pw[c][3]);
 }
 
-// The FP6 codes of a repacked Q4_0 / Q4_K matrix and Q4_0's scales beside them (QMat::g6), one thread per (expert, row tile, 32-block, row).
+// The FP6 codes of a repacked Q4_0 / Q4_K matrix and Q4_0's scales beside them (QMat::g6), one thread per (expert, row
+// tile, 32-block, row).
 __global__ void __launch_bounds__(256) k_g6_codes(QMat m, int KB, uint8_t* out) {
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= (size_t)m.n_mats * m.nrt * KB * 32) return;
@@ -617,7 +621,8 @@ __global__ void __launch_bounds__(256) k_g6_codes(QMat m, int KB, uint8_t* out) 
     }
     uint8_t* o = out + (t / HB) * (size_t)g6_half_unit(m.type);
     if (m.type == T_Q4_0)
-        *reinterpret_cast<uint32_t*>(o + 3072 + row * 16 + (b % HB) * 4) = *reinterpret_cast<const uint16_t*>(m.sc + (t * 32 + row) * 2);
+        *reinterpret_cast<uint32_t*>(o + 3072 + row * 16 + (b % HB) * 4) =
+            *reinterpret_cast<const uint16_t*>(m.sc + (t * 32 + row) * 2);
     uint32_t* oc = reinterpret_cast<uint32_t*>(o + (b % HB) * 768 + row * 12);
 #pragma unroll
     for (int w = 0; w < 3; ++w) {

@@ -907,7 +907,8 @@ k_gemv_down(QMat D, ActQ8 hq, const float* hf, int hf_ld, Groups grp, float* y, 
 // quantized by every block for itself while its first two weight units are in flight.  The Q8_0 of x costs a
 // block 16 KB from L2 (4096 columns) inside the latency of its weights; a launch of its own for it and one
 // per matrix cost four latencies in a row: q / k / v of 4096 columns (Q4_K, 4096 + 2 x 1024 rows)
-// 20.0 -> 9.8 us.
+// 20.0 -> 9.8 us, with 60 such sets in turn (850 MB: weights from HBM) 22 -> 10.9 us.  x must not change under it: the
+// caller hands it a copy where an output shares x's memory.
 struct QkvArgs {
     QMat W[3];     // unused ones: nrt 0
     float* out[3];

@@ -123,3 +123,18 @@ def test_fp16_down_workspace(moe):
     want = pairs * h + n * cfg.d_model * (3 * 4 + 1 + 8 / 32 + 2 + 48 / 256)
     assert used <= 1.02 * want + (32 << 20), (used, want)
     L.close()
+
+
+@pytest.mark.parametrize("name,n", [("qwen3moe", 600), ("dsv2lite_q50", 150), ("toy_q5k", 200)])
+def test_repeats_bit_for_bit(moe, name, n):
+    """The same call gives the same bits, also after calls of other sizes and values on the same workspace."""
+    cfg = synth.CONFIGS[name]
+    L = moe.MoELayer.from_weights(synth.make_layer(cfg))
+    x = synth.make_tokens(cfg, n)
+    print(f"[gpu] repeats {name} n={n}", flush=True)
+    first = L.forward(x)
+    for m, scale in ((n + 70, 1e4), (n - 33, 1e-4), (1, 1.0)):
+        L.forward(synth.make_tokens(cfg, m, seed=m) * np.float32(scale))
+        for a, b in zip(L.forward(x), first):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    L.close()
