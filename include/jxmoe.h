@@ -111,10 +111,10 @@ int jx_moe_init(int32_t device);
  * per-expert residency of LFRUTierManager::get_resident/admit_expert,
  * src/tier.cpp:41-122, and PILOT streaming, src/pilot_io.cpp:182-212: every
  * expert stays resident in HBM).
- * Device memory: the tensors in their own size; Q4_K and Q5_K matrices 0.25 bytes
- * per weight more (a table for prompts); and, while three quarters of the device
- * stay free behind them, 0.75 (Q4_K) or 0.88 (Q4_0) bytes per weight of codes that
- * make prompts 3 to 15% faster with the same results.  Neither fails the call: what
+ * Device memory: the tensors in their own size; Q4_K and Q5_K matrices 0.25 and 0.31
+ * bytes per weight more (a table for prompts); and, while three quarters of the device
+ * stay free behind them, 0.75 (Q4_K, Q5_K) or 0.88 (Q4_0) bytes per weight of codes that
+ * make prompts 3 to 20% faster with the same results.  Neither fails the call: what
  * the device has no room for is left out.  JX_GEMM_CODES=0 in the environment leaves
  * the codes out. */
 int jx_moe_layer_create(const jx_moe_layer_desc* desc, jx_moe_layer** out);

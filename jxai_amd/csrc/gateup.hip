@@ -9,21 +9,22 @@
 //   acc = fma(S, P, acc), 16 per lane
 // so no accumulator is rescaled.  Forms of S, which give the same bits:
 //   from the packed blocks  v_mfma_i32_32x32x32_i8 on the Q8_0 quants as they are and on the weights' quants as bytes,
-//        unpacked in registers (a block's bytes feed both pair tiles): Q4_K and Q5_K q, Q8_0 q, Q4_0 16 (q - 8) (a nibble
+//        unpacked in registers (a block's bytes feed both pair tiles): Q4_K q, Q5_K q - 16, Q8_0 q, Q4_0 16 (q - 8) (a nibble
 //        in the upper half of its byte, the sign bit flipped; the result's 1/16 is exact).  |S| < 2^20: exact as the
 //        fp32 that the fma takes (16 conversions a tile: with them 37 vector instructions, which bound the kernel).
-//   from the FP6 codes  v_mfma_scale_f32_32x32x64_f8f6f4 on a second copy of Q4_0 and Q4_K weights (QMat::g6, 0.88 and 0.75 B
-//        per weight; built where device memory is plentiful).  A: the weight q (Q4_0: q - 8) is one FP6 e2m3 digit (0..15 with
-//        a sign are the codes themselves in units of 1/8).  B: the Q8_0 quant is 16 a + b with |a|, |b| <= 8, two BF6
+//   from the FP6 codes  v_mfma_scale_f32_32x32x64_f8f6f4 on a second copy of Q4_0, Q4_K and Q5_K weights (QMat::g6, 0.75 to 0.88 B
+//        per weight; built where device memory is plentiful).  A: the weight q (Q4_0: q - 8, Q5_K: q - 16) is one FP6 e2m3
+//        digit (0..16 with a sign are the codes themselves in units of 1/8).  B: the Q8_0 quant is 16 a + b with |a|, |b| <= 8, two BF6
 //        e3m2 digits (3 significant bits; 16 a is a shift of the exponent).  A lane half holds 16 elements: its a's, then
 //        its b's, against its weights twice (three register copies per 32 weights instead of loading them in both halves:
 //        Mixtral-shaped 2048 tokens gate/up 1336 -> 1194 us).  No conversion of the result: |S| < 2^17, exact in fp32.
 //        Per step from the blocks and from the codes: Mixtral-shaped 150 / 512 / 2048 tokens 356 / 673 / 2075 and 343 /
-//        656 / 1907 us, Qwen1.5-shaped 200 / 700 / 2048 tokens 211 / 284 / 491 and 203 / 248 / 439 us.
+//        656 / 1907 us (its Q5_K form 437 / 795 / 2385 and 372 / 688 / 1996), Qwen1.5-shaped 200 / 700 / 2048 tokens 211 /
+//        284 / 491 and 203 / 248 / 439 us.
 // P is exact up to one rounding: the fp16 scales themselves (dx; Q4_0 and Q8_0 d), d * sc_j as an exact
 // fp16 hi + lo pair from the table built at upload (QMat::bt).  The Q4_K / Q5_K min term
-// -dmin * sum_j m_j * (dx_j * sum q_j) is three bf16
-// MFMAs on the exact 2- and 3-piece splits of its factors once per super-block, straight into acc.  Only the fp32 rounding of
+// -dmin * sum_j m_j * (dx_j * sum q_j) (Q5_K: plus 16 d sc_j for the offset) is three bf16
+// MFMAs on 2- and 3-piece splits of its factors once per super-block, straight into acc.  Only the fp32 rounding of
 // the accumulation differs from the reference; it matters, because h = SiLU(g) * u is
 // re-quantized to Q8_0 (a relative error of 2^-11 in g and u moves ~1.4% of h's quants by
 // one step, ~2.6e-3 relative in the layer output).
@@ -61,19 +62,19 @@ constexpr int GU_BN = 64;     // pairs per workgroup
 constexpr int GU_WAVES = 4;   // row-tile slots
 
 // One staged half-unit of GU_BN activation rows.
-template <bool F6, bool MIN>
+template <bool F6, int NP>
 struct GuStage {
     static constexpr int PB = F6 ? 256 : 128;  // bytes per row: codes and scales (ActH::q6), or quants
     uint8_t q[GU_BN * PB];                     // row r, chunk c at chunk c ^ (r % (PB / 16))
     float sx[F6 ? 4 : GU_BN * 8];              // [block pair][row][2 blocks](scale, sum)
-    uint16_t xm[MIN ? 3 * GU_BN * 8 : 8];      // [piece][row][8 sub-blocks] bf16 of dx * sum(q)
-    // the waves' min-term weight pieces: gate hi, gate lo, up hi, up lo, each [32 rows][16 B]
-    uint8_t wm[MIN ? GU_WAVES * 2048 : 16];
+    uint16_t xm[NP ? 3 * GU_BN * 8 : 8];       // [piece][row][8 sub-blocks] bf16 of dx * sum(q)
+    // the waves' min-term weight pieces: gate hi, gate mid, up hi, up mid and with three gate lo, up lo, each [32 rows][16 B]
+    uint8_t wm[NP ? GU_WAVES * NP * 1024 : 16];
 };
 
-template <bool F6, bool MIN>
+template <bool F6, int NP>
 struct alignas(16) GuSmem {
-    GuStage<F6, MIN> st[2];
+    GuStage<F6, NP> st[2];
     int src[GU_BN];  // token of each staged pair
 };
 
@@ -140,14 +141,16 @@ struct BgOut {
 // Q4_0: both halves of the block) or two (K-quants: the low and the high nibbles of 16 bytes) at a time.
 template <int TYPE, bool F6>
 struct Ring {
-    static_assert(!F6 || TYPE == T_Q4_0 || TYPE == T_Q4_K, "types with codes");
+    static_assert(!F6 || TYPE == T_Q4_0 || TYPE == T_Q4_K || TYPE == T_Q5_K, "types with codes");
     static constexpr bool KQ = TYPE == T_Q4_K || TYPE == T_Q5_K, PAIR = KQ && !F6;
+    static constexpr bool FIFTH = TYPE == T_Q5_K && !F6;  // the fifth bits beside the nibbles
+    static constexpr int NP = !KQ ? 0 : block_table_pieces(TYPE);
     static constexpr bool QUAD = KQ || F6;  // a half-unit's four scales in one load (else each block's d beside its quants)
     static constexpr int N = PAIR ? HB / 2 : HB;                          // loads of quants per half-unit
     static constexpr int BYTES = F6 ? 768 : TYPE == T_Q4_0 ? 512 : 1024;  // of a row tile per load
     static constexpr int HU = N * BYTES + (F6 && !KQ ? 512 : 0);          // and half-unit (Q4_0 codes: their scales behind)
     // all loads per half-unit of both row tiles: quants, scales, fifth bits
-    static constexpr int LOADS = 2 * (N + (QUAD ? TYPE == T_Q5_K ? 2 : 1 : HB));
+    static constexpr int LOADS = 2 * (N + (QUAD ? FIFTH ? 2 : 1 : HB));
     // The half-unit's DMAs go out after block 2's weights have arrived (PAIR): the compiler's counted waits for the
     // ring do not know of them, and with a ring of two loads a wait for its second one would wait for DMAs just
     // issued (Mixtral-shaped 512 tokens 752 -> 714 us).
@@ -168,10 +171,11 @@ __device__ __forceinline__ v4i unpack(v4i w, v4i fifth, int j, bool odd, int sh)
             r[i] = (int)(((v << sh) & 0xF0F0F0F0u) ^ 0x80808080u);
         } else if constexpr (TYPE != T_Q8_0) {
             uint32_t q = (j & 1 ? v >> 4 : v) & 0x0F0F0F0Fu;
-            if constexpr (TYPE == T_Q5_K) {
+            if constexpr (TYPE == T_Q5_K) {  // q - 16: the nibble, and 0xF0 (15 x 0x10) where the fifth bit is clear
                 const uint32_t f = (uint32_t)fifth[i];  // bit J of a byte: sub-block J
                 const int J = (odd ? 4 : 0) + j;
-                q |= (J >= 4 ? f >> (J - 4) : f << (4 - J)) & 0x10101010u;
+                const uint32_t c = ~(J >= 4 ? f >> (J - 4) : f << (4 - J)) & 0x10101010u;
+                q |= (c << 4) - c;
             }
             r[i] = (int)q;
         }
@@ -199,10 +203,11 @@ __global__ void __launch_bounds__(GU_WAVES * 64) __attribute__((amdgpu_waves_per
 k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut o) {
     using Rg = Ring<TYPE, F6>;
     constexpr bool KQ = Rg::KQ;
-    using St = GuStage<F6, KQ>;
+    constexpr int NP = Rg::NP, BTS = BT_MIN + NP * 512;  // the table's min pieces, bytes per super-block
+    using St = GuStage<F6, NP>;
     constexpr int PB = St::PB, CPP = PB / 16, PPI = 64 / CPP;  // row bytes, chunks, rows per DMA
     constexpr int PER = GU_BN / PPI / GU_WAVES;                // 1 KB DMAs per wave and half-unit
-    __shared__ GuSmem<F6, KQ> sm;
+    __shared__ GuSmem<F6, NP> sm;
     int ti, sub, rg;
     // the grid covers the tile upper bound; the items of the tiles that exist are spread over the XCDs as if
     // the grid were exact, and the rest exit
@@ -260,10 +265,12 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
         const QMat& W = GATEUP && i ? W1 : W0;
         const int rt = GATEUP ? rt0 : min(rt0 + i, W.nrt - 1);
         wb[i] = (F6 ? W.g6 + (size_t)e * W.g6_es : W.qs + (size_t)e * W.qs_es) + (size_t)rt * H * Rg::HU;
-        wsb[i] = KQ ? W.bt + (size_t)e * W.bt_es + (size_t)rt * in.KU * BT_SB
+        wsb[i] = KQ ? W.bt + (size_t)e * W.bt_es + (size_t)rt * in.KU * BTS
                     : W.sc + (size_t)e * W.sc_es + (size_t)rt * KB * 64;
-        wxb[i] = TYPE == T_Q5_K ? W.ex + (size_t)e * W.ex_es + (size_t)rt * in.KU * 1024 : nullptr;
+        wxb[i] = Rg::FIFTH ? W.ex + (size_t)e * W.ex_es + (size_t)rt * in.KU * 1024 : nullptr;
     }
+
+    const uint8_t* wlo = NP == 3 ? (g ? wsb[1] : wsb[0]) + BT_MIN + 1024 + n * 16 : nullptr;
 
     // LDS address of a stage's parts
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)&sm;
@@ -279,11 +286,12 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
             dma16g(dma_base(xsrc + (size_t)h * (HB * 8) + wave * 16), xoff, S + offsetof(St, sx) + wave * (GU_BN * 16));
         if constexpr (KQ) {
             if (h & 1) {  // the super-block's min-term pieces, used at the end of its second half
-                const uint32_t sb = (uint32_t)(h >> 1) * BT_SB;
-                const uint32_t d = S + offsetof(St, wm) + wave * 2048;
+                const uint32_t sb = (uint32_t)(h >> 1) * BTS;
+                const uint32_t d = S + offsetof(St, wm) + wave * (NP * 1024);
                 gbyte *m0 = dma_base(wsb[0] + sb + BT_MIN), *m1 = dma_base(wsb[1] + sb + BT_MIN);
                 dma16g(m0, (uint32_t)lane * 16, d);
                 dma16g(m1, (uint32_t)lane * 16, d + 1024);
+                if constexpr (NP == 3) dma16v(wlo + sb, d + 2048);
                 if (wave > 0)
                     dma16g(dma_base(psrc + (size_t)(h >> 1) * 48 + (wave - 1) * 16), poff,
                            S + offsetof(St, xm) + (wave - 1) * (GU_BN * 16));
@@ -322,9 +330,9 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const size_t sb = (size_t)(uint32_t)(h >> 1);
-                wsc[odd][i] = gload<v4i>(scalar(KQ ? wsb[i] + sb * BT_SB + odd * 512
+                wsc[odd][i] = gload<v4i>(scalar(KQ ? wsb[i] + sb * BTS + odd * 512
                                                    : wb[i] + (size_t)(uint32_t)h * Rg::HU + Rg::N * Rg::BYTES) + o1);
-                if constexpr (TYPE == T_Q5_K) fifth[odd][i] = gload<v4i>(scalar(wxb[i] + sb * 1024) + o0);
+                if constexpr (Rg::FIFTH) fifth[odd][i] = gload<v4i>(scalar(wxb[i] + sb * 1024) + o0);
             }
     };
     // acc of tile (i, t) takes the sums of set c
@@ -434,27 +442,29 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
         fold(1, NT - 1, 1);
         if constexpr (KQ) {
             if (odd) {
-                // acc += sum_j (dx_j sum q_j)(-dmin m_j), the six products of the weight's two pieces and the
-                // activation's three in three MFMAs, (MFMA, lane half) -> (weight piece, activation piece):
-                // (0,0) h.h (0,1) h.m (1,0) l.h (1,1) l.m (2,0) h.l (2,1) l.l
-                const uint8_t* wm = cur.wm + wave * 2048 + n * 16;
+                // acc += sum_j (dx_j sum q_j)(-dmin m_j) in three MFMAs, (MFMA, lane half) -> (weight piece,
+                // activation piece).  Two exact weight pieces (h, m), all products:
+                //   (0,0) h.h (0,1) h.m (1,0) m.h (1,1) m.m (2,0) h.l (2,1) m.l
+                // Three (Q5_K), the six of nine above 2^-24 relative:
+                //   (0,0) h.h (0,1) h.m (1,0) m.h (1,1) h.l (2,0) l.h (2,1) m.m
+                const uint8_t* wm = cur.wm + wave * (NP * 1024) + n * 16;
                 b8 x0[2], x1[2];
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     const uint16_t* xp = cur.xm + (32 * t + n) * 8;
                     x0[t] = *reinterpret_cast<const b8*>(xp + (g ? 1 : 0) * GU_BN * 8);
-                    x1[t] = *reinterpret_cast<const b8*>(xp + 2 * GU_BN * 8);
+                    x1[t] = *reinterpret_cast<const b8*>(xp + (NP == 3 && !g ? 0 : 2) * GU_BN * 8);
                 }
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     const b8 w0 = *reinterpret_cast<const b8*>(wm + i * 1024);
-                    const b8 w1 = *reinterpret_cast<const b8*>(wm + i * 1024 + 512);
-                    const b8 w2 = *reinterpret_cast<const b8*>(wm + i * 1024 + (g ? 512 : 0));
+                    const b8 w1 = *reinterpret_cast<const b8*>(wm + i * 1024 + (NP == 3 && g ? 0 : 512));
+                    const b8 w2 = *reinterpret_cast<const b8*>(wm + (g ? i * 1024 + 512 : NP == 3 ? 2048 + i * 512 : i * 1024));
 #pragma unroll
                     for (int t = 0; t < NT; ++t) {
                         acc[i][t] = mfma_min<GATEUP>(w0, x0[t], acc[i][t]);
-                        acc[i][t] = mfma_min<GATEUP>(w1, x0[t], acc[i][t]);
-                        acc[i][t] = mfma_min<GATEUP>(w2, x1[t], acc[i][t]);
+                        acc[i][t] = mfma_min<GATEUP>(w1, NP == 3 ? x1[t] : x0[t], acc[i][t]);
+                        acc[i][t] = mfma_min<GATEUP>(w2, NP == 3 ? x0[t] : x1[t], acc[i][t]);
                     }
                 }
             }
@@ -551,8 +561,9 @@ k_bgemm(QMat W0, QMat W1, GuIn in, Groups grp, int R, int n_items, int RC, BgOut
 __device__ __forceinline__ float nearest_bf16(float v) { return __uint_as_float((__float_as_uint(v) + 0x8000u) & 0xFFFF0000u); }
 
 // The table of a repacked Q4_K / Q5_K matrix (QMat::bt), one thread per (expert, row tile, super-block, row): the 8
-// sub-blocks' d * sc_j as an exact fp16 hi + lo pair, and -dmin * m_j as an exact bf16 hi + lo pair (both products have 17
-// bits: past the 8 of the nearest bf16 an integer of magnitude 2^8 at most is left).  A scale past fp16 sets *over (d above
+// sub-blocks' d * sc_j as an exact fp16 hi + lo pair, and -dmin * m_j as an exact bf16 pair (both products have 17
+// bits: past the 8 of the nearest bf16 an integer of magnitude 2^8 at most is left); Q5_K, whose quants are taken from
+// q - 16, -dmin * m_j + 16 d * sc_j in three pieces.  A scale past fp16 sets *over (d above
 // 1000: no model's; such a matrix then has no table).
 __global__ void __launch_bounds__(256) k_block_table(QMat m, uint8_t* out, int* over) {
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -561,7 +572,8 @@ __global__ void __launch_bounds__(256) k_block_table(QMat m, uint8_t* out, int* 
     const int row = (int)(idx % 32);
     const uint4 hd = ld16(m.sc + (t * 32 + row) * 16);
     const float d = f16_to_f32(hd.x & 0xFFFFu), dmin = f16_to_f32(hd.x >> 16);
-    uint32_t pw[2][4] = {}, sw[8];
+    uint32_t pw[3][4] = {}, sw[8];
+    const int np = block_table_pieces(m.type);
     bool bad = false;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -572,21 +584,27 @@ __global__ void __launch_bounds__(256) k_block_table(QMat m, uint8_t* out, int* 
         bad |= !(__builtin_fabsf((float)h) < __builtin_inff());
         const _Float16 l = (_Float16)(scale - (float)h);  // exact: scale is a multiple of 2^-24 of 17 bits at most
         sw[j] = (uint32_t)__builtin_bit_cast(uint16_t, h) | (uint32_t)__builtin_bit_cast(uint16_t, l) << 16;
-        const float v = -dmin * (float)mv, vh = nearest_bf16(v), vl = v - vh;
-        pw[0][j / 2] |= (__float_as_uint(vh) >> 16) << (16 * (j & 1));
-        pw[1][j / 2] |= (__float_as_uint(vl) >> 16) << (16 * (j & 1));
+        uint16_t pc[3] = {};
+        if (np == 3) {
+            split3(__builtin_fmaf(16.0f * d, (float)sc, -dmin * (float)mv), pc[0], pc[1], pc[2]);
+        } else {
+            const float v = -dmin * (float)mv, vh = nearest_bf16(v);
+            pc[0] = (uint16_t)(__float_as_uint(vh) >> 16);
+            pc[1] = (uint16_t)(__float_as_uint(v - vh) >> 16);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) pw[c][j / 2] |= (uint32_t)pc[c] << (16 * (j & 1));
     }
     if (bad) atomicOr(over, 1);
-    uint8_t* o = out + t * BT_SB + row * 16;
+    uint8_t* o = out + t * (size_t)(BT_MIN + np * 512) + row * 16;
 #pragma unroll
     for (int c = 0; c < 2; ++c)
         *reinterpret_cast<uint4*>(o + c * 512) = make_uint4(sw[4 * c], sw[4 * c + 1], sw[4 * c + 2], sw[4 * c + 3]);
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int c = 0; c < np; ++c)
         *reinterpret_cast<uint4*>(o + BT_MIN + c * 512) = make_uint4(pw[c][0], pw[c][1], pw[c][2], pw[c][3]);
 }
 
-// The FP6 codes of a repacked Q4_0 / Q4_K matrix and Q4_0's scales beside them (QMat::g6), one thread per (expert, row
+// The FP6 codes of a repacked Q4_0 / Q4_K / Q5_K matrix and Q4_0's scales beside them (QMat::g6), one thread per (expert, row
 // tile, 32-block, row).
 __global__ void __launch_bounds__(256) k_g6_codes(QMat m, int KB, uint8_t* out) {
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -609,6 +627,14 @@ __global__ void __launch_bounds__(256) k_g6_codes(QMat m, int KB, uint8_t* out) 
         const uint32_t w[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
 #pragma unroll
         for (int i = 0; i < 8; ++i) lo[i] = (w[i] >> (j & 1 ? 4 : 0)) & 0x0F0F0F0Fu;
+        if (m.type == T_Q5_K) {
+            off = 16;
+            const uint8_t* ex = m.ex + (er * m.nkb + (b >> 3)) * 1024 + row * 16;
+            const uint4 h0 = ld16(ex), h1 = ld16(ex + 512);
+            const uint32_t hb[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) lo[i] |= ((hb[i] >> j) & 0x01010101u) << 4;
+        }
     }
     uint32_t c[6] = {0, 0, 0, 0, 0, 0};  // two parts of 16 codes
 #pragma unroll
@@ -651,14 +677,18 @@ bool launch_form(const QMat& w0, const QMat& w1, const ActQ8& xq, const ActH& xh
     GuIn in{xh.q6, nullptr, reinterpret_cast<const uint8_t*>(xh.xp), w0.cols, (w0.cols + 255) / 256};
     if (w0.g6 && w1.g6) {
         if (!in.q) return false;
-        if (w0.type == T_Q4_0) {
-            if (few) launch_t<T_Q4_0, true, GATEUP, true>(w0, w1, in, grp, tiles_ub, o, st);
-            else launch_t<T_Q4_0, true, GATEUP, false>(w0, w1, in, grp, tiles_ub, o, st);
-        } else {
-            if (few) launch_t<T_Q4_K, true, GATEUP, true>(w0, w1, in, grp, tiles_ub, o, st);
-            else launch_t<T_Q4_K, true, GATEUP, false>(w0, w1, in, grp, tiles_ub, o, st);
+        auto go = [&](auto type) {
+            constexpr int T = decltype(type)::value;
+            if (few) launch_t<T, true, GATEUP, true>(w0, w1, in, grp, tiles_ub, o, st);
+            else launch_t<T, true, GATEUP, false>(w0, w1, in, grp, tiles_ub, o, st);
+            return true;
+        };
+        switch (w0.type) {
+            case T_Q4_0: return go(std::integral_constant<int, T_Q4_0>{});
+            case T_Q4_K: return go(std::integral_constant<int, T_Q4_K>{});
+            case T_Q5_K: return go(std::integral_constant<int, T_Q5_K>{});
+            default: return false;
         }
-        return true;
     }
     if (!xq.q || !xq.s) return false;
     in.q = reinterpret_cast<const uint8_t*>(xq.q);

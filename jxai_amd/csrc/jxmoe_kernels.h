@@ -55,15 +55,15 @@ struct QMat {
     // fp16 operand scales s1 of the 8 sub-blocks.
     const uint8_t* mn = nullptr;
     size_t mn_es = 0;  // per-expert stride (bytes)
-    // Q4_K / Q5_K table for the block GEMM (launch_block_table): per (expert, row tile, super-block) BT_SB bytes =
-    // 2 half-units x [32 rows][4 sub-blocks] scales d * sc_j as fp16 hi | lo << 16, then at BT_MIN 2 x [32 rows][16 B], the
-    // bf16 pieces (hi, lo) of the 8 sub-blocks' factors -dmin m_j of dx * sum(q).
+    // Q4_K / Q5_K table for the block GEMM (launch_block_table): per (expert, row tile, super-block)
+    // 2 half-units x [32 rows][4 sub-blocks] scales d * sc_j as fp16 hi | lo << 16, then at BT_MIN [32 rows][16 B] for each
+    // of block_table_pieces bf16 pieces of the 8 sub-blocks' factors of dx * sum(q): -dmin m_j (Q5_K: + 16 d sc_j).
     const uint8_t* bt = nullptr;
     size_t bt_es = 0;
-    // Q4_0 / Q4_K, where device memory is plentiful: the quants as FP6 codes for the block GEMM (launch_g6_codes), per
+    // Q4_0 / Q4_K / Q5_K, where device memory is plentiful: the quants as FP6 codes for the block GEMM (launch_g6_codes), per
     // (expert, row tile, half-unit of 128 columns) [4 blocks][2 parts of 16 elements][32 rows][12 B], then for Q4_0
-    // [32 rows][4 blocks] scales d (fp16 in 32 bits).  Code of value v (q - 8 / q): sign << 5 | |v|, element i of a part
-    // at bit 6 i.
+    // [32 rows][4 blocks] scales d (fp16 in 32 bits).  Code of value v (q - 8 / q / q - 16): sign << 5 | |v|, element i
+    // of a part at bit 6 i.
     const uint8_t* g6 = nullptr;
     size_t g6_es = 0;
     // Gated activation applied to this matrix's outputs when it is the gate of
@@ -75,8 +75,9 @@ struct QMat {
     int valid_rows = 0;
 };
 constexpr size_t QMAT_PAD = 8192;
-constexpr int BT_SB = 2048, BT_MIN = 1024;
-constexpr int g6_half_unit(int type) { return type == T_Q4_0 ? 3584 : 3072; }
+constexpr int BT_MIN = 1024;
+__host__ __device__ constexpr int block_table_pieces(int type) { return type == T_Q5_K ? 3 : 2; }
+__host__ __device__ constexpr int g6_half_unit(int type) { return type == T_Q4_0 ? 3584 : 3072; }
 
 // Q8_0 activations on the device: q [rows][K] int8, s [rows][K/32] = (fp16-truncated
 // scale as fp32, sum of the 32 quants as fp32).
@@ -279,10 +280,10 @@ bool launch_mfma_down_block(const QMat& dn, const ActQ8& hq, const ActH& hh, con
                             hipStream_t st, int KS = 1, size_t ystride = 0, bool few = false);
 // `few`: the average expert has fewer than BG_FEW pairs, most of its parts one pair tile.
 constexpr int BG_FEW = 24;
-// Fill m.bt (n_mats * nrt * nkb * BT_SB bytes) from a repacked Q4_K / Q5_K matrix (cols % 256 == 0).  *over is set
+// Fill m.bt (n_mats * nrt * nkb * (BT_MIN + 512 pieces) bytes) from a repacked Q4_K / Q5_K matrix (cols % 256 == 0).  *over is set
 // where a scale passes fp16: the table is then not usable.
 void launch_block_table(const QMat& m, uint8_t* bt, int* over, hipStream_t st);
-// Fill m.g6 (n_mats * nrt * cols / 128 * g6_half_unit bytes) from a repacked Q4_0 / Q4_K matrix (cols % 128 == 0).
+// Fill m.g6 (n_mats * nrt * cols / 128 * g6_half_unit bytes) from a repacked Q4_0 / Q4_K / Q5_K matrix (cols % 128 == 0).
 void launch_g6_codes(const QMat& m, uint8_t* g6, hipStream_t st);
 // The fp16 down GEMM, KS as above.  small: few pairs per expert (the
 // 64-pair tile form at more workgroups per CU).

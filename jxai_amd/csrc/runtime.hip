@@ -140,8 +140,8 @@ enum class Gemm { none, gateup, down };
 // What a matrix-core GEMM reads beside an uploaded matrix, all of it for speed only: where the device has no memory left
 // for a part, the matrix goes without.
 //   Q4_K / Q5_K: the block GEMM's table over Q8_0 activations; otherwise (fp32 h, or a scale past fp16) the fp16 GEMM's
-//   for a down.  0.25 B per weight each; without one the projection takes the GEMVs.
-//   Q4_0 / Q4_K with Q8_0 activations: FP6 codes, 0.88 / 0.75 B per weight.  The block GEMM gives the same bits without
+//   for a down.  0.25 B per weight (the block GEMM's of Q5_K 0.31); without one the projection takes the GEMVs.
+//   Q4_0 / Q4_K / Q5_K with Q8_0 activations: FP6 codes, 0.88 / 0.75 / 0.75 B per weight.  The block GEMM gives the same bits without
 //   them from the blocks themselves (gateup.hip), so they are built only while CODES_FREE of the device stays free
 //   behind them: models of more layers than that keep the memory for their weights and caches.
 constexpr double CODES_FREE = 0.75;
@@ -161,7 +161,7 @@ hipError_t build_gemm_tables(DevMat& out, Gemm gemm, bool q8, bool codes, hipStr
     if (kq && q8) {
         int* over = nullptr;
         int host_over = 0;
-        m.bt_es = (size_t)m.nrt * m.nkb * jx::BT_SB;
+        m.bt_es = (size_t)m.nrt * m.nkb * (jx::BT_MIN + 512 * jx::block_table_pieces(m.type));
         if ((e = alloc(out.bt, m.bt_es * m.n_mats)) != hipSuccess) return e;
         if (out.bt) {
             if ((e = hipMalloc(&over, sizeof(int))) != hipSuccess) return e;
@@ -190,7 +190,7 @@ hipError_t build_gemm_tables(DevMat& out, Gemm gemm, bool q8, bool codes, hipStr
         }
         m.mn = out.mn;
     }
-    if (codes && q8 && m.cols % 128 == 0 && (m.type == jx::T_Q4_0 || (m.type == jx::T_Q4_K && m.bt))) {
+    if (codes && q8 && m.cols % 128 == 0 && (m.type == jx::T_Q4_0 || m.bt)) {
         size_t left = 0, total = 0;
         m.g6_es = (size_t)m.nrt * (m.cols / 128) * jx::g6_half_unit(m.type);
         if ((e = hipMemGetInfo(&left, &total)) != hipSuccess) return e;

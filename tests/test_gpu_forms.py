@@ -33,8 +33,8 @@ def held(moe, lw):
     return (used - (32 << 20)) / (3.0 * lw.cfg.n_experts * lw.cfg.d_model * lw.cfg.d_ff)
 
 
-# bytes per weight of the blocks and (K-quants) the 0.25 of the table; the codes take 0.75 to 0.88 more
-@pytest.mark.parametrize("fmt,least,codes", [(F.Q4_0, 0.5625, 0.875), (F.Q4_K, 0.8125, 0.75), (F.Q5_K, 0.9375, 0.0),
+# bytes per weight of the blocks and (K-quants) the 0.25 or 0.31 of the table; the codes take 0.75 to 0.88 more
+@pytest.mark.parametrize("fmt,least,codes", [(F.Q4_0, 0.5625, 0.875), (F.Q4_K, 0.8125, 0.75), (F.Q5_K, 1.0, 0.75),
                                              (F.Q8_0, 1.0625, 0.0)])
 def test_memory_without_codes(moe, monkeypatch, fmt, least, codes):
     """The second copy of the weights is only built while three quarters of the device stay free behind it."""
@@ -55,7 +55,7 @@ def test_memory_without_codes(moe, monkeypatch, fmt, least, codes):
 # the same edges as the gate/up's: half-units, ragged row tiles, 64-pair parts; 24 pairs per expert and more take
 # the two-tile loop throughout
 @pytest.mark.parametrize("fmt,d,ff", [(F.Q4_0, 128, 32), (F.Q4_0, 384, 416), (F.Q4_0, 640, 384), (F.Q4_K, 256, 256),
-                                      (F.Q4_K, 768, 1280)])
+                                      (F.Q4_K, 768, 1280), (F.Q5_K, 256, 256), (F.Q5_K, 768, 1280)])
 def test_forms_same_bits(moe, monkeypatch, fmt, d, ff):
     """Products from the FP6 codes and from the blocks: the same integer sums, scale products and order."""
     lw = synth.make_layer(synth.LayerConfig(f"forms_{fmt}_{d}_{ff}", d, 3, 2, ff, fmt, d_ff_shared=256))
